@@ -39,28 +39,17 @@ HBM_PEAK_GBS = 8000.0
 # once, and 12 B of binning keys (cell id written and read, index): 256 + 224 + 12 = 492 B.
 STEP_BYTES = 256 + 224 + 12
 # The same 492 B split over the step's kernels, each compulsory byte counted in the first kernel
-# that touches it: the binning passes take the 12 B of keys; predict reads the read-only set and
-# the fields of the leap-frog predictor (h, flags, pos, vel, S, rho, T and their rates: 192 B);
-# the interaction kernel reads the rest of the mutable set (eps_pl, eps_pl_dot, fc, ft, n: 64 B)
-# and writes the whole mutable set (224 B). Everything else a kernel moves (neighbour records,
-# the start state read again by the update, cell tables) is traffic above the algorithmic bytes.
-KERNEL_BYTES = {"binning": 12, "predict": 192, "interact": 64 + 224}
+# that touches it: the binning takes the 12 B of keys; the interaction kernel reads the state and
+# writes the mutable set (480 B). Everything else a kernel moves (neighbour records, cell tables,
+# window candidates read by two work-groups) is traffic above the algorithmic bytes.
+KERNEL_BYTES = {"binning": 12, "interact": 256 + 224}
 assert sum(KERNEL_BYTES.values()) == STEP_BYTES
-# the split variant: the sums kernel reads nothing compulsory beyond what the interaction kernel
-# is credited with; its 288 B are credited to the pair (sums + update)
-# HBM bytes per particle of one launch of the fused interaction kernel on thermal_contact_150k,
-# by precision, pair loop, XCD chunk length and LDS stage limit (0: the full 2048 candidates),
-# measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE passes and scaled by a 512 MiB copy (the
-# commands and tables are in profiles/traffic_thermal_contact_150k.md); a table of measurements,
-# not measured in this run, and reported as `traffic` only for the tuning it was measured with
-MEASURED_TRAFFIC = {("kb_interact", "fp32c", 0, 8, 0): 664, ("kb_interact", "fp32c", 0, 32, 0): 612,
-                    ("kb_interact", "fp32c", 1, 8, 0): 647, ("kb_interact", "fp32c", 1, 32, 0): 599,
-                    ("kb_interact", "fp64", 0, 8, 0): 826, ("kb_interact", "fp64", 0, 32, 0): 743,
-                    ("kb_interact", "fp64", 1, 8, 0): 794, ("kb_interact", "fp64", 1, 32, 0): 691,
-                    ("kb_interact", "fp32c", 0, 8, 1536): 669, ("kb_interact", "fp32c", 0, 32, 1536): 615,
-                    ("kb_interact", "fp32c", 1, 8, 1536): 656, ("kb_interact", "fp32c", 1, 32, 1536): 600,
-                    ("kb_interact", "fp64", 0, 8, 1536): 846, ("kb_interact", "fp64", 0, 32, 1536): 748,
-                    ("kb_interact", "fp64", 1, 8, 1536): 826, ("kb_interact", "fp64", 1, 32, 1536): 695}
+# HBM bytes per particle of one launch of the interaction kernel on thermal_contact_150k, by
+# precision, XCD chunk length and LDS stage limit (0: all candidates), measured with rocprofv3
+# --pmc FETCH_SIZE / WRITE_SIZE passes and scaled by a 512 MiB copy (the commands and tables are in
+# profiles/traffic_thermal_contact_150k.md); a table of measurements, not measured in this run, and
+# reported as `traffic` only for the tuning it was measured with
+MEASURED_TRAFFIC = {}
 MEASURED_TRAFFIC_SOURCE = ("table: rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, thermal_contact_150k, fused interaction, "
                            "profiles/traffic_thermal_contact_150k.md")
 
@@ -355,18 +344,15 @@ def main() -> int:
     head = "fp32c" if "fp32c" in res else "fp64"
     r = res[head]
     N = r["N"]
-    split = r["tuning"]["split_interact"]
-    # the dominant kernel: the fused interaction, or the sums + update pair of the split variant
-    kname = "kb_sums+kb_update" if split else "kb_interact"
+    kname = "kb_interact"
     kbytes = KERNEL_BYTES["interact"]
     # --profile-steps 0 (kernel-trace runs) skips the event-timed phases, and with them the
     # kernel's roofline
-    t_int = (r["phases"]["interact"] + r["phases"]["update"]) * 1e-3 if r["phases"] else None
+    t_int = r["phases"]["interact"] * 1e-3 if r["phases"] else None
     achieved = N * kbytes / t_int / 1e9 if t_int else None
-    tkey = ("kb_interact", head, r["tuning"]["compact_pairs"], r["tuning"].get("xcd_chunk", 8),
-            r["tuning"]["stage_limit"])
+    tkey = ("kb_interact", head, r["tuning"].get("xcd_chunk", 8), r["tuning"]["stage_limit"])
     traffic = None
-    if args.workload == "thermal_contact_150k" and not split and tkey in MEASURED_TRAFFIC:
+    if args.workload == "thermal_contact_150k" and tkey in MEASURED_TRAFFIC:
         traffic = MEASURED_TRAFFIC[tkey] * N
     step_s = r["wall"] / args.steps
     result = {
@@ -383,7 +369,6 @@ def main() -> int:
         "dtype": "f32 (Kahan-compensated neighbour sums) + f64 state" if head == "fp32c" else "f64",
         "data": "synthetic",
         "config": {"workload": args.workload, "n_particles": N, "n_tool": r["info"].n_tool,
-                   "split_interact": split, "compact_pairs": r["tuning"]["compact_pairs"],
                    "num_cell": r["info"].num_cell, "precision": head,
                    "thermal": THERMAL_OF_WORKLOAD.get(args.workload, "see pymfc.workload")},
         "roofline": {"bound": "hbm", "kernel": kname, "achieved": achieved, "peak": HBM_PEAK_GBS,

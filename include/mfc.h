@@ -241,12 +241,11 @@ int mfc_sync(mfc_sim *sim);
 
 /* run nsteps steps without graphs, timing each phase with HIP events on the handle's
  * stream; ms[phase] receives the mean milliseconds per step of: 0 binning (cell offsets and
- * counting sort), 1 gather/predict/EOS/artificial stress, 2 the fused interaction kernel
- * (neighbour sums + per-particle update + contact + the next step's cell ids and counts), or
- * the neighbour-sum kernel when split_interact is set, 3 the update kernel (split_interact
- * only, else 0; it then computes the next step's cell ids), 4 tool-force reduction. Phases 2
- * and 3 are the kernels' own durations (events recorded by their dispatch); the others are
- * measured between events on the stream and include the gaps between launches. */
+ * counting sort), 1 always 0 (the predictor, EOS and artificial stress are part of phase 2),
+ * 2 the interaction kernel (neighbour sums, per-particle update, contact, the next step's cell
+ * ids, counts and neighbour records), 3 always 0, 4 tool-force reduction. Phase 2 is the kernel's
+ * own duration (events recorded by its dispatch); the others are measured between events on the
+ * stream and include the gaps between launches. */
 #define MFC_PROFILE_PHASES 5
 int mfc_profile(mfc_sim *sim, int nsteps, double *ms);
 
@@ -319,22 +318,20 @@ int mfc_vjp_backward(mfc_sim *sim, const double cot[2], double grad[6]);
 int mfc_vjp(mfc_sim *sim, mfc_vjp_req *req, double grad[6]);
 
 /* launch configuration of the step kernels (results do not depend on it: every variant
- * evaluates the same expressions in the same order). split_interact = 0 (default): one fused
- * interaction kernel; 1: a neighbour-sum kernel and a per-particle update kernel with the sums
- * stored in between (fewer registers per kernel, 224 B more traffic per particle).
- * compact_pairs = 1: each lane first marks its in-support neighbours in a bit mask, then runs
- * the pair terms of the marked ones in order; 0 (default): the pair terms run inside the window
- * walk. stage_limit: the most window candidates a tile of 256 particles copies into LDS
- * (0 = MFC_STAGE_CAP); a tile whose candidates span more sorted indices reads them from the
- * records in memory. xcd_chunk: the interaction kernels deal their tiles to the 8 XCDs in chunks
- * of this many consecutive tiles (1..MFC_XCD_CHUNK_MAX; 0 = 8); longer chunks fetch fewer
- * neighbour columns into two L2s, shorter ones balance the XCDs better. The Python package's
- * autotuner (pymfc.autotune) times the combinations on a live handle and keeps the fastest.
- * sort_fast and sort_list bound the counting sort's paths (0 = the defaults; no autotuned
- * setting: they exist so that every path of the sort can be run on any cut): a chunk of cells
- * with at most sort_fast particles (1..MFC_SORT_FAST_MAX) sorts them in registers and LDS, a
- * denser one walks its particle list with a bucket in memory, and a chunk with more than
- * sort_list particles (>= 1) passes over every particle's cell id instead of its list. */
+ * evaluates the same expressions in the same order). lanes: threads per particle of the
+ * interaction, 1, 4 or 8 (0: by the number of particles that are stepped together; more lanes
+ * shorten a particle's chain of operations where the particles alone would not fill the chip).
+ * stage_limit: the most window candidates a patch of cells copies into LDS (0 or anything above
+ * what the kernel has room for: all of them); a patch with more reads them from the records in
+ * memory. xcd_chunk: the interaction deals its patches to the 8 XCDs in chunks of this many
+ * (1..MFC_XCD_CHUNK_MAX; 0 = 8). split_interact and compact_pairs (0 or 1) selected other kernels
+ * of the interaction once; they are accepted and change nothing. The Python package's autotuner
+ * (pymfc.autotune) times the combinations on a live handle and keeps the fastest. sort_fast and
+ * sort_list bound the counting sort's paths (0 = the defaults; no autotuned setting: they exist so
+ * that every path of the sort can be run on any cut): a chunk of cells with at most sort_fast
+ * particles (1..MFC_SORT_FAST_MAX) sorts them in registers and LDS, a denser one walks its
+ * particle list with a bucket in memory, and a chunk with more than sort_list particles (>= 1)
+ * passes over every particle's cell id instead of its list. */
 #define MFC_STAGE_CAP 2048
 #define MFC_XCD_CHUNK_MAX 64
 #define MFC_SORT_FAST_MAX 1536
@@ -345,7 +342,8 @@ typedef struct mfc_tuning {
   int xcd_chunk;
   int sort_fast;
   int sort_list;
-  int reserved[2];
+  int lanes;
+  int reserved[1];
 } mfc_tuning;
 int mfc_set_tuning(mfc_sim *sim, const mfc_tuning *tuning);
 int mfc_get_tuning(const mfc_sim *sim, mfc_tuning *tuning);

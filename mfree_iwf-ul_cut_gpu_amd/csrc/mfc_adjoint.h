@@ -31,7 +31,7 @@ namespace adj {
 MFC_HD double sq(double x) { return x * x; }
 
 // ------------------------------------------------------------------ neighbour record
-// fields of the FP64 neighbour record (16 doubles per particle, written by the predict kernel)
+// fields of the FP64 neighbour record (16 doubles per particle)
 enum { R_X = 0, R_Y, R_FLAGS, R_H, R_U, R_V, R_RHO, R_VOL, R_AXX, R_AXY, R_AYY, R_RXX, R_RXY, R_RYY, R_C, R_T };
 
 // neighbour sums of one particle

@@ -81,6 +81,11 @@ struct adj_args {
   uint64_t *live_state[2];
   uint64_t *live_pos;
   int *live_keys;                   // the handle's sorted cell ids
+  int *chunk_sums[2];               // the handle's chunk sums
+  int nscan;
+  int *pcnt;                        // and patch counts
+  int npatch;
+  int *plen;                        // 2 list lengths
   mfc_tool_state *live_tool;        // 2 replay tool states
   const snapshot *ckpt, *seg;       // checkpoints of the tape, and the start states of a segment
 };
@@ -93,7 +98,8 @@ struct adj_args {
 
 // ------------------------------------------------------------------ checkpoint copies
 // dir 0: a snapshot (ckpt[idx] or seg[idx]) into replay set 0, the positional block, the cell
-// ids and replay tool 0; dir 1: replay set wa, the positional block, the cell ids and replay
+// ids and replay tool 0, and the chunk sums and patch counts cleared for the binning of that
+// state; dir 1: replay set wa, the positional block, the cell ids and replay
 // tool wa into seg[idx]. Grid (copy_blocks, instances).
 __global__ __launch_bounds__(256) void kb_adj_copy(const adj_args *__restrict__ D, int dir, int from_ckpt, int idx,
                                                    int wa) {
@@ -112,9 +118,17 @@ __global__ __launch_bounds__(256) void kb_adj_copy(const adj_args *__restrict__ 
   for (size_t q = i0; q < d.state_words; q += stride) dst_s[q] = src_s[q];
   for (size_t q = i0; q < d.pos_words; q += stride) dst_p[q] = src_p[q];
   for (size_t q = i0; q < (size_t)d.k.N; q += stride) dst_k[q] = src_k[q];
+  if (!dir)
+    for (size_t q = i0; q < (size_t)d.nscan; q += stride) d.chunk_sums[0][q] = d.chunk_sums[1][q] = 0;
+  if (!dir)
+    for (size_t q = i0; q < (size_t)d.npatch; q += stride) d.pcnt[q] = 0;
   if (i0 == 0) {
-    if (dir) *sn.tool = d.live_tool[lw];
-    else d.live_tool[0] = *sn.tool;
+    if (dir) {
+      *sn.tool = d.live_tool[lw];
+    } else {
+      d.live_tool[0] = *sn.tool;
+      d.plen[0] = d.plen[1] = 0;
+    }
   }
 }
 
@@ -125,8 +139,8 @@ __global__ __launch_bounds__(64) void kb_adj_acc_slot(inst_args *__restrict__ re
   const int q = blockIdx.x * 64 + threadIdx.x;
   if (q >= n) return;
   double *a = D[q].acc_seg + (size_t)slot * D[q].acc_stride;
-  rep[q].acc = a; rep[q].acc_out = a;
-  rep[n + q].acc = a; rep[n + q].acc_out = a;
+  rep[q].acc_out = a;
+  rep[n + q].acc_out = a;
 }
 
 // ------------------------------------------------------------------ B1: per-particle tail
@@ -340,7 +354,7 @@ struct adj_work {
   mfc_tool_state *toolw = nullptr;      // 2
   double *partials = nullptr, *force_last = nullptr, *hist = nullptr;
   int64_t *ctr = nullptr;
-  int *pending = nullptr;
+  int *pending = nullptr, *gflag = nullptr;
   int *keys_keep = nullptr;  // the handle's cell ids, kept across the replay of the backward pass
   double *acc_seg = nullptr, *lam_acc = nullptr, *lam_s[2] = {nullptr, nullptr}, *lam_n = nullptr, *g_s = nullptr,
          *g_rec = nullptr, *theta_part = nullptr, *theta_acc = nullptr;
@@ -409,7 +423,8 @@ int setup_work(mfc_sim *s, int nsteps, int K, int w0, int w1) {
     if ((rc = w->alloc(&w->work[0], state_block_bytes(N))) || (rc = w->alloc(&w->work[1], state_block_bytes(N))) ||
         (rc = w->alloc(&w->posw, positional_block_bytes(N))) || (rc = w->alloc(&w->toolw, 2)) ||
         (rc = w->alloc(&w->partials, 16 * (size_t)s->ntiles)) || (rc = w->alloc(&w->force_last, 2)) ||
-        (rc = w->alloc(&w->hist, 2)) || (rc = w->alloc(&w->ctr, 1)) || (rc = w->alloc(&w->pending, 1)) ||
+        (rc = w->alloc(&w->hist, 2)) || (rc = w->alloc(&w->ctr, 1)) || (rc = w->alloc(&w->pending, 2)) ||
+        (rc = w->alloc(&w->gflag, 4 * (size_t)s->ntiles)) ||
         (rc = w->alloc(&w->keys_keep, n)) ||
         (rc = w->alloc(&w->acc_seg, (size_t)K * (L_N + 1) * n)) || (rc = w->alloc(&w->lam_acc, L_N * n)) ||
         (rc = w->alloc(&w->lam_s[0], TS_N * n)) || (rc = w->alloc(&w->lam_s[1], TS_N * n)) ||
@@ -419,7 +434,8 @@ int setup_work(mfc_sim *s, int nsteps, int K, int w0, int w1) {
       return rc;
     // the replay's force reduction keeps no history (cap 0) but counts steps
     HIP_TRY(hipMemsetAsync(w->ctr, 0, sizeof(int64_t), s->stream));
-    HIP_TRY(hipMemsetAsync(w->pending, 0, sizeof(int), s->stream));
+    HIP_TRY(hipMemsetAsync(w->pending, 0, 2 * sizeof(int), s->stream));
+    HIP_TRY(hipMemsetAsync(w->gflag, 0, 4 * sizeof(int) * (size_t)s->ntiles, s->stream));
   }
   w->nsteps = nsteps;
   w->w0 = w0;
@@ -510,15 +526,20 @@ int adj_backward(mfc_sim *const *sims, int n, const batch_work &fw, hipStream_t 
       a.cur = p ? B : A;
       a.nxt = p ? A : B;
       a.b = s->bins;
+      a.b.bsum = s->chunk_sums[p];
+      a.b.bsum_next = s->chunk_sums[1 - p];
+      a.b.plen = s->plen + p;
+      a.b.plen_next = s->plen + 1 - p;
       a.pos = P;
-      a.r = s->recs;
+      a.r = s->recs[p];
+      a.rn = s->recs[1 - p];
       a.tool_in = w->toolw + p;
       a.tool_out = w->toolw + 1 - p;
-      a.f = {w->partials, w->force_last, w->hist, 0, w->ctr, w->pending};  // no history, counted
-      a.acc = a.acc_out = w->acc_seg;  // pointed at each step's slot by kb_adj_acc_slot
+      a.f = {w->partials, w->gflag, w->force_last, w->hist, 0, w->ctr, w->pending + p, w->pending + 1 - p};  // no history, counted
+      a.acc_out = w->acc_seg;  // pointed at each step's slot by kb_adj_acc_slot
       a.ntiles = s->ntiles;
       a.nscan = scan_blocks(s->k.ncell_table);
-      a.bin_next = 0;
+      a.npatch_items = s->npatch_items;
     }
     adj_args &d = da[i];
     std::memset(&d, 0, sizeof(d));
@@ -527,7 +548,7 @@ int adj_backward(mfc_sim *const *sims, int n, const batch_work &fw, hipStream_t 
     d.st = B.px;  // the sorted start state, TS_* order with stride N
     d.flags = B.flags;
     d.pos = P;
-    d.rec = s->recs.rec;
+    d.rec = s->recs[0].rec;  // the reverse steps run from parity 0
     d.key_sorted = s->bins.key_sorted;
     d.offsets = s->bins.offsets;
     d.perm = s->bins.perm;
@@ -550,6 +571,12 @@ int adj_backward(mfc_sim *const *sims, int n, const batch_work &fw, hipStream_t 
     d.live_state[1] = (uint64_t *)w->work[1];
     d.live_pos = (uint64_t *)w->posw;
     d.live_keys = s->bins.key_sorted;
+    d.chunk_sums[0] = s->chunk_sums[0];
+    d.chunk_sums[1] = s->chunk_sums[1];
+    d.nscan = scan_blocks(s->k.ncell_table);
+    d.pcnt = s->bins.pcnt;
+    d.npatch = s->npatch_max;
+    d.plen = s->plen;
     d.live_tool = w->toolw;
     for (int c = 0; c < nck; c++) snaps[(size_t)i * (nck + K) + c] = w->ckpt[c];
     for (int c = 0; c < K; c++) snaps[(size_t)i * (nck + K) + nck + c] = w->seg[c];
@@ -584,14 +611,13 @@ int adj_backward(mfc_sim *const *sims, int n, const batch_work &fw, hipStream_t 
       HIP_TRY(hipMemsetAsync(w->lam_n, 0, sizeof(double) * 2 * N, st));
       HIP_TRY(hipMemsetAsync(w->theta_acc, 0, sizeof(double) * 6, st));
       HIP_TRY(hipMemcpyAsync(w->keys_keep, s->bins.key_sorted, sizeof(int) * N, hipMemcpyDeviceToDevice, st));
-      // every binning of the pass counts into cleared chunk sums and leaves them cleared; the
-      // handle's chunk sums hold the next step's counts: clear them, and bin the handle's state
-      // again at its next step
-      HIP_TRY(hipMemsetAsync(s->bins.bsum, 0, sizeof(int) * (size_t)scan_blocks(s->k.ncell_table), st));
+      // the pass bins its states into the handle's tables and overwrites its records: both are
+      // computed again at the handle's next step
       s->keys_fresh = false;
     }
-    const batch_work rw[2] = {{d_rep, n, fw.tiles, fw.ntiles, fw.chunks, fw.nchunks, false, fw.v, false, false},
-                              {d_rep + n, n, fw.tiles, fw.ntiles, fw.chunks, fw.nchunks, false, fw.v, false, false}};
+    batch_work rw[2] = {fw, fw};
+    rw[0].args = d_rep;
+    rw[1].args = d_rep + n;
     const dim3 gcopy(copy_blocks, n), gt(padded(fw.ntiles)), gpull(padded(fw.ntiles * PULL_LANES));
     const dim3 gslot((n + 63) / 64);
     int cur = 0;  // lam_s[cur] holds the adjoint of the end state of the step being reversed
@@ -601,10 +627,11 @@ int adj_backward(mfc_sim *const *sims, int n, const batch_work &fw, hipStream_t 
       // replay the segment, keeping the start of each of its steps
       int wa = 0;
       hipLaunchKernelGGL(kb_adj_copy, gcopy, dim3(256), 0, st, d_da, 0, 1, sg, 0);
+      launch_batch_hash(rw[0], st);
+      launch_batch_records(rw[0], st);
       for (int t = t0; t < t1; t++) {
         hipLaunchKernelGGL(kb_adj_copy, gcopy, dim3(256), 0, st, d_da, 1, 0, t - t0, wa);
         hipLaunchKernelGGL(kb_adj_acc_slot, gslot, dim3(64), 0, st, d_rep, d_da, n, t - t0);
-        launch_batch_hash(rw[wa], st);
         launch_batch_step(rw[wa], st);  // the interaction keeps its sums in the step's slot
         wa = 1 - wa;
       }

@@ -70,10 +70,111 @@ void enqueue_step(mfc_sim *s, int c) { mfc::launch_batch_step(s->work(c), s->str
 
 int ensure_keys(mfc_sim *s) {
   if (s->keys_fresh) return MFC_OK;
-  HIP_TRY(hipMemsetAsync(s->bins.bsum, 0, sizeof(int) * (size_t)mfc::scan_blocks(s->k.ncell_table), s->stream));
+  HIP_TRY(hipMemsetAsync(s->chunk_sums[s->cur], 0, sizeof(int) * (size_t)mfc::scan_blocks(s->k.ncell_table), s->stream));
+  HIP_TRY(hipMemsetAsync(s->bins.pcnt, 0, sizeof(int) * (size_t)s->npatch_max, s->stream));
+  HIP_TRY(hipMemsetAsync(s->plen, 0, 2 * sizeof(int), s->stream));
   mfc::launch_batch_hash(s->work(s->cur), s->stream);
+  mfc::launch_batch_records(s->work(s->cur), s->stream);
   s->keys_fresh = true;
   return MFC_OK;
+}
+
+void sort_items(std::vector<int2> &items, mfc_sim *const *sims, int n) {
+  const int groups_per_tile = mfc::TILE / 64;
+  for (int i = 0; i < n; i++) {
+    for (int q = 0; q * mfc::PLIST_SECTION < sims[i]->npatch_max; q++) items.push_back(make_int2(i, mfc::SORT_ITEM_PATCHES - q));
+    items.push_back(make_int2(i, mfc::SORT_ITEM_TOOL));
+    const int blocks = (groups_per_tile * sims[i]->ntiles + mfc::FORCE_GROUPS - 1) / mfc::FORCE_GROUPS;
+    for (int q = 0; q < blocks; q++) items.push_back(make_int2(i, mfc::SORT_ITEM_FORCE - q));
+  }
+  for (int i = 0; i < n; i++)
+    for (int q = 0; q < mfc::scan_blocks(sims[i]->k.ncell_table); q++) items.push_back(make_int2(i, q));
+}
+
+void patch_items(std::vector<int2> &items, mfc_sim *const *sims, int n) {
+  for (int i = 0; i < n; i++) items.push_back(make_int2(i, mfc::PATCH_ITEM_FORCE));
+  for (int i = 0; i < n; i++)
+    for (int q = 0; q < sims[i]->npatch_items; q++) items.push_back(make_int2(i, q));
+}
+
+// Measured, us per step with 1 / 4 / 8 threads per particle (FP64; FP32C): 6k 48 / 34 / 32
+// (39 / 30 / 29), 7.6k 50 / 34 / 30 (38 / 29 / 27), 27k 55 / 50 / 62 (43 / 38 / 43), 37k 62 / 53 / 62
+// (51 / 45 / 51), 71k 67 / 80 / 107 (47 / 60 / 72): more threads pay as long as they find idle SIMDs
+int interaction_lanes(int64_t total) {
+  return total > 48000 ? 1 : total > 13000 ? 4 : 8;
+}
+
+namespace {
+
+// rows and columns of the patches for `lanes` threads per particle: the largest near-square
+// rectangle of cells that a full lattice (cells of h = hdx dx: hdx^2 particles each) fills with at
+// most TILE / lanes particles, a lattice line more than the whole ones on each side included, and
+// whose windows fit the LDS stage
+void patch_shape(double hdx, bool f32, int lanes, int &s, int &w) {
+  const int most = mfc::TILE / lanes, cap = mfc::patch_cap(f32, lanes);
+  auto lines = [&](int cells, double more) { return (int)(cells * hdx + more); };
+  auto fits = [&](int a, int b) {
+    const double more = lanes == 1 ? 1. : 0.5;
+    return lines(a, more) * lines(b, more) <= most && lines(a + 4, 1.) * lines(b + 4, 1.) <= cap && b + 4 <= mfc::PATCH_COLS &&
+           (b + 4) * (a + 5) <= mfc::PATCH_TABLE;
+  };
+  s = w = 1;
+  for (;;) {
+    if (s >= w && fits(s, w + 1)) w++;
+    else if (fits(s + 1, w)) s++;
+    else if (fits(s, w + 1)) w++;
+    else break;
+  }
+}
+
+int64_t patch_bound(const mfc::dev_consts &k, int s, int w) {
+  if (!k.adaptive) return (int64_t)((k.gnx + w - 1) / w) * ((k.gny + s - 1) / s);
+  // any nx by ny cells with nx ny < ncell_table: (nx / w + 1) (ny / s + 1)
+  const int64_t t = k.ncell_table;
+  return t / ((int64_t)s * w) + t / (s < w ? s : w) + 2;
+}
+
+}  // namespace
+
+void set_patches(mfc_sim *s, int lanes) {
+  int a, b;
+  patch_shape(s->cfg.hdx, s->recs[0].f32, lanes, a, b);
+  s->lanes = lanes;
+  s->k.patch_s = a;
+  s->k.patch_w = b;
+  s->k.patch_slots = mfc::TILE / lanes;
+  // the entries of the initial particles' patches and half as many again: the particles spread
+  // over more patches as the run goes on. A work item past the list's end leaves at once, and
+  // entries past the work items' are taken by the slower path
+  const mfc::dev_consts &k = s->k;
+  const int rows = (k.gny + a - 1) / a, cols = (k.gnx + b - 1) / b;
+  std::vector<int> in((size_t)rows * cols, 0);
+  for (int i = 0; i < k.N; i++) {
+    const int gx = (int)((s->sc.px[i] - k.bbmin_x) / k.cell), gy = (int)((s->sc.py[i] - k.bbmin_y) / k.cell);
+    const int cx = gx < 0 ? 0 : gx < k.gnx ? gx : k.gnx - 1, cy = gy < 0 ? 0 : gy < k.gny ? gy : k.gny - 1;
+    in[(size_t)(cx / b) * rows + cy / a]++;
+  }
+  int64_t entries = 0;
+  for (int n : in) entries += (n + k.patch_slots - 1) / k.patch_slots;
+  const int64_t bound = patch_bound(k, a, b) + k.N / k.patch_slots, want = entries + entries / 2 + 32;
+  s->npatch_items = (int)(want < bound ? want : bound);
+  if (s->npatch_items > s->npatch_items_max) s->npatch_items_max = s->npatch_items;
+}
+
+int upload_descriptors(mfc_sim *s) {
+  HIP_TRY(hipStreamSynchronize(s->stream));
+  for (int c = 0; c < 2; c++) {
+    const mfc::inst_args a = instance_args(s, c);
+    HIP_TRY(hipMemcpy(s->slot[c], &a, sizeof(a), hipMemcpyHostToDevice));
+  }
+  return MFC_OK;
+}
+
+void check_uniform_h(mfc_sim *s, const double *h) {
+  bool same = h[0] == h[0];
+  for (int i = 1; i < s->k.N && same; i++) same = h[i] == h[0];
+  s->k.uniform_h = same;
+  s->k.h0 = h[0];
 }
 
 static_assert(mfc::XCD_CHUNK_MAX == MFC_XCD_CHUNK_MAX, "XCD chunk bound of the header and the kernels");
@@ -87,11 +188,13 @@ int check_tuning(const mfc_tuning *t) {
     return fail(MFC_E_INVALID, "xcd_chunk must be in 0.." + std::to_string(mfc::XCD_CHUNK_MAX));
   if (t->sort_fast < 0 || t->sort_fast > MFC_SORT_FAST_MAX)
     return fail(MFC_E_INVALID, "sort_fast must be in 0.." + std::to_string(MFC_SORT_FAST_MAX));
+  if (t->lanes != 0 && t->lanes != 1 && t->lanes != 4 && t->lanes != 8)
+    return fail(MFC_E_INVALID, "lanes must be 0, 1, 4 or 8");
   if (t->sort_list < 0) return fail(MFC_E_INVALID, "sort_list must be >= 0");
   return MFC_OK;
 }
 
-// each step's tool force is reduced by the next step's first kernel; this reduces the last one
+// each step's tool force is reduced by the next step's sort launch; this reduces the last one
 void finish_steps(mfc_sim *s) { mfc::launch_batch_force(s->work(s->cur), s->stream); }
 
 mfc::inst_args instance_args(const mfc_sim *s, int c) {
@@ -101,16 +204,20 @@ mfc::inst_args instance_args(const mfc_sim *s, int c) {
   a.cur = s->set[c];
   a.nxt = s->set[1 - c];
   a.b = s->bins;
+  a.b.bsum = s->chunk_sums[c];
+  a.b.bsum_next = s->chunk_sums[1 - c];
+  a.b.plen = s->plen + c;
+  a.b.plen_next = s->plen + 1 - c;
   a.pos = s->pos;
-  a.r = s->recs;
+  a.r = s->recs[c];
+  a.rn = s->recs[1 - c];
   a.tool_in = s->tool + c;
   a.tool_out = s->tool + (1 - c);
-  a.f = s->force();
-  a.acc = s->acc;
+  a.f = s->force(c);
   a.geo = s->geo;
   a.ntiles = s->ntiles;
   a.nscan = mfc::scan_blocks(s->k.ncell_table);
-  a.bin_next = 1;
+  a.npatch_items = s->npatch_items;
   return a;
 }
 
@@ -213,7 +320,7 @@ int mfc_create(const mfc_config *cfg, mfc_sim **out) {
   const int N = c.N;
   s->ntiles = (N + mfc::TILE - 1) / mfc::TILE;
   s->precision = cfg->precision;
-  s->recs.f32 = cfg->precision == MFC_PREC_FP32C;
+  s->recs[0].f32 = s->recs[1].f32 = cfg->precision == MFC_PREC_FP32C;
 
   auto bail = [&](int code) { mfc_destroy(s); return code; };
   if (hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) != hipSuccess) return bail(fail(MFC_E_HIP, "stream"));
@@ -224,7 +331,8 @@ int mfc_create(const mfc_config *cfg, mfc_sim **out) {
   if ((rc = s->alloc(&b.key, N)) || (rc = s->alloc(&b.key_sorted, N)) ||
       (rc = s->alloc(&b.offsets, (size_t)c.ncell_table + 1)) ||
       (rc = s->alloc(&b.bucket, N)) || (rc = s->alloc(&b.perm, N)) || (rc = s->alloc(&b.spos, N)) ||
-      (rc = s->alloc(&b.bsum, (mfc::scan_blocks(c.ncell_table) + 3) & ~3)) || (rc = s->alloc(&b.clamped, 1)) ||
+      (rc = s->alloc(&s->chunk_sums[0], (mfc::scan_blocks(c.ncell_table) + 3) & ~3)) ||
+      (rc = s->alloc(&s->chunk_sums[1], (mfc::scan_blocks(c.ncell_table) + 3) & ~3)) || (rc = s->alloc(&b.clamped, 1)) ||
       (rc = s->alloc(&b.clist, (size_t)mfc::scan_blocks(c.ncell_table) * mfc::chunk_list_cap(N))) ||
       (rc = s->alloc(&s->geo, 1)) || (c.rothlin && (rc = s->alloc(&b.offsets_r, (size_t)c.ncell_table + 1))))
     return bail(rc);
@@ -234,17 +342,30 @@ int mfc_create(const mfc_config *cfg, mfc_sim **out) {
     if ((rc = s->alloc(&pb, positional_block_bytes(N)))) return bail(rc);
     carve_positional(pb, N, p);
   }
-  if ((rc = s->alloc(&s->recs.posd, N)) || (rc = s->alloc(&s->recs.vfl, N))) return bail(rc);
-  if (s->recs.f32) {
-    if ((rc = s->alloc(&s->recs.rec32, (size_t)16 * N))) return bail(rc);
-  } else if ((rc = s->alloc(&s->recs.rec, (size_t)mfc::REC * N))) {
+  for (int lanes : {1, 4, 8}) {
+    int a, w;
+    patch_shape(cfg->hdx, s->recs[0].f32, lanes, a, w);
+    const int64_t n = patch_bound(k, a, w);
+    if (n > s->npatch_max) s->npatch_max = (int)n;
+  }
+  if ((rc = s->alloc(&b.pcnt, s->npatch_max)) ||
+      (rc = s->alloc(&b.plist, (size_t)s->npatch_max + (size_t)N / (mfc::TILE / 8) + 1)) || (rc = s->alloc(&s->plen, 2)))
     return bail(rc);
+  for (int lanes : {1, 4, 8}) set_patches(s, lanes);  // the largest work table
+  set_patches(s, interaction_lanes(N));
+  check_uniform_h(s, s->sc.h.data());
+  for (mfc::drecords &r : s->recs) {
+    if ((rc = s->alloc(&r.vfl, N))) return bail(rc);
+    if (r.f32) {
+      if ((rc = s->alloc(&r.rec32, (size_t)mfc::REC32_PIECES * N))) return bail(rc);
+    } else if ((rc = s->alloc(&r.rec, (size_t)mfc::REC * N))) {
+      return bail(rc);
+    }
   }
   if ((rc = s->alloc(&s->tool, 2)) ||
       (rc = s->alloc(&s->partials, (size_t)16 * s->ntiles)) || (rc = s->alloc(&s->force_last, 2)) ||
       (rc = s->alloc(&s->hist, (size_t)2 * HIST_CAP)) || (rc = s->alloc(&s->hist_ctr, 1)) ||
-      (rc = s->alloc(&s->force_pending, 1)) ||
-      (rc = s->alloc(&s->acc, (size_t)mfc::ACC_N * N)))
+      (rc = s->alloc(&s->force_pending, 2)) || (rc = s->alloc(&s->force_groups, (size_t)4 * s->ntiles)))
     return bail(rc);
   // zero everything, then upload the initial state (particle_gpu.cu:20-125)
   {
@@ -280,32 +401,34 @@ int mfc_create(const mfc_config *cfg, mfc_sim **out) {
         (b.offsets_r && hipMemsetAsync(b.offsets_r, 0, sizeof(int) * ((size_t)c.ncell_table + 1), s->stream) != hipSuccess) ||
         hipMemsetAsync(b.clamped, 0, sizeof(unsigned long long), s->stream) != hipSuccess ||
         hipMemsetAsync(s->hist_ctr, 0, sizeof(int64_t), s->stream) != hipSuccess ||
-        hipMemsetAsync(s->force_pending, 0, sizeof(int), s->stream) != hipSuccess ||
-        hipMemsetAsync(b.bsum, 0, sizeof(int) * (size_t)mfc::scan_blocks(c.ncell_table), s->stream) != hipSuccess ||
-        hipMemsetAsync(s->force_last, 0, 2 * sizeof(double), s->stream) != hipSuccess ||
-        (s->recs.rec && hipMemsetAsync(s->recs.rec, 0, sizeof(double) * mfc::REC * (size_t)N, s->stream) != hipSuccess) ||
-        hipMemsetAsync(s->recs.posd, 0, sizeof(double2) * (size_t)N, s->stream) != hipSuccess ||
-        hipMemsetAsync(s->recs.vfl, 0, sizeof(int) * (size_t)N, s->stream) != hipSuccess ||
-        (s->recs.rec32 && hipMemsetAsync(s->recs.rec32, 0, sizeof(float) * 16 * (size_t)N, s->stream) != hipSuccess))
+        hipMemsetAsync(s->force_pending, 0, 2 * sizeof(int), s->stream) != hipSuccess ||
+        hipMemsetAsync(s->force_groups, 0, sizeof(int) * 4 * (size_t)s->ntiles, s->stream) != hipSuccess ||
+        hipMemsetAsync(s->chunk_sums[0], 0, sizeof(int) * (size_t)mfc::scan_blocks(c.ncell_table), s->stream) != hipSuccess ||
+        hipMemsetAsync(s->chunk_sums[1], 0, sizeof(int) * (size_t)mfc::scan_blocks(c.ncell_table), s->stream) != hipSuccess ||
+        hipMemsetAsync(s->force_last, 0, 2 * sizeof(double), s->stream) != hipSuccess)
       return bail(fail(MFC_E_HIP, "memset"));
     mfc_tool_state t2[2] = {S.tool, S.tool};
     if (up(s->tool, t2, sizeof(t2)) != hipSuccess) return bail(fail(MFC_E_HIP, "upload tool"));
     const mfc::grid_geo g0 = {c.bbmin_x, c.bbmin_y, c.cell, c.gnx, c.gny, c.num_cell, 0};
     if (up(s->geo, &g0, sizeof(g0)) != hipSuccess) return bail(fail(MFC_E_HIP, "upload grid"));
     // descriptors and work tables of the step kernels (a batch of one)
-    const int nscan = mfc::scan_blocks(c.ncell_table);
-    std::vector<int2> tiles(s->ntiles), chunks(nscan);
+    std::vector<int2> tiles(s->ntiles), chunks, patches;
     for (int t = 0; t < s->ntiles; t++) tiles[t] = make_int2(0, t);
-    for (int q = 0; q < nscan; q++) chunks[q] = make_int2(0, q);
-    s->nchunks = nscan;
+    sort_items(chunks, &s, 1);
+    patch_items(patches, &s, 1);
+    s->nchunks = (int)chunks.size();
+    s->npatches = (int)patches.size();
     mfc::inst_args a2[2] = {instance_args(s, 0), instance_args(s, 1)};
     if ((rc = s->alloc(&s->dargs, 2)) || (rc = s->alloc(&s->dtiles, (size_t)s->ntiles)) ||
-        (rc = s->alloc(&s->dchunks, (size_t)nscan)))
+        (rc = s->alloc(&s->dchunks, chunks.size())) || (rc = s->alloc(&s->dpatches, 1 + (size_t)s->npatch_items_max)))
       return bail(rc);
     if (up(s->dargs, a2, sizeof(a2)) != hipSuccess ||
         up(s->dtiles, tiles.data(), sizeof(int2) * tiles.size()) != hipSuccess ||
-        up(s->dchunks, chunks.data(), sizeof(int2) * chunks.size()) != hipSuccess)
+        up(s->dchunks, chunks.data(), sizeof(int2) * chunks.size()) != hipSuccess ||
+        up(s->dpatches, patches.data(), sizeof(int2) * patches.size()) != hipSuccess)
       return bail(fail(MFC_E_HIP, "upload of the step tables"));
+    s->slot[0] = s->dargs;
+    s->slot[1] = s->dargs + 1;
     if (hipStreamSynchronize(s->stream) != hipSuccess) return bail(fail(MFC_E_HIP, "sync"));
   }
   *out = s;
@@ -322,8 +445,16 @@ int mfc_set_tuning(mfc_sim *s, const mfc_tuning *t) {
   s->k.stage_limit = t->stage_limit;
   s->k.sort_fast = t->sort_fast;
   s->k.sort_list = t->sort_list;
-  mfc::inst_args a2[2] = {instance_args(s, 0), instance_args(s, 1)};
-  HIP_TRY(hipMemcpy(s->dargs, a2, sizeof(a2), hipMemcpyHostToDevice));
+  const int lanes = t->lanes ? t->lanes : interaction_lanes(s->k.N);
+  if (lanes != s->lanes) {
+    std::vector<int2> patches;
+    set_patches(s, lanes);
+    patch_items(patches, &s, 1);
+    HIP_TRY(hipMemcpy(s->dpatches, patches.data(), sizeof(int2) * patches.size(), hipMemcpyHostToDevice));
+    s->npatches = (int)patches.size();
+    s->keys_fresh = false;  // the patches' counts are those of the old shape
+  }
+  if ((rc = upload_descriptors(s))) return rc;
   for (int p = 0; p < 2; p++)
     if (s->graph[p]) {
       (void)hipGraphExecDestroy(s->graph[p]);
@@ -366,11 +497,11 @@ int mfc_step(mfc_sim *s, int nsteps) {
 int mfc_profile(mfc_sim *s, int nsteps, double *ms) {
   if (!s || !ms || nsteps < 1) return fail(MFC_E_INVALID, "bad argument");
   if (s->batched) return fail(MFC_E_INVALID, "instance of a batch: step it with mfc_batch_step");
-  // ev: the phase boundaries on the stream; kt: the interaction kernels' own start and end
-  constexpr int NE = MFC_PROFILE_PHASES + 1;
-  hipEvent_t ev[NE], kt[4];
+  // ev: the phase boundaries on the stream; kt: the interaction kernel's own start and end
+  constexpr int NE = 4, NK = 2;
+  hipEvent_t ev[NE], kt[NK];
   for (int q = 0; q < NE; q++) HIP_TRY(hipEventCreate(&ev[q]));
-  for (int q = 0; q < 4; q++) HIP_TRY(hipEventCreate(&kt[q]));
+  for (int q = 0; q < NK; q++) HIP_TRY(hipEventCreate(&kt[q]));
   double acc[MFC_PROFILE_PHASES] = {0., 0., 0., 0., 0.};
   int rc = ensure_keys(s);
   for (int it = 0; it < nsteps && rc == MFC_OK; it++) {
@@ -379,35 +510,24 @@ int mfc_profile(mfc_sim *s, int nsteps, double *ms) {
     (void)hipEventRecord(ev[0], s->stream);
     mfc::launch_batch_binning(w, s->stream);
     (void)hipEventRecord(ev[1], s->stream);
-    mfc::launch_batch_predict(w, s->stream);
+    mfc::launch_batch_interact(w, s->stream, kt[0], kt[1]);
     (void)hipEventRecord(ev[2], s->stream);
-    if (w.v.split) {
-      mfc::launch_batch_sums(w, s->stream, kt[0], kt[1]);
-      (void)hipEventRecord(ev[3], s->stream);
-      mfc::launch_batch_update(w, s->stream, kt[2], kt[3]);
-    } else {
-      mfc::launch_batch_interact_fused(w, s->stream, kt[0], kt[1]);
-      (void)hipEventRecord(ev[3], s->stream);
-    }
-    (void)hipEventRecord(ev[4], s->stream);
-    mfc::launch_batch_force(w, s->stream);
-    (void)hipEventRecord(ev[5], s->stream);
+    mfc::launch_batch_force(s->work(n), s->stream);
+    (void)hipEventRecord(ev[3], s->stream);
     s->cur = n;
     s->step++;
     if (hipEventSynchronize(ev[NE - 1]) != hipSuccess) { rc = fail(MFC_E_HIP, "event sync"); break; }
     float t[MFC_PROFILE_PHASES] = {0.f, 0.f, 0.f, 0.f, 0.f};
     if (hipEventElapsedTime(&t[0], ev[0], ev[1]) != hipSuccess ||
-        hipEventElapsedTime(&t[1], ev[1], ev[2]) != hipSuccess ||
         hipEventElapsedTime(&t[2], kt[0], kt[1]) != hipSuccess ||
-        (w.v.split && hipEventElapsedTime(&t[3], kt[2], kt[3]) != hipSuccess) ||
-        hipEventElapsedTime(&t[4], ev[4], ev[5]) != hipSuccess) {
+        hipEventElapsedTime(&t[4], ev[2], ev[3]) != hipSuccess) {
       rc = fail(MFC_E_HIP, "event time");
       break;
     }
     for (int q = 0; q < MFC_PROFILE_PHASES; q++) acc[q] += t[q];
   }
   for (int q = 0; q < NE; q++) (void)hipEventDestroy(ev[q]);
-  for (int q = 0; q < 4; q++) (void)hipEventDestroy(kt[q]);
+  for (int q = 0; q < NK; q++) (void)hipEventDestroy(kt[q]);
   if (rc) return rc;
   for (int q = 0; q < MFC_PROFILE_PHASES; q++) ms[q] = acc[q] / nsteps;
   return MFC_OK;
@@ -546,7 +666,11 @@ int mfc_set_field(mfc_sim *s, int field, const void *host, size_t bytes) {
   const size_t es = field_is_int(field) ? sizeof(int) : sizeof(double);
   if (bytes != (size_t)N * nc * es) return fail(MFC_E_RANGE, "buffer size does not match the field");
   HIP_TRY(hipStreamSynchronize(s->stream));
-  s->keys_fresh = false;  // positions and flags decide the binning
+  s->keys_fresh = false;  // positions and flags decide the binning, the other fields enter the records
+  if (field == MFC_FIELD_H) {
+    check_uniform_h(s, (const double *)host);
+    if ((rc = upload_descriptors(s))) return rc;
+  }
   if (nc == 1) {
     HIP_TRY(hipMemcpy(ptr[0], host, es * N, hipMemcpyHostToDevice));
     return MFC_OK;

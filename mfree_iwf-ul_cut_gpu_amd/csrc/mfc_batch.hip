@@ -17,20 +17,26 @@ struct mfc_batch {
   std::vector<mfc_sim *> sims;
   hipStream_t stream = nullptr;
   bool f32 = false;
-  mfc_tuning tuning = {0, 0, 0, 0, 0, 0, {0, 0}};
+  mfc_tuning tuning = {};
   mfc::inst_args *args[2] = {nullptr, nullptr};  // descriptors per start parity (device)
-  int2 *tiles = nullptr, *chunks = nullptr;
-  int ntiles = 0, nchunks = 0;
+  int2 *tiles = nullptr, *chunks = nullptr, *patches = nullptr;
+  int ntiles = 0, nchunks = 0, npatches = 0;
+  int lanes = 1;  // threads per particle of the interaction
+  int auto_lanes() const {
+    int64_t total = 0;
+    for (const mfc_sim *s : sims) total += s->k.N;
+    return interaction_lanes(total);  // the instances run together
+  }
   int cur = 0;
   int64_t step = 0;
   hipGraphExec_t graph[2] = {nullptr, nullptr};
 
   bool adaptive = false;  // some instance has an adaptive grid
+  bool pse = false;       // some instance conducts heat by PSE
   bool rothlin = false;   // some instance uses grid_gpu_rothlin's ranges
   mfc::batch_work work(int parity) const {
-    return {args[parity], (int)sims.size(), tiles, ntiles, chunks, nchunks, f32,
-            {tuning.split_interact != 0, tuning.compact_pairs != 0, tuning.xcd_chunk ? tuning.xcd_chunk : mfc::XCD_CHUNK},
-            adaptive, rothlin};
+    return {args[parity], (int)sims.size(), tiles, ntiles, chunks, nchunks, patches, npatches, f32,
+            {lanes, tuning.xcd_chunk ? tuning.xcd_chunk : mfc::XCD_CHUNK}, adaptive, pse, rothlin};
   }
   void drop_graphs() {
     for (int p = 0; p < 2; p++)
@@ -54,7 +60,7 @@ void batch_release(mfc_batch *b) {
     s->stream = nullptr;  // the batch's stream, destroyed below
     mfc_destroy(s);
   }
-  for (void *p : {(void *)b->args[0], (void *)b->args[1], (void *)b->tiles, (void *)b->chunks})
+  for (void *p : {(void *)b->args[0], (void *)b->args[1], (void *)b->tiles, (void *)b->chunks, (void *)b->patches})
     if (p) (void)hipFree(p);
   if (b->stream) (void)hipStreamDestroy(b->stream);
   delete b;
@@ -80,16 +86,19 @@ int build_batch_graph(mfc_batch *b, int parity) {
   return MFC_OK;
 }
 
-// the binning of every instance's current state (computed by the last step's interaction),
+// the binning and records of every instance's current state (computed by the last step's interaction),
 // recomputed for all instances when any of them lacks it
 int batch_keys(mfc_batch *b) {
   bool fresh = true;
   for (mfc_sim *s : b->sims) fresh = fresh && s->keys_fresh;
   if (fresh) return MFC_OK;
   for (mfc_sim *s : b->sims) {
-    HIP_TRY(hipMemsetAsync(s->bins.bsum, 0, sizeof(int) * (size_t)mfc::scan_blocks(s->k.ncell_table), b->stream));
+    HIP_TRY(hipMemsetAsync(s->bins.pcnt, 0, sizeof(int) * (size_t)s->npatch_max, b->stream));
+    HIP_TRY(hipMemsetAsync(s->plen, 0, 2 * sizeof(int), b->stream));
+    HIP_TRY(hipMemsetAsync(s->chunk_sums[b->cur], 0, sizeof(int) * (size_t)mfc::scan_blocks(s->k.ncell_table), b->stream));
   }
   mfc::launch_batch_hash(b->work(b->cur), b->stream);
+  mfc::launch_batch_records(b->work(b->cur), b->stream);
   for (mfc_sim *s : b->sims) s->keys_fresh = true;
   return MFC_OK;
 }
@@ -135,29 +144,40 @@ int mfc_batch_create(const mfc_config *cfgs, int n, mfc_batch **out) {
     s->use_graphs = false;
     b->adaptive = b->adaptive || s->k.adaptive;
     b->rothlin = b->rothlin || s->k.rothlin;
+    b->pse = b->pse || s->k.pse;
   }
-  std::vector<int2> tiles, chunks;
+  std::vector<int2> tiles, chunks, patches;
   std::vector<mfc::inst_args> a0(n), a1(n);
+  b->lanes = b->auto_lanes();
+  size_t patch_items_max = n;
   for (int i = 0; i < n; i++) {
-    const mfc_sim *s = b->sims[i];
+    mfc_sim *s = b->sims[i];
+    set_patches(s, b->lanes);
+    patch_items_max += s->npatch_items_max;
     a0[i] = instance_args(s, 0);
     a1[i] = instance_args(s, 1);
     for (int t = 0; t < a0[i].ntiles; t++) tiles.push_back(make_int2(i, t));
-    for (int c = 0; c < a0[i].nscan; c++) chunks.push_back(make_int2(i, c));
   }
+  sort_items(chunks, b->sims.data(), n);
+  patch_items(patches, b->sims.data(), n);
+  b->npatches = (int)patches.size();
   b->ntiles = (int)tiles.size();
   b->nchunks = (int)chunks.size();
   if (hipMalloc(&b->args[0], sizeof(mfc::inst_args) * n) != hipSuccess ||
       hipMalloc(&b->args[1], sizeof(mfc::inst_args) * n) != hipSuccess ||
       hipMalloc(&b->tiles, sizeof(int2) * tiles.size()) != hipSuccess ||
-      hipMalloc(&b->chunks, sizeof(int2) * chunks.size()) != hipSuccess)
+      hipMalloc(&b->chunks, sizeof(int2) * chunks.size()) != hipSuccess ||
+      hipMalloc(&b->patches, sizeof(int2) * patch_items_max) != hipSuccess)
     return bail(fail(MFC_E_NOMEM, "hipMalloc (batch tables)"));
   if (hipMemcpyAsync(b->args[0], a0.data(), sizeof(mfc::inst_args) * n, hipMemcpyHostToDevice, b->stream) ||
       hipMemcpyAsync(b->args[1], a1.data(), sizeof(mfc::inst_args) * n, hipMemcpyHostToDevice, b->stream) ||
       hipMemcpyAsync(b->tiles, tiles.data(), sizeof(int2) * tiles.size(), hipMemcpyHostToDevice, b->stream) ||
       hipMemcpyAsync(b->chunks, chunks.data(), sizeof(int2) * chunks.size(), hipMemcpyHostToDevice, b->stream) ||
+      hipMemcpyAsync(b->patches, patches.data(), sizeof(int2) * patches.size(), hipMemcpyHostToDevice, b->stream) ||
       hipStreamSynchronize(b->stream))
     return bail(fail(MFC_E_HIP, "upload of the batch tables"));
+  for (int i = 0; i < n; i++)
+    for (int c = 0; c < 2; c++) b->sims[i]->slot[c] = b->args[c] + i;
   *out = b;
   return MFC_OK;
 }
@@ -179,6 +199,18 @@ int mfc_batch_set_tuning(mfc_batch *b, const mfc_tuning *t) {
   HIP_TRY(hipStreamSynchronize(b->stream));
   b->tuning = *t;
   const size_t n = b->sims.size();
+  const int lanes = t->lanes ? t->lanes : b->auto_lanes();
+  if (lanes != b->lanes) {
+    std::vector<int2> patches;
+    for (mfc_sim *s : b->sims) {
+      set_patches(s, lanes);
+      s->keys_fresh = false;  // the patches' counts are those of the old shape
+    }
+    patch_items(patches, b->sims.data(), (int)n);
+    HIP_TRY(hipMemcpy(b->patches, patches.data(), sizeof(int2) * patches.size(), hipMemcpyHostToDevice));
+    b->npatches = (int)patches.size();
+    b->lanes = lanes;
+  }
   std::vector<mfc::inst_args> a0(n), a1(n);
   for (size_t i = 0; i < n; i++) {
     mfc_sim *s = b->sims[i];

@@ -163,6 +163,8 @@ int mfc_load(const char *path, mfc_sim **out) {
   const unsigned char *p = buf.data();
   s->cur = 0;
   if (hipMemcpy(s->set[0].px, p, L.state, hipMemcpyHostToDevice) != hipSuccess) return bail(fail(MFC_E_HIP, "upload"));
+  check_uniform_h(s, (const double *)p + (s->set[0].h - s->set[0].px));
+  if ((rc = upload_descriptors(s))) return bail(rc);
   p += L.state;
   if (hipMemcpy(s->pos.nx, p, L.positional, hipMemcpyHostToDevice) != hipSuccess) return bail(fail(MFC_E_HIP, "upload"));
   p += L.positional;

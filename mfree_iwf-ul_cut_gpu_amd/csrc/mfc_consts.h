@@ -24,6 +24,11 @@ struct dev_consts {
   int jc_tanh;        // the secant's flow stress: tanh-modified JC (the yield test keeps plain JC)
   double tanh_a, tanh_b, tanh_c, tanh_d;
   int plastic;        // Johnson-Cook return on
+  // the interaction's patches: patch_s rows x patch_w columns of cells
+  int patch_s, patch_w;
+  int patch_slots;    // particles a work-group takes at a time
+  int uniform_h;      // every particle's h is h0
+  double h0;
   int stage_limit;    // most window candidates a tile stages in LDS (0: all it has room for)
   int sort_fast;      // most particles of a chunk the sort holds in registers (0: all it can)
   int sort_list;      // most list entries a chunk of the sort reads (0: all the list holds)

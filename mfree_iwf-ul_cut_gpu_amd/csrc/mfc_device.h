@@ -428,24 +428,34 @@ __device__ inline bool contact_force(const dev_consts &k, const mfc_tool_state &
 }
 
 // one incremental tool move by dt: end points, line coefficients, fillet centre
-// (tool.cpp:211-221, geometric_primitives.cpp:70-85)
-__device__ inline void tool_move(mfc_tool_state &t, double dt) {
-  double sx = dt * t.vel[0], sy = dt * t.vel[1];
-#pragma unroll
-  for (int i = 0; i < 5; i++) {
-    if (i >= t.num_seg) break;
-    double lx = t.left[i][0] + sx, ly = t.left[i][1] + sy;
-    double rx = t.right[i][0] + sx, ry = t.right[i][1] + sy;
-    t.left[i][0] = lx; t.left[i][1] = ly; t.right[i][0] = rx; t.right[i][1] = ry;
-    double det = lx * 1. - 1. * rx;
-    if (fabs(det) < 1e-12) { t.vertical[i] = 1; t.line_a[i] = 1.7976931348623157e308; t.line_b[i] = lx; }
-    else {
-      t.vertical[i] = 0;
-      t.line_a[i] = (ly * 1. - 1. * ry) / det;
-      t.line_b[i] = (ry * lx - rx * ly) / det;
+// (tool.cpp:211-221, geometric_primitives.cpp:70-85). The work-group copies the state, then
+// thread i moves segment i and thread 5 the fillet: one thread moving all of them takes longer
+// than a chunk of the sort that runs beside it
+__device__ inline void tool_move(const mfc_tool_state *__restrict__ in, mfc_tool_state *__restrict__ out, double dt) {
+  constexpr int WORDS = sizeof(mfc_tool_state) / sizeof(int);
+  static_assert(sizeof(mfc_tool_state) % sizeof(int) == 0, "the tool state is copied in words");
+  for (int q = threadIdx.x; q < WORDS; q += blockDim.x)
+    reinterpret_cast<int *>(out)[q] = reinterpret_cast<const int *>(in)[q];
+  __syncthreads();
+  const double sx = dt * in->vel[0], sy = dt * in->vel[1];
+  const int i = threadIdx.x;
+  if (i < 5 && i < in->num_seg) {
+    const double lx = in->left[i][0] + sx, ly = in->left[i][1] + sy;
+    const double rx = in->right[i][0] + sx, ry = in->right[i][1] + sy;
+    out->left[i][0] = lx; out->left[i][1] = ly; out->right[i][0] = rx; out->right[i][1] = ry;
+    const double det = lx * 1. - 1. * rx;
+    if (fabs(det) < 1e-12) {
+      out->vertical[i] = 1; out->line_a[i] = 1.7976931348623157e308; out->line_b[i] = lx;
+    } else {
+      out->vertical[i] = 0;
+      out->line_a[i] = (ly * 1. - 1. * ry) / det;
+      out->line_b[i] = (ry * lx - rx * ly) / det;
     }
   }
-  if (t.has_fillet) { t.fillet_p[0] = t.fillet_p[0] + sx; t.fillet_p[1] = t.fillet_p[1] + sy; }
+  if (i == 5 && in->has_fillet) {
+    out->fillet_p[0] = in->fillet_p[0] + sx;
+    out->fillet_p[1] = in->fillet_p[1] + sy;
+  }
 }
 
 }  // namespace mfc

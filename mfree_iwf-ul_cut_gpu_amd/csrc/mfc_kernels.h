@@ -27,11 +27,17 @@ struct dbins {
   int *bucket;       // particle indices grouped by cell, unordered inside a cell
   int *perm;         // sorted position -> current position
   int *spos;         // current position -> sorted position
-  int *bsum;         // particles counted in each scan chunk of cells, zero between steps
+  int *bsum;         // particles counted in each scan chunk of cells (the start state's)
+  int *bsum_next;    // the same for the next step: cleared by the sort, counted by the interaction
   int2 *clist;       // per scan chunk, (current position, cell id) of the particles counted in
                      // its cells, in arrival order (ccap entries per chunk; a chunk that counts
                      // more finds them by a pass over all particles)
   int ccap;
+  int *pcnt;         // per patch of cells: particles of the next step's start state in it
+  int2 *plist;       // the interaction's work: (patch, part) for every patch_slots particles of a
+                     // patch, in ascending order (written by the sort launch, which clears pcnt)
+  int *plen;         // its length
+  int *plen_next;    // the next step's, cleared by the sort launch
   int *offsets_r;    // MFC_GRID_ROTHLIN: the ranges rebuilt from the sorted ids (the step reads these)
   unsigned long long *clamped;  // binned particles whose position lay outside the grid on an axis
 };
@@ -41,35 +47,43 @@ struct dpositional {
   double *nx, *ny, *p, *rxx, *rxy, *ryy;
 };
 
-constexpr int REC = 16;    // doubles per neighbour record
+constexpr int REC = 16;    // doubles per neighbour record (FP64; FP32C: floats)
 constexpr int ACC_N = 14;  // neighbour sums per particle
 
-// neighbour records written by the predict kernel and read by the interaction kernel, in
-// sorted order: posd (FP64 predicted position) and vfl (flags of the record) for the window
-// walk, and the pair record, rec (16 doubles per particle, FP64 path) or rec32 (16 floats,
-// FP32C path)
+// neighbour records in the storage order of the start state (sorted index j is particle
+// perm[j]): rec (FP64 path, 128 bytes: x y flags h u v rho vol Axx Axy Ayy Rxx Rxy Ryy c T) or
+// rec32 (FP32C path, 64 bytes: x y in FP64, then u v rho vol Axx Axy Ayy c Rxx Rxy Ryy T), and the
+// flags of the record, vfl. h is the state's (it does not change). The interaction writes those
+// of the next step into the other of two sets
 struct drecords {
   bool f32;
   double *rec;
-  double2 *posd;
+  float4 *rec32;
   int *vfl;
-  float *rec32;
 };
+constexpr int REC32_PIECES = 4;  // float4 per FP32C record
 
-// window candidates of a tile that the interaction kernels stage in LDS (positions and flags,
-// 20 bytes each); a tile whose candidates span more sorted indices reads them from memory
-constexpr int STAGE_CAP = MFC_STAGE_CAP;
+// The interaction runs over patches: rectangles of cells whose particles one work-group of TILE
+// threads takes, `lanes` threads per particle. The records of every window candidate of a patch
+// (its cells and two more on each side) are staged in LDS: up to PATCH_CAP of them; a patch with
+// more candidates (or of a state whose h is not uniform) reads them from memory.
+constexpr int PATCH_TABLE = 256;  // cell starts a patch holds in LDS: (patch_w + 4) (patch_s + 5) at most
+constexpr int PATCH_COLS = 24;    // patch_w + 4 at most
+__host__ __device__ constexpr int patch_cap(bool f32, int lanes) { return lanes > 1 ? 256 : f32 ? 512 : 488; }
 
-// tool-force reduction: per-tile partials written by the interaction kernel, reduced by the
-// force-final pass (the next step's first kernel, or a kernel of its own after the last step),
-// which appends F to the history
+// tool-force reduction: the interaction flags the groups of 64 particles (storage order) in which
+// some contact or friction force is not zero; the next step's sort launch sums those groups from
+// the state (the others' sums are zero) and its interaction launch adds the group sums up, or one
+// kernel does both after the last step. F is appended to the history
 struct dforce {
-  double *partials;      // 4 per wave of 64 particles: sum fc.x, fc.y, ft.x, ft.y
+  double *partials;      // 4 per group of 64 particles: sum fc.x, fc.y, ft.x, ft.y
+  int *gflag;            // per group: 1 when it has a force
   double *force_last;    // F of the last step
   double *hist;          // force history, 2 per step, cap entries
   int64_t cap;
   int64_t *ctr;          // steps recorded
-  int *pending;          // 1: the partials of a step are not yet reduced
+  int *pending;          // 1: the force of the step that produced the start state is not yet reduced
+  int *pending_next;     // the same for the state this step produces
 };
 
 // the particle flags of the state (FIXED, BLANKED, TOOL)
@@ -80,9 +94,8 @@ constexpr int FLAG_NONFINITE = 8;
 
 // launch variant of the interaction (results are identical for every variant)
 struct variant {
-  bool split;    // sums kernel + update kernel instead of one fused kernel
-  bool compact;  // per-lane mask of in-support neighbours before the pair loop
-  int chunk;     // tiles per XCD chunk of the interaction kernels' tile map (1..XCD_CHUNK_MAX)
+  int lanes;  // threads per particle: 1, 4 or 8
+  int chunk;  // work items per XCD chunk of the interaction's map (1..XCD_CHUNK_MAX)
 };
 
 // one instance of a batch as the batched kernels see it (an array of these lives in device
@@ -92,19 +105,17 @@ struct inst_args {
   dstate cur, nxt;  // state at the start of the step, and the sorted copy updated by the step
   dbins b;
   dpositional pos;
-  drecords r;
+  drecords r, rn;   // records of the start state, and of the next step's
   const mfc_tool_state *tool_in;
   mfc_tool_state *tool_out;
   dforce f;
-  double *acc;  // split interaction only
   double *acc_out;  // when set, the interaction also stores its neighbour sums there (ACC_N
                     // arrays of N doubles), then each particle's secant result (N doubles,
                     // wave_returns); the reverse mode's replay keeps them
   grid_geo *geo;  // adaptive grid: the geometry of the current step (written by the device)
   int ntiles;   // particle tiles of TILE
   int nscan;    // scan chunks of the cell table
-  int bin_next;  // 1: the interaction bins the next step's start state (0: the reverse mode's
-                 // replay, which bins every restored state itself)
+  int npatch_items;  // patch work items of the instance: item q takes the entries q, q + npatch_items, ... of plist
 };
 
 // the work of one batched step: instance descriptors and (instance, block) work tables
@@ -113,32 +124,40 @@ struct batch_work {
   int n;
   const int2 *tiles;      // (instance, particle tile) for every tile of every instance
   int ntiles;
-  const int2 *chunks;     // (instance, scan chunk) for every chunk of every cell table
+  const int2 *chunks;     // (instance, scan chunk) for every chunk of every cell table, and each
+                          // instance's SORT_ITEM_* (push_sort_items)
   int nchunks;
+  const int2 *patches;    // (instance, patch item), and each instance's SORT_ITEM_FORCE first
+  int npatches;
   bool f32;
   variant v;
   bool adaptive;          // some instance has an adaptive grid (a geometry pass starts the step)
-  bool rothlin;           // some instance uses grid_gpu_rothlin's cell ranges (a pass after predict)
+  bool pse;               // some instance conducts heat by PSE
+  bool rothlin;           // some instance uses grid_gpu_rothlin's cell ranges (a pass after the sort)
 };
 
-// one step of every instance of a batch: 3 (fused) or 4 (split) launches, and its phases. The
-// cell ids, chunk lists and chunk sums of a step's start state are computed by the previous
-// step's interaction; launch_batch_hash computes them from the state itself (chunk sums zeroed
-// before)
+// one step of every instance of a batch: 2 launches, and its phases. The
+// cell ids, chunk lists, chunk sums and neighbour records of a step's start state are computed by
+// the previous step's interaction; launch_batch_hash and launch_batch_records compute them from
+// the state itself (chunk sums zeroed before)
 void launch_batch_step(const batch_work &w, hipStream_t s);
 void launch_batch_hash(const batch_work &w, hipStream_t s);
 void launch_batch_binning(const batch_work &w, hipStream_t s);
-void launch_batch_predict(const batch_work &w, hipStream_t s);
-// predict that also writes the sorted copy of the start state into nxt (FP64 records; the
-// reverse mode reads it)
+void launch_batch_records(const batch_work &w, hipStream_t s);
+// the reverse mode's view of a step: the sorted copy of the start state (into nxt), the FP64
+// records in sorted order and the positional pressure and artificial stress
 void launch_batch_predict_gather(const batch_work &w, hipStream_t s);
 // with events t0 and t1 the launch records the kernel's own start and end in them
 // (hipExtLaunchKernelGGL), which times the kernel without the gap before it
-void launch_batch_interact_fused(const batch_work &w, hipStream_t s, hipEvent_t t0 = nullptr,
-                                 hipEvent_t t1 = nullptr);
-void launch_batch_sums(const batch_work &w, hipStream_t s, hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr);
-void launch_batch_update(const batch_work &w, hipStream_t s, hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr);
+void launch_batch_interact(const batch_work &w, hipStream_t s, hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr);
 void launch_batch_force(const batch_work &w, hipStream_t s);
+// work items of the sort launch beside the chunks (negative, where a chunk's index stands)
+constexpr int SORT_ITEM_TOOL = -1;     // the tool's move
+constexpr int SORT_ITEM_FORCE = -2;    // and below: the group sums of a block of FORCE_GROUPS groups
+constexpr int FORCE_GROUPS = 64;
+constexpr int SORT_ITEM_PATCHES = -(1 << 30);  // and below: the interaction's work from a section of patches
+constexpr int PLIST_SECTION = 1024;
+constexpr int PATCH_ITEM_FORCE = -1;   // of the interaction launch: the sum of the group sums
 int scan_chunk_cells();
 // entries of a scan chunk's particle list: 4 particles per cell of the chunk (a cell holds
 // about 2.25 at the lattice spacing), at most N

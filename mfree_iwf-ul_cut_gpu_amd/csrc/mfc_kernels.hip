@@ -1,37 +1,43 @@
 // mfc_kernels.hip — gfx950 kernels of one SPH cutting step (FP64 and FP32C).
 //
-// Per step (the reference's ~20 launches of leap_frog::step, leap_frog.cu:94-155, become 3):
+// Per step (the reference's ~20 launches of leap_frog::step, leap_frog.cu:94-155, become 2):
 //   sort         one work-group per chunk of cells: the cells' offsets, buckets and the rank of
 //                every particle in its cell, a stable counting sort by cell
 //                (thrust::sort_by_key + reorder_data_and_find_cell_start,
 //                grid_gpu_green.cu:22-116,177-201) from the cell ids (grid.cu:34-51), per-cell
 //                and per-chunk counts and the chunks' particle lists that the previous step's
 //                interaction computed for the updated state (hash_count computes them when the
-//                state was written from outside, and for every state the reverse mode's replay
-//                restores)
-//   predict      leap-frog predict (leap_frog.cu:30-66) + EOS
-//                (actions_gpu.cu:41-51) + artificial stress (:53-97) + neighbour record + tool
-//                move, in the start state's storage order; the work-group of the first tile
-//                also reduces the previous step's tool force (output.cu:30-39) from its tile
-//                partials
+//                state was written from outside, and for every state the reverse mode
+//                restores); a few more work-groups of the launch move the tool, list the patches of
+//                cells that hold particles and sum the previous step's tool force
+//                (output.cu:30-39) over groups of 64 particles
 //   interact     neighbour sums (interactions_gpu.cu:88-345) fused with every per-particle action
 //                that follows them in the step: Jaumann, continuity, momentum, advection, correct,
 //                friction heat, Johnson-Cook return, tool-particle move, contact, boundary
-//                conditions, NaN blanking, the gather into sorted order, and the per-wave partial
-//                sums of the tool force (or split into sums + update), and the cell ids and
-//                counts of the next step
-// After the last step of a call, force_final reduces the last step's tool force.
+//                conditions, NaN blanking and the gather into sorted order; then, for the next step,
+//                the cell ids and counts and each particle's neighbour record: leap-frog predict
+//                (leap_frog.cu:30-66), EOS (actions_gpu.cu:41-51) and artificial stress (:53-97)
+//                (records computes them when the state was written from outside). A work-group
+//                takes a patch of cells with its window candidates staged in LDS, with 1, 4 or 8
+//                threads per particle; one more adds up the previous step's force sums
+// After the last step of a call, force_final reduces the last step's tool force. The record of a
+// step could not be written by a kernel of the same step that also reads it (every particle's sums
+// need all its neighbours' records), but the previous interaction holds all it is made of in
+// registers: with a launch of its own, which read 19 of the 27 state fields again, the step took
+// 80 us instead of 72 (FP32C, 197k particles) and 63 instead of 53 (FP64, 6k).
 // Each body is a device function of its work index; the kb_* kernels run it over an
 // (instance, tile) work table for any number of instances (a single handle is a batch of one).
 //
 // Memory layout: the persistent particle state is a structure of arrays in cell-sorted order,
 // double-buffered across the step. Neighbour data are packed per particle into one 128-byte
-// record (two 64-byte lines; FP32C: 64 bytes plus the FP64 position) so that the divergent
-// per-lane neighbour reads are 16-byte vector loads from one cache line. Work-group to tile
+// record (FP64) or one of 64 bytes (FP32C, the position in FP64); the records stay where
+// the interaction wrote them (the storage order of the next step's start state) and are found
+// through the sort permutation. Work-group to tile
 // mapping is XCD-aware.
 #include <hip/hip_ext.h>
 
 #include <cfloat>
+#include <type_traits>
 
 #include "mfc_kernels.h"
 #include "mfc_pairs.h"
@@ -72,6 +78,11 @@ __device__ inline int block_exclusive_scan(int v, int &total) {
   return pre + x - v;
 }
 
+// patches of the grid: patch p holds the cell rows [r patch_s, (r + 1) patch_s) and the columns
+// [c patch_w, (c + 1) patch_w) with p = c patch_rows + r
+__device__ inline int patch_rows(const dev_consts &k) { return (k.gny + k.patch_s - 1) / k.patch_s; }
+__device__ inline int patch_total(const dev_consts &k) { return ((k.gnx + k.patch_w - 1) / k.patch_w) * patch_rows(k); }
+
 // ------------------------------------------------------------------------------- binning
 // Each kernel body is a device function of its work index, called by the batched kernel with
 // the index of an (instance, block) item of its work table.
@@ -111,12 +122,27 @@ __device__ inline void count_cell(int i, int h, int *__restrict__ key, int *__re
   if (c >= 0 && place < ccap) clist[(size_t)c * ccap + place] = make_int2(i, h);
 }
 
+// counts the particle of cell h in its patch (all 64 lanes of the wave; h = -1: no particle): one
+// atomic per run of equal patches in the wave
+__device__ inline void count_patch(const dev_consts &k, int h, int *__restrict__ pcnt) {
+  int p = -1;
+  if (h >= 0) {
+    const int gi = h / k.gny, gj = h - gi * k.gny;
+    p = (gi / k.patch_w) * patch_rows(k) + gj / k.patch_s;
+  }
+  const int lane = threadIdx.x & 63, prev = __shfl_up(p, 1, 64);
+  const bool head = lane == 0 || prev != p;
+  const unsigned long long after = lane == 63 ? 0ull : __ballot(head) & ~((2ull << lane) - 1ull);
+  if (head && p >= 0) atomicAdd(&pcnt[p], (after ? __ffsll((long long)after) - 1 : 64) - lane);
+}
+
 // cell id of every particle of the start state, counted in its chunk
 __device__ inline void hash_count(const dev_consts &k, int i, const double *__restrict__ px,
                                   const double *__restrict__ py, const int *__restrict__ flags,
                                   const dbins &b) {
   const int h = i < k.N ? particle_cell(k, px[i], py[i], flags[i], b.key_sorted[i], b.clamped) : -1;
   count_cell(i, h, b.key, b.bsum, b.clist, b.ccap);
+  count_patch(k, h, b.pcnt);
 }
 
 // The counting sort of one chunk of SCAN_CHUNK cells (SCAN_ITEMS per thread), by one work-group,
@@ -203,6 +229,7 @@ __device__ inline void sort_chunk(int blk, int N, int n, const dbins &b, int sor
     v[q] = cnt_l[l0 + q];
     sv += v[q];
   }
+  if (threadIdx.x == 0) b.bsum_next[blk] = 0;  // the interaction counts the next step's there
   int total;
   int o = block_exclusive_scan(sv, total) + carry;
 #pragma unroll
@@ -252,6 +279,66 @@ __device__ inline void sort_chunk(int blk, int N, int n, const dbins &b, int sor
   }
 }
 
+// the work of the interaction from the patches [PLIST_SECTION sec, + PLIST_SECTION), by one
+// work-group: for every patch that holds particles an entry (patch, part) per patch_slots of them.
+// A section's entries follow each other in ascending order, the sections in any (the results do
+// not depend on the order of the list). Clears the patches' counts
+constexpr int PLIST_BATCH = PLIST_SECTION / SCAN_THREADS;  // patches per thread
+__device__ inline void list_patches(const dev_consts &k, int sec, const dbins &b) {
+  const int np = patch_total(k);
+  const int p0 = sec * PLIST_SECTION + threadIdx.x * PLIST_BATCH;
+  if (sec == 0 && threadIdx.x == 0) *b.plen_next = 0;
+  if (sec * PLIST_SECTION >= np) return;
+  int f[PLIST_BATCH], cnt = 0;
+#pragma unroll
+  for (int u = 0; u < PLIST_BATCH; u++) f[u] = p0 + u < np ? b.pcnt[p0 + u] : 0;
+#pragma unroll
+  for (int u = 0; u < PLIST_BATCH; u++)
+    if (f[u]) {
+      b.pcnt[p0 + u] = 0;
+      f[u] = (f[u] + k.patch_slots - 1) / k.patch_slots;
+      cnt += f[u];
+    }
+  __shared__ int first;
+  int total;
+  int o = block_exclusive_scan(cnt, total);
+  if (total == 0) return;  // the same in every thread
+  if (threadIdx.x == 0) first = atomicAdd(b.plen, total);
+  __syncthreads();
+  o += first;
+#pragma unroll
+  for (int u = 0; u < PLIST_BATCH; u++)
+    for (int q = 0; q < f[u]; q++) b.plist[o++] = make_int2(p0 + u, q);
+}
+
+// sums of (fc.x, fc.y, ft.x, ft.y) over group g of 64 particles (storage order) of state st by one
+// wave: the halving-stride tree over the lanes (lane l adds lane l + s for s = 32, 16, ..., 1, so
+// lane 0 ends with the tree's root); lanes past N add zeros
+__device__ inline void force_group(int N, int g, const dstate &st, double *__restrict__ partials) {
+  const int lane = threadIdx.x & 63, i = 64 * g + lane;
+  double v0 = 0., v1 = 0., v2 = 0., v3 = 0.;
+  if (i < N) { v0 = st.fcx[i]; v1 = st.fcy[i]; v2 = st.ftx[i]; v3 = st.fty[i]; }
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) {
+    v0 = v0 + __shfl_down(v0, s, 64);
+    v1 = v1 + __shfl_down(v1, s, 64);
+    v2 = v2 + __shfl_down(v2, s, 64);
+    v3 = v3 + __shfl_down(v3, s, 64);
+  }
+  if (lane == 0) { partials[4 * g] = v0; partials[4 * g + 1] = v1; partials[4 * g + 2] = v2; partials[4 * g + 3] = v3; }
+}
+
+// the group sums of the groups [g0, g0 + n) (n <= 64) by one wave: zeros for the groups without a
+// force; clears the groups' flags
+__device__ inline void force_groups(int N, int g0, int n, const dstate &st, const dforce &fo) {
+  const int lane = threadIdx.x & 63, g = g0 + lane;
+  const bool in = lane < n && g < (N + TILE - 1) / TILE * (TILE / 64);  // the groups of whole tiles
+  const bool some = in && fo.gflag[g] != 0;
+  if (some) fo.gflag[g] = 0;
+  else if (in) reinterpret_cast<double4 *>(fo.partials)[g] = make_double4(0., 0., 0., 0.);
+  for (unsigned long long m = __ballot(some); m; m &= m - 1ull)
+    force_group(N, g0 + __builtin_ctzll(m), st, fo.partials);
+}
 
 // ------------------------------------------------------------------------------- predict
 // artificial stress in single precision without trigonometry: with d = sqrt((sxx-syy)^2 + 4 sxy^2),
@@ -275,118 +362,182 @@ __device__ inline void artificial_stress_f32(float rho, float p, float Sxx, floa
   Ryy = st2 * q1 + ct2 * q2;
 }
 
-// leap-frog init + predict, EOS, artificial stress and the neighbour record written at the
-// particle's sorted position (from the sort). Runs in the storage order of the start state (its
-// reads are coalesced). F32: the record is 16 floats (64 bytes) plus the FP64 predicted
-// position.
-template <bool F32, bool GATHER>
-__device__ inline void predict(const dev_consts &k, int t, const dbins &bins, const dstate &cur, const dstate &nxt,
-                               const dpositional &pos, const drecords &recs,
-                               const mfc_tool_state *__restrict__ tool_in, mfc_tool_state *__restrict__ tool_out) {
-  double *__restrict__ rec = recs.rec;
-  double2 *__restrict__ posd = recs.posd;
-  int *__restrict__ vfl = recs.vfl;
-  float *__restrict__ rec32 = recs.rec32;
-  if (t == 0 && threadIdx.x == 0) {
-    mfc_tool_state ts = *tool_in;
-    tool_move(ts, k.dt);
-    *tool_out = ts;
+// the fields a neighbour record is made of: a particle's state and the rates of the predictor
+struct rec_input {
+  double x, y, u, v, sxx, sxy, syy, rho, T, h;
+  double ptx, pty, vtx, vty, rhot, stxx, stxy, styy, Tt;
+  int fl;
+};
+
+__device__ inline rec_input load_rec_input(const dstate &c, int s) {
+  rec_input q;
+  q.x = c.px[s]; q.y = c.py[s]; q.u = c.vx[s]; q.v = c.vy[s];
+  q.sxx = c.sxx[s]; q.sxy = c.sxy[s]; q.syy = c.syy[s];
+  q.rho = c.rho[s]; q.T = c.T[s];
+  q.ptx = c.ptx[s]; q.pty = c.pty[s]; q.vtx = c.vtx[s]; q.vty = c.vty[s];
+  q.rhot = c.rhot[s]; q.stxx = c.stxx[s]; q.stxy = c.stxy[s]; q.styy = c.styy[s];
+  q.Tt = c.Tt[s];
+  q.fl = c.flags[s] & FLAG_MASK;
+  q.h = c.h[s];
+  return q;
+}
+
+// leap-frog init + predict (in place)
+__device__ inline void predict_input(const dev_consts &k, rec_input &q) {
+  if (q.fl & MFC_FLAG_BLANKED) return;  // leap_frog.cu:42-66
+  const double hdt = 0.5 * k.dt;
+  q.x = q.x + hdt * q.ptx; q.y = q.y + hdt * q.pty;
+  q.u = q.u + hdt * q.vtx; q.v = q.v + hdt * q.vty;
+  q.sxx = q.sxx + hdt * q.stxx; q.sxy = q.sxy + hdt * q.stxy; q.syy = q.syy + hdt * q.styy;
+  q.rho = q.rho + hdt * q.rhot;
+  q.T = q.T + hdt * q.Tt;
+}
+
+// the FP64 record of predicted input q with pressure p and artificial stress R, written at i
+__device__ inline void store_record(const dev_consts &k, const rec_input &q, double p, double rxx, double rxy,
+                                    double ryy, int i, const drecords &recs) {
+  const double r21 = 1. / (q.rho * q.rho);
+  double r[REC];
+  r[0] = q.x; r[1] = q.y;
+  r[3] = q.h;
+  r[4] = q.u; r[5] = q.v;
+  r[6] = q.rho;
+  r[7] = k.mass / q.rho;
+  r[8] = (q.sxx - p) * r21;
+  r[9] = q.sxy * r21;
+  r[10] = (q.syy - p) * r21;
+  r[11] = rxx; r[12] = rxy; r[13] = ryy;
+  r[14] = tsqrt(k, k.K / q.rho);
+  r[15] = q.T;
+  bool fin = true;
+#pragma unroll
+  for (int c = 0; c < REC; c++)
+    if (c != 2) fin = fin && finite_d(r[c]);
+  const int rfl = q.fl | (fin ? 0 : FLAG_NONFINITE);
+  r[2] = bits_to_double(rfl);
+  double2 *dst = reinterpret_cast<double2 *>(recs.rec + (size_t)REC * i);
+#pragma unroll
+  for (int c = 0; c < REC / 2; c++) dst[c] = make_double2(r[2 * c], r[2 * c + 1]);
+  recs.vfl[i] = rfl;
+}
+
+// leap-frog predict, EOS, artificial stress and the neighbour record of a particle in state q,
+// written at its storage index i. The pressure and artificial stress of a tool particle enter no sum (every term that
+// reads them skips pairs with one) and are 0 in its record.
+template <bool F32>
+__device__ inline void write_record(const dev_consts &k, rec_input q, int i, const drecords &recs) {
+  predict_input(k, q);
+  const bool tool = q.fl & MFC_FLAG_TOOL;
+  const double p = tool ? 0. : k.c0 * k.c0 * (q.rho - k.rho0);
+  if constexpr (F32) {
+    float fxx = 0.0f, fxy = 0.0f, fyy = 0.0f;
+    if (!tool)
+      artificial_stress_f32((float)q.rho, (float)p, (float)q.sxx, (float)q.sxy, (float)q.syy, (float)k.stress_eps, fxx,
+                            fxy, fyy);
+    const float rf = (float)q.rho, pf = (float)p;
+    const float r21 = 1.0f / (rf * rf);
+    float4 *dst = recs.rec32 + (size_t)REC32_PIECES * i;
+    *reinterpret_cast<double2 *>(dst) = make_double2(q.x, q.y);
+    dst[1] = make_float4((float)q.u, (float)q.v, rf, (float)(k.mass / q.rho));
+    dst[2] = make_float4(((float)q.sxx - pf) * r21, (float)q.sxy * r21, ((float)q.syy - pf) * r21,
+                         sqrtf((float)(k.K / q.rho)));
+    dst[3] = make_float4(fxx, fxy, fyy, (float)q.T);
+    recs.vfl[i] = q.fl;
+  } else {
+    double rxx = 0., rxy = 0., ryy = 0.;
+    if (!tool) artificial_stress(q.rho, p, q.sxx, q.sxy, q.syy, k.stress_eps, rxx, rxy, ryy, k.promote != 0);
+    store_record(k, q, p, rxx, rxy, ryy, i, recs);
   }
+}
+
+// the positional pressure and artificial stress of the step at sorted index i (the reference's
+// arrays p and R, which its sort does not permute: a tool particle leaves what the slot holds),
+// from the particle's record at storage index s
+template <bool F32>
+__device__ inline void store_positional(const dpositional &pos, int i, int s, double p, const drecords &recs) {
+  pos.p[i] = p;
+  if constexpr (F32) {
+    const float4 a3 = recs.rec32[(size_t)REC32_PIECES * s + 3];
+    pos.rxx[i] = a3.x; pos.rxy[i] = a3.y; pos.ryy[i] = a3.z;
+  } else {
+    const double *r = recs.rec + (size_t)REC * s;
+    pos.rxx[i] = r[11]; pos.rxy[i] = r[12]; pos.ryy[i] = r[13];
+  }
+}
+
+// the reverse mode's view of a step, in the storage order of the start state: the sorted copy of
+// the state, the FP64 record at the particle's sorted position and the positional arrays there
+__device__ inline void predict_gather(const dev_consts &k, int t, const dbins &bins, const dstate &cur,
+                                      const dstate &nxt, const dpositional &pos, const drecords &recs) {
   const int s = t * TILE + threadIdx.x;
   if (s >= k.N) return;
   const int i = bins.spos[s];
-  const double x0 = cur.px[s], y0 = cur.py[s], u0 = cur.vx[s], v0 = cur.vy[s];
-  const double sxx0 = cur.sxx[s], sxy0 = cur.sxy[s], syy0 = cur.syy[s];
-  const double rho0 = cur.rho[s], T0 = cur.T[s];
-  const double ptx = cur.ptx[s], pty = cur.pty[s], vtx = cur.vtx[s], vty = cur.vty[s];
-  const double rhot = cur.rhot[s], stxx = cur.stxx[s], stxy = cur.stxy[s], styy = cur.styy[s];
-  const double Tt = cur.Tt[s];
-  const int fl = cur.flags[s] & FLAG_MASK;
-  const double h = cur.h[s];
-  if constexpr (GATHER) {  // the sorted copy of the start state (the reverse mode reads it)
-    nxt.px[i] = x0; nxt.py[i] = y0; nxt.vx[i] = u0; nxt.vy[i] = v0;
-    nxt.sxx[i] = sxx0; nxt.sxy[i] = sxy0; nxt.syy[i] = syy0; nxt.szz[i] = cur.szz[s];
-    nxt.rho[i] = rho0; nxt.T[i] = T0; nxt.h[i] = h;
-    nxt.eps[i] = cur.eps[s]; nxt.epsd[i] = cur.epsd[s];
-    nxt.fcx[i] = cur.fcx[s]; nxt.fcy[i] = cur.fcy[s]; nxt.ftx[i] = cur.ftx[s]; nxt.fty[i] = cur.fty[s];
-    nxt.ptx[i] = ptx; nxt.pty[i] = pty; nxt.vtx[i] = vtx; nxt.vty[i] = vty;
-    nxt.rhot[i] = rhot; nxt.stxx[i] = stxx; nxt.stxy[i] = stxy; nxt.styy[i] = styy; nxt.stzz[i] = cur.stzz[s];
-    nxt.Tt[i] = Tt;
-    nxt.flags[i] = fl;
-    nxt.id[i] = cur.id[s];
-  }
-
-  double x = x0, y = y0, u = u0, v = v0, sxx = sxx0, sxy = sxy0, syy = syy0, rho = rho0, T = T0;
-  if (!(fl & MFC_FLAG_BLANKED)) {  // leap_frog.cu:42-66
-    const double hdt = 0.5 * k.dt;
-    x = x0 + hdt * ptx; y = y0 + hdt * pty;
-    u = u0 + hdt * vtx; v = v0 + hdt * vty;
-    sxx = sxx0 + hdt * stxx; sxy = sxy0 + hdt * stxy; syy = syy0 + hdt * styy;
-    rho = rho0 + hdt * rhot;
-    T = T0 + hdt * Tt;
-  }
-  // the positional values at i are recomputed below for every particle but the tool's, which
-  // keep what the slot holds (the reference's positional arrays are not permuted)
-  double p = 0., rxx = 0., rxy = 0., ryy = 0.;
-  if (fl & MFC_FLAG_TOOL) {
+  rec_input q = load_rec_input(cur, s);
+  nxt.px[i] = q.x; nxt.py[i] = q.y; nxt.vx[i] = q.u; nxt.vy[i] = q.v;
+  nxt.sxx[i] = q.sxx; nxt.sxy[i] = q.sxy; nxt.syy[i] = q.syy; nxt.szz[i] = cur.szz[s];
+  nxt.rho[i] = q.rho; nxt.T[i] = q.T; nxt.h[i] = q.h;
+  nxt.eps[i] = cur.eps[s]; nxt.epsd[i] = cur.epsd[s];
+  nxt.fcx[i] = cur.fcx[s]; nxt.fcy[i] = cur.fcy[s]; nxt.ftx[i] = cur.ftx[s]; nxt.fty[i] = cur.fty[s];
+  nxt.ptx[i] = q.ptx; nxt.pty[i] = q.pty; nxt.vtx[i] = q.vtx; nxt.vty[i] = q.vty;
+  nxt.rhot[i] = q.rhot; nxt.stxx[i] = q.stxx; nxt.stxy[i] = q.stxy; nxt.styy[i] = q.styy; nxt.stzz[i] = cur.stzz[s];
+  nxt.Tt[i] = q.Tt;
+  nxt.flags[i] = q.fl;
+  nxt.id[i] = cur.id[s];
+  predict_input(k, q);
+  double p, rxx, rxy, ryy;
+  if (q.fl & MFC_FLAG_TOOL) {
     p = pos.p[i]; rxx = pos.rxx[i]; rxy = pos.rxy[i]; ryy = pos.ryy[i];
-  }
-  if constexpr (F32) {
-    float fxx = (float)rxx, fxy = (float)rxy, fyy = (float)ryy;
-    if (!(fl & MFC_FLAG_TOOL)) {
-      p = k.c0 * k.c0 * (rho - k.rho0);
-      artificial_stress_f32((float)rho, (float)p, (float)sxx, (float)sxy, (float)syy, (float)k.stress_eps, fxx, fxy, fyy);
-      pos.p[i] = p; pos.rxx[i] = fxx; pos.rxy[i] = fxy; pos.ryy[i] = fyy;
-    }
-    const float rf = (float)rho, pf = (float)p;
-    const float r21 = 1.0f / (rf * rf);
-    float4 q0 = make_float4((float)u, (float)v, (float)h, rf);
-    float4 q1 = make_float4((float)(k.mass / rho), ((float)sxx - pf) * r21, (float)sxy * r21, ((float)syy - pf) * r21);
-    float4 q2 = make_float4(fxx, fxy, fyy, sqrtf((float)(k.K / rho)));
-    float4 q3 = make_float4((float)T, __int_as_float(fl), 0.0f, 0.0f);
-    float4 *dst = reinterpret_cast<float4 *>(rec32 + (size_t)16 * i);
-    dst[0] = q0; dst[1] = q1; dst[2] = q2; dst[3] = q3;
-    posd[i] = make_double2(x, y);
-    vfl[i] = fl;
-    return;
   } else {
-    if (!(fl & MFC_FLAG_TOOL)) {
-      p = k.c0 * k.c0 * (rho - k.rho0);
-      artificial_stress(rho, p, sxx, sxy, syy, k.stress_eps, rxx, rxy, ryy, k.promote != 0);
-      pos.p[i] = p; pos.rxx[i] = rxx; pos.rxy[i] = rxy; pos.ryy[i] = ryy;
-    }
+    p = k.c0 * k.c0 * (q.rho - k.rho0);
+    artificial_stress(q.rho, p, q.sxx, q.sxy, q.syy, k.stress_eps, rxx, rxy, ryy, k.promote != 0);
+    pos.p[i] = p; pos.rxx[i] = rxx; pos.rxy[i] = rxy; pos.ryy[i] = ryy;
   }
-  const double r21 = 1. / (rho * rho);
-  double r[REC];
-  r[0] = x; r[1] = y;
-  r[3] = h;
-  r[4] = u; r[5] = v;
-  r[6] = rho;
-  r[7] = k.mass / rho;
-  r[8] = (sxx - p) * r21;
-  r[9] = sxy * r21;
-  r[10] = (syy - p) * r21;
-  r[11] = rxx; r[12] = rxy; r[13] = ryy;
-  r[14] = tsqrt(k, k.K / rho);
-  r[15] = T;
-  bool fin = true;
-#pragma unroll
-  for (int q = 0; q < REC; q++)
-    if (q != 2) fin = fin && finite_d(r[q]);
-  const int rfl = fl | (fin ? 0 : FLAG_NONFINITE);
-  r[2] = bits_to_double(rfl);
-  double2 *dst = reinterpret_cast<double2 *>(rec + (size_t)REC * i);
-#pragma unroll
-  for (int q = 0; q < REC / 2; q++) dst[q] = make_double2(r[2 * q], r[2 * q + 1]);
-  posd[i] = make_double2(x, y);
-  vfl[i] = rfl;
+  store_record(k, q, p, rxx, rxy, ryy, i, recs);
 }
 
-// ------------------------------------------------------------------------------- interact
-// the sums kernels keep at least 3 waves per SIMD (at most 168 VGPRs): a 150k-particle step
-// has about 3 waves per SIMD in all, so all of them are resident at once
-#define SUMS_OCCUPANCY __attribute__((amdgpu_waves_per_eu(3)))
+// ------------------------------------------------------------------------------- descriptors
+// Fields of the instance descriptors read through the constant address space: the compiler
+// then takes the pointers loaded from them for global pointers and emits global loads, which
+// count only against the vector-memory wait counter, instead of flat loads, which also hold up
+// every wait for an LDS or scalar load. (A whole-struct copy loses that, hence the field lists.)
+// The descriptors do not change while a kernel runs.
+#define MFC_CONST(T) const __attribute__((address_space(4))) T
+#define MFC_F(f) o.f = c->f
+__device__ inline dstate load_state(MFC_CONST(dstate) * c) {
+  dstate o;
+  MFC_F(px); MFC_F(py); MFC_F(vx); MFC_F(vy); MFC_F(sxx); MFC_F(sxy); MFC_F(syy); MFC_F(szz); MFC_F(rho);
+  MFC_F(T); MFC_F(eps); MFC_F(epsd); MFC_F(h); MFC_F(fcx); MFC_F(fcy); MFC_F(ftx); MFC_F(fty); MFC_F(ptx);
+  MFC_F(pty); MFC_F(vtx); MFC_F(vty); MFC_F(rhot); MFC_F(stxx); MFC_F(stxy); MFC_F(styy); MFC_F(stzz); MFC_F(Tt);
+  MFC_F(flags); MFC_F(id);
+  return o;
+}
+__device__ inline dbins load_bins(MFC_CONST(dbins) * c) {
+  dbins o;
+  MFC_F(key); MFC_F(key_sorted); MFC_F(offsets); MFC_F(bucket); MFC_F(perm);
+  MFC_F(spos); MFC_F(bsum); MFC_F(bsum_next); MFC_F(pcnt); MFC_F(plist); MFC_F(plen); MFC_F(plen_next); MFC_F(clist); MFC_F(ccap); MFC_F(offsets_r); MFC_F(clamped);
+  return o;
+}
+__device__ inline dpositional load_pos(MFC_CONST(dpositional) * c) {
+  dpositional o;
+  MFC_F(nx); MFC_F(ny); MFC_F(p); MFC_F(rxx); MFC_F(rxy); MFC_F(ryy);
+  return o;
+}
+__device__ inline drecords load_recs(MFC_CONST(drecords) * c) {
+  drecords o;
+  MFC_F(f32); MFC_F(rec); MFC_F(rec32); MFC_F(vfl);
+  return o;
+}
+__device__ inline dforce load_force(MFC_CONST(dforce) * c) {
+  dforce o;
+  MFC_F(partials); MFC_F(gflag); MFC_F(pending_next); MFC_F(force_last); MFC_F(hist); MFC_F(cap); MFC_F(ctr); MFC_F(pending);
+  return o;
+}
+__device__ inline MFC_CONST(inst_args) * const_args(const inst_args *A, int q) {
+  return (MFC_CONST(inst_args) *)(A + q);
+}
+#undef MFC_F
 
+// ------------------------------------------------------------------------------- interact
 // compensated (Kahan) accumulation in single precision
 struct kahan {
   float s = 0.0f, c = 0.0f;
@@ -399,50 +550,253 @@ struct kahan {
   __device__ inline double value() const { return (double)s - (double)c; }
 };
 
-// FP32 neighbour sums with Kahan compensation (the same pair terms as pair_terms, rearranged
-// for single precision: hardware reciprocals and reciprocal square roots instead of divisions,
-// the particle mass and the factor 2 of Brookshaw taken out of the sums, e.gradW/r of Brookshaw
-// written as der*fac, which is its exact value, and the stress and viscosity terms of each
-// acceleration component added before their one compensated sum). Pair distances are formed in
-// FP64 and then rounded.
-template <bool COMPACT>
-__device__ inline void sums_f32(const dev_consts &k, int i, const double2 *__restrict__ posd,
-                                const float *__restrict__ rec32, const int *__restrict__ key_sorted,
-                                const int *__restrict__ offsets, const cand_src &cs, bool tool, double ta_d,
-                                bool run_mech, bool run_pse, pair_acc &acc, double &tpse) {
-  const float4 *ri = reinterpret_cast<const float4 *>(rec32 + (size_t)16 * i);
-  const float4 a0 = ri[0], a1 = ri[1], a2 = ri[2], a3 = ri[3];
-  const double2 pi = posd[i];
-  const float ui = a0.x, vi_ = a0.y, hi = a0.z, rhoi = a0.w;
-  const float Axx_i = a1.y, Axy_i = a1.z, Ayy_i = a1.w, Rxx_i = a2.x, Rxy_i = a2.y, Ryy_i = a2.z, ci = a2.w;
-  const float Tpred = a3.x;
-  const float ta = (float)ta_d;
-  const float Ti = ta != 0.0f ? Tpred : 0.0f;
-  const float h1 = 1.0f / hi;
-  const float fourh2 = 4.0f * hi * hi;
-  const float fac = (float)PI_FAC * h1 * h1;
-  const float inv_wd = (float)(1.0 / k.wdeltap);
-  const float eta2 = (float)(k.av_eta * k.av_eta);
-  const float alpha = (float)k.av_alpha, beta = (float)k.av_beta, xeps = (float)k.xsph_eps;
-  const float inv_h2 = h1 * h1;
-  const float pse_c = (float)(4. / M_PI) * inv_h2 * inv_h2;
-  const float massf = (float)k.mass;
-  // the stress and viscosity sums enter the acceleration only as sd0 + sd1 + vt0 and
-  // sd2 + sd3 + vt1 (actions_gpu.cu momentum), so they are accumulated as those two sums
-  kahan vd0, vd1, vd2, vd3, ax, ay, xt0, xt1, tl, tp;
-  const window w = make_window(k, offsets, key_sorted[i]);
-  // the mechanical and Brookshaw terms of one in-support neighbour
-  struct rec4 {
-    float4 b0, b1, b2, b3;
-  };
-  auto load_rec = [&](int j, rec4 &r) {
-    const float4 *rj = reinterpret_cast<const float4 *>(rec32 + (size_t)16 * j);
-    r.b0 = rj[0]; r.b1 = rj[1]; r.b2 = rj[2]; r.b3 = rj[3];
-  };
-  auto pair = [&](float dx, float dy, float rr2, const rec4 &r) {
-    const float4 b0 = r.b0, b1 = r.b1, b2 = r.b2, b3 = r.b3;
-    const int fj = __float_as_int(b3.y);
-    const float uj = b0.x, vj = b0.y, hj_ = b0.z, rhoj = b0.w, volj = b1.x;
+// a particle's FP32C record as the pair terms read it
+struct rec32 {
+  double x, y;
+  float u, v, rho, vol, Axx, Axy, Ayy, c, Rxx, Rxy, Ryy, T, h;
+};
+template <bool F32>
+using rec_t = std::conditional_t<F32, rec32, rec64>;
+
+// LDS of a work-group of the interaction (patch_cap, PATCH_TABLE and PATCH_COLS above). The records
+// lie in arrays of 16-byte pieces (FP64: xy uv rho/vol A A/R R c/T; FP32C: xy u v rho vol | A c |
+// R T), each one 16 bytes longer than a multiple of the banks, so that the lanes that stage the
+// pieces of a record write different banks. FP64 with one thread per particle keeps one of c and T
+// (X) and leaves the other in memory: with both only two work-groups would fit a CU instead of
+// three (53.9 of 160 KB).
+template <bool F32, int G>
+struct patch_mem {
+  static constexpr int CAP = patch_cap(F32, G);
+  static constexpr bool ALL_IN_LDS = F32 || G > 1;
+  static constexpr int PIECES = F32 ? 4 : ALL_IN_LDS ? 7 : 6;
+  // the terms of one pair per thread, exchanged between the threads of a particle: FP32C all nine,
+  // FP64 in two halves (an odd stride keeps the rows on different banks)
+  static constexpr int TERM_BYTES = G == 1 ? 0 : TILE * (F32 ? 9 * (int)sizeof(float) : 7 * (int)sizeof(double));
+  float4 piece[PIECES][CAP + 1];
+  double X[ALL_IN_LDS ? 1 : CAP];
+  int tag[CAP];
+  int flags;               // of all the candidates, and PATCH_DENSE
+  int table[PATCH_TABLE];  // LDS index of the first candidate of each cell (row-major in a column)
+  int col_first[PATCH_COLS + 1];  // of each staged column
+  int col_shift[PATCH_COLS];      // LDS index minus sorted index in each staged column
+  int own_first[PATCH_COLS + 1];  // number of the first particle of each own column
+  unsigned char list[G == 1 ? 1 : TILE / G][64];  // the pairs of a particle, as LDS indices
+  alignas(16) char terms[TERM_BYTES ? TERM_BYTES : 16];
+};
+
+// a column range of some window of the patch holds more candidates than a mask of sums_lds has bits
+constexpr int PATCH_DENSE = 16;
+
+// where a sum reads the window candidates from: a patch's copy in LDS (index: place in the copy)
+template <bool F32, int G>
+struct lds_source {
+  using mem = patch_mem<F32, G>;
+  const mem *m;
+  const double *rec;
+  double h0;
+  bool t_in_lds;  // what mem::X holds: T (some particle conducts heat), else c
+  __device__ inline double2 pos(int j) const { return reinterpret_cast<const double2 *>(m->piece[0])[j]; }
+  __device__ inline int tag(int j) const { return m->tag[j]; }
+  __device__ inline void cand(int j, double2 &p, int &t) const {
+    p = pos(j);
+    t = tag(j);
+  }
+  __device__ inline void heat(int j, int t, rec_t<F32> &q) const {  // T and rho
+    if constexpr (F32) {
+      q.rho = m->piece[1][j].z; q.T = m->piece[3][j].w;
+    } else {
+      q.rho = reinterpret_cast<const double2 *>(m->piece[2])[j].x;
+      if constexpr (mem::ALL_IN_LDS) q.T = reinterpret_cast<const double2 *>(m->piece[6])[j].y;
+      else q.T = t_in_lds ? m->X[j] : rec[(size_t)REC * tag_index(t) + 15];
+    }
+  }
+  __device__ inline void record(int j, rec_t<F32> &q) const {
+    if constexpr (F32) {
+      const float4 a = m->piece[1][j], b = m->piece[2][j], c = m->piece[3][j];
+      q.u = a.x; q.v = a.y; q.rho = a.z; q.vol = a.w;
+      q.Axx = b.x; q.Axy = b.y; q.Ayy = b.z; q.c = b.w;
+      q.Rxx = c.x; q.Rxy = c.y; q.Ryy = c.z; q.T = c.w;
+      q.h = (float)h0;
+    } else {
+      if constexpr (mem::ALL_IN_LDS) {
+        const double2 f = reinterpret_cast<const double2 *>(m->piece[6])[j];
+        q.c = f.x; q.T = f.y;
+      } else if (t_in_lds) {
+        q.c = rec[(size_t)REC * tag_index(m->tag[j]) + 14];
+        q.T = m->X[j];
+      } else {
+        q.c = m->X[j];
+        q.T = 0.;  // not read
+      }
+      const double2 a = reinterpret_cast<const double2 *>(m->piece[1])[j];
+      const double2 b = reinterpret_cast<const double2 *>(m->piece[2])[j];
+      const double2 c = reinterpret_cast<const double2 *>(m->piece[3])[j];
+      const double2 d = reinterpret_cast<const double2 *>(m->piece[4])[j];
+      const double2 e = reinterpret_cast<const double2 *>(m->piece[5])[j];
+      q.u = a.x; q.v = a.y; q.rho = b.x; q.vol = b.y;
+      q.Axx = c.x; q.Axy = c.y; q.Ayy = d.x; q.Rxx = d.y; q.Rxy = e.x; q.Ryy = e.y;
+      q.h = h0;
+    }
+  }
+};
+
+// or the records in memory through the sort permutation (index: sorted index)
+template <bool F32>
+struct mem_source {
+  const drecords &r;
+  const int *perm;
+  const double *h;  // the start state's
+  __device__ inline void cand(int j, double2 &p, int &tag) const {
+    const int s = perm[j];
+    if constexpr (F32) p = *reinterpret_cast<const double2 *>(r.rec32 + (size_t)REC32_PIECES * s);
+    else p = *reinterpret_cast<const double2 *>(r.rec + (size_t)REC * s);
+    tag = make_tag(s, r.vfl[s]);
+  }
+  __device__ inline void heat(int j, int tag, rec_t<F32> &q) const {
+    if constexpr (F32) {
+      const float4 *d = r.rec32 + (size_t)REC32_PIECES * tag_index(tag);
+      q.rho = d[1].z; q.T = d[3].w;
+    } else {
+      const double *d = r.rec + (size_t)REC * tag_index(tag);
+      q.rho = d[6]; q.T = d[15];
+    }
+  }
+  __device__ inline void record(int j, int tag, rec_t<F32> &q) const {
+    if constexpr (F32) {
+      const float4 *d = r.rec32 + (size_t)REC32_PIECES * tag_index(tag);
+      const float4 a = d[1], b = d[2], c = d[3];
+      q.u = a.x; q.v = a.y; q.rho = a.z; q.vol = a.w;
+      q.Axx = b.x; q.Axy = b.y; q.Ayy = b.z; q.c = b.w;
+      q.Rxx = c.x; q.Rxy = c.y; q.Ryy = c.z; q.T = c.w;
+      q.h = (float)h[tag_index(tag)];
+    } else {
+      const double *d = r.rec + (size_t)REC * tag_index(tag);
+      q.h = d[3]; q.u = d[4]; q.v = d[5]; q.rho = d[6]; q.vol = d[7];
+      q.Axx = d[8]; q.Axy = d[9]; q.Ayy = d[10]; q.Rxx = d[11]; q.Rxy = d[12]; q.Ryy = d[13];
+      q.c = d[14]; q.T = d[15];
+    }
+  }
+};
+
+// what a particle's sums need of itself beside its record
+struct sum_flags {
+  bool tool, nonfinite, run_mech, run_pse;
+  double ta;
+};
+
+// e^x with the operations of mfcm::exp, without its special cases for x in (-700, 0]
+__device__ inline double exp_neg(double x) {
+  if (!(x > -700. && x <= 0.)) return mfcm::exp(x);
+  const double kd = floor(x * mfcm::INV_LN2 + 0.5);
+  const double r = (x - kd * mfcm::LN2_HI) - kd * mfcm::LN2_LO;
+  return __builtin_ldexp(mfcm::exp_reduced(r), (int)kd);  // 2^k is exact
+}
+
+// FP64 sums of a particle: the support test and PSE term of a window candidate, and the terms of
+// a pair
+struct math64 {
+  using rec = rec64;
+  static constexpr int TERMS = 13;
+  const dev_consts &k;
+  const rec64 &a;
+  const sum_flags &f;
+  double h1, fourh2, fac, h2, inv_h2, pse_c, inv_wd;
+  __device__ inline math64(const dev_consts &k_, const rec64 &a_, const sum_flags &f_) : k(k_), a(a_), f(f_) {
+    h1 = 1 / a.h;
+    fourh2 = 4 * a.h * a.h;
+    fac = PI_FAC * h1 * h1;
+    h2 = a.h * a.h;
+    const double h4 = h2 * h2;
+    pse_c = 4. / (h4 * M_PI);
+    inv_h2 = 1. / h2;
+    inv_wd = 1. / k.wdeltap;
+  }
+  // outside the support the reference adds exact zeros, unless a value is non-finite
+  __device__ inline bool near(double2 p) const {
+    const double dx = a.x - p.x, dy = a.y - p.y;
+    const double rr2 = dx * dx + dy * dy;
+    return !(rr2 >= fourh2 || rr2 < 1e-8);
+  }
+  __device__ inline bool support(double2 p, int tag) const {
+    return !(tag & MFC_FLAG_BLANKED) && (near(p) || f.nonfinite || (tag & FLAG_NONFINITE));
+  }
+  template <bool FINITE>
+  __device__ inline double pse(double2 p, const rec64 &b) const {  // do_interactions_heat_pse (interactions_gpu.cu:130-139)
+    const double dx = a.x - p.x, dy = a.y - p.y;
+    const double xx = sqrt(dx * dx + dy * dy);
+    const double w2 = pse_c * (FINITE ? exp_neg(div_by(-xx * xx, h2, inv_h2)) : mfcm::exp(-xx * xx / (h2)));
+    return (b.T - a.T) * w2 * k.mass / b.rho;
+  }
+  template <bool FINITE>
+  __device__ inline pair_acc pair(double2 p, bool tool_j, rec64 &b) const {
+    b.x = p.x; b.y = p.y;
+    return pair_terms<FINITE>(k, a, f.tool, f.ta, h1, fourh2, fac, inv_wd, b, tool_j);
+  }
+};
+
+// FP32C sums with Kahan compensation (the same pair terms, rearranged for single precision:
+// hardware reciprocals and reciprocal square roots instead of divisions, the particle mass and
+// the factor 2 of Brookshaw taken out of the sums, e.gradW/r of Brookshaw written as der*fac,
+// which is its exact value, and the stress and viscosity terms of each acceleration component
+// added before their one compensated sum). Pair distances are formed in FP64 and then rounded.
+struct terms32 {
+  float vd0, vd1, vd2, vd3, ax, ay, xt0, xt1, tl;
+  bool mech;  // the first eight are added to the sums (tl when ta != 0)
+  __device__ inline void add_mech(float a0, float a1, float a2, float a3, float a4, float a5, float a6, float a7) {
+    vd0 = a0; vd1 = a1; vd2 = a2; vd3 = a3; ax = a4; ay = a5; xt0 = a6; xt1 = a7;
+    mech = true;
+  }
+  __device__ inline void add_heat(float t) { tl = t; }
+};
+// the sums themselves, by one thread
+struct sums32 {
+  kahan s[9];
+  __device__ inline void add_mech(float a0, float a1, float a2, float a3, float a4, float a5, float a6, float a7) {
+    s[0].add(a0); s[1].add(a1); s[2].add(a2); s[3].add(a3); s[4].add(a4); s[5].add(a5); s[6].add(a6); s[7].add(a7);
+  }
+  __device__ inline void add_heat(float t) { s[8].add(t); }
+};
+struct math32 {
+  using rec = rec32;
+  const dev_consts &k;
+  const rec32 &a;
+  const sum_flags &f;
+  float ta, Ti, h1, fourh2, fac, inv_wd, eta2, alpha, beta, xeps, inv_h2, pse_c, massf;
+  __device__ inline math32(const dev_consts &k_, const rec32 &a_, const sum_flags &f_) : k(k_), a(a_), f(f_) {
+    ta = (float)f.ta;
+    Ti = ta != 0.0f ? a.T : 0.0f;
+    h1 = 1.0f / a.h;
+    fourh2 = 4.0f * a.h * a.h;
+    fac = (float)PI_FAC * h1 * h1;
+    inv_wd = (float)(1.0 / k.wdeltap);
+    eta2 = (float)(k.av_eta * k.av_eta);
+    alpha = (float)k.av_alpha; beta = (float)k.av_beta; xeps = (float)k.xsph_eps;
+    inv_h2 = h1 * h1;
+    pse_c = (float)(4. / M_PI) * inv_h2 * inv_h2;
+    massf = (float)k.mass;
+  }
+  __device__ inline void distance(double2 p, float &dx, float &dy, float &rr2) const {
+    dx = (float)(a.x - p.x);
+    dy = (float)(a.y - p.y);
+    rr2 = __builtin_fmaf(dx, dx, dy * dy);
+  }
+  __device__ inline bool near(double2 p) const {
+    float dx, dy, rr2;
+    distance(p, dx, dy, rr2);
+    return !(rr2 >= fourh2 || rr2 < 1e-8f);
+  }
+  __device__ inline bool support(double2 p, int tag) const { return near(p) && !(tag & MFC_FLAG_BLANKED); }
+  template <bool>
+  __device__ inline float pse(double2 p, const rec32 &b) const {
+    float dx, dy, rr2;
+    distance(p, dx, dy, rr2);
+    const float w2 = pse_c * __expf(-rr2 * inv_h2);
+    return (b.T - a.T) * w2 * (massf * __builtin_amdgcn_rcpf(b.rho));
+  }
+  template <class SINK>
+  __device__ inline void pair(double2 p, bool tool_j, const rec32 &b, SINK &sink) const {
+    float dx, dy, rr2;
+    distance(p, dx, dy, rr2);
     const float inv_r = __builtin_amdgcn_rsqf(rr2);
     const float q = rr2 * inv_r * h1;
     float val, der;  // der = dW/dr / r without the factor fac
@@ -456,134 +810,292 @@ __device__ inline void sums_f32(const dev_consts &k, int i, const double2 *__res
     }
     const float w = val * fac, gr = der * fac;
     const float w_x = gr * dx, w_y = gr * dy;
-    if (!tool && !(fj & MFC_FLAG_TOOL)) {
-      const float tx = w_x * volj, ty = w_y * volj;
-      const float du = uj - ui, dv = vj - vi_;
-      vd0.add(du * tx); vd1.add(du * ty); vd2.add(dv * tx); vd3.add(dv * ty);
+    if (!f.tool && !tool_j) {
+      const float tx = w_x * b.vol, ty = w_y * b.vol;
+      const float du = b.u - a.u, dv = b.v - a.v;
       float fab = w * inv_wd;
       fab *= fab;
       fab *= fab;
-      const float sx = Axx_i + b1.y + fab * (Rxx_i + b2.x);
-      const float sy = Axy_i + b1.z + fab * (Rxy_i + b2.y);
-      const float sz = Ayy_i + b1.w + fab * (Ryy_i + b2.z);
+      const float sx = a.Axx + b.Axx + fab * (a.Rxx + b.Rxx);
+      const float sy = a.Axy + b.Axy + fab * (a.Rxy + b.Rxy);
+      const float sz = a.Ayy + b.Ayy + fab * (a.Ryy + b.Ryy);
       float fx = __builtin_fmaf(sx, w_x, sy * w_y), fy = __builtin_fmaf(sy, w_x, sz * w_y);
       const float vijx = -du, vijy = -dv;
       const float vdx = __builtin_fmaf(vijx, dx, vijy * dy);
-      const float inv_rhoij = 2.0f * __builtin_amdgcn_rcpf(rhoi + rhoj);
+      const float inv_rhoij = 2.0f * __builtin_amdgcn_rcpf(a.rho + b.rho);
       if (vdx < 0.0f) {
-        const float cij = 0.5f * (ci + b2.w);
-        const float hij = 0.5f * (hi + hj_);
+        const float cij = 0.5f * (a.c + b.c);
+        const float hij = 0.5f * (a.h + b.h);
         const float muij = hij * vdx * __builtin_amdgcn_rcpf(__builtin_fmaf(eta2 * hij, hij, rr2));
         const float piij = (-alpha * cij * muij + beta * muij * muij) * inv_rhoij;
         fx = __builtin_fmaf(-piij, w_x, fx);
         fy = __builtin_fmaf(-piij, w_y, fy);
       }
-      ax.add(fx); ay.add(fy);
       const float xs = -xeps * w * inv_rhoij;
-      xt0.add(xs * vijx); xt1.add(xs * vijy);
+      sink.add_mech(du * tx, du * ty, dv * tx, dv * ty, fx, fy, xs * vijx, xs * vijy);
     }
-    if (ta != 0.0f) tl.add(volj * (Ti - b3.x) * gr);
-  };
-  // what the walk loads per candidate ahead of its evaluation: FP64 position and flags (the
-  // temperature and density for PSE are read when the candidate is evaluated)
-  struct cand {
+    if (ta != 0.0f) sink.add_heat(b.vol * (Ti - b.T) * gr);
+  }
+};
+template <bool F32>
+using math_t = std::conditional_t<F32, math32, math64>;
+
+// the sums as update_particle takes them, from the FP32C sums s (in the order of terms32; the
+// stress and viscosity sums enter the acceleration only as sd0 + sd1 + vt0 and sd2 + sd3 + vt1
+// (actions_gpu.cu momentum), so they are accumulated as those two)
+__device__ inline pair_acc acc_of_sums32(const dev_consts &k, const double *s) {
+  return {s[0], s[1], s[2], s[3], k.mass * s[4], 0., k.mass * s[5], 0., 0., 0., k.mass * s[6], k.mass * s[7], 2.0 * s[8]};
+}
+
+__device__ inline void add_terms(pair_acc &acc, const pair_acc &t) {
+  acc.vd0 += t.vd0; acc.vd1 += t.vd1; acc.vd2 += t.vd2; acc.vd3 += t.vd3;
+  acc.sd0 += t.sd0; acc.sd1 += t.sd1; acc.sd2 += t.sd2; acc.sd3 += t.sd3;
+  acc.vt0 += t.vt0; acc.vt1 += t.vt1; acc.xt0 += t.xt0; acc.xt1 += t.xt1;
+  acc.tl += t.tl;
+}
+__device__ inline pair_acc acc_of(const dev_consts &k, const sums32 &q) {
+  double s[9];
+#pragma unroll
+  for (int c = 0; c < 9; c++) s[c] = q.s[c].value();
+  return acc_of_sums32(k, s);
+}
+__device__ inline double value_of(const kahan &s) { return s.value(); }
+__device__ inline double value_of(double s) { return s; }
+
+// The neighbour sums of a particle by one thread from the records in memory: the window's
+// candidates in order, which is the reference's (interactions_gpu.cu:219-331)
+template <bool F32>
+__device__ inline void sums_mem(const dev_consts &k, const mem_source<F32> &src, const window &w, const rec_t<F32> &a,
+                                const sum_flags &f, pair_acc &acc, double &tpse) {
+  const math_t<F32> mt(k, a, f);
+  std::conditional_t<F32, sums32, pair_acc> sum = {};
+  std::conditional_t<F32, kahan, double> tp = {};
+  for (int t = 0; t < w.total; t++) {
+    const int j = w.at(t);
     double2 p;
-    int f;
-  };
-  auto load = [&](int j, cand &c) {
-    c.p = cs.pos[j - cs.base];
-    c.f = cs.fl[j - cs.base];
-  };
-  // the PSE term of every window member, and the support test; true: j is a mechanical pair
-  auto visit = [&](int j, const cand &c, float &dx, float &dy, float &rr2) -> bool {
-    dx = (float)(pi.x - c.p.x);
-    dy = (float)(pi.y - c.p.y);
-    rr2 = __builtin_fmaf(dx, dx, dy * dy);
-    if (run_pse) {
-      const float Tj = rec32[(size_t)16 * j + 12], rhoj = rec32[(size_t)16 * j + 3];
-      const float w2 = pse_c * __expf(-rr2 * inv_h2);
-      tp.add((Tj - Tpred) * w2 * (massf * __builtin_amdgcn_rcpf(rhoj)));
+    int tag;
+    rec_t<F32> b;
+    src.cand(j, p, tag);
+    if (f.run_pse) {  // all members of the window
+      src.heat(j, tag, b);
+      if constexpr (F32) tp.add(mt.template pse<false>(p, b));
+      else tp += mt.template pse<false>(p, b);
     }
-    if (!run_mech) return false;
-    if (rr2 >= fourh2 || rr2 < 1e-8f) return false;
-    return !(c.f & MFC_FLAG_BLANKED);
-  };
-  // the window in groups of candidates, the loads of a group issued before its first candidate
-  // is evaluated; the order of evaluation is the candidates' order
-  if constexpr (!COMPACT) {
-    // direct walk: the support tests of a group come first, then the records of the group's
-    // in-support candidates are loaded together, then their pairs are evaluated in order
-    for (int t0 = 0; t0 < w.total; t0 += WALK_U32) {
-      int j[WALK_U32];
-      cand c[WALK_U32];
-      bool in[WALK_U32];
-      float dx[WALK_U32], dy[WALK_U32], rr2[WALK_U32];
-      rec4 r[WALK_U32];
-#pragma unroll
-      for (int u = 0; u < WALK_U32; u++) {
-        j[u] = w.at(t0 + u < w.total ? t0 + u : w.total - 1);
-        load(j[u], c[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < WALK_U32; u++) in[u] = t0 + u < w.total && visit(j[u], c[u], dx[u], dy[u], rr2[u]);
-#pragma unroll
-      for (int u = 0; u < WALK_U32; u++)
-        if (in[u]) load_rec(j[u], r[u]);
-#pragma unroll
-      for (int u = 0; u < WALK_U32; u++)
-        if (in[u]) pair(dx[u], dy[u], rr2[u], r[u]);
-    }
-  } else {
-    // masked walk: the support tests of up to 64 candidates set the bits of a per-lane mask,
-    // then the candidates of the set bits are evaluated in candidate order, the loads of the
-    // next one issued before the current one is evaluated. The wave runs the pair body about as
-    // often as its busiest lane has pairs instead of once per window candidate, with no list in
-    // memory (the sorted index of a bit is recomputed by window::at).
-    for (int c0 = 0; c0 < w.total; c0 += 64) {
-      const int n = w.total - c0 < 64 ? w.total - c0 : 64;
-      unsigned long long m = 0ull;
-      for (int u0 = 0; u0 < n; u0 += WALK_U) {
-        int j[WALK_U];
-        cand c[WALK_U];
-#pragma unroll
-        for (int u = 0; u < WALK_U; u++) {
-          j[u] = w.at(c0 + (u0 + u < n ? u0 + u : n - 1));
-          load(j[u], c[u]);
+    if (!f.run_mech || !mt.support(p, tag)) continue;
+    src.record(j, tag, b);
+    if constexpr (F32) mt.pair(p, (tag & MFC_FLAG_TOOL) != 0, b, sum);
+    else add_terms(sum, mt.template pair<false>(p, (tag & MFC_FLAG_TOOL) != 0, b));
+  }
+  if constexpr (F32) acc = acc_of(k, sum);
+  else acc = sum;
+  tpse = value_of(tp);
+}
+
+// The same by one thread from a patch's LDS copy, the window as 5 column ranges [b, e) of it. First
+// the support tests of every candidate set the bits of a mask per column, then the pairs of the
+// set bits are evaluated in order: the wave runs the pair body about as often as its busiest lane
+// has pairs instead of once per candidate. The test loops run column by column (about 80 rounds of
+// a wave for windows of 56 candidates, whose columns hold 8 or 16 by turns), because a candidate
+// numbered through the columns costs 11 instructions to find and one of a column none; in the
+// loop over the pairs a lane moves its next column's mask up when its current one is used up.
+// flags: what the patch's candidates have of TOOL and BLANKED (without PSE, the copy holds blanked
+// particles at infinity).
+constexpr int WALK_U = 4;  // candidates whose loads are issued together
+template <bool F32, int G, bool PSE>
+__device__ inline void sums_lds(const dev_consts &k, const lds_source<F32, G> &src, int flags, const int b[5],
+                                const int e[5], const rec_t<F32> &a, const sum_flags &f, pair_acc &acc, double &tpse) {
+  const math_t<F32> mt(k, a, f);
+  std::conditional_t<F32, sums32, pair_acc> sum = {};
+  std::conditional_t<F32, kahan, double> tp = {};
+  if constexpr (PSE) {
+    if (f.run_pse) {  // all members of the window, two at a time
+      const window w = window_of(b, e);
+      for (int t = 0; t < w.total; t += 2) {
+        const bool two = t + 1 < w.total;
+        const int j0 = w.at(t), j1 = w.at(two ? t + 1 : t);
+        rec_t<F32> c0, c1;
+        src.heat(j0, src.tag(j0), c0);
+        src.heat(j1, src.tag(j1), c1);
+        const auto v0 = mt.template pse<true>(src.pos(j0), c0), v1 = mt.template pse<true>(src.pos(j1), c1);
+        if constexpr (F32) {
+          tp.add(v0);
+          if (two) tp.add(v1);
+        } else {
+          tp += v0;
+          if (two) tp += v1;
         }
-#pragma unroll
-        for (int u = 0; u < WALK_U; u++) {
-          float dx, dy, rr2;
-          if (u0 + u < n && visit(j[u], c[u], dx, dy, rr2)) m |= 1ull << (u0 + u);
-        }
-      }
-      double2 pn;
-      rec4 rn;
-      if (m) {
-        const int jj = w.at(c0 + __builtin_ctzll(m));
-        pn = cs.pos[jj - cs.base];
-        load_rec(jj, rn);
-      }
-      while (m) {
-        m &= m - 1ull;
-        const double2 pj = pn;
-        const rec4 r = rn;
-        if (m) {
-          const int jj = w.at(c0 + __builtin_ctzll(m));
-          pn = cs.pos[jj - cs.base];
-          load_rec(jj, rn);
-        }
-        const float dx = (float)(pi.x - pj.x), dy = (float)(pi.y - pj.y);
-        pair(dx, dy, __builtin_fmaf(dx, dx, dy * dy), r);
       }
     }
   }
-  acc.vd0 = vd0.value(); acc.vd1 = vd1.value(); acc.vd2 = vd2.value(); acc.vd3 = vd3.value();
-  acc.sd0 = k.mass * ax.value(); acc.sd1 = 0.;
-  acc.sd2 = k.mass * ay.value(); acc.sd3 = 0.;
-  acc.vt0 = 0.; acc.vt1 = 0.;
-  acc.xt0 = k.mass * xt0.value(); acc.xt1 = k.mass * xt1.value();
-  acc.tl = 2.0 * tl.value();
-  tpse = tp.value();
+  unsigned m[5];
+  int at[5];
+#pragma unroll
+  for (int r = 0; r < 5; r++) {
+    const int n = f.run_mech ? e[r] - b[r] : 0;
+    unsigned mr = 0u;
+    for (int q = 0; q < n; q += WALK_U) {
+      double2 p[WALK_U];
+#pragma unroll
+      for (int u = 0; u < WALK_U; u++) p[u] = src.pos(b[r] + q + u);  // past the range: some other entry of the copy
+      unsigned hits = 0u;
+#pragma unroll
+      for (int u = 0; u < WALK_U; u++) {
+        bool hit = q + u < n;
+        if (PSE && (flags & MFC_FLAG_BLANKED)) hit = hit && !(src.tag(b[r] + q + u) & MFC_FLAG_BLANKED);
+        const bool in = mt.near(p[u]);
+        hits |= (hit & in) ? 1u << u : 0u;
+      }
+      mr |= hits << q;
+    }
+    m[r] = mr;
+    at[r] = b[r];
+  }
+#pragma unroll
+  for (int r = 3; r >= 0; r--)  // columns without a pair to the end
+    if (m[r] == 0u) {
+#pragma unroll
+      for (int q = r; q < 4; q++) { m[q] = m[q + 1]; at[q] = at[q + 1]; }
+      m[4] = 0u;
+    }
+  while (m[0]) {
+    const int j = at[0] + __builtin_ctz(m[0]);
+    m[0] &= m[0] - 1u;
+    const double2 p = src.pos(j);
+    rec_t<F32> c;
+    src.record(j, c);
+    bool tool_j = false;
+    if (flags & MFC_FLAG_TOOL) tool_j = src.tag(j) & MFC_FLAG_TOOL;  // the same branch in every lane
+    if (m[0] == 0u) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) { m[q] = m[q + 1]; at[q] = at[q + 1]; }
+      m[4] = 0u;
+    }
+    if constexpr (F32) mt.pair(p, tool_j, c, sum);
+    else add_terms(sum, mt.template pair<true>(p, tool_j, c));
+  }
+  if constexpr (F32) acc = acc_of(k, sum);
+  else acc = sum;
+  tpse = value_of(tp);
+}
+
+// LDS written by lanes of a wave and read by others of the same wave: DS operations of a wave
+// complete in order, so only the compiler has to keep theirs
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// The same sums by G neighbouring threads, for a state too small to fill the chip with one thread
+// per particle, where the length of a thread's chain of dependent operations is what a step takes.
+// The threads test G candidates at a time and list the pairs in order; then each evaluates one
+// pair, and every sum belongs to one of them, which adds the G pairs' terms in order through LDS:
+// the order of every sum, and so its bits, are sums_lds's. The sums end in out[0..ACC_N) (LDS).
+template <bool F32, int G>
+__device__ inline void sums_group(const dev_consts &k, const lds_source<F32, G> &src, const window &w,
+                                  const rec_t<F32> &a, const sum_flags &f, unsigned char *list, char *terms,
+                                  double *out) {
+  const math_t<F32> mt(k, a, f);
+  const int lane = threadIdx.x & 63, r = lane % G, g0 = lane - r;
+  constexpr int ROW = F32 ? 9 : 7;                  // terms per row
+  constexpr int PARTS = F32 ? 1 : 2;                // rows a pair's terms take, one after the other
+  constexpr int OWN = (ROW + G - 1) / G;            // sums per thread and part
+  using T = std::conditional_t<F32, float, double>;
+  T *row = reinterpret_cast<T *>(terms) + (size_t)lane * ROW;
+  const T *rows = reinterpret_cast<const T *>(terms) + (size_t)g0 * ROW;
+  std::conditional_t<F32, kahan, double> sum[PARTS][OWN] = {};
+  std::conditional_t<F32, kahan, double> tp = {};
+  for (int c0 = 0; c0 < w.total; c0 += 64) {
+    const int n = w.total - c0 < 64 ? w.total - c0 : 64;
+    int cnt = 0;
+    for (int u0 = 0; u0 < n; u0 += G) {
+      const bool in = u0 + r < n;
+      const int j = w.at(c0 + (in ? u0 + r : n - 1));
+      double2 p;
+      int tag;
+      src.cand(j, p, tag);
+      if (f.run_pse) {
+        rec_t<F32> b;
+        src.heat(j, tag, b);
+        const T v = mt.template pse<true>(p, b);
+#pragma unroll
+        for (int q = 0; q < G; q++) {
+          const T vq = __shfl(v, q, G);
+          if (u0 + q < n) {
+            if constexpr (F32) tp.add(vq);
+            else tp += vq;
+          }
+        }
+      }
+      const bool hit = f.run_mech && in && mt.support(p, tag);
+      const unsigned bits = (unsigned)(__ballot(hit) >> g0) & ((1u << G) - 1u);
+      if (hit) list[cnt + __popc(bits & ((1u << r) - 1u))] = (unsigned char)j;
+      cnt += __popc(bits);
+    }
+    wave_lds_fence();
+    for (int p0 = 0; p0 < cnt; p0 += G) {
+      const bool in = p0 + r < cnt;
+      const int j = list[in ? p0 + r : p0];
+      double2 p;
+      int tag;
+      rec_t<F32> b;
+      src.cand(j, p, tag);
+      src.record(j, b);
+      if constexpr (F32) {
+        terms32 t = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, false};
+        mt.pair(p, (tag & MFC_FLAG_TOOL) != 0, b, t);
+        row[0] = t.vd0; row[1] = t.vd1; row[2] = t.vd2; row[3] = t.vd3;
+        row[4] = t.ax; row[5] = t.ay; row[6] = t.xt0; row[7] = t.xt1; row[8] = t.tl;
+        const unsigned mech = (unsigned)(__ballot(in && t.mech) >> g0);
+        wave_lds_fence();
+#pragma unroll
+        for (int q = 0; q < G; q++) {
+#pragma unroll
+          for (int o = 0; o < OWN; o++) {
+            const int c = r + G * o;
+            const float v = rows[q * ROW + (c < ROW ? c : 0)];
+            if (c < 8 ? (mech >> q) & 1u : p0 + q < cnt && mt.ta != 0.0f) sum[0][o].add(v);
+          }
+        }
+        wave_lds_fence();
+      } else {
+        const pair_acc t = mt.template pair<true>(p, (tag & MFC_FLAG_TOOL) != 0, b);
+        const double tv[14] = {t.vd0, t.vd1, t.vd2, t.vd3, t.sd0, t.sd1, t.sd2,
+                               t.sd3, t.vt0, t.vt1, t.xt0, t.xt1, t.tl, 0.};
+#pragma unroll
+        for (int h = 0; h < PARTS; h++) {
+#pragma unroll
+          for (int c = 0; c < ROW; c++) row[c] = tv[h * ROW + c];
+          wave_lds_fence();
+#pragma unroll
+          for (int q = 0; q < G; q++) {
+#pragma unroll
+            for (int o = 0; o < OWN; o++) {
+              const int c = r + G * o;
+              const double v = rows[q * ROW + (c < ROW ? c : 0)];
+              if (p0 + q < cnt) sum[h][o] += v;
+            }
+          }
+          wave_lds_fence();
+        }
+      }
+    }
+  }
+  wave_lds_fence();
+#pragma unroll
+  for (int h = 0; h < PARTS; h++)
+#pragma unroll
+    for (int o = 0; o < OWN; o++) {
+      const int c = r + G * o;
+      if constexpr (F32) {
+        if (c < ROW) out[c] = sum[h][o].value();
+      } else {
+        if (c < ROW && h * ROW + c < ACC_N - 1) out[h * ROW + c] = sum[h][o];
+      }
+    }
+  if (r == 0) {
+    if constexpr (F32) out[ACC_N - 1] = tp.value();
+    else out[ACC_N - 1] = tp;
+  }
 }
 
 // a particle's Johnson-Cook return, left for the whole wave's secant after update_particle: the
@@ -600,10 +1112,12 @@ struct deferred_return {
 // returns the particle's fc and ft for the tool force. The secant of a Johnson-Cook return runs
 // for the whole wave after this call (finish_return); the other results do not depend on it
 // reads particle s of the unsorted start state src (s = perm[i]) and writes the updated
-// particle to position i of dst: the gather into sorted order happens here, once
+// particle to position i of dst: the gather into sorted order happens here, once. Also writes the
+// step's positional values and, with the state before a return, the next step's record (rn)
+template <bool F32>
 __device__ inline void update_particle(const dev_consts &k, int i, int s, const pair_acc &acc, double tpse,
                                        const dstate &src, const dstate &dst, const dpositional &pos,
-                                       const mfc_tool_state &tool_now, double fsum[4], double &x_out, double &y_out,
+                                       const drecords &r, const drecords &rn, const mfc_tool_state &tool_now, double fsum[4], double &x_out, double &y_out,
                                        int &fl_out, deferred_return &dr) {
   const bool pse = k.pse != 0;
   int fl = src.flags[s] & FLAG_MASK;
@@ -630,6 +1144,8 @@ __device__ inline void update_particle(const dev_consts &k, int i, int s, const 
     psxx = sxx0 + hdt * stxx; psxy = sxy0 + hdt * stxy; psyy = syy0 + hdt * styy; pszz = szz0 + hdt * stzz;
     prho = rho0 + hdt * rhot;
   }
+  const double p = k.c0 * k.c0 * (prho - k.rho0);  // EOS of the predicted density
+  if (!tool) store_positional<F32>(pos, i, s, p, r);
   // interaction outputs (interactions_gpu.cu:334-344, :143)
   if (run_mech) {
     ptx = acc.xt0; pty = acc.xt1; vtx = acc.vt0; vty = acc.vt1;
@@ -671,7 +1187,7 @@ __device__ inline void update_particle(const dev_consts &k, int i, int s, const 
     }
   }
   if (!tool && k.plastic) {
-    dr.need = plasticity_test(k, pos.p[i], sxx, sxy, syy, szz, eps, epsd, T, dr.in);
+    dr.need = plasticity_test(k, p, sxx, sxy, syy, szz, eps, epsd, T, dr.in);
     if (dr.need) {
       dr.fixed = fixed;
       dr.rho = rho; dr.sxx = sxx; dr.sxy = sxy; dr.syy = syy; dr.szz = szz;
@@ -698,7 +1214,8 @@ __device__ inline void update_particle(const dev_consts &k, int i, int s, const 
   }
   dst.px[i] = x; dst.py[i] = y; dst.vx[i] = u; dst.vy[i] = v;
   dst.sxx[i] = sxx; dst.sxy[i] = sxy; dst.syy[i] = syy; dst.szz[i] = szz;
-  dst.rho[i] = rho; dst.T[i] = T; dst.eps[i] = eps; dst.epsd[i] = epsd; dst.h[i] = src.h[s];
+  const double h = src.h[s];
+  dst.rho[i] = rho; dst.T[i] = T; dst.eps[i] = eps; dst.epsd[i] = epsd; dst.h[i] = h;
   dst.fcx[i] = fcx; dst.fcy[i] = fcy; dst.ftx[i] = ftx; dst.fty[i] = fty;
   dst.ptx[i] = ptx; dst.pty[i] = pty; dst.vtx[i] = vtx; dst.vty[i] = vty;
   dst.rhot[i] = rhot; dst.stxx[i] = stxx; dst.stxy[i] = stxy; dst.styy[i] = styy; dst.stzz[i] = stzz;
@@ -707,220 +1224,317 @@ __device__ inline void update_particle(const dev_consts &k, int i, int s, const 
   dst.id[i] = src.id[s];
   fsum[0] = fcx; fsum[1] = fcy; fsum[2] = ftx; fsum[3] = fty;
   x_out = x; y_out = y; fl_out = fl;
+  write_record<F32>(k, {x, y, u, v, sxx, sxy, syy, rho, T, h, ptx, pty, vtx, vty, rhot, stxx, stxy, styy, Tt, fl}, i,
+                    rn);
 }
 
 // the return of a particle that needed one, with the secant's dl: the stress, plastic strain and
 // rate and temperature at sorted index i (the thermal boundary condition after the return, as in
-// update_particle)
-__device__ inline void finish_return(const dev_consts &k, int i, double dl, deferred_return &dr, const dstate &dst) {
+// update_particle), and its record again with them
+template <bool F32>
+__device__ inline void finish_return(const dev_consts &k, int i, double dl, deferred_return &dr, const dstate &dst,
+                                     const drecords &rn) {
   plasticity_finish(k, dr.rho, dl, dr.in, dr.sxx, dr.sxy, dr.syy, dr.szz, dr.eps, dr.epsd, dr.T);
   if (k.thermal_bc && dr.fixed) dr.T = k.T_init;  // actions_gpu.cu:287-294
   dst.sxx[i] = dr.sxx; dst.sxy[i] = dr.sxy; dst.syy[i] = dr.syy; dst.szz[i] = dr.szz;
   dst.eps[i] = dr.eps; dst.epsd[i] = dr.epsd; dst.T[i] = dr.T;
+  // the other fields as update_particle stored them: few particles return, so reading them back
+  // costs less than keeping them in registers through the secant
+  rec_input q = load_rec_input(dst, i);
+  q.sxx = dr.sxx; q.sxy = dr.sxy; q.syy = dr.syy; q.T = dr.T;
+  write_record<F32>(k, q, i, rn);
 }
 
 // the deferred returns of the wave (all 64 lanes together); dl_out (the reverse mode's replay,
 // the same in every thread): each particle's secant result, -dl where its last update folded,
 // 0 for no return. F32: the FP32C path's secant (rr_secant_wave<true>)
 template <bool F32>
-__device__ inline void wave_returns(const dev_consts &k, int i, deferred_return &dr, const dstate &dst,
-                                    double *__restrict__ dl_out) {
+__device__ inline void wave_returns(const dev_consts &k, int i, bool live, deferred_return &dr, const dstate &dst,
+                                    const drecords &rn, double *__restrict__ dl_out) {
   bool folded;
   const double dl = rr_secant_wave<F32>(k, dr.need, dr.in, dr.eps, dr.T, folded);
-  if (dr.need) finish_return(k, i, dl, dr, dst);
-  if (dl_out && i < k.N) dl_out[i] = dr.need ? (folded ? -dl : dl) : 0.;
-}
-
-// the neighbour sums of particle i as pair_acc + PSE sum
-template <bool F32, bool COMPACT>
-__device__ inline void particle_sums(const dev_consts &k, int i, const double *__restrict__ rec,
-                                     const double2 *__restrict__ posd, const float *__restrict__ rec32,
-                                     const int *__restrict__ key_sorted, const int *__restrict__ offsets,
-                                     const cand_src &cs, int fl, pair_acc &acc, double &tpse) {
-  const bool pse = k.pse != 0;
-  const bool blank = fl & MFC_FLAG_BLANKED, tool = fl & MFC_FLAG_TOOL;
-  const double ta = pse ? 0. : (tool ? k.alpha_tool : k.alpha_wp);
-  const bool run_mech = !blank && (!pse || !tool);
-  const bool run_pse = !blank && pse && k.thermal_wp;
-  acc = {0., 0., 0., 0., 0., 0., 0., 0., 0., 0., 0., 0., 0.};
-  tpse = 0.;
-  if (run_mech || run_pse) {
-    if constexpr (F32)
-      sums_f32<COMPACT>(k, i, posd, rec32, key_sorted, offsets, cs, tool, ta, run_mech, run_pse, acc, tpse);
-    else
-      sums_f64<COMPACT>(k, i, rec, key_sorted, offsets, cs, tool, ta, run_mech, run_pse, acc, tpse);
-  }
-}
-
-// partial sums of the tool force per wave of 64 particles (storage order): the halving-stride
-// tree over the wave's lanes (lane k adds lane k + st for st = 32, 16, ..., 1, so lane 0 ends with
-// the tree's root), then lane 0 writes the wave's four sums at partials[4 * wave]. Every lane of
-// the wave calls it (lanes past N carry zeros).
-__device__ inline void force_partials(int wave, const double fsum[4], double *__restrict__ partials) {
-  double v0 = fsum[0], v1 = fsum[1], v2 = fsum[2], v3 = fsum[3];
-#pragma unroll
-  for (int st = 32; st > 0; st >>= 1) {
-    v0 = v0 + __shfl_down(v0, st, 64);
-    v1 = v1 + __shfl_down(v1, st, 64);
-    v2 = v2 + __shfl_down(v2, st, 64);
-    v3 = v3 + __shfl_down(v3, st, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    partials[4 * wave + 0] = v0; partials[4 * wave + 1] = v1;
-    partials[4 * wave + 2] = v2; partials[4 * wave + 3] = v3;
-  }
-}
-
-// LDS copy of the window candidates of a tile (positions and flags), when they fit
-struct stage_buf {
-  double2 pos[STAGE_CAP];
-  int fl[STAGE_CAP];
-};
-
-// [lo, hi): the sorted indices of every window candidate of the particles of tile t. The first
-// and the last cell of a particle's window (column-major cell ids) do not decrease along the
-// sorted order, so the first particle's window start and the last particle's window end bound
-// the tile; where a window is clipped at the first or last two columns of the grid the bound
-// is the start or the end of the table instead.
-__device__ inline int2 tile_span(const dev_consts &k, int t, const int *__restrict__ key_sorted,
-                                 const int *__restrict__ offsets) {
-  const int first = t * TILE;
-  const int last = (first + TILE < k.N ? first + TILE : k.N) - 1;
-  const int hf = key_sorted[first], hl = key_sorted[last];
-  const int gif = hf / k.gny, gjf = hf - gif * k.gny;
-  const int gil = hl / k.gny, gjl = hl - gil * k.gny;
-  const int lo = gif - 2 < 0 ? 0 : offsets[(gif - 2) * k.gny + (gjf - 2 < 0 ? 0 : gjf - 2)];
-  const int hi = gil + 3 > k.gnx ? k.N : offsets[(gil + 2) * k.gny + (gjl + 3 > k.gny ? k.gny : gjl + 3)];
-  return make_int2(lo, hi);
-}
-
-// copies the tile's candidates into st when they fit (the same decision in every thread) and
-// returns the sorted index of st's first entry, or -1 when they do not fit; ends with a
-// work-group barrier
-__device__ inline int stage_tile(const dev_consts &k, int t, const drecords &r, const int *__restrict__ key_sorted,
-                                 const int *__restrict__ offsets, stage_buf &st) {
-  const int2 sp = tile_span(k, t, key_sorted, offsets);
-  const int n = sp.y - sp.x;
-  const int cap = k.stage_limit > 0 && k.stage_limit < STAGE_CAP ? k.stage_limit : STAGE_CAP;
-  int lo = -1;
-  if (n <= cap) {
-    for (int q = threadIdx.x; q < n; q += TILE) {
-      st.pos[q] = r.posd[sp.x + q];
-      st.fl[q] = r.vfl[sp.x + q];
-    }
-    lo = sp.x;
-  }
-  __syncthreads();
-  return lo;
+  if (dr.need) finish_return<F32>(k, i, dl, dr, dst, rn);
+  if (dl_out && live) dl_out[i] = dr.need ? (folded ? -dl : dl) : 0.;
 }
 
 // the next step's first binning pass for the updated particle i (its storage position in the
-// next step): cell id and arrival slot, as hash_count would take them from the updated state;
-// bin == false: the next step bins its start state itself (the bins are passed by value so that
-// they stay in registers)
-__device__ inline void next_cell(const dev_consts &k, int i, bool live, double x, double y, int fl, const dbins next,
-                                 bool bin) {
-  if (!bin) return;  // the same in every thread
+// next step): cell id, arrival slot and patch, as hash_count would take them from the updated
+// state (the bins are passed by value so that they stay in registers). An adaptive grid bins the
+// next step's start state after its geometry pass instead.
+__device__ inline void next_cell(const dev_consts &k, int i, bool live, double x, double y, int fl, const dbins next) {
+  if (k.adaptive) return;  // the same in every thread
   const int h = live ? particle_cell(k, x, y, fl, next.key_sorted[i], next.clamped) : -1;
-  count_cell(i, h, next.key, next.bsum, next.clist, next.ccap);
+  count_cell(i, h, next.key, next.bsum_next, next.clist, next.ccap);
+  count_patch(k, h, next.pcnt);
 }
 
-// fused: sums + update in one pass (registers of both live in one kernel)
-template <bool F32, bool COMPACT>
-__device__ inline void interact(const dev_consts &k, int t, const drecords &r, const int *__restrict__ key_sorted,
-                                const int *__restrict__ offsets, const int *__restrict__ perm, const dstate &src,
-                                const dstate &dst, const dpositional &pos,
-                                const mfc_tool_state *__restrict__ tool_now, const dforce &fo, const dbins next,
-                                bool bin_next, double *__restrict__ acc_out) {
-  __shared__ stage_buf st;
-  const int lo = stage_tile(k, t, r, key_sorted, offsets, st);
-  const int i = t * TILE + threadIdx.x;
-  double fsum[4] = {0., 0., 0., 0.};
-  double xn = 0., yn = 0.;
-  int fln = 0;
-  deferred_return dr;
-  dr.need = false;
-  if (i < k.N) {
-    const int s = perm[i];
-    const int fl = src.flags[s] & FLAG_MASK;
-    pair_acc acc;
-    double tpse;
-    // two call sites, so that each walk reads one kind of memory (LDS or global)
-    if (lo >= 0)
-      particle_sums<F32, COMPACT>(k, i, r.rec, r.posd, r.rec32, key_sorted, offsets, cand_src{st.pos, st.fl, lo}, fl,
-                                  acc, tpse);
-    else
-      particle_sums<F32, COMPACT>(k, i, r.rec, r.posd, r.rec32, key_sorted, offsets, cand_src{r.posd, r.vfl, 0}, fl,
-                                  acc, tpse);
-    if (acc_out) store_acc(acc_out, k.N, i, acc, tpse);  // the same in every thread
-    update_particle(k, i, s, acc, tpse, src, dst, pos, *tool_now, fsum, xn, yn, fln, dr);
-  }
-  wave_returns<F32>(k, i, dr, dst, acc_out ? acc_out + (size_t)ACC_N * k.N : nullptr);
-  next_cell(k, i, i < k.N, xn, yn, fln, next, bin_next);
-  force_partials(i >> 6, fsum, fo.partials);
-  if (t == 0 && threadIdx.x == 0) *fo.pending = 1;
+__device__ inline sum_flags flags_of(const dev_consts &k, int tag) {
+  const bool pse = k.pse != 0, blank = tag & MFC_FLAG_BLANKED, tool = tag & MFC_FLAG_TOOL;
+  sum_flags f;
+  f.tool = tool;
+  f.nonfinite = tag & FLAG_NONFINITE;
+  f.ta = pse ? 0. : (tool ? k.alpha_tool : k.alpha_wp);
+  f.run_mech = !blank && (!pse || !tool);
+  f.run_pse = !blank && pse && k.thermal_wp;
+  return f;
 }
 
-// split, first half: the neighbour sums of every particle into acc (ACC_N arrays of N doubles)
-template <bool F32, bool COMPACT>
-__device__ inline void sums(const dev_consts &k, int t, const drecords &r, const int *__restrict__ key_sorted,
-                            const int *__restrict__ offsets, const int *__restrict__ perm,
-                            const int *__restrict__ src_flags, double *__restrict__ acc) {
-  __shared__ stage_buf st;
-  const int lo = stage_tile(k, t, r, key_sorted, offsets, st);
-  const int i = t * TILE + threadIdx.x;
-  if (i >= k.N) return;
-  const int fl = src_flags[perm[i]] & FLAG_MASK;
-  pair_acc a;
-  double tpse;
-  if (lo >= 0)
-    particle_sums<F32, COMPACT>(k, i, r.rec, r.posd, r.rec32, key_sorted, offsets, cand_src{st.pos, st.fl, lo}, fl, a,
-                                tpse);
-  else
-    particle_sums<F32, COMPACT>(k, i, r.rec, r.posd, r.rec32, key_sorted, offsets, cand_src{r.posd, r.vfl, 0}, fl, a,
-                                tpse);
-  store_acc(acc, k.N, i, a, tpse);
-}
-
-// split, second half: the per-particle update from the stored sums (dl_out: as wave_returns)
+// everything that follows the sums for the particle at sorted index i (all 64 lanes of the wave;
+// live: the lane has one)
 template <bool F32>
-__device__ inline void update(const dev_consts &k, int t, const double *__restrict__ acc,
-                              const int *__restrict__ perm, const dstate &src, const dstate &dst,
-                              const dpositional &pos, const mfc_tool_state *__restrict__ tool_now, const dforce &fo,
-                              const dbins next, bool bin_next, double *__restrict__ dl_out) {
-  const int i = t * TILE + threadIdx.x;
+__device__ inline void finish_particle(const inst_args *ap, int i, bool live, const pair_acc &acc, double tpse) {
+  const inst_args &a = *ap;
+  MFC_CONST(inst_args) *c = const_args(ap, 0);
+  const dev_consts &k = a.k;
   double fsum[4] = {0., 0., 0., 0.};
   double xn = 0., yn = 0.;
   int fln = 0;
   deferred_return dr;
   dr.need = false;
-  if (i < k.N) {
-    pair_acc a;
-    double tpse;
-    load_acc(acc, k.N, i, a, tpse);
-    update_particle(k, i, perm[i], a, tpse, src, dst, pos, *tool_now, fsum, xn, yn, fln, dr);
+  double *acc_out = a.acc_out;
+  if (live) {
+    if (acc_out) store_acc(acc_out, k.N, i, acc, tpse);  // the same in every thread
+    update_particle<F32>(k, i, c->b.perm[i], acc, tpse, a.cur, a.nxt, a.pos, load_recs(&c->r), load_recs(&c->rn),
+                         *a.tool_out, fsum, xn, yn, fln, dr);
+    if (fsum[0] != 0. || fsum[1] != 0. || fsum[2] != 0. || fsum[3] != 0.) c->f.gflag[i >> 6] = 1;
   }
-  wave_returns<F32>(k, i, dr, dst, dl_out);
-  next_cell(k, i, i < k.N, xn, yn, fln, next, bin_next);
-  force_partials(i >> 6, fsum, fo.partials);
-  if (t == 0 && threadIdx.x == 0) *fo.pending = 1;
+  wave_returns<F32>(k, i, live, dr, a.nxt, load_recs(&c->rn), acc_out ? acc_out + (size_t)ACC_N * k.N : nullptr);
+  next_cell(k, i, live, xn, yn, fln, load_bins(&c->b));
 }
 
-constexpr int FF_BATCH = 8;  // wave partials a thread of force_final loads at a time
+// One patch of cells by one work-group, G threads per particle: the cell starts and the records of
+// the window candidates staged in LDS, the neighbour sums of its particles, and everything that
+// follows them in the step. Why patches: a tile of consecutive particles of the sorted order is a
+// strip along one grid column, whose windows hold about 1,500 candidates at 150k particles; the
+// 10 x 10 cells of a patch have about 440, so that whole records fit LDS and a pair reads no
+// memory (each gather of 16 bytes by 64 lanes from scattered records kept the address and data
+// path of the vector caches busy for about 50 cycles, 60-70 % of the kernel). What bounds it: with
+// one thread per particle a work-group of the 197k cut lives 42 us (FP32C; FP64 50), of which the
+// staging takes 8, the sums 17 (29), the update and the next record 13 (9) and the next binning 3;
+// its loads and stores move in a burst, since one round of work-groups fills the chip (FP32C four,
+// FP64 three to a CU). With 4 or 8 threads per particle the sums of 6k particles take 13 or 8 us
+// instead of 21 (FP64). Measured, us per step (tiles of the sorted order with candidate positions
+// in LDS and a launch for the records, then this): FP32C 6k 55 -> 29, 27k 68 -> 38, 71k 63 -> 48,
+// 197k 80 -> 60, 500k PSE 276 -> 179; FP64 6k 63 -> 32, 27k 77 -> 50, 71k 93 -> 68, 197k 137 -> 121,
+// 500k PSE 403 -> 378.
+// returns false, with nothing done, for a patch whose window candidates do not fit the stage or
+// whose state has no uniform h (interact_rest takes it)
+template <bool F32, int G, bool PSE>
+__device__ inline bool interact_patch(patch_mem<F32, G> &m, const inst_args *A, int inst, int patch, int part) {
+  const inst_args &a_ = A[inst];
+  MFC_CONST(inst_args) *c_ = const_args(&a_, 0);
+  const dev_consts &k = a_.k;
+  const drecords r = load_recs(&c_->r);
+  const int *__restrict__ offsets = k.rothlin ? c_->b.offsets_r : c_->b.offsets;
+  const int *__restrict__ perm = c_->b.perm;
+  const int *__restrict__ key_sorted = c_->b.key_sorted;
+  constexpr int SLOTS = TILE / G;  // particles at a time
+  const int tid = threadIdx.x;
+  const int nrb = patch_rows(k);
+  const int pc = patch / nrb, pr = patch - pc * nrb;
+  // own cells: rows [r0, r1), columns [g0, g1); staged: rows [s0, s1), columns [q0, q1)
+  const int r0 = pr * k.patch_s, r1 = r0 + k.patch_s < k.gny ? r0 + k.patch_s : k.gny;
+  const int g0 = pc * k.patch_w, g1 = g0 + k.patch_w < k.gnx ? g0 + k.patch_w : k.gnx;
+  const int s0 = r0 < 2 ? 0 : r0 - 2, s1 = r1 + 2 < k.gny ? r1 + 2 : k.gny;
+  const int q0 = g0 < 2 ? 0 : g0 - 2, q1 = g1 + 2 < k.gnx ? g1 + 2 : k.gnx;
+  const int ncol = q1 - q0, nrow = s1 - s0 + 1;  // cell starts per column, with the end of the last
+  const int te = tid / nrow;                     // the column of this thread's table entry
+  if (tid < ncol * nrow) m.table[tid] = offsets[(q0 + te) * k.gny + s0 + (tid - te * nrow)];
+  if (tid == 0) m.flags = 0;
+  __syncthreads();
+  if (tid < 64) {  // the first wave: where each column's candidates and own particles start
+    int first = 0, c = 0, o = 0;
+    if (tid < ncol) {
+      first = m.table[tid * nrow];
+      c = m.table[tid * nrow + nrow - 1] - first;
+      if (q0 + tid >= g0 && q0 + tid < g1) o = m.table[tid * nrow + r1 - s0] - m.table[tid * nrow + r0 - s0];
+    }
+    int xc = c, xo = o;
+#pragma unroll
+    for (int s = 1; s < 32; s <<= 1) {
+      const int yc = __shfl_up(xc, s, 64), yo = __shfl_up(xo, s, 64);
+      if (tid >= s) { xc += yc; xo += yo; }
+    }
+    if (tid <= ncol) {
+      m.col_first[tid] = xc - c;
+      m.own_first[tid] = xo - o;
+      if (tid < ncol) m.col_shift[tid] = xc - c - first;
+    }
+  }
+  __syncthreads();
+  const int ncand = m.col_first[ncol], nown = m.own_first[ncol];
+  constexpr int CAP = patch_mem<F32, G>::CAP;
+  const int cap = k.stage_limit > 0 && k.stage_limit < CAP ? k.stage_limit : CAP;
+  if (ncand > cap || !k.uniform_h) return false;  // the same in every thread
+  if (tid < ncol * nrow) {
+    const int last = (te + 1) * nrow - 1;
+    if (m.table[tid + 5 < last ? tid + 5 : last] - m.table[tid] > 32) atomicOr(&m.flags, PATCH_DENSE);
+  }
+  for (int q = tid; q < ncand; q += TILE) {
+    int c = 0;
+    for (int e = 1; e < ncol; e++) c += q >= m.col_first[e];
+    const int s = perm[q - m.col_shift[c]], fl = r.vfl[s];
+    m.tag[q] = make_tag(s, fl);
+    if (fl & ~MFC_FLAG_FIXED) atomicOr(&m.flags, fl & ~MFC_FLAG_FIXED);
+  }
+  __syncthreads();
+  const int flags = m.flags;
+  if (flags & (PATCH_DENSE | FLAG_NONFINITE)) return false;  // the same in every thread
+  const bool t_in_lds = k.alpha_wp != 0. || k.alpha_tool != 0.;
+  {
+    // the lanes take the 16-byte pieces of the records in turn, so that a load of a wave covers
+    // whole records
+    constexpr int LPR = F32 ? 4 : 8;  // lanes per record
+    const int pl = tid % LPR;
+    constexpr int STAGE_U = 4;
+    for (int q = tid / LPR; q < ncand; q += STAGE_U * (TILE / LPR)) {
+      float4 v[STAGE_U];
+#pragma unroll
+      for (int u = 0; u < STAGE_U; u++) {
+        const int c = q + u * (TILE / LPR);
+        const size_t s = tag_index(m.tag[c < ncand ? c : q]);
+        if constexpr (F32) v[u] = r.rec32[s * REC32_PIECES + pl];
+        else v[u] = reinterpret_cast<const float4 *>(r.rec)[s * (REC / 2) + pl];
+      }
+#pragma unroll
+      for (int u = 0; u < STAGE_U; u++) {
+        const int c = q + u * (TILE / LPR);
+        if (c >= ncand) break;
+        if (!PSE && (flags & MFC_FLAG_BLANKED) && pl == 0 && (m.tag[c] & MFC_FLAG_BLANKED))
+          reinterpret_cast<double2 &>(v[u]).x = __builtin_huge_val();
+        if constexpr (F32) {
+          m.piece[pl][c] = v[u];
+        } else if (pl != 1) {  // piece 1 of a record: flags (in the tag) and h (uniform)
+          const int p = pl == 0 ? 0 : pl - 1;
+          if (patch_mem<F32, G>::ALL_IN_LDS || p < 6) m.piece[p][c] = v[u];
+          else m.X[c] = t_in_lds ? reinterpret_cast<const double2 &>(v[u]).y : reinterpret_cast<const double2 &>(v[u]).x;
+        }
+      }
+    }
+    if (tid < ncol * nrow) m.table[tid] += m.col_shift[te];
+  }
+  __syncthreads();
+  // the sorted index, column and staged index of own particle number n
+  auto locate = [&](int n, int &col, int &li) -> int {
+    col = 0;
+    for (int e = 1; e < ncol; e++) col += n >= m.own_first[e];
+    li = m.table[col * nrow + r0 - s0] + (n - m.own_first[col]);
+    return li - m.col_shift[col];
+  };
+  const int base = part * SLOTS;
+  {
+    [[maybe_unused]] pair_acc acc;
+    [[maybe_unused]] double tpse = 0.;
+    const int n = base + tid / G;  // the particle whose sums this thread takes part in
+    const bool mine = n < nown;
+    [[maybe_unused]] int i_mine = 0;
+    // the exchange area of the wave; the sums of its particles end there too
+    constexpr int WAVE_BYTES = patch_mem<F32, G>::TERM_BYTES / (TILE / 64);
+    static_assert(G == 1 || WAVE_BYTES >= 64 / G * ACC_N * (int)sizeof(double), "a wave's sums fit its exchange area");
+    [[maybe_unused]] char *terms = m.terms + (size_t)(tid >> 6) * WAVE_BYTES;
+    [[maybe_unused]] double *out = reinterpret_cast<double *>(terms) + (size_t)((tid & 63) / G) * ACC_N;
+    if (mine) {
+      int col, li;
+      const int i = locate(n, col, li);
+      i_mine = i;
+      const int key = key_sorted[i];
+      double2 p;
+      int tag;
+      rec_t<F32> a;
+      const lds_source<F32, G> lds = {&m, r.rec, k.h0, t_in_lds};
+      lds.cand(li, p, tag);
+      lds.record(li, a);
+      a.x = p.x; a.y = p.y;
+      const sum_flags f = flags_of(k, tag);
+      auto at = [&](int c, int row) { return m.table[(c - q0) * nrow + row - s0]; };
+      const int gi = q0 + col, gj = key - gi * k.gny;
+      if constexpr (G == 1) {
+        int b[5], e[5];
+        window_ranges(k, gi, gj, at, b, e);
+        if (!f.run_mech && !f.run_pse)
+#pragma unroll
+          for (int q = 0; q < 5; q++) e[q] = b[q];
+        sums_lds<F32, G, PSE>(k, lds, flags, b, e, a, f, acc, tpse);
+      } else {
+        window w = make_window_at(k, gi, gj, at);
+        if (!f.run_mech && !f.run_pse) w.total = 0;
+        sums_group<F32, G>(k, lds, w, a, f, m.list[tid / G], terms, out);
+      }
+    }
+    // the update, one thread per particle: with G > 1 the first SLOTS threads
+    int i = i_mine;
+    bool live = mine;
+    if constexpr (G > 1) {
+      __syncthreads();
+      live = tid < SLOTS && base + tid < nown;
+      if (live) {
+        int col, li;
+        i = locate(base + tid, col, li);
+        // summed by wave tid / (64 / G)
+        const double *o = reinterpret_cast<const double *>(m.terms + (size_t)(tid / (64 / G)) * WAVE_BYTES) +
+                          (size_t)(tid % (64 / G)) * ACC_N;
+        if constexpr (F32) acc = acc_of_sums32(k, o);
+        else load_acc(o, 1, 0, acc, tpse);
+        tpse = o[ACC_N - 1];
+      }
+    }
+    if (G == 1 || tid < (SLOTS < 64 ? 64 : SLOTS))  // whole waves
+      finish_particle<F32>(A + inst, i, live, acc, tpse);
+  }
+  return true;
+}
 
-// tool force of the step from the wave partials, when the interaction of a step has left them
-// (pending): lane l adds the results of waves l, l + TILE, ... in ascending order, then the lane
-// sums are reduced by halving strides; F = sum(fc) + sum(ft). All threads of the work-group
-// call it.
-__device__ inline void force_final(int ntiles, const dforce &fo) {
-  if (*fo.pending == 0) return;  // the same value in every thread
-  __shared__ double red[4][TILE];
+// The patches that interact_patch leaves, and those past the end of the launch's work items: one
+// thread per particle over the records in memory. A call, so that this rare path takes no
+// registers from the kernel that holds it.
+template <bool F32>
+__device__ __attribute__((noinline)) void interact_rest(const inst_args *ap, int patch, int part) {
+  const inst_args &a_ = *ap;
+  const dev_consts &k = a_.k;
+  const dbins &b = a_.b;
+  const int *offsets = k.rothlin ? b.offsets_r : b.offsets;
+  const int nrb = patch_rows(k);
+  const int pc = patch / nrb, pr = patch - pc * nrb;
+  const int r0 = pr * k.patch_s, r1 = r0 + k.patch_s < k.gny ? r0 + k.patch_s : k.gny;
+  const int g0 = pc * k.patch_w, g1 = g0 + k.patch_w < k.gnx ? g0 + k.patch_w : k.gnx;
+  int n = (int)threadIdx.x < k.patch_slots ? part * k.patch_slots + (int)threadIdx.x : 0x7fffffff, i = -1;
+  for (int c = g0; c < g1; c++) {
+    const int first = offsets[c * k.gny + r0], count = offsets[c * k.gny + r1] - first;
+    if (i < 0 && n < count) i = first + n;
+    if (n != 0x7fffffff) n -= count;
+  }
+  const bool live = i >= 0;
+  pair_acc acc = {};
+  double tpse = 0.;
+  if (live) {
+    const mem_source<F32> mem = {a_.r, b.perm, a_.cur.h};
+    double2 p;
+    int tag;
+    rec_t<F32> a;
+    mem.cand(i, p, tag);
+    mem.record(i, tag, a);
+    a.x = p.x; a.y = p.y;
+    const sum_flags f = flags_of(k, tag);
+    window w = make_window(k, offsets, b.key_sorted[i]);
+    if (!f.run_mech && !f.run_pse) w.total = 0;
+    sums_mem<F32>(k, mem, w, a, f, acc, tpse);
+  }
+  finish_particle<F32>(ap, i, live, acc, tpse);
+}
+
+constexpr int FF_BATCH = 8;  // group sums a thread of force_final loads at a time
+
+// tool force of a step from its group sums: lane l of TILE adds the sums of the groups l,
+// l + TILE, ... in ascending order, then the lane sums are reduced by halving strides;
+// F = sum(fc) + sum(ft). The first TILE threads of the work-group do the adding, all of its
+// threads call it; red: 4 TILE doubles of LDS.
+__device__ inline void force_final(int ntiles, const dforce &fo, double (*red)[TILE]) {
   double a0 = 0., a1 = 0., a2 = 0., a3 = 0.;
-  // each thread adds the wave partials q = threadIdx.x, + TILE, + 2 TILE, ... in that order (4
-  // per tile), eight loads in flight at a time: this work-group is the first of the step's
-  // predict launch, and one load at a time made it that launch's last
+  // each thread adds the group sums q = threadIdx.x, + TILE, + 2 TILE, ... in that order (4
+  // per tile), eight loads in flight at a time: one load at a time made this work-group the last
+  // of its launch
   const double4 *__restrict__ p4 = reinterpret_cast<const double4 *>(fo.partials);
-  const int nq = 4 * ntiles;
+  const int nq = threadIdx.x < TILE ? 4 * ntiles : 0;
   for (int q0 = threadIdx.x; q0 < nq; q0 += TILE * FF_BATCH) {
     double4 v[FF_BATCH];
 #pragma unroll
@@ -931,8 +1545,10 @@ __device__ inline void force_final(int ntiles, const dforce &fo) {
         a0 = a0 + v[u].x; a1 = a1 + v[u].y; a2 = a2 + v[u].z; a3 = a3 + v[u].w;
       }
   }
-  red[0][threadIdx.x] = a0; red[1][threadIdx.x] = a1;
-  red[2][threadIdx.x] = a2; red[3][threadIdx.x] = a3;
+  if (threadIdx.x < TILE) {
+    red[0][threadIdx.x] = a0; red[1][threadIdx.x] = a1;
+    red[2][threadIdx.x] = a2; red[3][threadIdx.x] = a3;
+  }
   for (int s = TILE / 2; s > 0; s >>= 1) {
     __syncthreads();
     if (threadIdx.x < s) {
@@ -1017,60 +1633,6 @@ __global__ __launch_bounds__(TILE) void k_wear_final(int ntiles, const double *_
 }
 
 // ------------------------------------------------------------------------------- batched
-// Fields of the instance descriptors read through the constant address space: the compiler
-// then takes the pointers loaded from them for global pointers and emits global loads, which
-// count only against the vector-memory wait counter, instead of flat loads, which also hold up
-// every wait for an LDS or scalar load. (A whole-struct copy loses that, hence the field lists.)
-// The descriptors do not change while a kernel runs.
-#define MFC_CONST(T) const __attribute__((address_space(4))) T
-#define MFC_F(f) o.f = c->f
-__device__ inline dstate load_state(MFC_CONST(dstate) * c) {
-  dstate o;
-  MFC_F(px); MFC_F(py); MFC_F(vx); MFC_F(vy); MFC_F(sxx); MFC_F(sxy); MFC_F(syy); MFC_F(szz); MFC_F(rho);
-  MFC_F(T); MFC_F(eps); MFC_F(epsd); MFC_F(h); MFC_F(fcx); MFC_F(fcy); MFC_F(ftx); MFC_F(fty); MFC_F(ptx);
-  MFC_F(pty); MFC_F(vtx); MFC_F(vty); MFC_F(rhot); MFC_F(stxx); MFC_F(stxy); MFC_F(styy); MFC_F(stzz); MFC_F(Tt);
-  MFC_F(flags); MFC_F(id);
-  return o;
-}
-__device__ inline dbins load_bins(MFC_CONST(dbins) * c) {
-  dbins o;
-  MFC_F(key); MFC_F(key_sorted); MFC_F(offsets); MFC_F(bucket); MFC_F(perm);
-  MFC_F(spos); MFC_F(bsum); MFC_F(clist); MFC_F(ccap); MFC_F(offsets_r); MFC_F(clamped);
-  return o;
-}
-__device__ inline dpositional load_pos(MFC_CONST(dpositional) * c) {
-  dpositional o;
-  MFC_F(nx); MFC_F(ny); MFC_F(p); MFC_F(rxx); MFC_F(rxy); MFC_F(ryy);
-  return o;
-}
-__device__ inline drecords load_recs(MFC_CONST(drecords) * c) {
-  drecords o;
-  MFC_F(f32); MFC_F(rec); MFC_F(posd); MFC_F(vfl); MFC_F(rec32);
-  return o;
-}
-__device__ inline dforce load_force(MFC_CONST(dforce) * c) {
-  dforce o;
-  MFC_F(partials); MFC_F(force_last); MFC_F(hist); MFC_F(cap); MFC_F(ctr); MFC_F(pending);
-  return o;
-}
-__device__ inline MFC_CONST(inst_args) * const_args(const inst_args *A, int q) {
-  return (MFC_CONST(inst_args) *)(A + q);
-}
-__device__ inline inst_args load_args(const inst_args *A, int q) {
-  MFC_CONST(inst_args) *c = const_args(A, q);
-  inst_args o;
-  o.k = A[q].k;  // no pointers
-  o.cur = load_state(&c->cur);
-  o.nxt = load_state(&c->nxt);
-  o.b = load_bins(&c->b);
-  o.pos = load_pos(&c->pos);
-  o.r = load_recs(&c->r);
-  MFC_F(tool_in); MFC_F(tool_out);
-  o.f = load_force(&c->f);
-  MFC_F(acc); MFC_F(geo); MFC_F(ntiles); MFC_F(nscan);
-  return o;
-}
-#undef MFC_F
 
 // One launch per phase for all instances of a batch: block b takes work item xcd_tile(b) (the
 // interaction kernels: xcd_chunk_tile(b)) of the (instance, block) table, and runs the device
@@ -1081,7 +1643,7 @@ __global__ __launch_bounds__(256) void kb_hash_count(const inst_args *__restrict
   const int w = xcd_tile(blockIdx.x, nwork);
   if (w < 0) return;
   const int2 it = work[w];
-  const inst_args a = load_args(A, it.x);
+  const inst_args &a = A[it.x];
   if (a.k.adaptive) return;  // its step starts with the geometry pass, which bins the state
   hash_count(a.k, it.y * 256 + threadIdx.x, a.cur.px, a.cur.py, a.cur.flags, a.b);
 }
@@ -1154,34 +1716,57 @@ __global__ __launch_bounds__(GEO_THREADS) void kb_geometry(inst_args *__restrict
     hash_count(k, base + threadIdx.x, a.cur.px, a.cur.py, a.cur.flags, a.b);
 }
 
+// the sort of a chunk of cells, and the work items of an instance beside its chunks: the tool's
+// move, the list of its patches and the group sums of the previous step's tool force, if they are
+// still pending (the items come first in the work table, so that their work-groups start first)
 __global__ __launch_bounds__(SCAN_THREADS) void kb_sort(const inst_args *__restrict__ A, const int2 *__restrict__ work,
                                                          int nwork) {
   const int w = xcd_tile(blockIdx.x, nwork);
   if (w < 0) return;
   const int2 it = work[w];
   MFC_CONST(inst_args) *c = const_args(A, it.x);
+  if (it.y <= SORT_ITEM_PATCHES) {
+    list_patches(A[it.x].k, SORT_ITEM_PATCHES - it.y, load_bins(&c->b));
+    return;
+  }
+  if (it.y <= SORT_ITEM_FORCE) {
+    const dforce fo = load_force(&c->f);
+    if (*fo.pending == 0) return;  // the same value in every thread
+    constexpr int PER_WAVE = FORCE_GROUPS / (SCAN_THREADS / 64);
+    const int g0 = (SORT_ITEM_FORCE - it.y) * FORCE_GROUPS + (threadIdx.x >> 6) * PER_WAVE;
+    force_groups(A[it.x].k.N, g0, PER_WAVE, load_state(&c->cur), fo);
+    return;
+  }
+  if (it.y == SORT_ITEM_TOOL) {
+    tool_move(A[it.x].tool_in, A[it.x].tool_out, A[it.x].k.dt);
+    return;
+  }
   const dev_consts &k = A[it.x].k;
   sort_chunk(it.y, k.N, k.ncell_table, load_bins(&c->b), k.sort_fast, k.sort_list);
 }
 
-template <bool F32, bool GATHER>
-__global__ __launch_bounds__(TILE) void kb_predict(const inst_args *__restrict__ A, const int2 *__restrict__ work,
+// the records of a start state that no interaction wrote
+template <bool F32>
+__global__ __launch_bounds__(TILE) void kb_records(const inst_args *__restrict__ A, const int2 *__restrict__ work,
                                                    int nwork) {
   const int w = xcd_tile(blockIdx.x, nwork);
   if (w < 0) return;
   const int2 it = work[w];
-  // records, bins and the start state through the constant address space (global loads and
-  // stores); the other pointers through generic loads, where they are used (holding all of
-  // them would take more scalar registers than there are)
+  MFC_CONST(inst_args) *c = const_args(A, it.x);
+  const dev_consts &k = A[it.x].k;
+  const int s = it.y * TILE + threadIdx.x;
+  if (s >= k.N) return;
+  write_record<F32>(k, load_rec_input(load_state(&c->cur), s), s, load_recs(&c->r));
+}
+
+__global__ __launch_bounds__(TILE) void kb_predict_gather(const inst_args *__restrict__ A,
+                                                          const int2 *__restrict__ work, int nwork) {
+  const int w = xcd_tile(blockIdx.x, nwork);
+  if (w < 0) return;
+  const int2 it = work[w];
   const inst_args &a = A[it.x];
   MFC_CONST(inst_args) *c = const_args(A, it.x);
-  const dbins b = load_bins(&c->b);
-  predict<F32, GATHER>(a.k, it.y, b, load_state(&c->cur), a.nxt, a.pos, load_recs(&c->r), a.tool_in, a.tool_out);
-  // the chunk sums are consumed (the sort): cleared for the counts of the next step
-  for (int q = it.y * TILE + threadIdx.x; q < a.nscan; q += a.ntiles * TILE) b.bsum[q] = 0;
-  // the tool force of the previous step, if its partials are still pending (the first tile's
-  // work-group is dispatched first, so the longer kernel hides the reduction)
-  if (it.y == 0) force_final(a.ntiles, load_force(&c->f));
+  predict_gather(a.k, it.y, load_bins(&c->b), load_state(&c->cur), a.nxt, a.pos, load_recs(&c->r));
 }
 
 // The cell ranges of grid_gpu_rothlin (grid_gpu_rothlin.cu:28-127) rebuilt from the sorted cell
@@ -1210,49 +1795,40 @@ __global__ __launch_bounds__(256) void kb_rothlin_cells(const inst_args *__restr
     for (int q = h + 1; q <= hn; q++) b.offsets_r[q] = i + 1;
 }
 
-template <bool F32, bool COMPACT>
-__global__ __launch_bounds__(TILE) SUMS_OCCUPANCY void kb_interact(const inst_args *__restrict__ A, const int2 *__restrict__ work,
-                                                    int nwork, int chunk) {
+template <bool F32, int G, bool PSE>
+__global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(F32 ? 4 : 3))) void kb_interact(
+    const inst_args *__restrict__ A, const int2 *__restrict__ work, int nwork, int chunk) {
   const int w = xcd_chunk_tile(blockIdx.x, nwork, chunk);
   if (w < 0) return;
   const int2 it = work[w];
-  const inst_args &a = A[it.x];
   MFC_CONST(inst_args) *c = const_args(A, it.x);
-  const dbins b = load_bins(&c->b);
-  // an adaptive grid bins the next step's start state after its geometry pass instead
-  interact<F32, COMPACT>(a.k, it.y, load_recs(&c->r), b.key_sorted, a.k.rothlin ? b.offsets_r : b.offsets, b.perm,
-                         a.cur, a.nxt, a.pos, a.tool_out, a.f, b, a.bin_next && !a.k.adaptive, a.acc_out);
+  __shared__ patch_mem<F32, G> m;
+  if (it.y == PATCH_ITEM_FORCE) {
+    const dforce fo = load_force(&c->f);
+    // pending: the same value in every thread
+    if (*fo.pending != 0) force_final(c->ntiles, fo, reinterpret_cast<double(*)[TILE]>(&m));
+    if (threadIdx.x == 0) *fo.pending_next = 1;
+    return;
+  }
+  const int count = *c->b.plen, step = c->npatch_items;
+  if (it.y >= count) return;
+  const int2 p = c->b.plist[it.y];
+  if (!interact_patch<F32, G, PSE>(m, A, it.x, p.x, p.y)) interact_rest<F32>(A + it.x, p.x, p.y);
+  for (int q = it.y + step; q < count; q += step) interact_rest<F32>(A + it.x, c->b.plist[q].x, c->b.plist[q].y);
 }
 
-template <bool F32, bool COMPACT>
-__global__ __launch_bounds__(TILE) SUMS_OCCUPANCY void kb_sums(const inst_args *__restrict__ A, const int2 *__restrict__ work,
-                                                int nwork, int chunk) {
-  const int w = xcd_chunk_tile(blockIdx.x, nwork, chunk);
-  if (w < 0) return;
-  const int2 it = work[w];
-  const inst_args &a = A[it.x];
-  MFC_CONST(inst_args) *c = const_args(A, it.x);
-  const dbins b = load_bins(&c->b);
-  sums<F32, COMPACT>(a.k, it.y, load_recs(&c->r), b.key_sorted, a.k.rothlin ? b.offsets_r : b.offsets, b.perm,
-                     a.cur.flags, c->acc);
-}
-
-template <bool F32>
-__global__ __launch_bounds__(TILE) void kb_update(const inst_args *__restrict__ A, const int2 *__restrict__ work,
-                                                  int nwork) {
-  const int w = xcd_tile(blockIdx.x, nwork);
-  if (w < 0) return;
-  const int2 it = work[w];
-  const inst_args &a = A[it.x];
-  MFC_CONST(inst_args) *c = const_args(A, it.x);
-  const dbins b = load_bins(&c->b);
-  update<F32>(a.k, it.y, c->acc, b.perm, a.cur, a.nxt, a.pos, a.tool_out, a.f, b, a.bin_next && !a.k.adaptive,
-              a.acc_out ? a.acc_out + (size_t)ACC_N * a.k.N : nullptr);
-}
-
-__global__ __launch_bounds__(TILE) void kb_force_final(const inst_args *__restrict__ A) {
-  const inst_args a = load_args(A, blockIdx.x);
-  force_final(a.ntiles, a.f);
+// after the last step of a call: its tool force, by one work-group per instance
+constexpr int FORCE_LAST_THREADS = 1024;
+__global__ __launch_bounds__(FORCE_LAST_THREADS) void kb_force_final(const inst_args *__restrict__ A) {
+  MFC_CONST(inst_args) *c = const_args(A, blockIdx.x);
+  const dforce fo = load_force(&c->f);
+  if (*fo.pending == 0) return;  // the same value in every thread
+  const int N = A[blockIdx.x].k.N, ntiles = A[blockIdx.x].ntiles;
+  const dstate st = load_state(&c->cur);
+  for (int g0 = (threadIdx.x >> 6) * 64; 64 * g0 < N; g0 += FORCE_LAST_THREADS) force_groups(N, g0, 64, st, fo);
+  __syncthreads();  // the group sums
+  __shared__ double red[4][TILE];
+  force_final(ntiles, fo, red);
 }
 
 __global__ void k_device_math(int fn, const double *__restrict__ x, const double *__restrict__ y,
@@ -1285,10 +1861,6 @@ int scan_blocks(int num_cell) { return (num_cell + SCAN_CHUNK - 1) / SCAN_CHUNK;
 
 static int padded_tiles(int ntiles) { return ((ntiles + 7) / 8) * 8; }
 
-// the four instantiations of a kernel template <F32, COMPACT>
-#define MFC_PICK(kern, f32, compact) \
-  ((f32) ? ((compact) ? kern<true, true> : kern<true, false>) : ((compact) ? kern<false, true> : kern<false, false>))
-
 void launch_tool_wear(const dev_consts &k, const dstate &st, const dpositional &pos, double K, double alpha,
                       double tvx, double tvy, double *part, double *out, hipStream_t s) {
   const int nt = (k.N + TILE - 1) / TILE;
@@ -1314,68 +1886,49 @@ void launch_batch_binning(const batch_work &w, hipStream_t s) {
   if (w.adaptive)  // the descriptors are device memory of the batch; the geometry pass updates them
     hipLaunchKernelGGL(kb_geometry, dim3(w.n), dim3(GEO_THREADS), 0, s, const_cast<inst_args *>(w.args));
   hipLaunchKernelGGL(kb_sort, gc, dim3(SCAN_THREADS), 0, s, w.args, w.chunks, w.nchunks);
+  if (w.rothlin)
+    hipLaunchKernelGGL(kb_rothlin_cells, dim3(padded_tiles(w.ntiles)), dim3(256), 0, s, w.args, w.tiles, w.ntiles);
 }
 
-void launch_batch_predict(const batch_work &w, hipStream_t s) {
+void launch_batch_records(const batch_work &w, hipStream_t s) {
   const dim3 gt(padded_tiles(w.ntiles));
-  if (w.f32) hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_predict<true, false>), gt, dim3(TILE), 0, s, w.args, w.tiles, w.ntiles);
-  else hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_predict<false, false>), gt, dim3(TILE), 0, s, w.args, w.tiles, w.ntiles);
-  if (w.rothlin) hipLaunchKernelGGL(kb_rothlin_cells, gt, dim3(256), 0, s, w.args, w.tiles, w.ntiles);
+  if (w.f32) hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_records<true>), gt, dim3(TILE), 0, s, w.args, w.tiles, w.ntiles);
+  else hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_records<false>), gt, dim3(TILE), 0, s, w.args, w.tiles, w.ntiles);
 }
 
 void launch_batch_predict_gather(const batch_work &w, hipStream_t s) {
-  hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_predict<false, true>), dim3(padded_tiles(w.ntiles)), dim3(TILE), 0, s, w.args,
-                     w.tiles, w.ntiles);
+  hipLaunchKernelGGL(kb_predict_gather, dim3(padded_tiles(w.ntiles)), dim3(TILE), 0, s, w.args, w.tiles, w.ntiles);
 }
 
-// a batched launch over the work table, with the kernel's own start and end recorded in t0 and
-// t1 when they are given
 template <class K>
-static void launch_timed(K kern, dim3 grid, const batch_work &w, hipStream_t s, hipEvent_t t0, hipEvent_t t1) {
+static void launch_patches(K kern, const batch_work &w, hipStream_t s, hipEvent_t t0, hipEvent_t t1) {
+  const dim3 grid(chunked_blocks(w.npatches, w.v.chunk));
   if (t0)
-    hipExtLaunchKernelGGL(kern, grid, dim3(TILE), 0, s, t0, t1, 0, w.args, w.tiles, w.ntiles);
+    hipExtLaunchKernelGGL(kern, grid, dim3(TILE), 0, s, t0, t1, 0, w.args, w.patches, w.npatches, w.v.chunk);
   else
-    hipLaunchKernelGGL(kern, grid, dim3(TILE), 0, s, w.args, w.tiles, w.ntiles);
+    hipLaunchKernelGGL(kern, grid, dim3(TILE), 0, s, w.args, w.patches, w.npatches, w.v.chunk);
 }
 
-// the same for the interaction kernels, whose tile map takes the XCD chunk length
-template <class K>
-static void launch_chunked(K kern, const batch_work &w, hipStream_t s, hipEvent_t t0, hipEvent_t t1) {
-  const dim3 grid(chunked_blocks(w.ntiles, w.v.chunk));
-  if (t0)
-    hipExtLaunchKernelGGL(kern, grid, dim3(TILE), 0, s, t0, t1, 0, w.args, w.tiles, w.ntiles, w.v.chunk);
-  else
-    hipLaunchKernelGGL(kern, grid, dim3(TILE), 0, s, w.args, w.tiles, w.ntiles, w.v.chunk);
-}
-
-void launch_batch_sums(const batch_work &w, hipStream_t s, hipEvent_t t0, hipEvent_t t1) {
-  launch_chunked(MFC_PICK(kb_sums, w.f32, w.v.compact), w, s, t0, t1);
-}
-
-void launch_batch_update(const batch_work &w, hipStream_t s, hipEvent_t t0, hipEvent_t t1) {
-  if (w.f32) launch_timed(kb_update<true>, dim3(padded_tiles(w.ntiles)), w, s, t0, t1);
-  else launch_timed(kb_update<false>, dim3(padded_tiles(w.ntiles)), w, s, t0, t1);
-}
-
-void launch_batch_interact_fused(const batch_work &w, hipStream_t s, hipEvent_t t0, hipEvent_t t1) {
-  launch_chunked(MFC_PICK(kb_interact, w.f32, w.v.compact), w, s, t0, t1);
+void launch_batch_interact(const batch_work &w, hipStream_t s, hipEvent_t t0, hipEvent_t t1) {
+#define MFC_PICK(lanes, pse) (w.f32 ? kb_interact<true, lanes, pse> : kb_interact<false, lanes, pse>)
+#define MFC_PICK_PSE(lanes) launch_patches(w.pse ? MFC_PICK(lanes, true) : MFC_PICK(lanes, false), w, s, t0, t1)
+  switch (w.v.lanes) {
+    case 1: MFC_PICK_PSE(1); break;
+    case 4: MFC_PICK_PSE(4); break;
+    default: MFC_PICK_PSE(8); break;
+  }
 }
 
 void launch_batch_force(const batch_work &w, hipStream_t s) {
-  hipLaunchKernelGGL(kb_force_final, dim3(w.n), dim3(TILE), 0, s, w.args);
+  hipLaunchKernelGGL(kb_force_final, dim3(w.n), dim3(FORCE_LAST_THREADS), 0, s, w.args);
 }
 
-// one step; the cell ids and counts of its start state come from the previous step's interaction
-// (or launch_batch_hash), and its own interaction computes those of the next step
+// one step; the cell ids, counts and records of its start state come from the previous step's
+// interaction (or launch_batch_hash and launch_batch_records), and its own interaction computes
+// those of the next step
 void launch_batch_step(const batch_work &w, hipStream_t s) {
-  launch_batch_binning(w, s);  // also reduces the previous step's tool force
-  launch_batch_predict(w, s);
-  if (w.v.split) {
-    launch_batch_sums(w, s);
-    launch_batch_update(w, s);
-  } else {
-    launch_batch_interact_fused(w, s);
-  }
+  launch_batch_binning(w, s);  // also the tool's move, the patch list, the previous step's force groups
+  launch_batch_interact(w, s);
 }
 
 }  // namespace mfc

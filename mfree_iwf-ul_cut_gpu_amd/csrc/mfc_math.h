@@ -63,15 +63,8 @@ constexpr double SQRT3   = 1.7320508075688772;
 constexpr double TAN_PI12 = 0.2679491924311228;
 constexpr double SQRT2   = 1.4142135623730951;
 
-// e^x
-MFC_HD double exp(double x) {
-  if (is_nan(x)) return x;
-  if (x > 709.782712893384) return u2d(0x7ff0000000000000ULL);
-  if (x < -745.1332191019412) return 0.0;
-  double kd = floor(x * INV_LN2 + 0.5);
-  int k = (int)kd;
-  double r = (x - kd * LN2_HI) - kd * LN2_LO;
-  // Taylor coefficients 1/j!, j = 13 .. 2
+// e^r for |r| <= ln2/2: Taylor coefficients 1/j!, j = 13 .. 2
+MFC_HD double exp_reduced(double r) {
   double p = 1.6059043836821613e-10;            // 1/13!
   p = 2.08767569878681e-09 + r * p;             // 1/12!
   p = 2.505210838544172e-08 + r * p;            // 1/11!
@@ -84,12 +77,22 @@ MFC_HD double exp(double x) {
   p = 0.041666666666666664 + r * p;             // 1/4!
   p = 0.16666666666666666 + r * p;              // 1/3!
   p = 0.5 + r * p;                              // 1/2!
-  double e = 1.0 + (r + (r * r) * p);
+  return 1.0 + (r + (r * r) * p);
+}
+
+// e^x
+MFC_HD double exp(double x) {
+  if (is_nan(x)) return x;
+  if (x > 709.782712893384) return u2d(0x7ff0000000000000ULL);
+  if (x < -745.1332191019412) return 0.0;
+  double kd = floor(x * INV_LN2 + 0.5);
+  int k = (int)kd;
+  double r = (x - kd * LN2_HI) - kd * LN2_LO;
+  double e = exp_reduced(r);
   if (k > 1023) return (e * pow2i(1023)) * pow2i(k - 1023);
   if (k < -1022) return (e * pow2i(k + 54)) * pow2i(-54);
   return e * pow2i(k);
 }
-
 // natural logarithm
 MFC_HD double log(double x) {
   if (is_nan(x)) return x;

@@ -1,5 +1,5 @@
-// mfc_pairs.h — the FP64 neighbour sums of one particle, shared by the step kernels and the
-// adjoint's forward recomputation.
+// mfc_pairs.h — the cell window of a particle and the FP64 terms of one pair, shared by the step
+// kernels and the reverse mode.
 #pragma once
 
 #include "mfc_kernels.h"
@@ -8,18 +8,10 @@ namespace mfc {
 
 constexpr int REC_DOUBLES = 16;  // doubles per FP64 neighbour record
 
-// candidates of the window walk whose loads are issued together (FP32C direct walk: WALK_U32,
-// with their whole records)
-constexpr int WALK_U = 4;
-constexpr int WALK_U32 = 2;
-
-// where the window walk reads candidate positions and flags: candidate j at [j - base] of pos
-// and fl (the records in memory with base 0, or a tile's copy in LDS)
-struct cand_src {
-  const double2 *pos;
-  const int *fl;
-  int base;
-};
+// a tag: the index of a neighbour's record (storage order) and its flags
+constexpr int TAG_BITS = 4;  // FIXED, BLANKED, TOOL, NONFINITE
+__device__ inline int make_tag(int index, int flags) { return (int)(((unsigned)index << TAG_BITS) | (unsigned)flags); }
+__device__ inline unsigned tag_index(int tag) { return (unsigned)tag >> TAG_BITS; }
 
 // The 5 x 5 cell window around the cell of a particle (interactions_gpu.cu:219-229): up to 5
 // columns of the cell grid (clipped to the grid), each a contiguous range of the sorted order.
@@ -38,21 +30,26 @@ struct window {
   }
 };
 
-__device__ inline window make_window(const dev_consts &k, const int *__restrict__ offsets, int hsh) {
-  const int gi = hsh / k.gny, gj = hsh - gi * k.gny;
+// the up to 5 column ranges [b, e) of the window of a particle in cell column gi and row gj;
+// at(column, row) is the first index of a cell (the last one past the column's end for row gny)
+template <class AT>
+__device__ inline void window_ranges(const dev_consts &k, int gi, int gj, const AT &at, int b[5], int e[5]) {
   const int li = gi - 2 < 0 ? 0 : gi - 2;
   const int lj = gj - 2 < 0 ? 0 : gj - 2;
   const int hi = gi + 3 > k.gnx ? k.gnx : gi + 3;
   const int hj = gj + 3 > k.gny ? k.gny : gj + 3;
-  int b[5], e[5];
 #pragma unroll
   for (int r = 0; r < 5; r++) {
     const bool in = li + r < hi;
     const int ii = in ? li + r : hi - 1;
-    b[r] = offsets[ii * k.gny + lj];
-    e[r] = offsets[ii * k.gny + hj];
+    b[r] = at(ii, lj);
+    e[r] = at(ii, hj);
     if (!in) e[r] = b[r];
   }
+}
+
+// its candidates numbered through the ranges
+__device__ inline window window_of(const int b[5], const int e[5]) {
   window w;
   // d_r = b[r] - c_r with c_r the candidates before column r; e_r = d_r - d_(r-1)
   int c = e[0] - b[0];
@@ -63,6 +60,20 @@ __device__ inline window make_window(const dev_consts &k, const int *__restrict_
   w.c4 = c; w.e4 = b[4] - c - (b[3] - w.c3); c += e[4] - b[4];
   w.total = c;
   return w;
+}
+
+template <class AT>
+__device__ inline window make_window_at(const dev_consts &k, int gi, int gj, const AT &at) {
+  int b[5], e[5];
+  window_ranges(k, gi, gj, at, b, e);
+  return window_of(b, e);
+}
+
+
+// the window of a particle with cell id hsh over the cell ranges in memory
+__device__ inline window make_window(const dev_consts &k, const int *__restrict__ offsets, int hsh) {
+  const int gi = hsh / k.gny, gj = hsh - gi * k.gny;
+  return make_window_at(k, gi, gj, [&](int col, int row) { return offsets[col * k.gny + row]; });
 }
 
 __device__ inline double bits_to_double(int f) { return __longlong_as_double((long long)f); }
@@ -93,176 +104,91 @@ __device__ inline void load_acc(const double *__restrict__ acc, size_t N, int i,
   a.tl = acc[12 * N + i]; tpse = acc[13 * N + i];
 }
 
-// the body of the neighbour loop of do_interactions_monaghan for one pair
-// (interactions_gpu.cu:249-326 with cubic_spline kernels.cuh:30-70)
-__device__ inline void pair_terms(const dev_consts &k, pair_acc &a, double xi, double yi, double ui, double vi_,
-                                  double hi, double rhoi, double Axx_i, double Axy_i, double Ayy_i, double Rxx_i,
-                                  double Rxy_i, double Ryy_i, double ci, double Ti, bool tool_i, double ta,
-                                  double h1, double fourh2, double fac, const double *rj, double xj, double yj,
-                                  bool tool_j) {
-  const double2 *r2 = reinterpret_cast<const double2 *>(rj);
-  double2 q1 = r2[1], q2 = r2[2], q3 = r2[3], q4 = r2[4], q5 = r2[5], q6 = r2[6], q7 = r2[7];
-  const double hj = q1.y, uj = q2.x, vj = q2.y, rhoj = q3.x, volj = q3.y;
-  const double Axx_j = q4.x, Axy_j = q4.y, Ayy_j = q5.x, Rxx_j = q5.y, Rxy_j = q6.x, Ryy_j = q6.y;
-  const double cj = q7.x, Tj = (ta != 0.) ? q7.y : 0.;
+// a particle's FP64 record as the pair terms read it
+struct rec64 {
+  double x, y, u, v, rho, vol, Axx, Axy, Ayy, Rxx, Rxy, Ryy, c, T, h;
+};
+
+// a / b, correctly rounded, from y = 1 / b correctly rounded: a quotient and two corrections by the
+// exact remainder (the second one starts from a faithful quotient, which Markstein's theorem
+// (IBM J. Res. Dev. 34, 1990) takes to the rounded one). For finite a that is 0 or large enough
+// that its remainder does not underflow (|a| > 2^-960) and quotients in range; 5 operations
+// where a division takes 11.
+__device__ inline double div_by(double a, double b, double y) {
+  const double q0 = a * y;
+  const double q1 = __builtin_fma(__builtin_fma(-q0, b, a), y, q0);
+  return __builtin_fma(__builtin_fma(-q1, b, a), y, q1);
+}
+
+// the terms of one pair in the body of the neighbour loop of do_interactions_monaghan
+// (interactions_gpu.cu:249-326 with cubic_spline kernels.cuh:30-70), in the order and with the
+// operations of the reference's sums. A term that the reference does not add is 0: a sum starts
+// at +0 and adding +0 leaves every value it can take unchanged. FINITE: both records are finite and
+// the pair is in support, so the quotients by the same divisor can share its reciprocal (div_by;
+// their numerators are kernel values and coordinate differences). inv_wd = 1 / wdeltap.
+template <bool FINITE>
+__device__ inline pair_acc pair_terms(const dev_consts &k, const rec64 &a, bool tool_i, double ta, double h1,
+                                      double fourh2, double fac, double inv_wd, const rec64 &b, bool tool_j) {
+  pair_acc t = {0., 0., 0., 0., 0., 0., 0., 0., 0., 0., 0., 0., 0.};
   const double mass = k.mass;
   // cubic spline with h_i
   double w = 0., w_x = 0., w_y = 0.;
-  const double xij = xi - xj, yij = yi - yj;
+  const double xij = a.x - b.x, yij = a.y - b.y;
   const double rr2 = xij * xij + yij * yij;
-  if (!(rr2 >= fourh2 || rr2 < 1e-8)) {
+  if (FINITE || !(rr2 >= fourh2 || rr2 < 1e-8)) {
     double der, val;
     double rad = tsqrt(k, rr2);
     double q = rad * h1;
+    double num;  // of der: one division for both pieces of the spline
     if (q > 1) {
       double m = 2 - q, m2 = m * m;
       val = 0.25 * m2 * m2 * m2;
-      der = -0.75 * m2 * h1 / rad;
+      num = -0.75 * m2 * h1;
     } else {
       val = 1 - 1.5 * q * q * (1 - 0.5 * q);
-      der = -3.0 * q * (1 - 0.75 * q) * h1 / rad;
+      num = -3.0 * q * (1 - 0.75 * q) * h1;
     }
+    der = num / rad;
     w = val * fac;
     w_x = der * xij * fac;
     w_y = der * yij * fac;
   }
   if (!tool_i && !tool_j) {
-    a.vd0 += (uj - ui) * w_x * volj;
-    a.vd1 += (uj - ui) * w_y * volj;
-    a.vd2 += (vj - vi_) * w_x * volj;
-    a.vd3 += (vj - vi_) * w_y * volj;
-    double fab = w / k.wdeltap;
+    t.vd0 = (b.u - a.u) * w_x * b.vol;
+    t.vd1 = (b.u - a.u) * w_y * b.vol;
+    t.vd2 = (b.v - a.v) * w_x * b.vol;
+    t.vd3 = (b.v - a.v) * w_y * b.vol;
+    double fab = FINITE ? div_by(w, k.wdeltap, inv_wd) : w / k.wdeltap;
     fab *= fab;
     fab *= fab;
-    const double Rx = fab * (Rxx_i + Rxx_j), Ry = fab * (Rxy_i + Rxy_j), Rz = fab * (Ryy_i + Ryy_j);
-    a.sd0 += mass * (Axx_i + Axx_j + Rx) * w_x;
-    a.sd1 += mass * (Axy_i + Axy_j + Ry) * w_y;
-    a.sd2 += mass * (Axy_i + Axy_j + Ry) * w_x;
-    a.sd3 += mass * (Ayy_i + Ayy_j + Rz) * w_y;
-    const double vijx = ui - uj, vijy = vi_ - vj;
+    const double Rx = fab * (a.Rxx + b.Rxx), Ry = fab * (a.Rxy + b.Rxy), Rz = fab * (a.Ryy + b.Ryy);
+    t.sd0 = mass * (a.Axx + b.Axx + Rx) * w_x;
+    t.sd1 = mass * (a.Axy + b.Axy + Ry) * w_y;
+    t.sd2 = mass * (a.Axy + b.Axy + Ry) * w_x;
+    t.sd3 = mass * (a.Ayy + b.Ayy + Rz) * w_y;
+    const double vijx = a.u - b.u, vijy = a.v - b.v;
     const double vijposij = vijx * xij + vijy * yij;
-    const double rhoij = 0.5 * (rhoi + rhoj);
+    const double rhoij = 0.5 * (a.rho + b.rho);
     if (vijposij < 0.) {
-      const double cij = 0.5 * (ci + cj);
-      const double hij = 0.5 * (hi + hj);
+      const double cij = 0.5 * (a.c + b.c);
+      const double hij = 0.5 * (a.h + b.h);
       const double muij = (hij * vijposij) / (rr2 + k.av_eta * k.av_eta * hij * hij);
       const double piij = (-k.av_alpha * cij * muij + k.av_beta * muij * muij) / rhoij;
-      a.vt0 += -mass * piij * w_x;
-      a.vt1 += -mass * piij * w_y;
+      t.vt0 = -mass * piij * w_x;
+      t.vt1 = -mass * piij * w_y;
     }
-    a.xt0 += -k.xsph_eps * w * mass / rhoij * vijx;
-    a.xt1 += -k.xsph_eps * w * mass / rhoij * vijy;
+    t.xt0 = -k.xsph_eps * w * mass / rhoij * vijx;
+    t.xt1 = -k.xsph_eps * w * mass / rhoij * vijy;
   }
   if (ta != 0.) {  // Brookshaw
     const double rij = sqrt(rr2);
     if (rij > 1e-8) {
-      const double eijx = xij / rij, eijy = yij / rij;
       const double rij1 = 1. / rij;
-      a.tl += 2.0 * volj * (Ti - Tj) * rij1 * (eijx * w_x + eijy * w_y);
+      const double eijx = FINITE ? div_by(xij, rij, rij1) : xij / rij, eijy = FINITE ? div_by(yij, rij, rij1) : yij / rij;
+      t.tl = 2.0 * b.vol * (a.T - b.T) * rij1 * (eijx * w_x + eijy * w_y);
     }
   }
-}
-
-// FP64 neighbour sums of particle i: the reference's loop over the 5 x 5 cell window
-// (interactions_gpu.cu:219-331), walked as 5 contiguous column ranges of the sorted order.
-// COMPACT: the window is walked first, marking the neighbours that contribute in a per-lane
-// bit mask, and the marked ones are evaluated afterwards in the same order, so that a wave runs
-// the pair body about as often as its busiest lane has pairs instead of once per window
-// candidate.
-template <bool COMPACT>
-__device__ inline void sums_f64(const dev_consts &k, int i, const double *__restrict__ rec,
-                                const int *__restrict__ key_sorted, const int *__restrict__ offsets,
-                                const cand_src &cs, bool tool, double ta, bool run_mech, bool run_pse, pair_acc &acc,
-                                double &tpse) {
-  const double2 *r2 = reinterpret_cast<const double2 *>(rec + (size_t)REC_DOUBLES * i);
-  double2 a0 = r2[0], a1 = r2[1], a2 = r2[2], a3 = r2[3], a4 = r2[4], a5 = r2[5], a6 = r2[6], a7 = r2[7];
-  const double xi = a0.x, yi = a0.y;
-  const int rfl = double_to_bits(a1.x);
-  const double hi = a1.y, ui = a2.x, vi_ = a2.y, rhoi = a3.x;
-  const double Axx_i = a4.x, Axy_i = a4.y, Ayy_i = a5.x, Rxx_i = a5.y, Rxy_i = a6.x, Ryy_i = a6.y;
-  const double ci = a7.x, Tpred = a7.y;
-  const bool nonfin_i = rfl & FLAG_NONFINITE;
-  const double Ti = (ta != 0.) ? Tpred : 0.;
-  const double h1 = 1 / hi;
-  const double fourh2 = 4 * hi * hi;
-  const double fac = PI_FAC * h1 * h1;
-  const double h2 = hi * hi, h4 = h2 * h2;
-  const double pse_c = 4. / (h4 * M_PI);
-  const window w = make_window(k, offsets, key_sorted[i]);
-  // what the walk loads per candidate ahead of its evaluation: position and flags (density and
-  // temperature for PSE are loaded when the candidate is evaluated, which keeps the registers
-  // of the group at 5 per candidate)
-  struct cand {
-    double2 p;
-    int f;
-  };
-  auto load = [&](int j, cand &c) {
-    c.p = cs.pos[j - cs.base];
-    c.f = cs.fl[j - cs.base];
-  };
-  // the PSE term of every window member and the test whether j adds to the mechanical sums
-  auto visit = [&](int j, const cand &c) -> bool {
-    const double xj = c.p.x, yj = c.p.y;
-    if (run_pse) {  // do_interactions_heat_pse (interactions_gpu.cu:130-139), all cell members
-      const double *rj = rec + (size_t)REC_DOUBLES * j;
-      const double dx = xi - xj, dy = yi - yj;
-      const double xx = sqrt(dx * dx + dy * dy);
-      const double w2 = pse_c * mfcm::exp(-xx * xx / (h2));
-      tpse += (rj[15] - Tpred) * w2 * k.mass / rj[6];
-    }
-    if (!run_mech) return false;
-    if (c.f & MFC_FLAG_BLANKED) return false;
-    const double dx = xi - xj, dy = yi - yj;
-    const double rr2 = dx * dx + dy * dy;
-    // outside the support the reference adds exact zeros, unless a value is non-finite
-    return !((rr2 >= fourh2 || rr2 < 1e-8) && !nonfin_i && !(c.f & FLAG_NONFINITE));
-  };
-  auto pair = [&](int j, double xj, double yj, int fj) {
-    pair_terms(k, acc, xi, yi, ui, vi_, hi, rhoi, Axx_i, Axy_i, Ayy_i, Rxx_i, Rxy_i, Ryy_i, ci, Ti, tool, ta, h1,
-               fourh2, fac, rec + (size_t)REC_DOUBLES * j, xj, yj, (fj & MFC_FLAG_TOOL) != 0);
-  };
-  // the window in groups of WALK_U candidates, the loads of a group issued before its first
-  // candidate is evaluated; the order of evaluation is the candidates' order
-  if constexpr (!COMPACT) {
-    for (int t0 = 0; t0 < w.total; t0 += WALK_U) {
-      int j[WALK_U];
-      cand c[WALK_U];
-#pragma unroll
-      for (int u = 0; u < WALK_U; u++) {
-        j[u] = w.at(t0 + u < w.total ? t0 + u : w.total - 1);
-        load(j[u], c[u]);
-      }
-#pragma unroll
-      for (int u = 0; u < WALK_U; u++)
-        if (t0 + u < w.total && visit(j[u], c[u])) pair(j[u], c[u].p.x, c[u].p.y, c[u].f);
-    }
-  } else {
-    // masked walk: the tests of up to 64 candidates set the bits of a per-lane mask, then the
-    // candidates of the set bits are evaluated in candidate order (the sorted index of a bit is
-    // recomputed by window::at, so no list is kept in memory)
-    for (int c0 = 0; c0 < w.total; c0 += 64) {
-      const int n = w.total - c0 < 64 ? w.total - c0 : 64;
-      unsigned long long m = 0ull;
-      for (int u0 = 0; u0 < n; u0 += WALK_U) {
-        int j[WALK_U];
-        cand c[WALK_U];
-#pragma unroll
-        for (int u = 0; u < WALK_U; u++) {
-          j[u] = w.at(c0 + (u0 + u < n ? u0 + u : n - 1));
-          load(j[u], c[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < WALK_U; u++)
-          if (u0 + u < n && visit(j[u], c[u])) m |= 1ull << (u0 + u);
-      }
-      while (m) {
-        const int jj = w.at(c0 + __builtin_ctzll(m));
-        m &= m - 1ull;
-        const double2 p = cs.pos[jj - cs.base];
-        pair(jj, p.x, p.y, cs.fl[jj - cs.base]);
-      }
-    }
-  }
+  return t;
 }
 
 }  // namespace mfc

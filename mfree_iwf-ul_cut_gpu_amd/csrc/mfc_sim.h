@@ -52,13 +52,18 @@ struct mfc_sim {
   mfc::dstate set[2];
   mfc::dbins bins = {};
   mfc::dpositional pos;
-  mfc::drecords recs = {false, nullptr, nullptr, nullptr};
+  mfc::drecords recs[2] = {};  // records of the start state of a step of parity 0 / 1
+  int *chunk_sums[2] = {nullptr, nullptr};  // bins.bsum of parity 0 / 1
+  int *plen = nullptr;                      // bins.plen of parity 0 / 1
   int precision = MFC_PREC_FP64;
   mfc_tool_state *tool = nullptr;  // two states, alternating each step
   double *partials = nullptr, *force_last = nullptr, *hist = nullptr;
   int64_t *hist_ctr = nullptr;
-  int *force_pending = nullptr;  // the last step's tool force is not yet reduced
-  mfc::dforce force() const { return {partials, force_last, hist, HIST_CAP, hist_ctr, force_pending}; }
+  int *force_pending = nullptr;  // per parity: the force of the step that produced it is not yet reduced
+  int *force_groups = nullptr;   // mfc::dforce::gflag
+  mfc::dforce force(int c) const {
+    return {partials, force_groups, force_last, hist, HIST_CAP, hist_ctr, force_pending + c, force_pending + 1 - c};
+  }
   int64_t hist_base = 0;           // steps recorded before the last history reset
   int cur = 0;                     // set holding the current state, and index of the current tool state
   int64_t step = 0;
@@ -66,24 +71,27 @@ struct mfc_sim {
   bool use_graphs = true;
   mfc::adj_work *adj = nullptr;    // reverse-mode tape of the last mfc_vjp_forward
   bool batched = false;            // instance of a batch: stepped by mfc_batch_step only
-  // bins.key/bsum/clist hold the binning of the current state (computed by the last step's
-  // interaction); false after creation and after anything else wrote the state or the bins
+  // bins.key/clist, the chunk sums and the records hold the binning and the neighbour records of
+  // the current state (computed by the last step's interaction); false after creation and after anything else wrote the state or the bins
   bool keys_fresh = false;
-  double *acc = nullptr;           // neighbour sums between the split interaction kernels
   double *wear_part = nullptr;     // tool wear: 4 doubles per tile, then the 4 results
   double wear_accum = 0.;          // accumulated wear, sum of dt * mean rate (tool_wear.cu:59)
-  mfc_tuning tuning = {0, 0, 0, 0, 0, 0, {0, 0}};
-  mfc::variant variant() const {
-    return {tuning.split_interact != 0, tuning.compact_pairs != 0, tuning.xcd_chunk ? tuning.xcd_chunk : mfc::XCD_CHUNK};
-  }
+  mfc_tuning tuning = {};
+  int lanes = 1;  // threads per particle of the interaction (set_patches)
+  mfc::variant variant() const { return {lanes, tuning.xcd_chunk ? tuning.xcd_chunk : mfc::XCD_CHUNK}; }
   // the step runs the batched kernels on a batch of one: descriptors of this handle for start
   // parity 0 and 1, and its (instance, block) work tables
   mfc::inst_args *dargs = nullptr;
-  int2 *dtiles = nullptr, *dchunks = nullptr;
-  int nchunks = 0;
+  mfc::inst_args *slot[2] = {nullptr, nullptr};  // where its descriptors are read from (a batch's for its instances)
+  int2 *dtiles = nullptr, *dchunks = nullptr, *dpatches = nullptr;
+  int nchunks = 0, npatches = 0;
+  int npatch_items = 0;            // patch work items (mfc::inst_args)
+  int npatch_items_max = 0;        // the most for any number of lanes
+  int npatch_max = 0;              // patches the buffers hold
   mfc::grid_geo *geo = nullptr;    // adaptive grid: the geometry of the last step (device)
   mfc::batch_work work(int c) const {
-    return {dargs + c, 1, dtiles, ntiles, dchunks, nchunks, recs.f32, variant(), k.adaptive != 0, k.rothlin != 0};
+    return {dargs + c, 1, dtiles, ntiles, dchunks, nchunks, dpatches, npatches, recs[0].f32, variant(),
+            k.adaptive != 0, k.pse != 0, k.rothlin != 0};
   }
 
   template <class T>
@@ -109,8 +117,19 @@ void carve_positional(void *base, int N, mfc::dpositional &p);
 // steps per captured hipGraph (even: a graph starts and ends on the same buffer parity)
 constexpr int GRAPH_STEPS = 8;
 void enqueue_step(mfc_sim *s, int c);
-// bins.key/bsum/clist of the current state, recomputed when keys_fresh is false
+// the binning and the records of the current state, recomputed when keys_fresh is false
 int ensure_keys(mfc_sim *s);
+// the work tables of the sort launch and of the interaction launch over a group of instances
+void sort_items(std::vector<int2> &items, mfc_sim *const *sims, int n);
+void patch_items(std::vector<int2> &items, mfc_sim *const *sims, int n);
+// threads per particle of the interaction for `total` particles stepped together, and a handle's
+// patches for that
+int interaction_lanes(int64_t total);
+void set_patches(mfc_sim *s, int lanes);
+// copies the handle's descriptors to where the kernels read them (synchronises its stream)
+int upload_descriptors(mfc_sim *s);
+// whether the current state's h is the same for every particle (host copy of the field)
+void check_uniform_h(mfc_sim *s, const double *h);
 void finish_steps(mfc_sim *s);
 int check_tuning(const mfc_tuning *t);
 // the batched kernels' view of a handle for start parity c

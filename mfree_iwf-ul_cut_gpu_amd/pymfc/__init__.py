@@ -121,9 +121,9 @@ SORT_FAST_MAX = 1536  # MFC_SORT_FAST_MAX: most particles of a chunk the sort ho
 GRAPH_STEPS = 8   # steps per captured hipGraph of a handle (one graph per buffer parity)
 
 
-# the launch configurations the autotuner tries: fused or split interaction, direct or compacted
-# pair loop, and the LDS stage limit (0: tiles stage up to STAGE_CAP candidates; n > 0: tiles
-# whose candidates span more than n sorted indices read them from memory; 1: no tile stages)
+# the launch configurations the autotuner tries: LDS stage limit (0: patches stage all the
+# candidates the kernel has room for; n > 0: patches with more than n read them from memory; 1: no
+# patch stages) and XCD chunk; split_interact and compact_pairs change nothing
 TUNING_SPACE = {"split_interact": (0, 1), "compact_pairs": (0, 1), "stage_limit": (0, 1536, 1), "xcd_chunk": (8, 32)}
 
 
@@ -168,7 +168,7 @@ class Tuning(C.Structure):
     """mfc_tuning (include/mfc.h)."""
     _fields_ = [("split_interact", C.c_int32), ("compact_pairs", C.c_int32), ("stage_limit", C.c_int32),
                 ("xcd_chunk", C.c_int32), ("sort_fast", C.c_int32), ("sort_list", C.c_int32),
-                ("reserved", C.c_int32 * 2)]
+                ("lanes", C.c_int32), ("reserved", C.c_int32 * 1)]
 
 
 THETA = ("jc_A", "jc_B", "jc_n", "jc_C", "jc_m", "mu")  # order of the adjoint's parameters
@@ -432,9 +432,10 @@ class Sim:
         return F
 
     def set_tuning(self, **kw) -> None:
-        """Launch configuration (results are independent of it): split_interact=0|1,
-        compact_pairs=0|1, stage_limit=0..STAGE_CAP (0: the full LDS stage),
-        xcd_chunk=0..XCD_CHUNK_MAX, sort_fast=0..SORT_FAST_MAX, sort_list>=0 (0: no bound)."""
+        """Launch configuration (results are independent of it): lanes=0|1|4|8 (0: by size),
+        stage_limit=0..STAGE_CAP (0: the full LDS stage), xcd_chunk=0..XCD_CHUNK_MAX,
+        sort_fast=0..SORT_FAST_MAX, sort_list>=0 (0: no bound); split_interact=0|1 and
+        compact_pairs=0|1 are accepted and change nothing."""
         t = Tuning()
         _check(lib().mfc_get_tuning(self._h, C.byref(t)), "mfc_get_tuning")
         for k, v in kw.items():
@@ -445,7 +446,7 @@ class Sim:
         t = Tuning()
         _check(lib().mfc_get_tuning(self._h, C.byref(t)), "mfc_get_tuning")
         return {"split_interact": t.split_interact, "compact_pairs": t.compact_pairs, "stage_limit": t.stage_limit,
-                "xcd_chunk": t.xcd_chunk, "sort_fast": t.sort_fast, "sort_list": t.sort_list}
+                "xcd_chunk": t.xcd_chunk, "sort_fast": t.sort_fast, "sort_list": t.sort_list, "lanes": t.lanes}
 
     def vjp_forward(self, nsteps: int, checkpoint_every: int, w0: int, w1: int) -> np.ndarray:
         """Run nsteps steps keeping a checkpoint every checkpoint_every steps; returns the mean
@@ -595,8 +596,7 @@ class Batch:
             pass
 
     def set_tuning(self, **kw) -> None:
-        """Launch configuration of every instance: split_interact=0|1, compact_pairs=0|1,
-        stage_limit=0..STAGE_CAP."""
+        """Launch configuration of every instance (as Sim.set_tuning)."""
         self._tuning.update({k: int(v) for k, v in kw.items()})
         t = Tuning()
         for k, v in self._tuning.items():

@@ -1,0 +1,110 @@
+"""The interaction over patches of cells: every number of threads per particle, and the path over the
+records in memory that takes what a patch's LDS copy does not (too many candidates, columns too
+dense for the masks, records that are not finite, an h that is not uniform, and entries past the
+launch's work items), against the oracle bit for bit (FP64) or each other (FP32C)."""
+import numpy as np
+import pytest
+
+import pymfc
+import oracle_binding as ob
+from parity import assert_bitwise, equal
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ["pos", "vel", "S", "rho", "p", "T", "eps_pl", "fc", "ft", "n", "R", "flags", "id", "hash"]
+
+
+def cut(prec=pymfc.PREC_FP64, thermal="contact", nx=61, ny=17, **kw):
+    return pymfc.cut_config(nx, ny, 10.0, thermal=thermal, speed_m_min=1000.0, jitter=0.01, precision=prec, **kw)
+
+
+@pytest.mark.parametrize("lanes", [1, 4, 8])
+@pytest.mark.parametrize("thermal", ["adiabatic", "contact", "pse"])
+def test_lanes_match_the_oracle(lanes, thermal):
+    cfg = cut(thermal=thermal)
+    g, o = pymfc.Sim(cfg), ob.OracleSim(cfg)
+    g.set_tuning(lanes=lanes)
+    assert g.tuning()["lanes"] == lanes
+    g.step(41)
+    o.step(41)
+    assert_bitwise(g, o, context=f"lanes {lanes}")
+    assert equal(g.force_history(), o.force_history())
+
+
+@pytest.mark.parametrize("thermal", ["adiabatic", "contact", "pse"])
+def test_fp32c_bits_do_not_depend_on_lanes(thermal):
+    cfg = cut(pymfc.PREC_FP32C, thermal=thermal)
+    runs = []
+    for lanes, limit in ((1, 0), (4, 0), (8, 0), (1, 1), (8, 1), (1, 400)):
+        g = pymfc.Sim(cfg)
+        g.set_tuning(lanes=lanes, stage_limit=limit)
+        g.step(41)
+        runs.append(g)
+    for g in runs[1:]:
+        for f in FIELDS:
+            assert equal(runs[0].field(f), g.field(f)), f
+        assert equal(runs[0].force_history(), g.force_history())
+
+
+def test_lanes_change_between_steps():
+    cfg = cut()
+    g, o = pymfc.Sim(cfg), ob.OracleSim(cfg)
+    for lanes in (1, 8, 4, 0):
+        g.set_tuning(lanes=lanes)
+        g.step(9)
+        o.step(9)
+    assert_bitwise(g, o, context="lanes changed")
+    with pytest.raises(pymfc.MfcError):
+        g.set_tuning(lanes=2)
+
+
+@pytest.mark.parametrize("lanes", [1, 4, 8])
+def test_uneven_h(lanes):
+    cfg = cut()
+    g, o = pymfc.Sim(cfg), ob.OracleSim(cfg)
+    g.set_tuning(lanes=lanes)
+    h = g.field("h")
+    h = h * (1.0 - 0.05 * (np.arange(h.size) % 3))
+    for s in (g, o):
+        s.set_field("h", h)
+        s.step(10)
+    assert_bitwise(g, o, context="uneven h")
+
+
+@pytest.mark.parametrize("lanes", [1, 4, 8])
+@pytest.mark.parametrize("place", ["scattered", "heaped"])
+def test_unusual_densities(lanes, place):
+    """Particles scattered over the whole grid fill many more patches than the initial lattice
+    (entries past the work items, windows of a few candidates); particles heaped into a few cells
+    fill several parts of a patch and more candidates than the LDS copy and the masks take."""
+    cfg = pymfc.config_rings(24)
+    g, o = pymfc.Sim(cfg), ob.OracleSim(cfg)
+    g.set_tuning(lanes=lanes)
+    rng = np.random.default_rng(7)
+    N = g.N
+    if place == "scattered":
+        pos = np.stack([rng.uniform(-0.19, 0.19, N), rng.uniform(-0.075, 0.075, N)], axis=1)
+    else:
+        pos = np.stack([rng.uniform(0.01, 0.022, N), rng.uniform(-0.01, 0.01, N)], axis=1)
+    for s in (g, o):
+        s.set_field("pos", pos)
+        s.step(3)
+    assert_bitwise(g, o, context=place)
+
+
+@pytest.mark.parametrize("lanes", [1, 4, 8])
+def test_nonfinite_and_blanked_neighbours(lanes):
+    cfg = cut(thermal="contact")
+    g, o = pymfc.Sim(cfg), ob.OracleSim(cfg)
+    g.set_tuning(lanes=lanes)
+    for s in (g, o):
+        s.step(10)
+    vt = o.field("vel_t")
+    free = np.nonzero(o.field("flags") == 0)[0]
+    vt[free[free.size // 2], 0] = np.nan
+    vt[free[free.size // 3], 1] = np.inf
+    for s in (g, o):
+        s.set_field("vel_t", vt)
+        s.step(20)
+    assert (o.field("flags") & pymfc.FLAG_BLANKED).sum() >= 1
+    assert_bitwise(g, o, context="non-finite")
