@@ -185,6 +185,110 @@ MFC_HD void pair_vjp(const dev_consts &k, const double *ri, const double *rj, bo
   if (want_j) { gj[R_X] -= b_xij; gj[R_Y] -= b_yij; }
 }
 
+// Both VJPs that link particle b with a neighbour a in support, for equal smoothing lengths: the
+// adjoint of b's record from the pair (b, a) of b's own sums (adjoints lb) and from the pair (a, b)
+// of a's (la); a side whose sums do not include the other passes zeros. The kernel value, its
+// gradient's factor, the stresses, the viscosity and the XSPH factor are the same for both pairs,
+// coordinate differences, velocity differences and kernel gradients change their sign: the terms
+// that are odd in them see lb - la, the even ones (velocity gradient, conduction) the sum weighted
+// with the other one's volume. Adds to gb what pair_vjp(b, a, want_i) and pair_vjp(a, b, want_j)
+// add. mech: neither is a tool particle; heat: the conduction sums are used.
+template <class RB, class RA, class LB, class LA>
+MFC_HD void pair_vjp_sym(const dev_consts &k, const RB &rb, const RA &ra, bool mech, bool heat, const LB &lb,
+                         const LA &la, double *gb) {
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma clang fp contract(fast)
+#endif
+  const double xij = rb(R_X) - ra(R_X), yij = rb(R_Y) - ra(R_Y);
+  const double rr2 = xij * xij + yij * yij;
+  const double h = rb(R_H);
+  const double r = sqrt(rr2), inv_r = 1.0 / r;
+  const double h1 = 1.0 / h, q = r * h1, fac = PI_FAC * h1 * h1;
+  double w, dw, F, dF;  // as spline()
+  if (q > 1) {
+    const double m = 2 - q, m2 = m * m;
+    w = fac * 0.25 * m2 * m2 * m2;
+    dw = fac * (-1.5) * m2 * m2 * m * h1;
+    F = fac * (-0.75) * m2 * h1 * inv_r;
+    dF = fac * (-0.75) * h1 * (-2.0 * m * h1 * inv_r - m2 * inv_r * inv_r);
+  } else {
+    w = fac * (1 - 1.5 * q * q * (1 - 0.5 * q));
+    dw = fac * h1 * (-3.0 * q + 2.25 * q * q);
+    F = fac * (-3.0) * h1 * h1 * (1 - 0.75 * q);
+    dF = fac * 2.25 * h1 * h1 * h1;
+  }
+  const double gx = F * xij, gy = F * yij, m = k.mass;
+  double b_w = 0, b_F = 0, b_gx = 0, b_gy = 0, b_xij = 0, b_yij = 0, b_rr2 = 0;
+  if (mech) {
+    const double du = ra(R_U) - rb(R_U), dv = ra(R_V) - rb(R_V);
+    const double Va = ra(R_VOL), Vb = rb(R_VOL);
+    const double L0 = lb(L_VD0) * Va + la(L_VD0) * Vb, L1 = lb(L_VD1) * Va + la(L_VD1) * Vb;
+    const double L2 = lb(L_VD2) * Va + la(L_VD2) * Vb, L3 = lb(L_VD3) * Va + la(L_VD3) * Vb;
+    double b_du = L0 * gx + L1 * gy, b_dv = L2 * gx + L3 * gy;
+    b_gx += L0 * du + L2 * dv;
+    b_gy += L1 * du + L3 * dv;
+    gb[R_VOL] += du * (la(L_VD0) * gx + la(L_VD1) * gy) + dv * (la(L_VD2) * gx + la(L_VD3) * gy);
+    const double wd1 = 1.0 / k.wdeltap, f1 = w * wd1, f2 = f1 * f1, fab = f2 * f2;
+    const double RX = rb(R_RXX) + ra(R_RXX), RY = rb(R_RXY) + ra(R_RXY), RZ = rb(R_RYY) + ra(R_RYY);
+    const double sx = rb(R_AXX) + ra(R_AXX) + fab * RX;
+    const double sy = rb(R_AXY) + ra(R_AXY) + fab * RY;
+    const double sz = rb(R_AYY) + ra(R_AYY) + fab * RZ;
+    const double S0 = lb(L_SD0) - la(L_SD0), S1 = lb(L_SD1) - la(L_SD1), S2 = lb(L_SD2) - la(L_SD2),
+                 S3 = lb(L_SD3) - la(L_SD3);
+    const double b_sx = m * S0 * gx, b_sy = m * (S1 * gy + S2 * gx), b_sz = m * S3 * gy;
+    b_gx += m * (S0 * sx + S2 * sy);
+    b_gy += m * (S1 * sy + S3 * sz);
+    const double b_fab = b_sx * RX + b_sy * RY + b_sz * RZ;
+    b_w += b_fab * 4.0 * f2 * f1 * wd1;
+    gb[R_AXX] += b_sx; gb[R_AXY] += b_sy; gb[R_AYY] += b_sz;
+    gb[R_RXX] += b_sx * fab; gb[R_RXY] += b_sy * fab; gb[R_RYY] += b_sz * fab;
+    const double vijx = -du, vijy = -dv;
+    const double vdx = vijx * xij + vijy * yij;
+    const double inv_rho = 1.0 / (0.5 * (rb(R_RHO) + ra(R_RHO)));
+    double b_rhoij = 0, b_vijx = 0, b_vijy = 0;
+    if (vdx < 0.) {
+      const double cij = 0.5 * (rb(R_C) + ra(R_C));
+      const double inv_D = 1.0 / (rr2 + k.av_eta * k.av_eta * h * h);
+      const double mu = h * vdx * inv_D;
+      const double Pi = (-k.av_alpha * cij * mu + k.av_beta * mu * mu) * inv_rho;
+      const double P = -m * Pi;
+      const double T0 = lb(L_VT0) - la(L_VT0), T1 = lb(L_VT1) - la(L_VT1);
+      const double b_Pi = -m * (T0 * gx + T1 * gy);
+      b_gx += T0 * P;
+      b_gy += T1 * P;
+      const double b_mu = b_Pi * (-k.av_alpha * cij + 2.0 * k.av_beta * mu) * inv_rho;
+      b_rhoij += -b_Pi * Pi * inv_rho;
+      const double b_vdx = b_mu * h * inv_D;
+      b_rr2 += -b_mu * mu * inv_D;
+      b_vijx += b_vdx * xij; b_vijy += b_vdx * yij;
+      b_xij += b_vdx * vijx; b_yij += b_vdx * vijy;
+      gb[R_C] += 0.5 * (b_Pi * (-k.av_alpha * mu) * inv_rho);
+    }
+    const double xf = -k.xsph_eps * m * inv_rho, xs = xf * w;
+    const double X0 = lb(L_XT0) - la(L_XT0), X1 = lb(L_XT1) - la(L_XT1);
+    const double b_xs = X0 * vijx + X1 * vijy;
+    b_vijx += X0 * xs; b_vijy += X1 * xs;
+    b_w += b_xs * xf;
+    b_rhoij += -b_xs * xs * inv_rho;
+    gb[R_U] -= b_du - b_vijx; gb[R_V] -= b_dv - b_vijy;
+    gb[R_RHO] += 0.5 * b_rhoij;
+  }
+  if (heat) {
+    const double dT = rb(R_T) - ra(R_T);
+    const double Lt = 2.0 * (lb(L_TL) * ra(R_VOL) - la(L_TL) * rb(R_VOL));
+    b_F += Lt * dT;
+    gb[R_T] += Lt * F;
+    gb[R_VOL] -= la(L_TL) * 2.0 * dT * F;
+  }
+  b_F += b_gx * xij + b_gy * yij;
+  b_xij += b_gx * F;
+  b_yij += b_gy * F;
+  b_rr2 += (b_w * dw + b_F * dF) * (0.5 * inv_r);
+  b_xij += 2.0 * xij * b_rr2;
+  b_yij += 2.0 * yij * b_rr2;
+  gb[R_X] += b_xij; gb[R_Y] += b_yij;
+}
+
 // one term of the PSE sum of particle i (interactions_gpu.cu:130-139, no cutoff, promoted):
 // (T_j - T_i) 4/(pi h^4) exp(-r^2/h^2) m / rho_j
 MFC_HD double pse_fwd(const dev_consts &k, const double *ri, const double *rj) {

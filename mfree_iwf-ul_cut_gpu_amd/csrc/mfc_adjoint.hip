@@ -4,35 +4,39 @@
 //
 // Tape: the state at the start of every K-th step (state block, positional block, stale cell
 // ids of blanked particles, tool) is copied into a checkpoint. The backward pass walks the
-// checkpoint segments from last to first; each segment is replayed forward with the step
-// kernels to recover the start state of each of its steps, and the steps are then reversed
-// one by one:
-//   F1  binning          cell ids and the stable counting sort of the restored state
-//   F2  predict          with the sorted copy of the start state (gather, predictor, EOS,
-//                        artificial stress, records)
-//   F3  sums             neighbour sums of every particle, kept from the segment's replay (the
-//                        replayed interaction stores them, one slot per step of the segment)
-//   B1  kb_adj_tail      VJP of everything after the sums, per particle (tail_vjp), and the
-//                        per-tile theta partials of the step (kb_adj_theta adds them up)
-//   B2  kb_adj_pull      VJP of the neighbour sums with respect to the records: each particle
-//                        pulls the contributions of the pairs it takes part in over the same
-//                        symmetric 5 x 5 cell window, in a fixed order (no atomics), the pairs
-//                        of the neighbours' sums and of its own sums in one walk
-//   B3  kb_adj_record    VJP of the record and predictor, then the scatter back to the
-//                        storage order of the previous step (inverse of the sort permutation)
+// checkpoint segments from last to first. Each segment is replayed forward with the step kernels,
+// whose descriptors (one per step of the segment) point each step's output at a slot of its own:
+// the next slot's start state and normals, this slot's sort (sorted cell ids, cell ranges,
+// permutation and its inverse, list of patches), its neighbour sums and secant results and the tool.
+// So the replay is two launches per step and nothing is computed or copied again for the reverse
+// steps, which take two each:
+//   kb_adj_tail     the VJP of the record and predictor of the step after (record_vjp) and the
+//                   gather of its result through the inverse of its sort, then the VJP of
+//                   everything after the neighbour sums of this step (tail_vjp), per particle, its
+//                   record for the pull, and the per-tile theta partials
+//   kb_adj_pull     VJP of the neighbour sums with respect to the records: each particle pulls the
+//                   contributions of the pairs it takes part in over its symmetric 5 x 5 cell
+//                   window, in a fixed order (no atomics); one more work-group per instance adds up
+//                   the theta partials
+// and kb_adj_record takes the segment's first step back to the storage order of its start state.
+// (With a copy of each replayed state, and the binning, sort, sorted state and records of the
+// reversed step computed again, a replayed and reversed step took 12 launches, and launching them
+// took longer than running them.)
 // The positional contact normal (read by the friction heat of the next step at the same sorted
 // index) carries its adjoint from step to step without permutation, like its forward value.
 //
 // A group of instances that ran the same taped forward (one handle, or the instances of a
 // batch) is reversed together: every phase, the checkpoint copies included, is one launch over
-// the group's (instance, tile) work table, with per-instance descriptors in device memory, as
-// the batched forward step runs. Each instance computes exactly what it computes alone.
+// the group's work tables, with per-instance descriptors in device memory, as the batched forward
+// step runs. Each instance computes exactly what it computes alone.
 //
 // Derivatives follow the smooth map of promote_fp64 = 1 with a tight secant tolerance; the
 // handle must use FP64 records.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
+#include <memory>
 #include <vector>
 
 #include "mfc_adjoint.h"
@@ -61,33 +65,33 @@ int padded(int ntiles) { return ((ntiles + 7) / 8) * 8; }
 
 static_assert(L_N == ACC_N, "a replay slot holds the interaction's neighbour sums in the tail's order");
 
-// one instance of the backward pass as its kernels see it (device memory, one per instance)
+constexpr int LAM = 16;  // doubles per particle of lam_acc (ACC_N, padded to whole 16-byte pieces)
+
+// one instance of the backward pass as its kernels see it (device memory, one per instance). The
+// slots of the segment's steps follow each other in each array; state has one more, for the
+// last step's end state, as have normal and tool
 struct adj_args {
   dev_consts k;
   int ntiles;
-  const double *st;                 // sorted start state of the reversed step (TS_* order, stride N)
-  const int *flags;                 // its flags
-  dpositional pos;                  // replay positional block
-  const double *rec;                // FP64 neighbour records
-  const int *key_sorted, *offsets, *perm;
-  const mfc_tool_state *tool_now;   // the tool after the reversed step's move
-  double *acc_seg;                  // the replay's neighbour sums and secant results, one slot of
-                                    // (ACC_N + 1) x N per step
-  size_t acc_stride;                // doubles per slot
-  double *lam_acc, *lam_s[2], *lam_n, *g_s, *g_rec, *theta_part, *theta_acc;
+  char *state;                      // start states in storage order (state_block_bytes each)
+  size_t state_bytes;
+  double *normal;                   // normals before the step, nx then ny (2 N)
+  int *perm, *spos, *key_sorted;    // N each
+  int *offsets;                     // num_cell + 1 each
+  int2 *plist;                      // list of patches (list_len each) and its length
+  int *plen;
+  int list_len, ncell1;
+  mfc_tool_state *tool;             // before the step's move
+  double *acc;                      // neighbour sums and secant results, (ACC_N + 1) N each
+  double *lam;                      // adjoint of a segment's end state, in the storage order of the next one's start
+  double *lam_n;                    // adjoint of the positional normals
+  double *g_s[2];                   // adjoint of the sorted start state by parity of the slot
+  double *lam_acc, *rec, *g_rec;    // LAM, REC_DOUBLES and REC_DOUBLES per particle, sorted order
+  double *theta_part, *theta_acc;
   double Fb[2];                     // cotangent over the window length
-  // checkpoint copies: the live replay buffers and the instance's snapshots
-  size_t state_words, pos_words;    // 8-byte words of a state block and of a positional block
-  uint64_t *live_state[2];
-  uint64_t *live_pos;
-  int *live_keys;                   // the handle's sorted cell ids
-  int *chunk_sums[2];               // the handle's chunk sums
-  int nscan;
-  int *pcnt;                        // and patch counts
-  int npatch;
-  int *plen;                        // 2 list lengths
-  mfc_tool_state *live_tool;        // 2 replay tool states
-  const snapshot *ckpt, *seg;       // checkpoints of the tape, and the start states of a segment
+  const snapshot *ckpt;
+  int *chunk_sums[2], *pcnt;        // the handle's binning scratch
+  int nscan, npatch;
 };
 
 // an instance's descriptor read through the constant address space: the pointers loaded from it
@@ -97,59 +101,60 @@ struct adj_args {
     *(const __attribute__((address_space(4))) adj_args *)(D + (q))
 
 // ------------------------------------------------------------------ checkpoint copies
-// dir 0: a snapshot (ckpt[idx] or seg[idx]) into replay set 0, the positional block, the cell
-// ids and replay tool 0, and the chunk sums and patch counts cleared for the binning of that
-// state; dir 1: replay set wa, the positional block, the cell ids and replay
-// tool wa into seg[idx]. Grid (copy_blocks, instances).
-__global__ __launch_bounds__(256) void kb_adj_copy(const adj_args *__restrict__ D, int dir, int from_ckpt, int idx,
-                                                   int wa) {
+// the checkpoint of segment sg into slot 0, and the binning scratch cleared for the
+// binning of that state. Grid (copy_blocks, instances).
+__global__ __launch_bounds__(256) void kb_adj_restore(const adj_args *__restrict__ D, int sg) {
   MFC_ADJ_ARGS(d, blockIdx.y);
-  const snapshot sn = from_ckpt ? d.ckpt[idx] : d.seg[idx];
-  const int lw = dir ? wa : 0;
-  uint64_t *ls = d.live_state[lw];
-  const uint64_t *src_s = dir ? ls : (const uint64_t *)sn.state;
-  uint64_t *dst_s = dir ? (uint64_t *)sn.state : ls;
-  const uint64_t *src_p = dir ? d.live_pos : (const uint64_t *)sn.pos;
-  uint64_t *dst_p = dir ? (uint64_t *)sn.pos : d.live_pos;
-  const int *src_k = dir ? d.live_keys : sn.keys;
-  int *dst_k = dir ? sn.keys : d.live_keys;
+  const snapshot sn = d.ckpt[sg];
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  for (size_t q = i0; q < d.state_words; q += stride) dst_s[q] = src_s[q];
-  for (size_t q = i0; q < d.pos_words; q += stride) dst_p[q] = src_p[q];
-  for (size_t q = i0; q < (size_t)d.k.N; q += stride) dst_k[q] = src_k[q];
-  if (!dir)
-    for (size_t q = i0; q < (size_t)d.nscan; q += stride) d.chunk_sums[0][q] = d.chunk_sums[1][q] = 0;
-  if (!dir)
-    for (size_t q = i0; q < (size_t)d.npatch; q += stride) d.pcnt[q] = 0;
+  const size_t N = d.k.N;
+  uint64_t *st = (uint64_t *)d.state;
+  const uint64_t *src = (const uint64_t *)sn.state;
+  for (size_t q = i0; q < d.state_bytes / sizeof(uint64_t); q += stride) st[q] = src[q];
+  const double *pos = (const double *)sn.pos;  // nx, ny first
+  for (size_t q = i0; q < 2 * N; q += stride) d.normal[q] = pos[q];
+  for (size_t q = i0; q < N; q += stride) d.key_sorted[q] = sn.keys[q];
+  for (size_t q = i0; q < (size_t)d.nscan; q += stride) d.chunk_sums[0][q] = d.chunk_sums[1][q] = 0;
+  for (size_t q = i0; q < (size_t)d.npatch; q += stride) d.pcnt[q] = 0;
   if (i0 == 0) {
-    if (dir) {
-      *sn.tool = d.live_tool[lw];
-    } else {
-      d.live_tool[0] = *sn.tool;
-      d.plen[0] = d.plen[1] = 0;
-    }
+    d.tool[0] = *sn.tool;
+    d.plen[0] = 0;
   }
 }
 
-// points the replay descriptors of both parities at the neighbour-sum slot of a step (one
-// thread per instance; the next launches read the descriptors after this one completes)
-__global__ __launch_bounds__(64) void kb_adj_acc_slot(inst_args *__restrict__ rep, const adj_args *__restrict__ D,
-                                                      int n, int slot) {
-  const int q = blockIdx.x * 64 + threadIdx.x;
-  if (q >= n) return;
-  double *a = D[q].acc_seg + (size_t)slot * D[q].acc_stride;
-  rep[q].acc_out = a;
-  rep[n + q].acc_out = a;
+// a checkpoint of the current state (the sources of one handle)
+__global__ __launch_bounds__(256) void k_adj_save(snapshot sn, const uint64_t *__restrict__ state, size_t state_words,
+                                                  const uint64_t *__restrict__ pos, size_t pos_words,
+                                                  const int *__restrict__ keys, int N,
+                                                  const mfc_tool_state *__restrict__ tool) {
+  const size_t stride = (size_t)gridDim.x * blockDim.x;
+  const size_t i0 = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  for (size_t q = i0; q < state_words; q += stride) ((uint64_t *)sn.state)[q] = state[q];
+  for (size_t q = i0; q < pos_words; q += stride) ((uint64_t *)sn.pos)[q] = pos[q];
+  for (size_t q = i0; q < (size_t)N; q += stride) sn.keys[q] = keys[q];
+  if (i0 == 0) *sn.tool = *tool;
 }
 
 // ------------------------------------------------------------------ B1: per-particle tail
-// st: sorted start state; acc: the step's neighbour sums (slot of the segment's replay);
-// lam_s[cur]: adjoint of the end state of the step (same layout); lam_n: adjoint of the positional
-// normal written by this step (in) and of the one read by it (out); in_win: the step's force is
-// in the loss window
+__device__ inline const double *slot_state(const __attribute__((address_space(4))) adj_args &d, int slot) {
+  return (const double *)(d.state + (size_t)slot * d.state_bytes);
+}
+__device__ inline const int *slot_flags(const __attribute__((address_space(4))) adj_args &d, int slot) {
+  return (const int *)(slot_state(d, slot) + (size_t)DSTATE_DOUBLES * d.k.N);
+}
+// EOS pressure of the predicted density (0 for a tool particle: no sum reads it)
+__device__ inline double eos_pressure(const dev_consts &k, const double *s, int flags) {
+  if (flags & MFC_FLAG_TOOL) return 0.;
+  const double rho = flags & MFC_FLAG_BLANKED ? s[TS_RHO] : s[TS_RHO] + 0.5 * k.dt * s[TS_RHOT];
+  return k.c0 * k.c0 * (rho - k.rho0);
+}
+
+// step `slot` of the segment; last: the segment's last step, whose end state's adjoint is in lam
+// (else it comes from step slot + 1); in_win: its force is in the loss window. lam_n: adjoint of the positional normal written by this step
+// (in) and of the one read by it (out)
 __global__ __launch_bounds__(TILE) void kb_adj_tail(const adj_args *__restrict__ D, const int2 *__restrict__ work,
-                                                    int nwork, int cur, int in_win, int slot) {
+                                                    int nwork, int slot, int last, int in_win) {
   const int w = xcd_tile(blockIdx.x, nwork);
   if (w < 0) return;
   const int2 it = work[w];
@@ -158,31 +163,55 @@ __global__ __launch_bounds__(TILE) void kb_adj_tail(const adj_args *__restrict__
   const int t = it.y;
   const int i = t * TILE + threadIdx.x;
   const size_t N = k.N;
-  const double *__restrict__ acc = d.acc_seg + (size_t)slot * d.acc_stride;
   double th[6] = {0., 0., 0., 0., 0., 0.};
   if (i < k.N) {
+    double ob[TS_N];
+    if (last) {
+#pragma unroll
+      for (int q = 0; q < TS_N; q++) ob[q] = d.lam[q * N + i];
+    } else {  // particle i of this step's end state is at a in the next step's sorted order
+      const int a = d.spos[(size_t)(slot + 1) * N + i];
+      const double *__restrict__ st = slot_state(d, slot + 1);
+      const double *__restrict__ gs = d.g_s[(slot + 1) & 1];
+      double s[TS_N], br[REC_DOUBLES];
+#pragma unroll
+      for (int q = 0; q < TS_N; q++) { s[q] = st[q * N + i]; ob[q] = gs[q * N + a]; }
+      const double2 *__restrict__ g2 = reinterpret_cast<const double2 *>(d.g_rec + (size_t)REC_DOUBLES * a);
+#pragma unroll
+      for (int q = 0; q < REC_DOUBLES / 2; q++) { const double2 v = g2[q]; br[2 * q] = v.x; br[2 * q + 1] = v.y; }
+      const int fl = slot_flags(d, slot + 1)[i] & FLAG_MASK;
+      record_vjp(k, s, fl, eos_pressure(k, s, fl), br, ob);
+    }
+    const int sidx = d.perm[(size_t)slot * N + i];
+    const double *__restrict__ st = slot_state(d, slot);
     tail_in in;
 #pragma unroll
-    for (int q = 0; q < TS_N; q++) in.s[q] = d.st[q * N + i];
-    in.p = d.pos.p[i];
-    in.nx = d.pos.nx[i];
-    in.ny = d.pos.ny[i];
-    in.flags = d.flags[i];
+    for (int q = 0; q < TS_N; q++) in.s[q] = st[q * N + sidx];
+    in.flags = slot_flags(d, slot)[sidx] & FLAG_MASK;
+    in.p = eos_pressure(k, in.s, in.flags);
+    const double *__restrict__ nn = d.normal + (size_t)slot * 2 * N;
+    in.nx = nn[i];
+    in.ny = nn[N + i];
     in.pse_flag_zero = k.pse_quirk && i >= k.N / 2;
+    const double *__restrict__ acc = d.acc + (size_t)slot * (L_N + 1) * N;
 #pragma unroll
     for (int q = 0; q < L_N; q++) in.acc[q] = acc[q * N + i];
     in.dl_rec = acc[L_N * N + i];
-    const double *lam_s = d.lam_s[cur];
-    double ob[TS_N];
+    double p = in.p, R3[3] = {0., 0., 0.}, rec[REC_DOUBLES];
+    record_fwd(k, in.s, in.flags, p, R3, rec);
+    rec[R_FLAGS] = bits_to_double(in.flags);
+    double2 *__restrict__ rdst = reinterpret_cast<double2 *>(d.rec + (size_t)REC_DOUBLES * i);
 #pragma unroll
-    for (int q = 0; q < TS_N; q++) ob[q] = lam_s[q * N + i];
+    for (int q = 0; q < REC_DOUBLES / 2; q++) rdst[q] = make_double2(rec[2 * q], rec[2 * q + 1]);
     const double nbx = d.lam_n[i], nby = d.lam_n[N + i];
     tail_grad g;
-    tail_vjp(k, *d.tool_now, in, ob, nbx, nby, in_win ? d.Fb[0] : 0., in_win ? d.Fb[1] : 0., g, nullptr);
+    tail_vjp(k, d.tool[slot + 1], in, ob, nbx, nby, in_win ? d.Fb[0] : 0., in_win ? d.Fb[1] : 0., g, nullptr);
+    double *__restrict__ gs = d.g_s[slot & 1];
 #pragma unroll
-    for (int q = 0; q < TS_N; q++) d.g_s[q * N + i] = g.s[q];
+    for (int q = 0; q < TS_N; q++) gs[q * N + i] = g.s[q];
+    double2 *__restrict__ ldst = reinterpret_cast<double2 *>(d.lam_acc + (size_t)LAM * i);
 #pragma unroll
-    for (int q = 0; q < L_N; q++) d.lam_acc[q * N + i] = g.acc[q];
+    for (int q = 0; q < L_N / 2; q++) ldst[q] = make_double2(g.acc[2 * q], g.acc[2 * q + 1]);
     d.lam_n[i] = g.nx;
     d.lam_n[N + i] = g.ny;
 #pragma unroll
@@ -205,11 +234,9 @@ __global__ __launch_bounds__(TILE) void kb_adj_tail(const adj_args *__restrict__
   }
 }
 
-// adds the step's theta partials of instance blockIdx.x to its running totals: lane l sums the
-// tiles l, l + TILE, ... in ascending order, lane sums reduced by halving strides
-__global__ __launch_bounds__(TILE) void kb_adj_theta(const adj_args *__restrict__ D) {
-  MFC_ADJ_ARGS(d, blockIdx.x);
-  __shared__ double red[6][TILE];
+// adds the step's theta partials of an instance to its running totals: lane l sums the tiles l,
+// l + TILE, ... in ascending order, lane sums reduced by halving strides; red: 6 TILE doubles of LDS
+__device__ inline void add_theta(const __attribute__((address_space(4))) adj_args &d, double (*red)[TILE]) {
   double a[6] = {0., 0., 0., 0., 0., 0.};
   for (int u = threadIdx.x; u < d.ntiles; u += TILE)
 #pragma unroll
@@ -229,95 +256,246 @@ __global__ __launch_bounds__(TILE) void kb_adj_theta(const adj_args *__restrict_
 // ------------------------------------------------------------------ B2: pull over pairs
 // For each window member a of particle b, both kinds of pair that link them: the pairs (a, b) of
 // a's sums that include b, with the adjoint of a's sums, and the pairs (b, a) of b's own sums,
-// with b's adjoint; a's record is loaded once for both, and g_rec[b] is written. (Two passes,
-// one per kind, kept fewer records live per lane at the same 2 waves per SIMD and walked every
-// window twice: 71 + 62 us per step against 113 us for the one pass on the 37.5k cut.)
-// PULL_LANES consecutive lanes share a particle: lane r takes the window candidates r,
-// r + PULL_LANES, ... (numbered column by column, as the forward walk numbers them), and the
-// lanes' partial sums are added by a butterfly of shuffles, which gives every lane the same bits
-// (((g0 + g1) + (g2 + g3)) + ...). The pass is latency-bound (a long dependent chain of record
-// loads and pair adjoints per particle, 2 waves per SIMD at its 256 VGPRs; forcing 3 waves
-// spills 336 bytes per lane and takes 40 % longer), so more lanes per particle shorten the
-// chain. The count is fixed, so that an instance's gradient has the same bits alone and in a
-// batch. Measured backward pass, ms per step with 2 / 4 / 8 lanes: 6k particles 0.357 / 0.317 /
-// 0.286, 37.5k 0.340 / 0.313 / 0.295, the 32-instance batch of 577k 1.80 / 1.88 / 1.92 (the
-// calibration cuts are the ones the reverse mode is for). A block takes the PULL_LANES-th part
-// of a tile: grid padded(ntiles * PULL_LANES).
+// with b's adjoint, in one evaluation (pair_vjp_sym). PULL_LANES neighbouring lanes share a
+// particle: they list its pairs in the window's order, lane r takes the pairs r, r + PULL_LANES,
+// ..., and the lanes' partial sums are added by a butterfly of shuffles, which gives every lane the
+// same bits (((g0 + g1) + (g2 + g3)) + ...). The count is fixed, and so is the lanes' split of a
+// window, so that an instance's gradient has the same bits alone and in a batch. A work-group takes
+// a part of a patch of cells, as the interaction does, with the records and the adjoints of the sums
+// of its window candidates staged in LDS (240 bytes each; three work-groups to a CU): read from
+// memory per pair, by one work-group per 32 particles of the sorted order, they were 30 gathers of
+// 64 scattered lines, and the pass took 95 us at 37.5k particles.
 constexpr int PULL_LANES = 8;
+constexpr int PULL_CAP = 192;  // window candidates a work-group stages
+constexpr int PULL_PIECES = REC_DOUBLES / 2 + ACC_N / 2;  // 16-byte pieces: the record, then the adjoints
 
-__global__ __launch_bounds__(TILE) void kb_adj_pull(const adj_args *__restrict__ D, const int2 *__restrict__ work,
-                                                    int nwork) {
-  const int u = xcd_tile(blockIdx.x, nwork * PULL_LANES);
-  if (u < 0) return;
-  const int2 it = work[u / PULL_LANES];
-  MFC_ADJ_ARGS(d, it.x);
-  const dev_consts &k = D[it.x].k;
-  const int r = threadIdx.x % PULL_LANES;
-  const int b = it.y * TILE + (u % PULL_LANES) * (TILE / PULL_LANES) + threadIdx.x / PULL_LANES;
-  const bool live = b < k.N;  // the lanes of a particle stay together for the shuffles
-  const size_t N = k.N;
-  const double *__restrict__ rec = d.rec;
-  const int *__restrict__ flags = d.flags;
-  const double *__restrict__ lam_acc = d.lam_acc;
-  double *__restrict__ g_rec = d.g_rec;
-  const bool pse = k.pse != 0;
-  double rb[REC_DOUBLES], gb[REC_DOUBLES], lb[L_N], dummy[REC_DOUBLES];
-  const int bb = live ? b : 0;
-#pragma unroll
-  for (int q = 0; q < REC_DOUBLES; q++) {
-    rb[q] = rec[REC_DOUBLES * (size_t)bb + q];
-    gb[q] = 0.;
-  }
-#pragma unroll
-  for (int q = 0; q < L_N; q++) lb[q] = lam_acc[q * N + bb];
-  const int fb = flags[bb];
-  const bool blank_b = fb & MFC_FLAG_BLANKED, tool_b = fb & MFC_FLAG_TOOL;
-  const double ta_b = pse ? 0. : (tool_b ? k.alpha_tool : k.alpha_wp);
-  const bool mech_b = !blank_b && (!pse || !tool_b);
-  const bool pse_b = !blank_b && pse && k.thermal_wp;
-  const window w = make_window(k, d.offsets, d.key_sorted[bb]);
-  const int total = live ? w.total : 0;
-  for (int t = r; t < total; t += PULL_LANES) {
-    const int a = w.at(t);
-    if (a == b) continue;
-    const int fa = flags[a];
-    const bool blank_a = fa & MFC_FLAG_BLANKED, tool_a = fa & MFC_FLAG_TOOL;
-    const bool mech_a = !blank_a && (!pse || !tool_a);
-    const bool pse_a = !blank_a && pse && k.thermal_wp;
-    const double *pa = rec + REC_DOUBLES * (size_t)a;
-    const double dx = pa[R_X] - rb[R_X], dy = pa[R_Y] - rb[R_Y];
-    const double rr2 = dx * dx + dy * dy;
-    const double ha = pa[R_H], hb = rb[R_H];
-    const bool mech1 = mech_a && !blank_b && rr2 < 4 * ha * ha && rr2 >= 1e-8;  // a's sums include b
-    const bool mech2 = mech_b && !blank_a && rr2 < 4 * hb * hb && rr2 >= 1e-8;  // b's sums include a
-    if (!mech1 && !pse_a && !mech2 && !pse_b) continue;
-    double ra[REC_DOUBLES];
-#pragma unroll
-    for (int q = 0; q < REC_DOUBLES; q++) ra[q] = pa[q];
-    if (mech1 || pse_a) {
-      double la[L_N];
-#pragma unroll
-      for (int q = 0; q < L_N; q++) la[q] = lam_acc[q * N + a];
-      const double ta_a = pse ? 0. : (tool_a ? k.alpha_tool : k.alpha_wp);
-      if (mech1) pair_vjp(k, ra, rb, tool_a, tool_b, ta_a, la, false, true, dummy, gb);
-      if (pse_a) pse_vjp(k, ra, rb, la[L_TPSE], false, true, dummy, gb);
-    }
-    if (mech2) pair_vjp(k, rb, ra, tool_b, tool_a, ta_b, lb, true, false, gb, dummy);
-    if (pse_b) pse_vjp(k, rb, ra, lb[L_TPSE], true, false, gb, dummy);
-  }
+struct pull_mem {
+  double2 piece[PULL_PIECES][PULL_CAP + 1];
+  int table[PATCH_TABLE];
+  int col_first[PATCH_COLS + 1], col_shift[PATCH_COLS], own_first[PATCH_COLS + 1];
+  unsigned char list[TILE / PULL_LANES][64];
+};
+
+// a pair of window members by their flags: whether the sums of a take b when it is in a's support
+// (and not at the same place), and those of b take a
+struct pull_pair {
+  bool of_a, of_b;
+};
+__device__ inline pull_pair pull_flags(const dev_consts &k, int fa, int fb) {
+  const bool blank = (fa | fb) & MFC_FLAG_BLANKED, pse = k.pse != 0;
+  return {!blank && (!pse || !(fa & MFC_FLAG_TOOL)), !blank && (!pse || !(fb & MFC_FLAG_TOOL))};
+}
+
+// the lanes' sums of a particle added and written (every lane of the particle calls it)
+__device__ inline void pull_store(double *gb, int r, double *__restrict__ dst) {
 #pragma unroll
   for (int st = 1; st < PULL_LANES; st <<= 1)
 #pragma unroll
-    for (int q = 0; q < REC_DOUBLES; q++) gb[q] = gb[q] + __shfl_xor(gb[q], st, 64);
-  if (live && r == 0) {
+    for (int q = 0; q < REC_DOUBLES; q++) gb[q] = gb[q] + __shfl_xor(gb[q], st, PULL_LANES);
+  if (r == 0) {
 #pragma unroll
-    for (int q = 0; q < REC_DOUBLES; q++) g_rec[q * N + b] = gb[q];
+    for (int q = 0; q < REC_DOUBLES / 2; q++)
+      reinterpret_cast<double2 *>(dst)[q] = make_double2(gb[2 * q], gb[2 * q + 1]);
   }
 }
 
+// one entry of the list from the records in memory: what the staged path does not take (more
+// candidates than the stage holds, an h that is not uniform, entries past the work items). Lane r
+// tests and takes the candidates r, r + PULL_LANES, ...
+__device__ inline void pull_rest(const adj_args *__restrict__ D, int inst, int slot, int patch, int part) {
+  MFC_ADJ_ARGS(d, inst);
+  const dev_consts &k = D[inst].k;
+  const size_t N = k.N;
+  const int *__restrict__ offsets = d.offsets + (size_t)slot * d.ncell1, *__restrict__ keys = d.key_sorted + (size_t)slot * N;
+  const int nrb = patch_rows(k), pc = patch / nrb, pr = patch - pc * nrb;
+  const int r0 = pr * k.patch_s, r1 = r0 + k.patch_s < k.gny ? r0 + k.patch_s : k.gny;
+  const int c0 = pc * k.patch_w, c1 = c0 + k.patch_w < k.gnx ? c0 + k.patch_w : k.gnx;
+  const int r = threadIdx.x % PULL_LANES;
+  int n = part * k.patch_slots + (int)threadIdx.x / PULL_LANES, b = -1;
+  for (int c = c0; c < c1 && b < 0; c++) {
+    const int first = offsets[c * k.gny + r0], count = offsets[c * k.gny + r1] - first;
+    if (n < count) b = first + n;
+    n -= count;
+  }
+  if (b < 0) return;  // whole groups of lanes
+  const double *__restrict__ rec = d.rec, *__restrict__ lam = d.lam_acc;
+  const double *rb = rec + (size_t)REC_DOUBLES * b, *lb = lam + (size_t)LAM * b;
+  double gb[REC_DOUBLES], dummy[REC_DOUBLES];
+#pragma unroll
+  for (int q = 0; q < REC_DOUBLES; q++) gb[q] = 0.;
+  const int fb = double_to_bits(rb[R_FLAGS]);
+  const bool pse = k.pse != 0, tool_b = fb & MFC_FLAG_TOOL;
+  const double ta_b = pse ? 0. : (tool_b ? k.alpha_tool : k.alpha_wp);
+  const bool pse_b = !(fb & MFC_FLAG_BLANKED) && pse && k.thermal_wp;
+  const window w = make_window(k, offsets, keys[b]);
+  for (int t = r; t < w.total; t += PULL_LANES) {
+    const int a = w.at(t);
+    if (a == b) continue;
+    asm volatile("" ::: "memory");  // b's record is read again for each pair: kept, it spills
+    const double *ra = rec + (size_t)REC_DOUBLES * a, *la = lam + (size_t)LAM * a;
+    const int fa = double_to_bits(ra[R_FLAGS]);
+    const bool tool_a = fa & MFC_FLAG_TOOL;
+    const double dx = ra[R_X] - rb[R_X], dy = ra[R_Y] - rb[R_Y], rr2 = dx * dx + dy * dy;
+    const pull_pair m = pull_flags(k, fa, fb);
+    const double ha = ra[R_H], hb = rb[R_H];
+    const bool of_a = m.of_a && rr2 < 4 * ha * ha && rr2 >= 1e-8, of_b = m.of_b && rr2 < 4 * hb * hb && rr2 >= 1e-8;
+    const bool pse_a = !(fa & MFC_FLAG_BLANKED) && pse && k.thermal_wp;
+    const double ta_a = pse ? 0. : (tool_a ? k.alpha_tool : k.alpha_wp);
+    if (of_a) pair_vjp(k, ra, rb, tool_a, tool_b, ta_a, la, false, true, dummy, gb);
+    if (pse_a) pse_vjp(k, ra, rb, la[L_TPSE], false, true, dummy, gb);
+    asm volatile("" ::: "memory");
+    if (of_b) pair_vjp(k, rb, ra, tool_b, tool_a, ta_b, lb, true, false, gb, dummy);
+    if (pse_b) pse_vjp(k, rb, ra, lb[L_TPSE], true, false, gb, dummy);
+  }
+  pull_store(gb, r, d.g_rec + (size_t)REC_DOUBLES * b);
+}
+
+// returns false, with nothing done, for an entry that pull_rest takes
+__device__ inline bool pull_patch(pull_mem &m, const adj_args *__restrict__ D, int inst, int slot, int patch, int part) {
+  MFC_ADJ_ARGS(d, inst);
+  const dev_consts &k = D[inst].k;
+  const size_t N = k.N;
+  const int *__restrict__ offsets = d.offsets + (size_t)slot * d.ncell1;
+  const int tid = threadIdx.x;
+  const int nrb = patch_rows(k), pc = patch / nrb, pr = patch - pc * nrb;
+  const int r0 = pr * k.patch_s, r1 = r0 + k.patch_s < k.gny ? r0 + k.patch_s : k.gny;
+  const int g0 = pc * k.patch_w, g1 = g0 + k.patch_w < k.gnx ? g0 + k.patch_w : k.gnx;
+  const int s0 = r0 < 2 ? 0 : r0 - 2, s1 = r1 + 2 < k.gny ? r1 + 2 : k.gny;
+  const int q0 = g0 < 2 ? 0 : g0 - 2, q1 = g1 + 2 < k.gnx ? g1 + 2 : k.gnx;
+  const int ncol = q1 - q0, nrow = s1 - s0 + 1;
+  const int te = tid / nrow;
+  if (tid < ncol * nrow) m.table[tid] = offsets[(q0 + te) * k.gny + s0 + (tid - te * nrow)];
+  __syncthreads();
+  if (tid < 64) {
+    int first = 0, c = 0, o = 0;
+    if (tid < ncol) {
+      first = m.table[tid * nrow];
+      c = m.table[tid * nrow + nrow - 1] - first;
+      if (q0 + tid >= g0 && q0 + tid < g1) o = m.table[tid * nrow + r1 - s0] - m.table[tid * nrow + r0 - s0];
+    }
+    int xc = c, xo = o;
+#pragma unroll
+    for (int s = 1; s < 32; s <<= 1) {
+      const int yc = __shfl_up(xc, s, 64), yo = __shfl_up(xo, s, 64);
+      if (tid >= s) { xc += yc; xo += yo; }
+    }
+    if (tid <= ncol) {
+      m.col_first[tid] = xc - c;
+      m.own_first[tid] = xo - o;
+      if (tid < ncol) m.col_shift[tid] = xc - c - first;
+    }
+  }
+  __syncthreads();
+  const int ncand = m.col_first[ncol], nown = m.own_first[ncol];
+  const int cap = k.stage_limit > 0 && k.stage_limit < PULL_CAP ? k.stage_limit : PULL_CAP;
+  if (ncand > cap || !k.uniform_h) return false;  // the same in every thread
+  // the pieces of a candidate's record and adjoints by neighbouring lanes (15 of each 16)
+  const int pl = tid % 16;
+  for (int q = tid / 16; q < ncand; q += TILE / 16) {
+    int c = 0;
+    for (int e = 1; e < ncol; e++) c += q >= m.col_first[e];
+    const size_t j = q - m.col_shift[c];
+    if (pl < REC_DOUBLES / 2) m.piece[pl][q] = reinterpret_cast<const double2 *>(d.rec)[j * (REC_DOUBLES / 2) + pl];
+    else if (pl < PULL_PIECES)
+      m.piece[pl][q] = reinterpret_cast<const double2 *>(d.lam_acc)[j * (LAM / 2) + pl - REC_DOUBLES / 2];
+  }
+  if (tid < ncol * nrow) m.table[tid] += m.col_shift[te];
+  __syncthreads();
+  const int n = part * (TILE / PULL_LANES) + tid / PULL_LANES;
+  if (n >= nown) return true;  // whole groups of lanes
+  const int lane = tid & 63, r = lane % PULL_LANES, gl = lane - r;
+  int col = 0;
+  for (int e = 1; e < ncol; e++) col += n >= m.own_first[e];
+  const int li = m.table[col * nrow + r0 - s0] + (n - m.own_first[col]);
+  const int b = li - m.col_shift[col];
+  auto load = [&](int j, double *rec, double *la) {
+#pragma unroll
+    for (int q = 0; q < REC_DOUBLES / 2; q++) { const double2 v = m.piece[q][j]; rec[2 * q] = v.x; rec[2 * q + 1] = v.y; }
+#pragma unroll
+    for (int q = 0; q < L_N / 2; q++) { const double2 v = m.piece[REC_DOUBLES / 2 + q][j]; la[2 * q] = v.x; la[2 * q + 1] = v.y; }
+  };
+  double gb[REC_DOUBLES];
+#pragma unroll
+  for (int q = 0; q < REC_DOUBLES; q++) gb[q] = 0.;
+  const double2 pb = m.piece[0][li];
+  const int fb = double_to_bits(m.piece[R_FLAGS / 2][li].x);
+  const bool pse = k.pse != 0, tool_b = fb & MFC_FLAG_TOOL;
+  const bool pse_b = !(fb & MFC_FLAG_BLANKED) && pse && k.thermal_wp;
+  const double ta_b = pse ? 0. : (tool_b ? k.alpha_tool : k.alpha_wp);
+  const int gi = q0 + col, gj = d.key_sorted[(size_t)slot * N + b] - gi * k.gny;
+  const window w = make_window_at(k, gi, gj, [&](int c, int row) { return m.table[(c - q0) * nrow + row - s0]; });
+  unsigned char *list = m.list[tid / PULL_LANES];
+  for (int b0 = 0; b0 < w.total; b0 += 64) {
+    const int nb = w.total - b0 < 64 ? w.total - b0 : 64;
+    int cnt = 0;
+    for (int u0 = 0; u0 < nb; u0 += PULL_LANES) {
+      const bool in = u0 + r < nb;
+      const int a = w.at(b0 + (in ? u0 + r : nb - 1));
+      const double2 pa = m.piece[0][a];
+      const int fa = double_to_bits(m.piece[R_FLAGS / 2][a].x);
+      const double dx = pa.x - pb.x, dy = pa.y - pb.y, rr2 = dx * dx + dy * dy;
+      const pull_pair pm = pull_flags(k, fa, fb);
+      const bool hit = in && a != li && pm.of_a && pm.of_b && rr2 < 4 * k.h0 * k.h0 && rr2 >= 1e-8;
+      const unsigned bits = (unsigned)(__ballot(hit) >> gl) & ((1u << PULL_LANES) - 1u);
+      if (hit) list[cnt + __popc(bits & ((1u << r) - 1u))] = (unsigned char)a;
+      cnt += __popc(bits);
+      if (pse && in && a != li) {
+        const bool pse_a = !(fa & MFC_FLAG_BLANKED) && k.thermal_wp;
+        if (pse_a || pse_b) {
+          double ra[REC_DOUBLES], la[LAM], rb[REC_DOUBLES], lb[LAM], dummy[REC_DOUBLES];
+          load(a, ra, la);
+          load(li, rb, lb);
+          if (pse_a) pse_vjp(k, ra, rb, la[L_TPSE], false, true, dummy, gb);
+          if (pse_b) pse_vjp(k, rb, ra, lb[L_TPSE], true, false, gb, dummy);
+        }
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the list, by lanes of the same wave
+    __builtin_amdgcn_wave_barrier();
+    for (int p = r; p < cnt; p += PULL_LANES) {
+      // both records are read from LDS where a value is used: held in registers across the pair (the
+      // particle's own across the pairs) they spill
+      const int a = list[p];
+      const bool tool_a = double_to_bits(m.piece[R_FLAGS / 2][a].x) & MFC_FLAG_TOOL;
+      // the mechanical sums of both take a pair without a tool particle; each conduction sum
+      // counts where its particle conducts
+      const double ta_a = pse ? 0. : (tool_a ? k.alpha_tool : k.alpha_wp);
+      auto rec = [&](int j, int q) { return q % 2 ? m.piece[q / 2][j].y : m.piece[q / 2][j].x; };
+      auto adj = [&](int j, double ta, int q) { return q == L_TL && ta == 0. ? 0. : rec(j, REC_DOUBLES + q); };
+      pair_vjp_sym(
+          k, [&](int q) { return rec(li, q); }, [&](int q) { return rec(a, q); }, !tool_a && !tool_b,
+          ta_a != 0. || ta_b != 0., [&](int q) { return adj(li, ta_b, q); }, [&](int q) { return adj(a, ta_a, q); }, gb);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  pull_store(gb, r, d.g_rec + (size_t)REC_DOUBLES * b);
+  return true;
+}
+
+__global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(3))) void kb_adj_pull(
+    const adj_args *__restrict__ D, const inst_args *__restrict__ rep, const int2 *__restrict__ work, int nwork, int slot) {
+  const int u = xcd_chunk_tile(blockIdx.x, nwork);
+  if (u < 0) return;
+  const int2 it = work[u];
+  MFC_ADJ_ARGS(d, it.x);
+  __shared__ pull_mem m;
+  if (it.y == PATCH_ITEM_FORCE) {  // the work table's other item, in the pull the theta partials
+    add_theta(d, reinterpret_cast<double(*)[TILE]>(&m));
+    return;
+  }
+  const int count = d.plen[slot], step = rep[it.x].npatch_items;
+  if (it.y >= count) return;
+  const int2 *__restrict__ plist = d.plist + (size_t)slot * d.list_len;
+  const int2 p = plist[it.y];
+  const bool staged = pull_patch(m, D, it.x, slot, p.x, p.y);
+  for (int q = staged ? it.y + step : it.y; q < count; q += step) pull_rest(D, it.x, slot, plist[q].x, plist[q].y);
+}
+
 // ------------------------------------------------------------------ B3: record VJP + unsort
+// the segment's first step: the adjoint of its start state into storage order
 __global__ __launch_bounds__(TILE) void kb_adj_record(const adj_args *__restrict__ D, const int2 *__restrict__ work,
-                                                      int nwork, int cur) {
+                                                      int nwork) {
   const int w = xcd_tile(blockIdx.x, nwork);
   if (w < 0) return;
   const int2 it = work[w];
@@ -326,38 +504,65 @@ __global__ __launch_bounds__(TILE) void kb_adj_record(const adj_args *__restrict
   const int a = it.y * TILE + threadIdx.x;
   if (a >= k.N) return;
   const size_t N = k.N;
+  const int dst = d.perm[a];
+  const double *__restrict__ st = slot_state(d, 0);
   double s[TS_N], gs[TS_N], br[REC_DOUBLES];
 #pragma unroll
-  for (int q = 0; q < TS_N; q++) { s[q] = d.st[q * N + a]; gs[q] = d.g_s[q * N + a]; }
+  for (int q = 0; q < TS_N; q++) { s[q] = st[q * N + dst]; gs[q] = d.g_s[0][q * N + a]; }
 #pragma unroll
-  for (int q = 0; q < REC_DOUBLES; q++) br[q] = d.g_rec[q * N + a];
-  record_vjp(k, s, d.flags[a], d.pos.p[a], br, gs);
-  const int dst = d.perm[a];
-  double *lam_prev = d.lam_s[1 - cur];
+  for (int q = 0; q < REC_DOUBLES; q++) br[q] = d.g_rec[(size_t)REC_DOUBLES * a + q];
+  const int fl = slot_flags(d, 0)[dst] & FLAG_MASK;
+  record_vjp(k, s, fl, eos_pressure(k, s, fl), br, gs);
 #pragma unroll
-  for (int q = 0; q < TS_N; q++) lam_prev[q * N + dst] = gs[q];
+  for (int q = 0; q < TS_N; q++) d.lam[q * N + dst] = gs[q];
 }
-
 
 }  // namespace
 
 // ------------------------------------------------------------------ workspace
+constexpr int ADJ_LANES = PULL_LANES;  // threads per particle of the replayed interaction: the
+                                       // pull takes the same patches
+
+// device memory of the backward pass of a group of instances, kept between calls with the first
+// instance's workspace; the descriptors are written at every call
+struct adj_group {
+  std::vector<int> items;       // work items of each instance's patches
+  int nck = 0;
+  char *mem = nullptr;
+  inst_args *rep = nullptr;     // K x n replay descriptors
+  adj_args *adj = nullptr;      // n
+  snapshot *snaps = nullptr;    // n x nck
+  int2 *patches = nullptr;
+  int npatches = 0;
+  ~adj_group() {
+    if (mem) (void)hipFree(mem);
+  }
+};
+
 struct adj_work {
-  int N = 0, nsteps = 0, K = 1, w0 = 0, w1 = 0;
+  int N = 0, nsteps = 0, K = 0, w0 = 0, w1 = 0;  // K set when everything is allocated
   bool valid = false;
   int64_t hist0 = 0;  // force-history index of the first step of the run
   double Fmean[2] = {0., 0.};
   std::vector<void *> allocs;
-  std::vector<snapshot> ckpt, seg;
-  char *work[2] = {nullptr, nullptr};   // replay state blocks
-  char *posw = nullptr;                 // replay positional block
-  mfc_tool_state *toolw = nullptr;      // 2
+  std::vector<snapshot> ckpt;
+  // the slots of a segment's steps (adj_args)
+  char *state = nullptr;
+  double *normal = nullptr;
+  int *perm = nullptr, *spos = nullptr, *key_sorted = nullptr, *offsets = nullptr, *plen = nullptr;
+  int2 *plist = nullptr;
+  mfc_tool_state *tool = nullptr;
+  double *acc = nullptr;
+  patch_plan patches = {};
+  int uniform_h = 0;  // of the recorded run's states
+  double h0 = 0.;
+  char *posw = nullptr;                 // replay positional block (pressure and artificial stress)
   double *partials = nullptr, *force_last = nullptr, *hist = nullptr;
   int64_t *ctr = nullptr;
   int *pending = nullptr, *gflag = nullptr;
-  int *keys_keep = nullptr;  // the handle's cell ids, kept across the replay of the backward pass
-  double *acc_seg = nullptr, *lam_acc = nullptr, *lam_s[2] = {nullptr, nullptr}, *lam_n = nullptr, *g_s = nullptr,
+  double *lam = nullptr, *lam_n = nullptr, *g_s[2] = {nullptr, nullptr}, *lam_acc = nullptr, *rec = nullptr,
          *g_rec = nullptr, *theta_part = nullptr, *theta_acc = nullptr;
+  std::unique_ptr<adj_group> group;     // of the group that this instance is the first of
 
   template <class T>
   int alloc(T **p, size_t n) {
@@ -385,57 +590,41 @@ void adj_free(adj_work *w) { delete w; }
 
 namespace {
 
-int save(hipStream_t st, const snapshot &d, const void *state, const void *pos, const int *keys,
-         const mfc_tool_state *tool, int N) {
-  HIP_TRY(hipMemcpyAsync(d.state, state, state_block_bytes(N), hipMemcpyDeviceToDevice, st));
-  HIP_TRY(hipMemcpyAsync(d.pos, pos, positional_block_bytes(N), hipMemcpyDeviceToDevice, st));
-  HIP_TRY(hipMemcpyAsync(d.keys, keys, sizeof(int) * (size_t)N, hipMemcpyDeviceToDevice, st));
-  HIP_TRY(hipMemcpyAsync(d.tool, tool, sizeof(mfc_tool_state), hipMemcpyDeviceToDevice, st));
-  return MFC_OK;
-}
-
-int restore(hipStream_t st, const snapshot &s, void *state, void *pos, int *keys, mfc_tool_state *tool, int N) {
-  HIP_TRY(hipMemcpyAsync(state, s.state, state_block_bytes(N), hipMemcpyDeviceToDevice, st));
-  HIP_TRY(hipMemcpyAsync(pos, s.pos, positional_block_bytes(N), hipMemcpyDeviceToDevice, st));
-  HIP_TRY(hipMemcpyAsync(keys, s.keys, sizeof(int) * (size_t)N, hipMemcpyDeviceToDevice, st));
-  HIP_TRY(hipMemcpyAsync(tool, s.tool, sizeof(mfc_tool_state), hipMemcpyDeviceToDevice, st));
-  return MFC_OK;
-}
-
 int setup_work(mfc_sim *s, int nsteps, int K, int w0, int w1) {
   const int N = s->k.N;
   adj_work *w = s->adj;
   const int nck = (nsteps + K - 1) / K;
   const bool reuse = w && w->N == N && w->K == K && (int)w->ckpt.size() >= nck;
   if (!reuse) {
+    HIP_TRY(hipStreamSynchronize(s->stream));  // nothing queued uses the old one
     adj_free(w);
     w = s->adj = new adj_work();
     w->N = N;
-    w->K = K;
     int rc;
     w->ckpt.resize(nck);
     for (auto &c : w->ckpt)
       if ((rc = w->alloc_snapshot(c))) return rc;
-    w->seg.resize(K);
-    for (auto &c : w->seg)
-      if ((rc = w->alloc_snapshot(c))) return rc;
-    const size_t n = (size_t)N;
-    if ((rc = w->alloc(&w->work[0], state_block_bytes(N))) || (rc = w->alloc(&w->work[1], state_block_bytes(N))) ||
-        (rc = w->alloc(&w->posw, positional_block_bytes(N))) || (rc = w->alloc(&w->toolw, 2)) ||
+    const size_t n = (size_t)N, k = (size_t)K;
+    w->patches = plan_patches(s, ADJ_LANES);
+    if ((rc = w->alloc(&w->state, (k + 1) * state_block_bytes(N))) || (rc = w->alloc(&w->normal, (k + 1) * 2 * n)) ||
+        (rc = w->alloc(&w->perm, k * n)) || (rc = w->alloc(&w->spos, k * n)) || (rc = w->alloc(&w->key_sorted, k * n)) ||
+        (rc = w->alloc(&w->offsets, k * ((size_t)s->k.ncell_table + 1))) || (rc = w->alloc(&w->plen, k + 1)) ||
+        (rc = w->alloc(&w->plist, k * w->patches.list)) || (rc = w->alloc(&w->tool, k + 1)) ||
+        (rc = w->alloc(&w->acc, k * (L_N + 1) * n)) ||
+        (rc = w->alloc(&w->posw, positional_block_bytes(N))) ||
         (rc = w->alloc(&w->partials, 16 * (size_t)s->ntiles)) || (rc = w->alloc(&w->force_last, 2)) ||
         (rc = w->alloc(&w->hist, 2)) || (rc = w->alloc(&w->ctr, 1)) || (rc = w->alloc(&w->pending, 2)) ||
-        (rc = w->alloc(&w->gflag, 4 * (size_t)s->ntiles)) ||
-        (rc = w->alloc(&w->keys_keep, n)) ||
-        (rc = w->alloc(&w->acc_seg, (size_t)K * (L_N + 1) * n)) || (rc = w->alloc(&w->lam_acc, L_N * n)) ||
-        (rc = w->alloc(&w->lam_s[0], TS_N * n)) || (rc = w->alloc(&w->lam_s[1], TS_N * n)) ||
-        (rc = w->alloc(&w->lam_n, 2 * n)) || (rc = w->alloc(&w->g_s, TS_N * n)) ||
-        (rc = w->alloc(&w->g_rec, REC_DOUBLES * n)) || (rc = w->alloc(&w->theta_part, 6 * (size_t)s->ntiles)) ||
-        (rc = w->alloc(&w->theta_acc, 6)))
+        (rc = w->alloc(&w->gflag, 4 * (size_t)s->ntiles)) || (rc = w->alloc(&w->lam, TS_N * n)) ||
+        (rc = w->alloc(&w->lam_n, 2 * n)) || (rc = w->alloc(&w->g_s[0], TS_N * n)) ||
+        (rc = w->alloc(&w->g_s[1], TS_N * n)) || (rc = w->alloc(&w->lam_acc, LAM * n)) ||
+        (rc = w->alloc(&w->rec, REC_DOUBLES * n)) || (rc = w->alloc(&w->g_rec, REC_DOUBLES * n)) ||
+        (rc = w->alloc(&w->theta_part, 6 * (size_t)s->ntiles)) || (rc = w->alloc(&w->theta_acc, 6)))
       return rc;
     // the replay's force reduction keeps no history (cap 0) but counts steps
     HIP_TRY(hipMemsetAsync(w->ctr, 0, sizeof(int64_t), s->stream));
     HIP_TRY(hipMemsetAsync(w->pending, 0, 2 * sizeof(int), s->stream));
     HIP_TRY(hipMemsetAsync(w->gflag, 0, 4 * sizeof(int) * (size_t)s->ntiles, s->stream));
+    w->K = K;
   }
   w->nsteps = nsteps;
   w->w0 = w0;
@@ -444,10 +633,78 @@ int setup_work(mfc_sim *s, int nsteps, int K, int w0, int w1) {
   return MFC_OK;
 }
 
-}  // namespace
-}  // namespace mfc
+// the group's device memory and work table, kept while a call's instances have the same work items
+int setup_group(mfc_sim *const *sims, int n, hipStream_t st) {
+  adj_work *w0 = sims[0]->adj;
+  const int K = w0->K, nck = (w0->nsteps + K - 1) / K;
+  std::vector<int> per(n);
+  for (int i = 0; i < n; i++) per[i] = sims[i]->adj->patches.items;
+  adj_group *g = w0->group.get();
+  if (g && g->items == per && g->nck >= nck) return MFC_OK;
+  HIP_TRY(hipStreamSynchronize(st));  // nothing queued uses the old one
+  w0->group.reset(new adj_group());
+  g = w0->group.get();
+  g->items = per;
+  g->nck = nck;
+  std::vector<int2> items;
+  for (int i = 0; i < n; i++) items.push_back(make_int2(i, PATCH_ITEM_FORCE));
+  for (int i = 0; i < n; i++)
+    for (int q = 0; q < per[i]; q++) items.push_back(make_int2(i, q));
+  g->npatches = (int)items.size();
+  auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  const size_t b_rep = up(sizeof(inst_args) * (size_t)K * n), b_adj = up(sizeof(adj_args) * n);
+  const size_t b_sn = up(sizeof(snapshot) * (size_t)n * nck), b_pt = up(sizeof(int2) * items.size());
+  const hipError_t e = hipMalloc(&g->mem, b_rep + b_adj + b_sn + b_pt);
+  if (e != hipSuccess) {
+    g->mem = nullptr;
+    w0->group.reset();
+    return fail(MFC_E_NOMEM, std::string("hipMalloc (adjoint group): ") + hipGetErrorString(e));
+  }
+  char *p = g->mem;
+  g->rep = (inst_args *)p; p += b_rep;
+  g->adj = (adj_args *)p; p += b_adj;
+  g->snaps = (snapshot *)p; p += b_sn;
+  g->patches = (int2 *)p;
+  if (hipMemcpy(g->patches, items.data(), sizeof(int2) * items.size(), hipMemcpyHostToDevice) != hipSuccess) {
+    w0->group.reset();
+    return fail(MFC_E_HIP, "upload of the adjoint's work table");
+  }
+  return MFC_OK;
+}
 
-namespace mfc {
+// segment sg of len steps: the replay, then the reverse steps
+void enqueue_segment(const adj_group &g, const adj_work &w, const batch_work &fw, int sg, int len, int copy_blocks,
+                     hipStream_t st) {
+  const int n = (int)g.items.size();
+  batch_work rw = fw;
+  rw.patches = g.patches;
+  rw.npatches = g.npatches;
+  rw.v.lanes = ADJ_LANES;
+  rw.args = g.rep;
+  const dim3 gt(padded(fw.ntiles)), gp(chunked_blocks(g.npatches));
+  hipLaunchKernelGGL(kb_adj_restore, dim3(copy_blocks, n), dim3(256), 0, st, g.adj, sg);
+  launch_batch_hash(rw, st);
+  launch_batch_records(rw, st);
+  for (int j = 0; j < len; j++) {
+    rw.args = g.rep + (size_t)j * n;
+    launch_batch_step(rw, st);
+  }
+  for (int j = len - 1; j >= 0; j--) {
+    const int t = sg * w.K + j;
+    hipLaunchKernelGGL(kb_adj_tail, gt, dim3(TILE), 0, st, g.adj, fw.tiles, fw.ntiles, j, (int)(j == len - 1),
+                       (int)(t >= w.w0 && t < w.w1));
+    hipLaunchKernelGGL(kb_adj_pull, gp, dim3(TILE), 0, st, g.adj, g.rep, g.patches, g.npatches, j);
+  }
+  hipLaunchKernelGGL(kb_adj_record, gt, dim3(TILE), 0, st, g.adj, fw.tiles, fw.ntiles);
+}
+
+// about 8 words of a state block per thread
+int copy_blocks_of(int N) {
+  const size_t want = (state_block_bytes(N) / sizeof(uint64_t) + 2047) / 2048;
+  return want < 16 ? 16 : (want > 1024 ? 1024 : (int)want);
+}
+
+}  // namespace
 
 int adj_begin(mfc_sim *s, int nsteps, int checkpoint_every, int w0, int w1) {
   if (nsteps < 1 || checkpoint_every < 1 || w0 < 0 || w1 <= w0 || w1 > nsteps)
@@ -465,14 +722,22 @@ int adj_begin(mfc_sim *s, int nsteps, int checkpoint_every, int w0, int w1) {
   if (base + nsteps > HIST_CAP) return fail(MFC_E_INVALID, "force history full: reset it before the run");
   if ((rc = setup_work(s, nsteps, checkpoint_every, w0, w1))) return rc;
   s->adj->hist0 = base;
+  s->adj->uniform_h = s->k.uniform_h;
+  s->adj->h0 = s->k.h0;
   return MFC_OK;
 }
+
+int adj_segment(const mfc_sim *s) { return s->adj->K; }
 
 int adj_checkpoint(mfc_sim *s, int t) {
   adj_work *w = s->adj;
   if (t % w->K) return MFC_OK;
-  const int c = s->cur;
-  return save(s->stream, w->ckpt[t / w->K], s->set[c].px, s->pos.nx, s->bins.key_sorted, s->tool + c, s->k.N);
+  const int c = s->cur, N = s->k.N;
+  hipLaunchKernelGGL(k_adj_save, dim3(copy_blocks_of(N)), dim3(256), 0, s->stream, w->ckpt[t / w->K],
+                     (const uint64_t *)s->set[c].px, state_block_bytes(N) / sizeof(uint64_t),
+                     (const uint64_t *)s->pos.nx, positional_block_bytes(N) / sizeof(uint64_t),
+                     (const int *)s->bins.key_sorted, N, (const mfc_tool_state *)(s->tool + c));
+  return MFC_OK;
 }
 
 int adj_finish(mfc_sim *s, double Fmean[2]) {
@@ -502,168 +767,115 @@ int adj_backward(mfc_sim *const *sims, int n, const batch_work &fw, hipStream_t 
     if (w->nsteps != w0->nsteps || w->K != w0->K || w->w0 != w0->w0 || w->w1 != w0->w1)
       return fail(MFC_E_INVALID, "the instances recorded different runs");
   }
-  const int nsteps = w0->nsteps, K = w0->K;
-  const int nck = (nsteps + K - 1) / K;
-  // descriptors: replay steps of start parity 0 and 1 (inst_args, the step kernels' view, with
-  // the replay buffers as state and no binning of the next step), the backward kernels' view
-  // (adj_args), and each instance's checkpoints and segment snapshots
-  std::vector<inst_args> rep(2 * (size_t)n);
+  int rc = setup_group(sims, n, st);
+  if (rc) return rc;
+  adj_group &g = *w0->group;
+  const int nsteps = w0->nsteps, K = w0->K, nseg = (nsteps + K - 1) / K;
+  const int slots = K < nsteps ? K : nsteps;
+  // the descriptors: a replay step each (inst_args, the step kernels' view of a slot), the reverse
+  // kernels' view of the instance, and its checkpoints
+  std::vector<inst_args> rep((size_t)slots * n);
   std::vector<adj_args> da(n);
-  std::vector<snapshot> snaps((size_t)n * (nck + K));
+  std::vector<snapshot> snaps((size_t)n * nseg);
+  int maxN = 0;
   for (int i = 0; i < n; i++) {
     mfc_sim *s = sims[i];
     adj_work *w = s->adj;
     const int N = s->k.N;
-    dstate A, B;
-    dpositional P;
-    carve_state(w->work[0], N, A);
-    carve_state(w->work[1], N, B);
-    carve_positional(w->posw, N, P);
-    for (int p = 0; p < 2; p++) {
-      inst_args &a = rep[(size_t)p * n + i];
+    const size_t sb = state_block_bytes(N), nc1 = (size_t)s->k.ncell_table + 1;
+    maxN = N > maxN ? N : maxN;
+    dev_consts k = s->k;
+    k.patch_s = w->patches.s;
+    k.patch_w = w->patches.w;
+    k.patch_slots = w->patches.slots;
+    k.uniform_h = w->uniform_h;
+    k.h0 = w->h0;
+    for (int j = 0; j < slots; j++) {
+      inst_args &a = rep[(size_t)j * n + i];
       std::memset(&a, 0, sizeof(a));
-      a.k = s->k;
-      a.cur = p ? B : A;
-      a.nxt = p ? A : B;
+      const int p = j & 1;
+      a.k = k;
+      carve_state(w->state + j * sb, N, a.cur);
+      carve_state(w->state + (j + 1) * sb, N, a.nxt);
       a.b = s->bins;
+      a.b.key_sorted = w->key_sorted + (size_t)j * N;
+      a.b.perm = w->perm + (size_t)j * N;
+      a.b.spos = w->spos + (size_t)j * N;
+      a.b.offsets = w->offsets + j * nc1;
+      a.b.plist = w->plist + (size_t)j * w->patches.list;
+      a.b.plen = w->plen + j;
+      a.b.plen_next = w->plen + j + 1;
       a.b.bsum = s->chunk_sums[p];
       a.b.bsum_next = s->chunk_sums[1 - p];
-      a.b.plen = s->plen + p;
-      a.b.plen_next = s->plen + 1 - p;
-      a.pos = P;
+      carve_positional(w->posw, N, a.pos);
+      a.pos.nx = w->normal + (size_t)j * 2 * N;
+      a.pos.ny = a.pos.nx + N;
+      a.pos.nx_out = a.pos.nx + 2 * (size_t)N;
+      a.pos.ny_out = a.pos.nx + 3 * (size_t)N;
       a.r = s->recs[p];
       a.rn = s->recs[1 - p];
-      a.tool_in = w->toolw + p;
-      a.tool_out = w->toolw + 1 - p;
+      a.tool_in = w->tool + j;
+      a.tool_out = w->tool + j + 1;
       a.f = {w->partials, w->gflag, w->force_last, w->hist, 0, w->ctr, w->pending + p, w->pending + 1 - p};  // no history, counted
-      a.acc_out = w->acc_seg;  // pointed at each step's slot by kb_adj_acc_slot
+      a.acc_out = w->acc + (size_t)j * (L_N + 1) * N;
       a.ntiles = s->ntiles;
       a.nscan = scan_blocks(s->k.ncell_table);
-      a.npatch_items = s->npatch_items;
+      a.npatch_items = w->patches.items;
     }
     adj_args &d = da[i];
     std::memset(&d, 0, sizeof(d));
-    d.k = s->k;
+    d.k = k;
     d.ntiles = s->ntiles;
-    d.st = B.px;  // the sorted start state, TS_* order with stride N
-    d.flags = B.flags;
-    d.pos = P;
-    d.rec = s->recs[0].rec;  // the reverse steps run from parity 0
-    d.key_sorted = s->bins.key_sorted;
-    d.offsets = s->bins.offsets;
-    d.perm = s->bins.perm;
-    d.tool_now = w->toolw + 1;
-    d.acc_seg = w->acc_seg;
-    d.acc_stride = (size_t)(L_N + 1) * N;
-    d.lam_acc = w->lam_acc;
-    d.lam_s[0] = w->lam_s[0];
-    d.lam_s[1] = w->lam_s[1];
-    d.lam_n = w->lam_n;
-    d.g_s = w->g_s;
-    d.g_rec = w->g_rec;
-    d.theta_part = w->theta_part;
-    d.theta_acc = w->theta_acc;
+    d.state = w->state;
+    d.state_bytes = sb;
+    d.normal = w->normal;
+    d.perm = w->perm; d.spos = w->spos; d.key_sorted = w->key_sorted;
+    d.offsets = w->offsets;
+    d.plist = w->plist; d.plen = w->plen;
+    d.list_len = w->patches.list; d.ncell1 = (int)nc1;
+    d.tool = w->tool;
+    d.acc = w->acc;
+    d.lam = w->lam; d.lam_n = w->lam_n;
+    d.g_s[0] = w->g_s[0]; d.g_s[1] = w->g_s[1];
+    d.lam_acc = w->lam_acc; d.rec = w->rec; d.g_rec = w->g_rec;
+    d.theta_part = w->theta_part; d.theta_acc = w->theta_acc;
     d.Fb[0] = cot[2 * i] / (w->w1 - w->w0);
     d.Fb[1] = cot[2 * i + 1] / (w->w1 - w->w0);
-    d.state_words = state_block_bytes(N) / sizeof(uint64_t);
-    d.pos_words = positional_block_bytes(N) / sizeof(uint64_t);
-    d.live_state[0] = (uint64_t *)w->work[0];
-    d.live_state[1] = (uint64_t *)w->work[1];
-    d.live_pos = (uint64_t *)w->posw;
-    d.live_keys = s->bins.key_sorted;
-    d.chunk_sums[0] = s->chunk_sums[0];
-    d.chunk_sums[1] = s->chunk_sums[1];
-    d.nscan = scan_blocks(s->k.ncell_table);
+    d.ckpt = g.snaps + (size_t)i * nseg;
+    d.chunk_sums[0] = s->chunk_sums[0]; d.chunk_sums[1] = s->chunk_sums[1];
     d.pcnt = s->bins.pcnt;
+    d.nscan = scan_blocks(s->k.ncell_table);
     d.npatch = s->npatch_max;
-    d.plen = s->plen;
-    d.live_tool = w->toolw;
-    for (int c = 0; c < nck; c++) snaps[(size_t)i * (nck + K) + c] = w->ckpt[c];
-    for (int c = 0; c < K; c++) snaps[(size_t)i * (nck + K) + nck + c] = w->seg[c];
+    for (int c = 0; c < nseg; c++) snaps[(size_t)i * nseg + c] = w->ckpt[c];
   }
-  auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-  const size_t b_rep = up(sizeof(inst_args) * rep.size()), b_da = up(sizeof(adj_args) * da.size());
-  const size_t b_sn = up(sizeof(snapshot) * snaps.size());
-  char *dmem = nullptr;
-  HIP_TRY(hipMalloc(&dmem, b_rep + b_da + b_sn));
-  inst_args *d_rep = (inst_args *)dmem;
-  adj_args *d_da = (adj_args *)(dmem + b_rep);
-  snapshot *d_sn = (snapshot *)(dmem + b_rep + b_da);
-  for (int i = 0; i < n; i++) {
-    da[i].ckpt = d_sn + (size_t)i * (nck + K);
-    da[i].seg = da[i].ckpt + nck;
-  }
-  // copy grid: about 8 words of the largest state block per thread
-  int maxN = 0;
-  for (int i = 0; i < n; i++) maxN = sims[i]->k.N > maxN ? sims[i]->k.N : maxN;
-  const size_t want = (state_block_bytes(maxN) / sizeof(uint64_t) + 2047) / 2048;
-  const int copy_blocks = want < 16 ? 16 : (want > 1024 ? 1024 : (int)want);
-  int rc = MFC_OK;
+  const int copy_blocks = copy_blocks_of(maxN);
   auto run = [&]() -> int {
-    HIP_TRY(hipMemcpyAsync(d_rep, rep.data(), sizeof(inst_args) * rep.size(), hipMemcpyHostToDevice, st));
-    HIP_TRY(hipMemcpyAsync(d_da, da.data(), sizeof(adj_args) * da.size(), hipMemcpyHostToDevice, st));
-    HIP_TRY(hipMemcpyAsync(d_sn, snaps.data(), sizeof(snapshot) * snaps.size(), hipMemcpyHostToDevice, st));
+    HIP_TRY(hipMemcpyAsync(g.rep, rep.data(), sizeof(inst_args) * rep.size(), hipMemcpyHostToDevice, st));
+    HIP_TRY(hipMemcpyAsync(g.adj, da.data(), sizeof(adj_args) * da.size(), hipMemcpyHostToDevice, st));
+    HIP_TRY(hipMemcpyAsync(g.snaps, snaps.data(), sizeof(snapshot) * snaps.size(), hipMemcpyHostToDevice, st));
     for (int i = 0; i < n; i++) {
       mfc_sim *s = sims[i];
       adj_work *w = s->adj;
       const size_t N = (size_t)s->k.N;
-      HIP_TRY(hipMemsetAsync(w->lam_s[0], 0, sizeof(double) * TS_N * N, st));
+      HIP_TRY(hipMemsetAsync(w->lam, 0, sizeof(double) * TS_N * N, st));
       HIP_TRY(hipMemsetAsync(w->lam_n, 0, sizeof(double) * 2 * N, st));
       HIP_TRY(hipMemsetAsync(w->theta_acc, 0, sizeof(double) * 6, st));
-      HIP_TRY(hipMemcpyAsync(w->keys_keep, s->bins.key_sorted, sizeof(int) * N, hipMemcpyDeviceToDevice, st));
-      // the pass bins its states into the handle's tables and overwrites its records: both are
+      // the pass bins its states with the handle's scratch and overwrites its records: both are
       // computed again at the handle's next step
       s->keys_fresh = false;
     }
-    batch_work rw[2] = {fw, fw};
-    rw[0].args = d_rep;
-    rw[1].args = d_rep + n;
-    const dim3 gcopy(copy_blocks, n), gt(padded(fw.ntiles)), gpull(padded(fw.ntiles * PULL_LANES));
-    const dim3 gslot((n + 63) / 64);
-    int cur = 0;  // lam_s[cur] holds the adjoint of the end state of the step being reversed
-    const int nseg = nck;
     for (int sg = nseg - 1; sg >= 0; sg--) {
-      const int t0 = sg * K, t1 = (t0 + K < nsteps) ? t0 + K : nsteps;
-      // replay the segment, keeping the start of each of its steps
-      int wa = 0;
-      hipLaunchKernelGGL(kb_adj_copy, gcopy, dim3(256), 0, st, d_da, 0, 1, sg, 0);
-      launch_batch_hash(rw[0], st);
-      launch_batch_records(rw[0], st);
-      for (int t = t0; t < t1; t++) {
-        hipLaunchKernelGGL(kb_adj_copy, gcopy, dim3(256), 0, st, d_da, 1, 0, t - t0, wa);
-        hipLaunchKernelGGL(kb_adj_acc_slot, gslot, dim3(64), 0, st, d_rep, d_da, n, t - t0);
-        launch_batch_step(rw[wa], st);  // the interaction keeps its sums in the step's slot
-        wa = 1 - wa;
-      }
-      // reverse the steps of the segment
-      for (int t = t1 - 1; t >= t0; t--) {
-        hipLaunchKernelGGL(kb_adj_copy, gcopy, dim3(256), 0, st, d_da, 0, 0, t - t0, 0);
-        launch_batch_hash(rw[0], st);
-        launch_batch_binning(rw[0], st);
-        launch_batch_predict_gather(rw[0], st);
-        const int in_win = t >= w0->w0 && t < w0->w1;
-        hipLaunchKernelGGL(kb_adj_tail, gt, dim3(TILE), 0, st, d_da, fw.tiles, fw.ntiles, cur, in_win, t - t0);
-        hipLaunchKernelGGL(kb_adj_theta, dim3(n), dim3(TILE), 0, st, d_da);
-        hipLaunchKernelGGL(kb_adj_pull, gpull, dim3(TILE), 0, st, d_da, fw.tiles, fw.ntiles);
-        hipLaunchKernelGGL(kb_adj_record, gt, dim3(TILE), 0, st, d_da, fw.tiles, fw.ntiles, cur);
-        cur = 1 - cur;
-      }
+      const int len = sg == nseg - 1 ? nsteps - sg * K : K;
+      enqueue_segment(g, *w0, fw, sg, len, copy_blocks, st);
     }
     HIP_TRY(hipGetLastError());
-    for (int i = 0; i < n; i++) {
-      mfc_sim *s = sims[i];
-      adj_work *w = s->adj;
-      // the replay overwrote the handle's cell ids, which blanked particles keep into the next step
-      HIP_TRY(hipMemcpyAsync(s->bins.key_sorted, w->keys_keep, sizeof(int) * (size_t)s->k.N, hipMemcpyDeviceToDevice,
-                             st));
-      HIP_TRY(hipMemcpyAsync(grad + 6 * i, w->theta_acc, sizeof(double) * 6, hipMemcpyDeviceToHost, st));
-    }
+    for (int i = 0; i < n; i++)
+      HIP_TRY(hipMemcpyAsync(grad + 6 * i, sims[i]->adj->theta_acc, sizeof(double) * 6, hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
     return MFC_OK;
   };
   rc = run();
-  if (rc) (void)hipStreamSynchronize(st);  // nothing queued may still read the descriptors
-  (void)hipFree(dmem);
+  if (rc) (void)hipStreamSynchronize(st);  // nothing queued may still read the descriptors' host copies
   return rc;
 }
 
@@ -678,11 +890,9 @@ int mfc_vjp_forward(mfc_sim *s, int nsteps, int checkpoint_every, int w0, int w1
   if (s->batched) return fail(MFC_E_INVALID, "instance of a batch: use mfc_batch_vjp_forward");
   int rc = adj_begin(s, nsteps, checkpoint_every, w0, w1);
   if (rc || (rc = ensure_keys(s))) return rc;
-  for (int t = 0; t < nsteps; t++) {
-    if ((rc = adj_checkpoint(s, t))) return rc;
-    enqueue_step(s, s->cur);
-    s->cur = 1 - s->cur;
-    s->step++;
+  const int K = mfc::adj_segment(s);
+  for (int t = 0; t < nsteps; t += K) {
+    if ((rc = adj_checkpoint(s, t)) || (rc = queue_steps(s, nsteps - t < K ? nsteps - t : K))) return rc;
   }
   finish_steps(s);
   HIP_TRY(hipGetLastError());

@@ -64,6 +64,7 @@ void carve_positional(void *base, int N, mfc::dpositional &p) {
   double *b = (double *)base;
   p.nx = b; p.ny = b + N; p.p = b + 2 * (size_t)N;
   p.rxx = b + 3 * (size_t)N; p.rxy = b + 4 * (size_t)N; p.ryy = b + 5 * (size_t)N;
+  p.nx_out = p.nx; p.ny_out = p.ny;
 }
 
 void enqueue_step(mfc_sim *s, int c) { mfc::launch_batch_step(s->work(c), s->stream); }
@@ -136,13 +137,10 @@ int64_t patch_bound(const mfc::dev_consts &k, int s, int w) {
 
 }  // namespace
 
-void set_patches(mfc_sim *s, int lanes) {
+patch_plan plan_patches(const mfc_sim *s, int lanes) {
   int a, b;
   patch_shape(s->cfg.hdx, s->recs[0].f32, lanes, a, b);
-  s->lanes = lanes;
-  s->k.patch_s = a;
-  s->k.patch_w = b;
-  s->k.patch_slots = mfc::TILE / lanes;
+  const int slots = mfc::TILE / lanes;
   // the entries of the initial particles' patches and half as many again: the particles spread
   // over more patches as the run goes on. A work item past the list's end leaves at once, and
   // entries past the work items' are taken by the slower path
@@ -155,9 +153,18 @@ void set_patches(mfc_sim *s, int lanes) {
     in[(size_t)(cx / b) * rows + cy / a]++;
   }
   int64_t entries = 0;
-  for (int n : in) entries += (n + k.patch_slots - 1) / k.patch_slots;
-  const int64_t bound = patch_bound(k, a, b) + k.N / k.patch_slots, want = entries + entries / 2 + 32;
-  s->npatch_items = (int)(want < bound ? want : bound);
+  for (int n : in) entries += (n + slots - 1) / slots;
+  const int64_t bound = patch_bound(k, a, b) + k.N / slots, want = entries + entries / 2 + 32;
+  return {a, b, slots, (int)(want < bound ? want : bound), (int)(patch_bound(k, a, b) + k.N / slots + 1)};
+}
+
+void set_patches(mfc_sim *s, int lanes) {
+  const patch_plan p = plan_patches(s, lanes);
+  s->lanes = lanes;
+  s->k.patch_s = p.s;
+  s->k.patch_w = p.w;
+  s->k.patch_slots = p.slots;
+  s->npatch_items = p.items;
   if (s->npatch_items > s->npatch_items_max) s->npatch_items_max = s->npatch_items;
 }
 
@@ -268,6 +275,26 @@ int copy_out(mfc_sim *s, void *dst, const void *src, size_t bytes) {
 }
 
 }  // namespace
+
+int queue_steps(mfc_sim *s, int nsteps) {
+  int rc;
+  int done = 0;
+  if (s->use_graphs && nsteps >= GRAPH_STEPS) {
+    while (nsteps - done >= GRAPH_STEPS) {
+      int par = s->cur;
+      if (!s->graph[par] && (rc = build_graph(s, par))) return rc;
+      HIP_TRY(hipGraphLaunch(s->graph[par], s->stream));
+      done += GRAPH_STEPS;
+      s->step += GRAPH_STEPS;
+    }
+  }
+  for (; done < nsteps; done++) {
+    enqueue_step(s, s->cur);
+    s->cur = 1 - s->cur;
+    s->step++;
+  }
+  return MFC_OK;
+}
 
 extern "C" {
 
@@ -473,22 +500,7 @@ int mfc_step(mfc_sim *s, int nsteps) {
   if (!s || nsteps < 0) return fail(MFC_E_INVALID, "bad argument");
   if (s->batched) return fail(MFC_E_INVALID, "instance of a batch: step it with mfc_batch_step");
   int rc = ensure_keys(s);
-  if (rc) return rc;
-  int done = 0;
-  if (s->use_graphs && nsteps >= GRAPH_STEPS) {
-    while (nsteps - done >= GRAPH_STEPS) {
-      int par = s->cur;
-      if (!s->graph[par] && (rc = build_graph(s, par))) return rc;
-      HIP_TRY(hipGraphLaunch(s->graph[par], s->stream));
-      done += GRAPH_STEPS;
-      s->step += GRAPH_STEPS;
-    }
-  }
-  for (; done < nsteps; done++) {
-    enqueue_step(s, s->cur);
-    s->cur = 1 - s->cur;
-    s->step++;
-  }
+  if (rc || (rc = queue_steps(s, nsteps))) return rc;
   finish_steps(s);
   HIP_TRY(hipGetLastError());
   return MFC_OK;

@@ -45,6 +45,8 @@ struct dbins {
 // positional (not permuted) arrays, as particle_gpu::{n,p,R} (particle_gpu.h:39-47)
 struct dpositional {
   double *nx, *ny, *p, *rxx, *rxy, *ryy;
+  double *nx_out, *ny_out;  // where the step's normals go: nx and ny, or (the reverse mode's replay,
+                            // which keeps the normals each step starts from) arrays of their own
 };
 
 constexpr int REC = 16;    // doubles per neighbour record (FP64; FP32C: floats)
@@ -144,9 +146,6 @@ void launch_batch_step(const batch_work &w, hipStream_t s);
 void launch_batch_hash(const batch_work &w, hipStream_t s);
 void launch_batch_binning(const batch_work &w, hipStream_t s);
 void launch_batch_records(const batch_work &w, hipStream_t s);
-// the reverse mode's view of a step: the sorted copy of the start state (into nxt), the FP64
-// records in sorted order and the positional pressure and artificial stress
-void launch_batch_predict_gather(const batch_work &w, hipStream_t s);
 // with events t0 and t1 the launch records the kernel's own start and end in them
 // (hipExtLaunchKernelGGL), which times the kernel without the gap before it
 void launch_batch_interact(const batch_work &w, hipStream_t s, hipEvent_t t0 = nullptr, hipEvent_t t1 = nullptr);

@@ -78,11 +78,6 @@ __device__ inline int block_exclusive_scan(int v, int &total) {
   return pre + x - v;
 }
 
-// patches of the grid: patch p holds the cell rows [r patch_s, (r + 1) patch_s) and the columns
-// [c patch_w, (c + 1) patch_w) with p = c patch_rows + r
-__device__ inline int patch_rows(const dev_consts &k) { return (k.gny + k.patch_s - 1) / k.patch_s; }
-__device__ inline int patch_total(const dev_consts &k) { return ((k.gnx + k.patch_w - 1) / k.patch_w) * patch_rows(k); }
-
 // ------------------------------------------------------------------------------- binning
 // Each kernel body is a device function of its work index, called by the batched kernel with
 // the index of an (instance, block) item of its work table.
@@ -465,36 +460,6 @@ __device__ inline void store_positional(const dpositional &pos, int i, int s, do
   }
 }
 
-// the reverse mode's view of a step, in the storage order of the start state: the sorted copy of
-// the state, the FP64 record at the particle's sorted position and the positional arrays there
-__device__ inline void predict_gather(const dev_consts &k, int t, const dbins &bins, const dstate &cur,
-                                      const dstate &nxt, const dpositional &pos, const drecords &recs) {
-  const int s = t * TILE + threadIdx.x;
-  if (s >= k.N) return;
-  const int i = bins.spos[s];
-  rec_input q = load_rec_input(cur, s);
-  nxt.px[i] = q.x; nxt.py[i] = q.y; nxt.vx[i] = q.u; nxt.vy[i] = q.v;
-  nxt.sxx[i] = q.sxx; nxt.sxy[i] = q.sxy; nxt.syy[i] = q.syy; nxt.szz[i] = cur.szz[s];
-  nxt.rho[i] = q.rho; nxt.T[i] = q.T; nxt.h[i] = q.h;
-  nxt.eps[i] = cur.eps[s]; nxt.epsd[i] = cur.epsd[s];
-  nxt.fcx[i] = cur.fcx[s]; nxt.fcy[i] = cur.fcy[s]; nxt.ftx[i] = cur.ftx[s]; nxt.fty[i] = cur.fty[s];
-  nxt.ptx[i] = q.ptx; nxt.pty[i] = q.pty; nxt.vtx[i] = q.vtx; nxt.vty[i] = q.vty;
-  nxt.rhot[i] = q.rhot; nxt.stxx[i] = q.stxx; nxt.stxy[i] = q.stxy; nxt.styy[i] = q.styy; nxt.stzz[i] = cur.stzz[s];
-  nxt.Tt[i] = q.Tt;
-  nxt.flags[i] = q.fl;
-  nxt.id[i] = cur.id[s];
-  predict_input(k, q);
-  double p, rxx, rxy, ryy;
-  if (q.fl & MFC_FLAG_TOOL) {
-    p = pos.p[i]; rxx = pos.rxx[i]; rxy = pos.rxy[i]; ryy = pos.ryy[i];
-  } else {
-    p = k.c0 * k.c0 * (q.rho - k.rho0);
-    artificial_stress(q.rho, p, q.sxx, q.sxy, q.syy, k.stress_eps, rxx, rxy, ryy, k.promote != 0);
-    pos.p[i] = p; pos.rxx[i] = rxx; pos.rxy[i] = rxy; pos.ryy[i] = ryy;
-  }
-  store_record(k, q, p, rxx, rxy, ryy, i, recs);
-}
-
 // ------------------------------------------------------------------------------- descriptors
 // Fields of the instance descriptors read through the constant address space: the compiler
 // then takes the pointers loaded from them for global pointers and emits global loads, which
@@ -519,7 +484,7 @@ __device__ inline dbins load_bins(MFC_CONST(dbins) * c) {
 }
 __device__ inline dpositional load_pos(MFC_CONST(dpositional) * c) {
   dpositional o;
-  MFC_F(nx); MFC_F(ny); MFC_F(p); MFC_F(rxx); MFC_F(rxy); MFC_F(ryy);
+  MFC_F(nx); MFC_F(ny); MFC_F(p); MFC_F(rxx); MFC_F(rxy); MFC_F(ryy); MFC_F(nx_out); MFC_F(ny_out);
   return o;
 }
 __device__ inline drecords load_recs(MFC_CONST(drecords) * c) {
@@ -1197,11 +1162,15 @@ __device__ inline void update_particle(const dev_consts &k, int i, int s, const 
   if (tool) {  // update_tool_particles (tool_gpu.cu:210-221)
     x += k.dt * k.tool_vx;
     y += k.dt * k.tool_vy;
+    if (pos.nx_out != pos.nx) {  // the same in every thread; a tool particle leaves what the slot holds
+      pos.nx_out[i] = pos.nx[i];
+      pos.ny_out[i] = pos.ny[i];
+    }
   }
   if (!tool) {
     double nx, ny;
     contact_force(k, tool_now, x, y, u, v, fcx, fcy, ftx, fty, nx, ny);
-    pos.nx[i] = nx; pos.ny[i] = ny;
+    pos.nx_out[i] = nx; pos.ny_out[i] = ny;
     if (fixed) {  // actions_gpu.cu:296-311
       u = 0.; v = 0.; fcx = 0.; fcy = 0.; ptx = 0.; pty = 0.; vtx = 0.; vty = 0.;
     }
@@ -1759,16 +1728,6 @@ __global__ __launch_bounds__(TILE) void kb_records(const inst_args *__restrict__
   write_record<F32>(k, load_rec_input(load_state(&c->cur), s), s, load_recs(&c->r));
 }
 
-__global__ __launch_bounds__(TILE) void kb_predict_gather(const inst_args *__restrict__ A,
-                                                          const int2 *__restrict__ work, int nwork) {
-  const int w = xcd_tile(blockIdx.x, nwork);
-  if (w < 0) return;
-  const int2 it = work[w];
-  const inst_args &a = A[it.x];
-  MFC_CONST(inst_args) *c = const_args(A, it.x);
-  predict_gather(a.k, it.y, load_bins(&c->b), load_state(&c->cur), a.nxt, a.pos, load_recs(&c->r));
-}
-
 // The cell ranges of grid_gpu_rothlin (grid_gpu_rothlin.cu:28-127) rebuilt from the sorted cell
 // ids: the lane at the end of each run of equal ids (where unique_by_key_copy starts the next run)
 // writes the run's end into the offsets of its cell's successor and of every empty cell up to the
@@ -1894,10 +1853,6 @@ void launch_batch_records(const batch_work &w, hipStream_t s) {
   const dim3 gt(padded_tiles(w.ntiles));
   if (w.f32) hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_records<true>), gt, dim3(TILE), 0, s, w.args, w.tiles, w.ntiles);
   else hipLaunchKernelGGL(HIP_KERNEL_NAME(kb_records<false>), gt, dim3(TILE), 0, s, w.args, w.tiles, w.ntiles);
-}
-
-void launch_batch_predict_gather(const batch_work &w, hipStream_t s) {
-  hipLaunchKernelGGL(kb_predict_gather, dim3(padded_tiles(w.ntiles)), dim3(TILE), 0, s, w.args, w.tiles, w.ntiles);
 }
 
 template <class K>

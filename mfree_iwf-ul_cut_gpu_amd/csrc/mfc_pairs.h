@@ -8,6 +8,11 @@ namespace mfc {
 
 constexpr int REC_DOUBLES = 16;  // doubles per FP64 neighbour record
 
+// patches of the grid: patch p holds the cell rows [r patch_s, (r + 1) patch_s) and the columns
+// [c patch_w, (c + 1) patch_w) with p = c patch_rows + r
+__device__ inline int patch_rows(const dev_consts &k) { return (k.gny + k.patch_s - 1) / k.patch_s; }
+__device__ inline int patch_total(const dev_consts &k) { return ((k.gnx + k.patch_w - 1) / k.patch_w) * patch_rows(k); }
+
 // a tag: the index of a neighbour's record (storage order) and its flags
 constexpr int TAG_BITS = 4;  // FIXED, BLANKED, TOOL, NONFINITE
 __device__ inline int make_tag(int index, int flags) { return (int)(((unsigned)index << TAG_BITS) | (unsigned)flags); }

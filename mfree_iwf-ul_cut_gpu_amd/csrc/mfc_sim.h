@@ -34,6 +34,7 @@ void adj_free(adj_work *w);
 // allocate, keep the state at the start of step t when t is a checkpoint, and mean the window
 int adj_begin(mfc_sim *s, int nsteps, int checkpoint_every, int w0, int w1);
 int adj_checkpoint(mfc_sim *s, int t);
+int adj_segment(const mfc_sim *s);  // steps between its checkpoints
 int adj_finish(mfc_sim *s, double Fmean[2]);
 // the backward pass of a group of instances that recorded the same run (steps, checkpoint
 // interval, window): one handle, or the instances of a batch, reversed together with one launch
@@ -125,12 +126,20 @@ void patch_items(std::vector<int2> &items, mfc_sim *const *sims, int n);
 // threads per particle of the interaction for `total` particles stepped together, and a handle's
 // patches for that
 int interaction_lanes(int64_t total);
+struct patch_plan {
+  int s, w, slots;  // rows and columns of cells, particles a work-group takes at a time
+  int items;        // work items of the interaction launch
+  int list;         // entries the list of patches can have
+};
+patch_plan plan_patches(const mfc_sim *s, int lanes);
 void set_patches(mfc_sim *s, int lanes);
 // copies the handle's descriptors to where the kernels read them (synchronises its stream)
 int upload_descriptors(mfc_sim *s);
 // whether the current state's h is the same for every particle (host copy of the field)
 void check_uniform_h(mfc_sim *s, const double *h);
 void finish_steps(mfc_sim *s);
+// nsteps steps of a handle whose binning is fresh (hipGraph replays where there are enough)
+int queue_steps(mfc_sim *s, int nsteps);
 int check_tuning(const mfc_tuning *t);
 // the batched kernels' view of a handle for start parity c
 mfc::inst_args instance_args(const mfc_sim *s, int c);

@@ -108,3 +108,25 @@ def test_nonfinite_and_blanked_neighbours(lanes):
         s.step(20)
     assert (o.field("flags") & pymfc.FLAG_BLANKED).sum() >= 1
     assert_bitwise(g, o, context="non-finite")
+
+
+@pytest.mark.parametrize("thermal", ["adiabatic", "contact", "pse"])
+def test_gradient_of_both_pull_paths(thermal):
+    """The reverse step's pull from the LDS copy (both terms of a pair in one evaluation) and from the
+    records in memory, over segments of unequal length. Each contribution differs by some tens of
+    rounding errors, there are about 50 per particle and step, and 30 steps follow each other:
+    30 * 50 * 50 * 1.1e-16 = 8e-12 of the largest component, and two decades for the cancellation
+    within the sums."""
+    cfg = cut(thermal=thermal)
+    cfg.promote_fp64, cfg.secant_tol = 1, 1e-14
+    grads = []
+    for limit in (0, 1):
+        g = pymfc.Sim(cfg)
+        g.set_tuning(stage_limit=limit)
+        g.step(30)
+        F = g.vjp_forward(30, 13, 10, 30)
+        grads.append((F, g.vjp_backward([1.0, 0.5])))
+    assert equal(grads[0][0], grads[1][0])
+    a, b = grads[0][1], grads[1][1]
+    assert np.all(np.isfinite(a)) and np.abs(a).max() > 0
+    assert np.abs(a - b).max() <= 1e-9 * np.abs(a).max()
