@@ -154,56 +154,6 @@ __device__ inline double sigma_yield_tanh(const dev_consts &k, double eps_pl, do
   return TA * TB * TC * TD;
 }
 
-// residual of the radial return (plasticity.cuh:74-83); the flow stress is the model of the
-// function pointer m_s_yield (plasticity.cuh:72), which only this residual uses. The same
-// expressions as sigma_yield / sigma_yield_tanh, with the constants passed in registers: the
-// secant below calls it twice per iteration, and as an outlined function it keeps the step
-// kernels' register budget (inlined, two interleaved residuals would cost them occupancy), while
-// taking its constants from the caller instead of reloading them from the instance descriptor in
-// memory at every call, which made a wave with a long return the last of the interaction launch
-__device__ __attribute__((noinline)) double rr_residual_jc(double dl, double norm, double eps0, double TC, double A,
-                                                          double B, double n, double C, double edr, double dt,
-                                                          double G) {
-  const double s23 = sqrt(2.0 / 3.0);
-  double e = eps0 + s23 * fmax(dl, 0.);
-  double ed = s23 * fmax(dl, 0.) / dt;
-  double TA = A + B * mfcm::pow(e, n);
-  double TB = 1.0;
-  double es = ed / edr;
-  if (es > 1.0) TB = 1.0 + C * mfcm::log(es);
-  else TB = mfcm::pow((1.0 + es), C);
-  double sY = TA * TB * TC;
-  return norm - 2 * G * dl - s23 * sY;
-}
-
-// The same residual for the FP32C path, with the device library's pow and log: FP64 throughout
-// (the return stays in double precision), but not the oracle's own pow and log, whose bits the
-// FP64 path must reproduce; the library's are about half the instructions and branch-free, and
-// the secant's chain of residuals sets the end of the interaction launch late in a cut.
-__device__ __attribute__((noinline)) double rr_residual_jc_lib(double dl, double norm, double eps0, double TC,
-                                                              double A, double B, double n, double C, double edr,
-                                                              double dt, double G) {
-  const double s23 = sqrt(2.0 / 3.0);
-  double e = eps0 + s23 * fmax(dl, 0.);
-  double ed = s23 * fmax(dl, 0.) / dt;
-  double TA = A + B * pow(e, n);
-  double TB = 1.0;
-  double es = ed / edr;
-  if (es > 1.0) TB = 1.0 + C * log(es);
-  else TB = pow((1.0 + es), C);
-  double sY = TA * TB * TC;
-  return norm - 2 * G * dl - s23 * sY;
-}
-
-__device__ __attribute__((noinline)) double rr_residual_tanh(const dev_consts &k, double dl, double norm, double eps0,
-                                                            double t, double TC) {
-  const double s23 = sqrt(2.0 / 3.0);
-  double e = eps0 + s23 * fmax(dl, 0.);
-  double ed = s23 * fmax(dl, 0.) / k.dt;
-  double sY = sigma_yield_tanh(k, e, ed, t, TC);
-  return norm - 2 * k.G * dl - s23 * sY;
-}
-
 // Johnson-Cook plasticity by radial return on one particle (actions_gpu.cu:226-285), in three
 // parts: the yield test (plasticity_test), the secant for dl (rr_secant_wave, for all the
 // returning particles of a wave at once), and the return itself (plasticity_finish).
@@ -260,16 +210,137 @@ __device__ inline int nth_set_bit(unsigned long long m, int n) {
   return b;
 }
 
-// The secant iteration of the radial return (plasticity.cuh:85-119) for every returning particle
-// of a wave, two lanes per particle: the lanes 2r and 2r + 1 take the r-th returning particle of
-// the pass (up to 32 per pass) and evaluate the two residuals of an iteration at once, g(dl) and
-// g(1.01 dl), exchanging them by a shuffle; both then take the same secant update (dl - g/slope,
-// negative iterates folded to -0.1 dl, stop when the step is below the tolerance or after 101
-// iterations), so each particle gets the iterates of a one-lane secant, bit for bit, in half the
-// dependent chain. Called by all 64 lanes of the wave together; need marks the lanes whose
-// particle returns, with their inputs. Returns dl on those lanes, and in folded whether the last
-// update took the fold branch (the reverse mode differentiates the fold's fixed point there).
-// LIB (the FP32C path): plain Johnson-Cook residuals with the device library's pow and log.
+// a / b, correctly rounded, from y = 1 / b correctly rounded: a quotient and two corrections by the
+// exact remainder (the second one starts from a faithful quotient, which Markstein's theorem
+// (IBM J. Res. Dev. 34, 1990) takes to the rounded one). For finite a that is 0 or large enough
+// that its remainder does not underflow (|a| > 2^-960) and quotients in range; 5 operations
+// where a division takes 11.
+__device__ inline double div_by(double a, double b, double y) {
+  const double q0 = a * y;
+  const double q1 = __builtin_fma(__builtin_fma(-q0, b, a), y, q0);
+  return __builtin_fma(__builtin_fma(-q1, b, a), y, q1);
+}
+
+// a double of lane (lane ^ X) of the same four lanes
+template <int X>
+__device__ inline double quad_xor(double v) {
+  constexpr int P = (0 ^ X) | (1 ^ X) << 2 | (2 ^ X) << 4 | (3 ^ X) << 6;  // quad_perm
+  const uint64_t u = mfcm::d2u(v);
+  const unsigned lo = __builtin_amdgcn_mov_dpp((int)(unsigned)u, P, 0xf, 0xf, true);
+  const unsigned hi = __builtin_amdgcn_mov_dpp((int)(unsigned)(u >> 32), P, 0xf, 0xf, true);
+  return mfcm::u2d((uint64_t)hi << 32 | lo);
+}
+
+// The secant iteration of the radial return (plasticity.cuh:85-119) from dl, with the residual :74-83
+// at dl in the even lane of a particle and at 1.01 dl in the odd one, exchanged. All lanes of the
+// particle take the same secant update (dl - g/slope, negative iterates folded to -0.1 dl, stop when
+// the step is below the tolerance or after 101 iterations), so each particle gets the iterates of a
+// one-lane secant, bit for bit. Returns dl, or -dl where the last update took the fold.
+template <class F>
+__device__ inline double secant(double dl, double tol, const F &residual) {
+  const bool second = threadIdx.x & 1;
+  int iter = 0;
+  while (true) {
+    const double dl1 = dl * 1.01;
+    const double gx = residual(second ? dl1 : dl);
+    const double gy = quad_xor<1>(gx);
+    const double g = second ? gy : gx, g1 = second ? gx : gy;
+    const double slope = (g - g1) / (dl - dl1);
+    const double dl_old = dl;
+    dl = dl - g / slope;
+    const bool fold = dl < 0.;
+    if (fold) dl = -0.1 * dl;
+    if (fabs(dl - dl_old) < tol || iter > 100) return fold ? -dl : dl;
+    iter++;
+  }
+}
+
+// One lane's part of the Johnson-Cook flow stress TA TB TC (sigma_yield): the strain factor TA, or
+// the rate factor TB (rate), at the strain e and the relative rate es. One evaluation of the
+// logarithm's series serves both.
+__device__ inline double jc_part(bool rate, double e, double es, double A, double B, double n, double C) {
+  const bool lg = rate && es > 1.0;
+  const double x = !rate ? e : lg ? es : 1.0 + es, y = rate ? C : n;
+  double v;
+  if (x > 0.0 && !mfcm::is_inf(x) && mfcm::abs_d(y) <= 1e290) {  // as mfcm::log and mfcm::pow there
+    int k;
+    double f, s, R;
+    mfcm::log_series(x, k, f, s, R);
+    v = mfcm::log_of(k, f, s, R);
+    if (!lg) v = mfcm::pow_of(k, f, s, R, y);
+  } else if (x == 0.0 && y > 0.0) {
+    v = 0.0;
+  } else {
+    v = lg ? mfcm::log(x) : mfcm::pow(x, y);
+  }
+  return !rate ? A + B * v : lg ? 1.0 + C * v : v;
+}
+
+// The FP64 path's secant, four lanes per particle: lane bit 1 takes one of the two factors of the flow
+// stress that depend on dl. What bounds it is one iteration's chain of dependent FP64 operations (about
+// 300 instructions, 220 of them FP64, 0.7 us): a wave with a long return is the last of its launch (a
+// fold at a tolerance of 1e-14 runs to 101 iterations, the steps of a cut at 1e-6 to 16). With both
+// factors in one lane, full divisions by dt and the reference rate and the pow's special cases on
+// the way an iteration took 1.7 us; a taped and reversed step of the 37.5k cut with 20-100 folding
+// returns 600 us, now 410, of the 6k cut 475, now 280. The loop is in the outlined function so that
+// the polynomials' constants stay in registers through it (evaluated by a function called in the loop
+// they were loaded again each time, and the two cuts took 480 and 320 us).
+__device__ __attribute__((noinline)) double rr_secant_jc(const dev_consts &k, double dl, double norm, double eps0,
+                                                        double TC) {
+  const double A = k.jc_A, B = k.jc_B, n = k.jc_n, C = k.jc_C, edr = k.jc_eps_dot_ref, dt = k.dt, G = k.G;
+  const double s23 = sqrt(2.0 / 3.0);
+  const bool rate = threadIdx.x & 2;
+  const double ydt = 1.0 / dt, yedr = 1.0 / edr;
+  // dt and edr in a range where div_by's quotients are those of the division
+  const bool in_range = dt > 0x1p-400 && dt < 0x1p400 && edr > 0x1p-400 && edr < 0x1p400;
+  return secant(dl, k.secant_tol, [&](double x) {
+    const double inc = s23 * fmax(x, 0.);
+    double ed, es;
+    if (in_range && (inc == 0. || (inc > 0x1p-100 && inc < 0x1p100))) {
+      ed = div_by(inc, dt, ydt);
+      es = div_by(ed, edr, yedr);
+    } else {
+      ed = inc / dt;
+      es = ed / edr;
+    }
+    const double T = jc_part(rate, eps0 + inc, es, A, B, n, C);
+    return norm - 2 * G * x - s23 * (T * quad_xor<2>(T) * TC);
+  });
+}
+
+// the residual with the tanh-modified flow stress
+__device__ __attribute__((noinline)) double rr_residual_tanh(const dev_consts &k, double dl, double norm, double eps0,
+                                                            double t, double TC) {
+  const double s23 = sqrt(2.0 / 3.0);
+  double e = eps0 + s23 * fmax(dl, 0.);
+  double ed = s23 * fmax(dl, 0.) / k.dt;
+  double sY = sigma_yield_tanh(k, e, ed, t, TC);
+  return norm - 2 * k.G * dl - s23 * sY;
+}
+
+// The FP32C path's residual, with the device library's pow and log: FP64 throughout (the return
+// stays in double precision), but not the oracle's own pow and log, whose bits the FP64 path must
+// reproduce. Outlined, with its constants in registers
+__device__ __attribute__((noinline)) double rr_residual_jc_lib(double dl, double norm, double eps0, double TC,
+                                                              double A, double B, double n, double C, double edr,
+                                                              double dt, double G) {
+  const double s23 = sqrt(2.0 / 3.0);
+  double e = eps0 + s23 * fmax(dl, 0.);
+  double ed = s23 * fmax(dl, 0.) / dt;
+  double TA = A + B * pow(e, n);
+  double TB = 1.0;
+  double es = ed / edr;
+  if (es > 1.0) TB = 1.0 + C * log(es);
+  else TB = pow((1.0 + es), C);
+  double sY = TA * TB * TC;
+  return norm - 2 * G * dl - s23 * sY;
+}
+
+// The secant for every returning particle of a wave: neighbouring lanes (4, or 2 with the residuals of the
+// FP32C path and of the tanh model) take a returning particle of the pass each. Called by all 64 lanes of the wave
+// together; need marks the lanes whose particle returns, with their inputs. Returns dl on those
+// lanes, and in folded whether the last update took the fold branch (the reverse mode differentiates
+// the fold's fixed point there). LIB: the FP32C path.
 template <bool LIB>
 __device__ inline double rr_secant_wave(const dev_consts &k, bool need, const rr_input &in, double eps0, double t,
                                         bool &folded) {
@@ -280,46 +351,30 @@ __device__ inline double rr_secant_wave(const dev_consts &k, bool need, const rr
   const double A = k.jc_A, B = k.jc_B, n = k.jc_n, C = k.jc_C, edr = k.jc_eps_dot_ref, dt = k.dt, G = k.G;
   const double tol = k.secant_tol;
   const bool tanh_model = k.jc_tanh != 0;
+  const int lanes_log2 = LIB || tanh_model ? 1 : 2, per_pass = 64 >> lanes_log2;
   while (pending) {  // the same in every lane
     const int cnt = __popcll(pending);
-    const int take = cnt < 32 ? cnt : 32;
+    const int take = cnt < per_pass ? cnt : per_pass;
     const unsigned long long pass = take == cnt ? pending : pending & ((1ull << nth_set_bit(pending, take)) - 1);
-    const int slot = lane >> 1;
+    const int slot = lane >> lanes_log2;
     const bool active = slot < take;
     const int owner = active ? nth_set_bit(pass, slot) : lane;
     const double norm = __shfl(in.norm, owner, 64), TC = __shfl(in.TC, owner, 64);
     const double e0 = __shfl(eps0, owner, 64), tt = __shfl(t, owner, 64);
     double dl = __shfl(in.init, owner, 64);
-    int fold = 0;
     if (active) {
-      const bool second = lane & 1;
-      int iter = 0;
-      while (true) {
-        const double dl1 = dl * 1.01;
-        const double x = second ? dl1 : dl;
-        const double gx = tanh_model ? rr_residual_tanh(k, x, norm, e0, tt, TC)
-                          : LIB      ? rr_residual_jc_lib(x, norm, e0, TC, A, B, n, C, edr, dt, G)
-                                     : rr_residual_jc(x, norm, e0, TC, A, B, n, C, edr, dt, G);
-        const double gy = __shfl_xor(gx, 1, 64);
-        const double g = second ? gy : gx, g1 = second ? gx : gy;
-        const double slope = (g - g1) / (dl - dl1);
-        const double dl_old = dl;
-        dl = dl - g / slope;
-        fold = dl < 0.;
-        if (fold) dl = -0.1 * dl;
-        if (fabs(dl - dl_old) < tol) break;
-        if (iter > 100) break;
-        iter++;
-      }
+      if (tanh_model) dl = secant(dl, tol, [&](double x) { return rr_residual_tanh(k, x, norm, e0, tt, TC); });
+      else if constexpr (LIB)
+        dl = secant(dl, tol, [&](double x) { return rr_residual_jc_lib(x, norm, e0, TC, A, B, n, C, edr, dt, G); });
+      else dl = rr_secant_jc(k, dl, norm, e0, TC);
     }
-    // the owner of slot r reads the result of lane 2r
+    // the owner of slot r reads the result of the slot's first lane
     const bool mine = (pass >> lane) & 1ull;
-    const int src = mine ? 2 * __popcll(pass & ((1ull << lane) - 1)) : lane;
+    const int src = mine ? __popcll(pass & ((1ull << lane) - 1)) << lanes_log2 : lane;
     const double got = __shfl(dl, src, 64);
-    const int got_fold = __shfl(fold, src, 64);
     if (mine) {
-      out = got;
-      folded = got_fold != 0;
+      out = fabs(got);
+      folded = got < 0.;
     }
     pending &= ~pass;
   }

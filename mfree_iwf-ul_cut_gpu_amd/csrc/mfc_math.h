@@ -45,6 +45,21 @@ MFC_HD double abs_d(double x) { return u2d(d2u(x) & 0x7fffffffffffffffULL); }
 // 2^k for k in [-1022, 1023], exact.
 MFC_HD double pow2i(int k) { return u2d((uint64_t)(k + 1023) << 52); }
 
+// a / b where neither operand nor the quotient is near the ends of the exponent range: on the GPU
+// the Newton iterations for 1/b and the corrected quotient that its division expands to, without the
+// scaling and special cases around them (correctly rounded, as the division)
+MFC_HD double quotient(double a, double b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  double y = __builtin_amdgcn_rcp(b);
+  y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+  y = __builtin_fma(__builtin_fma(-b, y, 1.0), y, y);
+  const double q = a * y;
+  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+#else
+  return a / b;
+#endif
+}
+
 constexpr double LN2_HI  = 0.6931471806019545;        // 0x3fe62e42ff000000 (32 bits)
 constexpr double LN2_LO  = -4.2009150726810846e-11;   // ln2 - LN2_HI
 constexpr double INV_LN2 = 1.4426950408889634;
@@ -82,6 +97,13 @@ MFC_HD double exp_reduced(double r) {
 
 // e^x
 MFC_HD double exp(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  // without branches: the scaling is one instruction, exact or rounded once, as below
+  const double kd = floor(x * INV_LN2 + 0.5);
+  const double r = (x - kd * LN2_HI) - kd * LN2_LO;
+  const double v = __builtin_ldexp(exp_reduced(r), (int)kd);
+  return is_nan(x) ? x : x > 709.782712893384 ? u2d(0x7ff0000000000000ULL) : x < -745.1332191019412 ? 0.0 : v;
+#else
   if (is_nan(x)) return x;
   if (x > 709.782712893384) return u2d(0x7ff0000000000000ULL);
   if (x < -745.1332191019412) return 0.0;
@@ -92,24 +114,21 @@ MFC_HD double exp(double x) {
   if (k > 1023) return (e * pow2i(1023)) * pow2i(k - 1023);
   if (k < -1022) return (e * pow2i(k + 54)) * pow2i(-54);
   return e * pow2i(k);
+#endif
 }
-// natural logarithm
-MFC_HD double log(double x) {
-  if (is_nan(x)) return x;
-  if (x < 0.0) return u2d(0x7ff8000000000000ULL);
-  if (x == 0.0) return -u2d(0x7ff0000000000000ULL);
-  if (is_inf(x)) return x;
+// x = 2^e (1 + f) for x positive and finite, and the series R of log(1 + f) (above) with s = f/(2+f)
+MFC_HD void log_series(double x, int &e, double &f, double &s, double &R) {
   int eadj = 0;
   if (x < 2.2250738585072014e-308) { x = x * 18014398509481984.0; eadj = -54; }  // 2^54
   uint64_t u = d2u(x);
-  int e = (int)((u >> 52) & 0x7ff) - 1023 + eadj;
+  e = (int)((u >> 52) & 0x7ff) - 1023 + eadj;
   double m = u2d((u & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL);
   if (m > SQRT2) { m = m * 0.5; e += 1; }
-  double f = m - 1.0;
-  double s = f / (2.0 + f);
+  f = m - 1.0;
+  s = quotient(f, 2.0 + f);
   double z = s * s;
   // R = sum_{k=1..11} 2/(2k+1) z^k
-  double R = 0.08695652173913043;               // 2/23
+  R = 0.08695652173913043;                      // 2/23
   R = 0.09523809523809523 + z * R;              // 2/21
   R = 0.10526315789473684 + z * R;              // 2/19
   R = 0.11764705882352941 + z * R;              // 2/17
@@ -121,9 +140,27 @@ MFC_HD double log(double x) {
   R = 0.4 + z * R;                              // 2/5
   R = 0.6666666666666666 + z * R;               // 2/3
   R = z * R;
+}
+
+// log(x) from its series
+MFC_HD double log_of(int e, double f, double s, double R) {
   double hfsq = 0.5 * f * f;
   double dk = (double)e;
   return dk * LN2_HI - ((hfsq - (s * (hfsq + R) + dk * LN2_LO)) - f);
+}
+
+// natural logarithm
+MFC_HD double log(double x) {
+  if (x > 0.0 && !is_inf(x)) {
+    int e;
+    double f, s, R;
+    log_series(x, e, f, s, R);
+    return log_of(e, f, s, R);
+  }
+  if (is_nan(x)) return x;
+  if (x < 0.0) return u2d(0x7ff8000000000000ULL);
+  if (x == 0.0) return -u2d(0x7ff0000000000000ULL);
+  return x;
 }
 
 MFC_HD bool is_int(double y) { return floor(y) == y; }
@@ -133,11 +170,11 @@ MFC_HD bool is_odd_int(double y) {
   return h * 2.0 != y;
 }
 
-// Error-free transformations (Knuth two-sum, Dekker two-product with Veltkamp splitting).
-MFC_HD void two_sum(double a, double b, double &s, double &e) {
+// Error-free transformations (Dekker's two-sum for |a| >= |b| or a = 0, two-product by an FMA or, where
+// the machine may lack one, Dekker's with Veltkamp splitting: the same p and e)
+MFC_HD void fast_two_sum(double a, double b, double &s, double &e) {
   s = a + b;
-  double bb = s - a;
-  e = (a - (s - bb)) + (b - bb);
+  e = b - (s - a);
 }
 MFC_HD void split(double a, double &hi, double &lo) {
   double c = 134217729.0 * a;  // 2^27 + 1
@@ -147,51 +184,56 @@ MFC_HD void split(double a, double &hi, double &lo) {
 }
 MFC_HD void two_prod(double a, double b, double &p, double &e) {
   p = a * b;
+#if defined(__HIP_DEVICE_COMPILE__)
+  e = __builtin_fma(a, b, -p);
+#else
   double ah, al, bh, bl;
   split(a, ah, al);
   split(b, bh, bl);
   e = (((ah * bh - p) + ah * bl) + al * bh) + al * bl;
+#endif
 }
 
-// log(x) as an unevaluated sum hi + lo (x finite, > 0), used by pow.
-MFC_HD void log_dd(double x, double &hi, double &lo) {
-  int eadj = 0;
-  if (x < 2.2250738585072014e-308) { x = x * 18014398509481984.0; eadj = -54; }
-  uint64_t u = d2u(x);
-  int e = (int)((u >> 52) & 0x7ff) - 1023 + eadj;
-  double m = u2d((u & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL);
-  if (m > SQRT2) { m = m * 0.5; e += 1; }
-  double f = m - 1.0;
-  double s = f / (2.0 + f);
-  double z = s * s;
-  double R = 0.08695652173913043;
-  R = 0.09523809523809523 + z * R;
-  R = 0.10526315789473684 + z * R;
-  R = 0.11764705882352941 + z * R;
-  R = 0.13333333333333333 + z * R;
-  R = 0.15384615384615385 + z * R;
-  R = 0.18181818181818182 + z * R;
-  R = 0.2222222222222222 + z * R;
-  R = 0.2857142857142857 + z * R;
-  R = 0.4 + z * R;
-  R = 0.6666666666666666 + z * R;
-  R = z * R;
+// log(x) from its series as an unevaluated sum hi + lo, used by pow. |f| < 0.42 and f^2/2 < 0.09
+// are below the terms they are added to (e LN2_HI, or f where e is 0)
+MFC_HD void log_dd(int e, double f, double s, double R, double &hi, double &lo) {
   double ff, ffe;
   two_prod(f, f, ff, ffe);
   double hfsq = 0.5 * ff, hfe = 0.5 * ffe;
   double corr = s * (hfsq + R) - hfe;   // log(1+f) = f - hfsq + corr
   double dk = (double)e;
   double s1, e1, s2, e2;
-  two_sum(dk * LN2_HI, f, s1, e1);
-  two_sum(s1, -hfsq, s2, e2);
+  fast_two_sum(dk * LN2_HI, f, s1, e1);
+  fast_two_sum(s1, -hfsq, s2, e2);
   double l = ((e1 + e2) + corr) + dk * LN2_LO;
   hi = s2 + l;
   lo = l - (hi - s2);
 }
 
-// x^y with IEEE 754 special cases; y log|x| is formed in double-double before exp.
+// x^y from the series of log(x); y log(x) is formed in double-double before exp
+MFC_HD double pow_of(int k, double f, double s, double R, double y) {
+  double lh, ll;
+  log_dd(k, f, s, R, lh, ll);
+  if (abs_d(y) > 1e290) return exp(y * lh);
+  double p, pe;
+  two_prod(y, lh, p, pe);
+  double plo = pe + y * ll;
+  double e = exp(p);
+  if (is_inf(e) || e == 0.0) return exp(p + plo);
+  return e + e * plo;
+}
+
+// x^y with IEEE 754 special cases
 MFC_HD double pow(double x, double y) {
   const double INF = u2d(0x7ff0000000000000ULL);
+  double v = 0.0;
+  if (abs_d(x) > 0.0 && !is_inf(x) && !is_inf(y)) {
+    int e;
+    double f, s, R;
+    log_series(abs_d(x), e, f, s, R);
+    v = pow_of(e, f, s, R, y);
+  }
+  if (x > 0.0 && !is_inf(x) && !is_inf(y) && !is_nan(y)) return v;
   if (y == 0.0) return 1.0;
   if (x == 1.0) return 1.0;
   if (is_nan(x) || is_nan(y)) return x + y;
@@ -212,21 +254,8 @@ MFC_HD double pow(double x, double y) {
     if (y > 0.0) return odd ? -INF : INF;
     return odd ? -0.0 : 0.0;
   }
-  double sgn = 1.0;
-  if (x < 0.0) {
-    if (!is_int(y)) return u2d(0x7ff8000000000000ULL);
-    if (is_odd_int(y)) sgn = -1.0;
-    x = -x;
-  }
-  double lh, ll;
-  log_dd(x, lh, ll);
-  if (abs_d(y) > 1e290) return sgn * exp(y * lh);
-  double p, pe;
-  two_prod(y, lh, p, pe);
-  double plo = pe + y * ll;
-  double e = exp(p);
-  if (is_inf(e) || e == 0.0) return sgn * exp(p + plo);
-  return sgn * (e + e * plo);
+  if (!is_int(y)) return u2d(0x7ff8000000000000ULL);
+  return is_odd_int(y) ? -v : v;
 }
 
 // atan(x)

@@ -114,17 +114,6 @@ struct rec64 {
   double x, y, u, v, rho, vol, Axx, Axy, Ayy, Rxx, Rxy, Ryy, c, T, h;
 };
 
-// a / b, correctly rounded, from y = 1 / b correctly rounded: a quotient and two corrections by the
-// exact remainder (the second one starts from a faithful quotient, which Markstein's theorem
-// (IBM J. Res. Dev. 34, 1990) takes to the rounded one). For finite a that is 0 or large enough
-// that its remainder does not underflow (|a| > 2^-960) and quotients in range; 5 operations
-// where a division takes 11.
-__device__ inline double div_by(double a, double b, double y) {
-  const double q0 = a * y;
-  const double q1 = __builtin_fma(__builtin_fma(-q0, b, a), y, q0);
-  return __builtin_fma(__builtin_fma(-q1, b, a), y, q1);
-}
-
 // the terms of one pair in the body of the neighbour loop of do_interactions_monaghan
 // (interactions_gpu.cu:249-326 with cubic_spline kernels.cuh:30-70), in the order and with the
 // operations of the reference's sums. A term that the reference does not add is 0: a sum starts
