@@ -605,7 +605,7 @@ int setup_work(mfc_sim *s, int nsteps, int K, int w0, int w1) {
     for (auto &c : w->ckpt)
       if ((rc = w->alloc_snapshot(c))) return rc;
     const size_t n = (size_t)N, k = (size_t)K;
-    w->patches = plan_patches(s, ADJ_LANES);
+    w->patches = patches_for(s, ADJ_LANES);
     if ((rc = w->alloc(&w->state, (k + 1) * state_block_bytes(N))) || (rc = w->alloc(&w->normal, (k + 1) * 2 * n)) ||
         (rc = w->alloc(&w->perm, k * n)) || (rc = w->alloc(&w->spos, k * n)) || (rc = w->alloc(&w->key_sorted, k * n)) ||
         (rc = w->alloc(&w->offsets, k * ((size_t)s->k.ncell_table + 1))) || (rc = w->alloc(&w->plen, k + 1)) ||

@@ -5,6 +5,7 @@
 // return data synchronise the handle's stream.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <string>
@@ -137,35 +138,50 @@ int64_t patch_bound(const mfc::dev_consts &k, int s, int w) {
 
 }  // namespace
 
-patch_plan plan_patches(const mfc_sim *s, int lanes) {
-  int a, b;
-  patch_shape(s->cfg.hdx, s->recs[0].f32, lanes, a, b);
-  const int slots = mfc::TILE / lanes;
-  // the entries of the initial particles' patches and half as many again: the particles spread
-  // over more patches as the run goes on. A work item past the list's end leaves at once, and
-  // entries past the work items' are taken by the slower path
+void plan_patches(mfc_sim *s) {
   const mfc::dev_consts &k = s->k;
-  const int rows = (k.gny + a - 1) / a, cols = (k.gnx + b - 1) / b;
-  std::vector<int> in((size_t)rows * cols, 0);
+  std::vector<int> cells((size_t)k.gnx * k.gny, 0);
   for (int i = 0; i < k.N; i++) {
     const int gx = (int)((s->sc.px[i] - k.bbmin_x) / k.cell), gy = (int)((s->sc.py[i] - k.bbmin_y) / k.cell);
     const int cx = gx < 0 ? 0 : gx < k.gnx ? gx : k.gnx - 1, cy = gy < 0 ? 0 : gy < k.gny ? gy : k.gny - 1;
-    in[(size_t)(cx / b) * rows + cy / a]++;
+    cells[(size_t)cx * k.gny + cy]++;
   }
-  int64_t entries = 0;
-  for (int n : in) entries += (n + slots - 1) / slots;
-  const int64_t bound = patch_bound(k, a, b) + k.N / slots, want = entries + entries / 2 + 32;
-  return {a, b, slots, (int)(want < bound ? want : bound), (int)(patch_bound(k, a, b) + k.N / slots + 1)};
+  for (int q = 0; q < 3; q++) {
+    patch_plan &p = s->plans[q];
+    p.lanes = PLAN_LANES[q];
+    patch_shape(s->cfg.hdx, s->recs[0].f32, p.lanes, p.s, p.w);
+    p.slots = mfc::TILE / p.lanes;
+    // the entries of the initial particles' patches and half as many again: the particles spread
+    // over more patches as the run goes on. A work item past the list's end leaves at once, and
+    // entries past the work items' are taken by the slower path
+    const int rows = (k.gny + p.s - 1) / p.s;
+    std::vector<int> in(rows);
+    int64_t entries = 0;
+    for (int c0 = 0; c0 < k.gnx; c0 += p.w) {
+      std::fill(in.begin(), in.end(), 0);
+      for (int c = c0; c < k.gnx && c < c0 + p.w; c++)
+        for (int r = 0, g = 0; r < rows; r++)
+          for (int e = 0; e < p.s && g < k.gny; e++, g++) in[r] += cells[(size_t)c * k.gny + g];
+      for (int n : in) entries += (n + p.slots - 1) / p.slots;
+    }
+    p.patches = patch_bound(k, p.s, p.w);
+    const int64_t bound = p.patches + k.N / p.slots, want = entries + entries / 2 + 32;
+    p.items = (int)(want < bound ? want : bound);
+    p.list = (int)bound + 1;
+  }
+}
+
+const patch_plan &patches_for(const mfc_sim *s, int lanes) {
+  return s->plans[lanes == PLAN_LANES[0] ? 0 : lanes == PLAN_LANES[1] ? 1 : 2];
 }
 
 void set_patches(mfc_sim *s, int lanes) {
-  const patch_plan p = plan_patches(s, lanes);
+  const patch_plan &p = patches_for(s, lanes);
   s->lanes = lanes;
   s->k.patch_s = p.s;
   s->k.patch_w = p.w;
   s->k.patch_slots = p.slots;
   s->npatch_items = p.items;
-  if (s->npatch_items > s->npatch_items_max) s->npatch_items_max = s->npatch_items;
 }
 
 int upload_descriptors(mfc_sim *s) {
@@ -268,7 +284,57 @@ int build_graph(mfc_sim *s, int parity) {
   return MFC_OK;
 }
 
+// Results leave through pinned memory of the handle, in pieces of which one is copied to the caller's
+// memory while the GPU writes the next. A copy straight into pageable memory took 20 us for a few
+// bytes, 48 us for 96 KB, 121 us for 288 KB and 909 us for 16 MB; through pinned memory it takes 12, 16, 24
+// and 600. READ_HALF: the copy of a piece of 1 MB (30 us) hides its 15 us of queueing and waiting.
+constexpr size_t READ_HALF = (size_t)1 << 20;
+
+// false where the pinned memory is not to be had: the callers then copy as they can
+bool open_stage(read_stage &r, int N) {
+  if (r.p) return true;
+  const size_t want = ((size_t)N * 4 * sizeof(double) + 4095) & ~(size_t)4095;  // the largest field
+  const size_t half = want < READ_HALF ? want : READ_HALF;
+  for (auto &e : r.done)
+    if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) e = nullptr;
+  void *p = nullptr;
+  if (!r.done[0] || !r.done[1] || hipHostMalloc(&p, 2 * half, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  r.p = (char *)p;
+  r.half = half;
+  return true;
+}
+
+// bytes to dst, in pieces of whole units: piece(offset, length, pinned) queues one. The stage is
+// open and its mutex held
+template <class F>
+int read_out(mfc_sim *s, void *dst, size_t bytes, size_t unit, const F &piece) {
+  read_stage &r = *s->reads;
+  const size_t step = r.half / unit * unit, n = (bytes + step - 1) / step;
+  auto length = [&](size_t c) { return bytes - c * step < step ? bytes - c * step : step; };
+  for (size_t c = 0; c <= n; c++) {
+    if (c < n) {
+      HIP_TRY(piece(c * step, length(c), r.p + (c & 1) * r.half));
+      HIP_TRY(hipEventRecord(r.done[c & 1], s->stream));
+    }
+    if (c > 0) {
+      const size_t d = c - 1;
+      HIP_TRY(hipEventSynchronize(r.done[d & 1]));
+      std::memcpy((char *)dst + d * step, r.p + (d & 1) * r.half, length(d));
+    }
+  }
+  return MFC_OK;
+}
+
 int copy_out(mfc_sim *s, void *dst, const void *src, size_t bytes) {
+  if (bytes == 0) return MFC_OK;
+  std::lock_guard<std::mutex> lock(s->reads->m);
+  if (open_stage(*s->reads, s->k.N))
+    return read_out(s, dst, bytes, sizeof(double), [&](size_t offset, size_t len, void *pinned) {
+      return hipMemcpyAsync(pinned, (const char *)src + offset, len, hipMemcpyDeviceToHost, s->stream);
+    });
   HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s->stream));
   HIP_TRY(hipStreamSynchronize(s->stream));
   return MFC_OK;
@@ -369,16 +435,14 @@ int mfc_create(const mfc_config *cfg, mfc_sim **out) {
     if ((rc = s->alloc(&pb, positional_block_bytes(N)))) return bail(rc);
     carve_positional(pb, N, p);
   }
-  for (int lanes : {1, 4, 8}) {
-    int a, w;
-    patch_shape(cfg->hdx, s->recs[0].f32, lanes, a, w);
-    const int64_t n = patch_bound(k, a, w);
-    if (n > s->npatch_max) s->npatch_max = (int)n;
+  plan_patches(s);
+  for (const patch_plan &q : s->plans) {
+    if (q.patches > s->npatch_max) s->npatch_max = (int)q.patches;
+    if (q.items > s->npatch_items_max) s->npatch_items_max = q.items;
   }
   if ((rc = s->alloc(&b.pcnt, s->npatch_max)) ||
       (rc = s->alloc(&b.plist, (size_t)s->npatch_max + (size_t)N / (mfc::TILE / 8) + 1)) || (rc = s->alloc(&s->plen, 2)))
     return bail(rc);
-  for (int lanes : {1, 4, 8}) set_patches(s, lanes);  // the largest work table
   set_patches(s, interaction_lanes(N));
   check_uniform_h(s, s->sc.h.data());
   for (mfc::drecords &r : s->recs) {
@@ -394,9 +458,9 @@ int mfc_create(const mfc_config *cfg, mfc_sim **out) {
       (rc = s->alloc(&s->hist, (size_t)2 * HIST_CAP)) || (rc = s->alloc(&s->hist_ctr, 1)) ||
       (rc = s->alloc(&s->force_pending, 2)) || (rc = s->alloc(&s->force_groups, (size_t)4 * s->ntiles)))
     return bail(rc);
-  // zero everything, then upload the initial state (particle_gpu.cu:20-125)
+  // zero everything, then upload the initial state (particle_gpu.cu:20-125); with the zeros uploaded
+  // too, creating a handle took 0.9 ms at 6k particles and 14 at 500k, now 0.4 and 10
   {
-    std::vector<double> zero(N, 0.);
     std::vector<int> ids(N);
     for (int i = 0; i < N; i++) ids[i] = i;
     auto up = [&](void *dst, const void *src, size_t bytes) {
@@ -404,12 +468,8 @@ int mfc_create(const mfc_config *cfg, mfc_sim **out) {
     };
     for (int q = 0; q < 2; q++) {
       mfc::dstate &d = s->set[q];
-      double *all[mfc::DSTATE_DOUBLES] = {d.px, d.py, d.vx, d.vy, d.sxx, d.sxy, d.syy, d.szz, d.rho,
-                                          d.T, d.eps, d.epsd, d.h, d.fcx, d.fcy, d.ftx, d.fty, d.ptx,
-                                          d.pty, d.vtx, d.vty, d.rhot, d.stxx, d.stxy, d.styy, d.stzz, d.Tt};
-      for (double *a : all)
-        if (up(a, zero.data(), sizeof(double) * N) != hipSuccess) return bail(fail(MFC_E_HIP, "upload"));
-      if (up(d.flags, zero.data(), sizeof(int) * N) != hipSuccess) return bail(fail(MFC_E_HIP, "upload"));
+      if (hipMemsetAsync(d.px, 0, state_block_bytes(N), s->stream) != hipSuccess)
+        return bail(fail(MFC_E_HIP, "memset"));
       if (up(d.id, ids.data(), sizeof(int) * N) != hipSuccess) return bail(fail(MFC_E_HIP, "upload"));
     }
     mfc::dstate &d = s->set[0];
@@ -420,10 +480,8 @@ int mfc_create(const mfc_config *cfg, mfc_sim **out) {
       return bail(fail(MFC_E_HIP, "upload"));
     if (!S.vx.empty() && (up(d.vx, S.vx.data(), sizeof(double) * N) || up(d.vy, S.vy.data(), sizeof(double) * N)))
       return bail(fail(MFC_E_HIP, "upload"));
-    double *pz[6] = {p.nx, p.ny, p.p, p.rxx, p.rxy, p.ryy};
-    for (double *a : pz)
-      if (up(a, zero.data(), sizeof(double) * N) != hipSuccess) return bail(fail(MFC_E_HIP, "upload"));
-    if (hipMemsetAsync(b.key_sorted, 0, sizeof(int) * N, s->stream) != hipSuccess ||
+    if (hipMemsetAsync(p.nx, 0, positional_block_bytes(N), s->stream) != hipSuccess ||
+        hipMemsetAsync(b.key_sorted, 0, sizeof(int) * N, s->stream) != hipSuccess ||
         hipMemsetAsync(b.offsets, 0, sizeof(int) * ((size_t)c.ncell_table + 1), s->stream) != hipSuccess ||
         (b.offsets_r && hipMemsetAsync(b.offsets_r, 0, sizeof(int) * ((size_t)c.ncell_table + 1), s->stream) != hipSuccess) ||
         hipMemsetAsync(b.clamped, 0, sizeof(unsigned long long), s->stream) != hipSuccess ||
@@ -602,8 +660,8 @@ int mfc_get_info(const mfc_sim *s, mfc_info *info) {
     info->grid_overflow = g.overflow;
   }
   unsigned long long oog = 0;
-  HIP_TRY(hipMemcpyAsync(&oog, s->bins.clamped, sizeof(oog), hipMemcpyDeviceToHost, s->stream));
-  HIP_TRY(hipStreamSynchronize(s->stream));
+  const int rc = copy_out(const_cast<mfc_sim *>(s), &oog, s->bins.clamped, sizeof(oog));  // its read stage
+  if (rc) return rc;
   info->out_of_grid = (int64_t)oog;
   return MFC_OK;
 }
@@ -656,6 +714,16 @@ int mfc_get_field(mfc_sim *s, int field, void *host, size_t bytes) {
       for (int i = 0; i < N; i++) f[i] &= (MFC_FLAG_FIXED | MFC_FLAG_BLANKED | MFC_FLAG_TOOL);
     }
     return MFC_OK;
+  }
+  {
+    std::lock_guard<std::mutex> lock(s->reads->m);
+    const size_t unit = sizeof(double) * nc;
+    if (open_stage(*s->reads, s->k.N))
+      return read_out(s, host, bytes, unit, [&](size_t offset, size_t len, void *pinned) {
+        mfc::launch_interleave(nc, (const double *const *)ptr, (int64_t)(offset / unit), (int64_t)(len / unit),
+                               (double *)pinned, s->stream);
+        return hipGetLastError();
+      });
   }
   std::vector<double> tmp((size_t)N);
   double *out = (double *)host;

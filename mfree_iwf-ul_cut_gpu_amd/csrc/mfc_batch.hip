@@ -141,6 +141,7 @@ int mfc_batch_create(const mfc_config *cfgs, int n, mfc_batch **out) {
     (void)hipStreamDestroy(s->stream);
     s->stream = b->stream;
     s->batched = true;
+    s->reads = b->sims[0]->reads;
     s->use_graphs = false;
     b->adaptive = b->adaptive || s->k.adaptive;
     b->rothlin = b->rothlin || s->k.rothlin;

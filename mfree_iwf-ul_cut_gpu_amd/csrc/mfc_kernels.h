@@ -167,6 +167,8 @@ int chunk_list_cap(int N);
 void launch_tool_wear(const dev_consts &k, const dstate &st, const dpositional &pos, double K, double alpha,
                       double tvx, double tvy, double *part, double *out, hipStream_t s);
 int scan_blocks(int num_cell);
+// out[i nc + c] = src[c][first + i], i < count (out may be pinned host memory)
+void launch_interleave(int nc, const double *const *src, int64_t first, int64_t count, double *out, hipStream_t s);
 void launch_device_math(int fn, const double *x, const double *y, double *out, int64_t n, hipStream_t s);
 
 }  // namespace mfc

@@ -1790,6 +1790,23 @@ __global__ __launch_bounds__(FORCE_LAST_THREADS) void kb_force_final(const inst_
   force_final(ntiles, fo, red);
 }
 
+// components of a field side by side, as the caller gets them: whole 16-byte stores over the host
+// link, which bounds it (55 GB/s)
+template <int NC>
+__global__ __launch_bounds__(256) void k_interleave(const double *__restrict__ a, const double *__restrict__ b,
+                                                    const double *__restrict__ c, const double *__restrict__ d,
+                                                    int64_t count, double *__restrict__ out) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x) {
+    if constexpr (NC == 3) {
+      out[3 * i] = a[i]; out[3 * i + 1] = b[i]; out[3 * i + 2] = c[i];
+    } else {
+      double2 *o = reinterpret_cast<double2 *>(out) + (NC / 2) * i;
+      o[0] = make_double2(a[i], b[i]);
+      if constexpr (NC == 4) o[1] = make_double2(c[i], d[i]);
+    }
+  }
+}
+
 __global__ void k_device_math(int fn, const double *__restrict__ x, const double *__restrict__ y,
                               double *__restrict__ out, int64_t n) {
   int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1826,6 +1843,15 @@ void launch_tool_wear(const dev_consts &k, const dstate &st, const dpositional &
   hipLaunchKernelGGL(k_wear_tiles, dim3(padded_tiles(nt)), dim3(TILE), 0, s, k.N, nt, st, pos.nx, pos.ny, K, alpha,
                      tvx, tvy, part);
   hipLaunchKernelGGL(k_wear_final, dim3(1), dim3(TILE), 0, s, nt, part, out);
+}
+
+void launch_interleave(int nc, const double *const *src, int64_t first, int64_t count, double *out, hipStream_t s) {
+  const dim3 g((unsigned)(count < 256 * 1024 ? (count + 255) / 256 : 1024)), b(256);
+  const double *p[4];
+  for (int c = 0; c < 4; c++) p[c] = c < nc ? src[c] + first : nullptr;
+  if (nc == 2) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_interleave<2>), g, b, 0, s, p[0], p[1], p[2], p[3], count, out);
+  else if (nc == 3) hipLaunchKernelGGL(HIP_KERNEL_NAME(k_interleave<3>), g, b, 0, s, p[0], p[1], p[2], p[3], count, out);
+  else hipLaunchKernelGGL(HIP_KERNEL_NAME(k_interleave<4>), g, b, 0, s, p[0], p[1], p[2], p[3], count, out);
 }
 
 void launch_device_math(int fn, const double *x, const double *y, double *out, int64_t n, hipStream_t s) {

@@ -1,6 +1,8 @@
 // mfc_sim.h — the simulation handle behind the C ABI (internal to the library).
 #pragma once
 
+#include <memory>
+#include <mutex>
 #include <hip/hip_runtime.h>
 
 #include <string>
@@ -43,6 +45,30 @@ int adj_finish(mfc_sim *s, double Fmean[2]);
 int adj_backward(mfc_sim *const *sims, int n, const batch_work &fw, hipStream_t st, const double *cot, double *grad);
 }  // namespace mfc
 
+// the patches of the grid for a number of threads per particle
+constexpr int PLAN_LANES[3] = {1, 4, 8};
+struct patch_plan {
+  int lanes;
+  int s, w, slots;  // rows and columns of cells, particles a work-group takes at a time
+  int items;        // work items of the interaction launch
+  int list;         // entries the list of patches can have
+  int64_t patches;  // patches the grid can have
+};
+
+// pinned memory that results pass through on their way to the caller: two pieces of `half` bytes,
+// allocated at the first read; readers take turns
+struct read_stage {
+  std::mutex m;
+  char *p = nullptr;
+  size_t half = 0;
+  hipEvent_t done[2] = {nullptr, nullptr};
+  ~read_stage() {
+    if (p) (void)hipHostFree(p);
+    for (hipEvent_t e : done)
+      if (e) (void)hipEventDestroy(e);
+  }
+};
+
 struct mfc_sim {
   mfc_config cfg;      // the configuration the handle was created from (checkpoints keep it)
   mfc::scenario sc;
@@ -75,6 +101,7 @@ struct mfc_sim {
   // bins.key/clist, the chunk sums and the records hold the binning and the neighbour records of
   // the current state (computed by the last step's interaction); false after creation and after anything else wrote the state or the bins
   bool keys_fresh = false;
+  std::shared_ptr<read_stage> reads = std::make_shared<read_stage>();  // one for the instances of a batch
   double *wear_part = nullptr;     // tool wear: 4 doubles per tile, then the 4 results
   double wear_accum = 0.;          // accumulated wear, sum of dt * mean rate (tool_wear.cu:59)
   mfc_tuning tuning = {};
@@ -89,6 +116,7 @@ struct mfc_sim {
   int npatch_items = 0;            // patch work items (mfc::inst_args)
   int npatch_items_max = 0;        // the most for any number of lanes
   int npatch_max = 0;              // patches the buffers hold
+  patch_plan plans[3] = {};        // for PLAN_LANES, from the initial particles
   mfc::grid_geo *geo = nullptr;    // adaptive grid: the geometry of the last step (device)
   mfc::batch_work work(int c) const {
     return {dargs + c, 1, dtiles, ntiles, dchunks, nchunks, dpatches, npatches, recs[0].f32, variant(),
@@ -126,12 +154,7 @@ void patch_items(std::vector<int2> &items, mfc_sim *const *sims, int n);
 // threads per particle of the interaction for `total` particles stepped together, and a handle's
 // patches for that
 int interaction_lanes(int64_t total);
-struct patch_plan {
-  int s, w, slots;  // rows and columns of cells, particles a work-group takes at a time
-  int items;        // work items of the interaction launch
-  int list;         // entries the list of patches can have
-};
-patch_plan plan_patches(const mfc_sim *s, int lanes);
+const patch_plan &patches_for(const mfc_sim *s, int lanes);
 void set_patches(mfc_sim *s, int lanes);
 // copies the handle's descriptors to where the kernels read them (synchronises its stream)
 int upload_descriptors(mfc_sim *s);

@@ -410,7 +410,10 @@ class Sim:
 
     @property
     def N(self) -> int:
-        return self.info.n_particles
+        n = self.__dict__.get("_n")
+        if n is None:  # a handle's particle count never changes
+            n = self._n = self.info.n_particles
+        return n
 
     def step(self, n: int = 1) -> None:
         _check(lib().mfc_step(self._h, int(n)), "mfc_step")
@@ -479,7 +482,7 @@ class Sim:
         fid, nc = FIELDS[name]
         N = self.N
         dt = np.int32 if name in INT_FIELDS else np.float64
-        out = np.zeros((N, nc) if nc > 1 else (N,), dtype=dt)
+        out = np.empty((N, nc) if nc > 1 else (N,), dtype=dt)
         _check(lib().mfc_get_field(self._h, fid, out.ctypes.data_as(C.c_void_p), out.nbytes), f"mfc_get_field({name})")
         return out
 
