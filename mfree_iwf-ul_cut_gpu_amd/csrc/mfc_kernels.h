@@ -71,7 +71,7 @@ constexpr int REC32_PIECES = 4;  // float4 per FP32C record
 // more candidates (or of a state whose h is not uniform) reads them from memory.
 constexpr int PATCH_TABLE = 256;  // cell starts a patch holds in LDS: (patch_w + 4) (patch_s + 5) at most
 constexpr int PATCH_COLS = 24;    // patch_w + 4 at most
-__host__ __device__ constexpr int patch_cap(bool f32, int lanes) { return lanes > 1 ? 256 : f32 ? 512 : 488; }
+__host__ __device__ constexpr int patch_cap(bool f32, int lanes) { return lanes > 1 ? 256 : f32 ? 512 : 484; }
 
 // tool-force reduction: the interaction flags the groups of 64 particles (storage order) in which
 // some contact or friction force is not zero; the next step's sort launch sums those groups from

@@ -526,9 +526,12 @@ using rec_t = std::conditional_t<F32, rec32, rec64>;
 // LDS of a work-group of the interaction (patch_cap, PATCH_TABLE and PATCH_COLS above). The records
 // lie in arrays of 16-byte pieces (FP64: xy uv rho/vol A A/R R c/T; FP32C: xy u v rho vol | A c |
 // R T), each one 16 bytes longer than a multiple of the banks, so that the lanes that stage the
-// pieces of a record write different banks. FP64 with one thread per particle keeps one of c and T
-// (X) and leaves the other in memory: with both only two work-groups would fit a CU instead of
-// three (53.9 of 160 KB).
+// pieces of a record write different banks. FP64 with one thread per particle has no room for both c
+// and T beside six pieces, the flags and the record's index, if three work-groups are to fit a
+// CU (53.9 of 160 KB). Where c is a float's value (promote = 0) it takes the index's place once the
+// record is staged; else one of the two (X) is there and c or T, whichever the sums read less, in
+// memory. (With the c of each pair gathered from memory, through a pointer that could be to either memory,
+// and full quotients and roots in the pair's terms the interaction of 197k particles took 116 us, now 104.)
 template <bool F32, int G>
 struct patch_mem {
   static constexpr int CAP = patch_cap(F32, G);
@@ -539,7 +542,8 @@ struct patch_mem {
   static constexpr int TERM_BYTES = G == 1 ? 0 : TILE * (F32 ? 9 * (int)sizeof(float) : 7 * (int)sizeof(double));
   float4 piece[PIECES][CAP + 1];
   double X[ALL_IN_LDS ? 1 : CAP];
-  int tag[CAP];
+  int tag[CAP];            // or, without ALL_IN_LDS and promote, c
+  unsigned char fl[ALL_IN_LDS ? 1 : CAP];  // the flags of the tag
   int flags;               // of all the candidates, and PATCH_DENSE
   int table[PATCH_TABLE];  // LDS index of the first candidate of each cell (row-major in a column)
   int col_first[PATCH_COLS + 1];  // of each staged column
@@ -557,11 +561,15 @@ template <bool F32, int G>
 struct lds_source {
   using mem = patch_mem<F32, G>;
   const mem *m;
-  const double *rec;
+  const __attribute__((address_space(1))) double *rec;  // a global pointer: no load of either memory
   double h0;
-  bool t_in_lds;  // what mem::X holds: T (some particle conducts heat), else c
+  bool c_in_tag;  // mem::X holds T and mem::tag c
+  bool t_in_lds;  // else mem::X holds T (some particle conducts heat), or c
   __device__ inline double2 pos(int j) const { return reinterpret_cast<const double2 *>(m->piece[0])[j]; }
-  __device__ inline int tag(int j) const { return m->tag[j]; }
+  __device__ inline int tag(int j) const {  // its flags
+    if constexpr (mem::ALL_IN_LDS) return m->tag[j];
+    else return m->fl[j];
+  }
   __device__ inline void cand(int j, double2 &p, int &t) const {
     p = pos(j);
     t = tag(j);
@@ -572,7 +580,8 @@ struct lds_source {
     } else {
       q.rho = reinterpret_cast<const double2 *>(m->piece[2])[j].x;
       if constexpr (mem::ALL_IN_LDS) q.T = reinterpret_cast<const double2 *>(m->piece[6])[j].y;
-      else q.T = t_in_lds ? m->X[j] : rec[(size_t)REC * tag_index(t) + 15];
+      else if (c_in_tag || t_in_lds) q.T = m->X[j];
+      else q.T = rec[(size_t)REC * tag_index(m->tag[j]) + 15];
     }
   }
   __device__ inline void record(int j, rec_t<F32> &q) const {
@@ -586,6 +595,9 @@ struct lds_source {
       if constexpr (mem::ALL_IN_LDS) {
         const double2 f = reinterpret_cast<const double2 *>(m->piece[6])[j];
         q.c = f.x; q.T = f.y;
+      } else if (c_in_tag) {
+        q.c = __int_as_float(m->tag[j]);
+        q.T = m->X[j];
       } else if (t_in_lds) {
         q.c = rec[(size_t)REC * tag_index(m->tag[j]) + 14];
         q.T = m->X[j];
@@ -692,10 +704,10 @@ struct math64 {
     const double w2 = pse_c * (FINITE ? exp_neg(div_by(-xx * xx, h2, inv_h2)) : mfcm::exp(-xx * xx / (h2)));
     return (b.T - a.T) * w2 * k.mass / b.rho;
   }
-  template <bool FINITE>
-  __device__ inline pair_acc pair(double2 p, bool tool_j, rec64 &b) const {
+  template <bool FINITE, class ADD>
+  __device__ inline void pair(double2 p, bool tool_j, rec64 &b, ADD &add) const {
     b.x = p.x; b.y = p.y;
-    return pair_terms<FINITE>(k, a, f.tool, f.ta, h1, fourh2, fac, inv_wd, b, tool_j);
+    pair_terms<FINITE>(k, a, f.tool, f.ta, h1, fourh2, fac, inv_wd, b, tool_j, add);
   }
 };
 
@@ -812,12 +824,6 @@ __device__ inline pair_acc acc_of_sums32(const dev_consts &k, const double *s) {
   return {s[0], s[1], s[2], s[3], k.mass * s[4], 0., k.mass * s[5], 0., 0., 0., k.mass * s[6], k.mass * s[7], 2.0 * s[8]};
 }
 
-__device__ inline void add_terms(pair_acc &acc, const pair_acc &t) {
-  acc.vd0 += t.vd0; acc.vd1 += t.vd1; acc.vd2 += t.vd2; acc.vd3 += t.vd3;
-  acc.sd0 += t.sd0; acc.sd1 += t.sd1; acc.sd2 += t.sd2; acc.sd3 += t.sd3;
-  acc.vt0 += t.vt0; acc.vt1 += t.vt1; acc.xt0 += t.xt0; acc.xt1 += t.xt1;
-  acc.tl += t.tl;
-}
 __device__ inline pair_acc acc_of(const dev_consts &k, const sums32 &q) {
   double s[9];
 #pragma unroll
@@ -833,7 +839,7 @@ template <bool F32>
 __device__ inline void sums_mem(const dev_consts &k, const mem_source<F32> &src, const window &w, const rec_t<F32> &a,
                                 const sum_flags &f, pair_acc &acc, double &tpse) {
   const math_t<F32> mt(k, a, f);
-  std::conditional_t<F32, sums32, pair_acc> sum = {};
+  std::conditional_t<F32, sums32, pair_sums> sum = {};
   std::conditional_t<F32, kahan, double> tp = {};
   for (int t = 0; t < w.total; t++) {
     const int j = w.at(t);
@@ -849,7 +855,7 @@ __device__ inline void sums_mem(const dev_consts &k, const mem_source<F32> &src,
     if (!f.run_mech || !mt.support(p, tag)) continue;
     src.record(j, tag, b);
     if constexpr (F32) mt.pair(p, (tag & MFC_FLAG_TOOL) != 0, b, sum);
-    else add_terms(sum, mt.template pair<false>(p, (tag & MFC_FLAG_TOOL) != 0, b));
+    else mt.template pair<false>(p, (tag & MFC_FLAG_TOOL) != 0, b, sum);
   }
   if constexpr (F32) acc = acc_of(k, sum);
   else acc = sum;
@@ -870,7 +876,7 @@ template <bool F32, int G, bool PSE>
 __device__ inline void sums_lds(const dev_consts &k, const lds_source<F32, G> &src, int flags, const int b[5],
                                 const int e[5], const rec_t<F32> &a, const sum_flags &f, pair_acc &acc, double &tpse) {
   const math_t<F32> mt(k, a, f);
-  std::conditional_t<F32, sums32, pair_acc> sum = {};
+  std::conditional_t<F32, sums32, pair_sums> sum = {};
   std::conditional_t<F32, kahan, double> tp = {};
   if constexpr (PSE) {
     if (f.run_pse) {  // all members of the window, two at a time
@@ -930,13 +936,12 @@ __device__ inline void sums_lds(const dev_consts &k, const lds_source<F32, G> &s
     src.record(j, c);
     bool tool_j = false;
     if (flags & MFC_FLAG_TOOL) tool_j = src.tag(j) & MFC_FLAG_TOOL;  // the same branch in every lane
-    if (m[0] == 0u) {
+    const bool used = m[0] == 0u;  // selects: under a branch every mask is moved twice
 #pragma unroll
-      for (int q = 0; q < 4; q++) { m[q] = m[q + 1]; at[q] = at[q + 1]; }
-      m[4] = 0u;
-    }
+    for (int q = 0; q < 4; q++) { m[q] = used ? m[q + 1] : m[q]; at[q] = used ? at[q + 1] : at[q]; }
+    m[4] = used ? 0u : m[4];
     if constexpr (F32) mt.pair(p, tool_j, c, sum);
-    else add_terms(sum, mt.template pair<true>(p, tool_j, c));
+    else mt.template pair<true>(p, tool_j, c, sum);
   }
   if constexpr (F32) acc = acc_of(k, sum);
   else acc = sum;
@@ -1023,9 +1028,9 @@ __device__ inline void sums_group(const dev_consts &k, const lds_source<F32, G> 
         }
         wave_lds_fence();
       } else {
-        const pair_acc t = mt.template pair<true>(p, (tag & MFC_FLAG_TOOL) != 0, b);
-        const double tv[14] = {t.vd0, t.vd1, t.vd2, t.vd3, t.sd0, t.sd1, t.sd2,
-                               t.sd3, t.vt0, t.vt1, t.xt0, t.xt1, t.tl, 0.};
+        pair_row terms_of;
+        mt.template pair<true>(p, (tag & MFC_FLAG_TOOL) != 0, b, terms_of);
+        const double *tv = terms_of.t;
 #pragma unroll
         for (int h = 0; h < PARTS; h++) {
 #pragma unroll
@@ -1284,8 +1289,8 @@ __device__ inline void finish_particle(const inst_args *ap, int i, bool live, co
 // FP64 three to a CU). With 4 or 8 threads per particle the sums of 6k particles take 13 or 8 us
 // instead of 21 (FP64). Measured, us per step (tiles of the sorted order with candidate positions
 // in LDS and a launch for the records, then this): FP32C 6k 55 -> 29, 27k 68 -> 38, 71k 63 -> 48,
-// 197k 80 -> 60, 500k PSE 276 -> 179; FP64 6k 63 -> 32, 27k 77 -> 50, 71k 93 -> 68, 197k 137 -> 121,
-// 500k PSE 403 -> 378.
+// 197k 80 -> 60, 500k PSE 276 -> 179; FP64 6k 63 -> 32, 27k 77 -> 50, 71k 93 -> 62, 197k 137 -> 110,
+// 500k PSE 403 -> 351.
 // returns false, with nothing done, for a patch whose window candidates do not fit the stage or
 // whose state has no uniform h (interact_rest takes it)
 template <bool F32, int G, bool PSE>
@@ -1344,12 +1349,13 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, const inst_args *A, 
     for (int e = 1; e < ncol; e++) c += q >= m.col_first[e];
     const int s = perm[q - m.col_shift[c]], fl = r.vfl[s];
     m.tag[q] = make_tag(s, fl);
+    if constexpr (!patch_mem<F32, G>::ALL_IN_LDS) m.fl[q] = (unsigned char)fl;
     if (fl & ~MFC_FLAG_FIXED) atomicOr(&m.flags, fl & ~MFC_FLAG_FIXED);
   }
   __syncthreads();
   const int flags = m.flags;
   if (flags & (PATCH_DENSE | FLAG_NONFINITE)) return false;  // the same in every thread
-  const bool t_in_lds = k.alpha_wp != 0. || k.alpha_tool != 0.;
+  const bool t_in_lds = k.alpha_wp != 0. || k.alpha_tool != 0., c_in_tag = k.promote == 0;
   {
     // the lanes take the 16-byte pieces of the records in turn, so that a load of a wave covers
     // whole records
@@ -1369,14 +1375,19 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, const inst_args *A, 
       for (int u = 0; u < STAGE_U; u++) {
         const int c = q + u * (TILE / LPR);
         if (c >= ncand) break;
-        if (!PSE && (flags & MFC_FLAG_BLANKED) && pl == 0 && (m.tag[c] & MFC_FLAG_BLANKED))
+        if (!PSE && (flags & MFC_FLAG_BLANKED) && pl == 0 &&
+            ((patch_mem<F32, G>::ALL_IN_LDS ? m.tag[c] : (int)m.fl[patch_mem<F32, G>::ALL_IN_LDS ? 0 : c]) & MFC_FLAG_BLANKED))
           reinterpret_cast<double2 &>(v[u]).x = __builtin_huge_val();
         if constexpr (F32) {
           m.piece[pl][c] = v[u];
         } else if (pl != 1) {  // piece 1 of a record: flags (in the tag) and h (uniform)
           const int p = pl == 0 ? 0 : pl - 1;
           if (patch_mem<F32, G>::ALL_IN_LDS || p < 6) m.piece[p][c] = v[u];
-          else m.X[c] = t_in_lds ? reinterpret_cast<const double2 &>(v[u]).y : reinterpret_cast<const double2 &>(v[u]).x;
+          else {
+            const double2 ct = reinterpret_cast<const double2 &>(v[u]);
+            m.X[c] = c_in_tag || t_in_lds ? ct.y : ct.x;
+            if (c_in_tag) m.tag[c] = __float_as_int((float)ct.x);  // read by the lanes of this wave only, before
+          }
         }
       }
     }
@@ -1410,7 +1421,7 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, const inst_args *A, 
       double2 p;
       int tag;
       rec_t<F32> a;
-      const lds_source<F32, G> lds = {&m, r.rec, k.h0, t_in_lds};
+      const lds_source<F32, G> lds = {&m, (const __attribute__((address_space(1))) double *)r.rec, k.h0, c_in_tag, t_in_lds};
       lds.cand(li, p, tag);
       lds.record(li, a);
       a.x = p.x; a.y = p.y;

@@ -114,24 +114,47 @@ struct rec64 {
   double x, y, u, v, rho, vol, Axx, Axy, Ayy, Rxx, Rxy, Ryy, c, T, h;
 };
 
+// sqrt of x far from the ends of the exponent range: the Goldschmidt iterations and corrections of the
+// division-free square root, without the scaling and special cases around them (correctly rounded)
+__device__ inline double root(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double s = x * y, h = 0.5 * y;
+  const double r = __builtin_fma(-h, s, 0.5);
+  s = __builtin_fma(s, r, s);
+  h = __builtin_fma(h, r, h);
+  s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
+  return __builtin_fma(__builtin_fma(-s, s, x), h, s);
+}
+// the same in single precision: the hardware's value (within one unit in the last place), or its
+// neighbour where x is beyond the midpoint to it
+__device__ inline float root32(float x) {
+  const float s = __builtin_amdgcn_sqrtf(x);
+  const float lo = __uint_as_float(__float_as_uint(s) - 1u), hi = __uint_as_float(__float_as_uint(s) + 1u);
+  float t = __builtin_fmaf(-lo, s, x) <= 0.0f ? lo : s;
+  return __builtin_fmaf(-hi, s, x) > 0.0f ? hi : t;
+}
+
 // the terms of one pair in the body of the neighbour loop of do_interactions_monaghan
 // (interactions_gpu.cu:249-326 with cubic_spline kernels.cuh:30-70), in the order and with the
-// operations of the reference's sums. A term that the reference does not add is 0: a sum starts
-// at +0 and adding +0 leaves every value it can take unchanged. FINITE: both records are finite and
-// the pair is in support, so the quotients by the same divisor can share its reciprocal (div_by;
-// their numerators are kernel values and coordinate differences). inv_wd = 1 / wdeltap.
-template <bool FINITE>
-__device__ inline pair_acc pair_terms(const dev_consts &k, const rec64 &a, bool tool_i, double ta, double h1,
-                                      double fourh2, double fac, double inv_wd, const rec64 &b, bool tool_j) {
-  pair_acc t = {0., 0., 0., 0., 0., 0., 0., 0., 0., 0., 0., 0., 0.};
+// operations of the reference's sums, given to add (pair_sums adds them up, pair_row keeps them).
+// A term that the reference does not add is left out, or 0 in a row: a sum starts at +0 and adding +0
+// leaves every value it can take unchanged. FINITE: both records are finite and the pair is in support, so
+// the quotients by the same divisor can share its reciprocal (div_by), and quotients and roots of
+// kernel values and distances need no scaling. inv_wd = 1 / wdeltap.
+template <bool FINITE, class ADD>
+__device__ inline void pair_terms(const dev_consts &k, const rec64 &a, bool tool_i, double ta, double h1,
+                                  double fourh2, double fac, double inv_wd, const rec64 &b, bool tool_j, ADD &add) {
   const double mass = k.mass;
+  auto over = [](double n, double d) { return FINITE ? mfcm::quotient(n, d) : n / d; };
   // cubic spline with h_i
   double w = 0., w_x = 0., w_y = 0.;
   const double xij = a.x - b.x, yij = a.y - b.y;
   const double rr2 = xij * xij + yij * yij;
   if (FINITE || !(rr2 >= fourh2 || rr2 < 1e-8)) {
     double der, val;
-    double rad = tsqrt(k, rr2);
+    double rad;
+    if constexpr (FINITE) rad = k.promote ? root(rr2) : (double)root32((float)rr2);
+    else rad = tsqrt(k, rr2);
     double q = rad * h1;
     double num;  // of der: one division for both pieces of the spline
     if (q > 1) {
@@ -142,24 +165,20 @@ __device__ inline pair_acc pair_terms(const dev_consts &k, const rec64 &a, bool 
       val = 1 - 1.5 * q * q * (1 - 0.5 * q);
       num = -3.0 * q * (1 - 0.75 * q) * h1;
     }
-    der = num / rad;
+    der = over(num, rad);
     w = val * fac;
     w_x = der * xij * fac;
     w_y = der * yij * fac;
   }
   if (!tool_i && !tool_j) {
-    t.vd0 = (b.u - a.u) * w_x * b.vol;
-    t.vd1 = (b.u - a.u) * w_y * b.vol;
-    t.vd2 = (b.v - a.v) * w_x * b.vol;
-    t.vd3 = (b.v - a.v) * w_y * b.vol;
     double fab = FINITE ? div_by(w, k.wdeltap, inv_wd) : w / k.wdeltap;
     fab *= fab;
     fab *= fab;
     const double Rx = fab * (a.Rxx + b.Rxx), Ry = fab * (a.Rxy + b.Rxy), Rz = fab * (a.Ryy + b.Ryy);
-    t.sd0 = mass * (a.Axx + b.Axx + Rx) * w_x;
-    t.sd1 = mass * (a.Axy + b.Axy + Ry) * w_y;
-    t.sd2 = mass * (a.Axy + b.Axy + Ry) * w_x;
-    t.sd3 = mass * (a.Ayy + b.Ayy + Rz) * w_y;
+    add.strain((b.u - a.u) * w_x * b.vol, (b.u - a.u) * w_y * b.vol, (b.v - a.v) * w_x * b.vol,
+               (b.v - a.v) * w_y * b.vol);
+    add.stress(mass * (a.Axx + b.Axx + Rx) * w_x, mass * (a.Axy + b.Axy + Ry) * w_y,
+               mass * (a.Axy + b.Axy + Ry) * w_x, mass * (a.Ayy + b.Ayy + Rz) * w_y);
     const double vijx = a.u - b.u, vijy = a.v - b.v;
     const double vijposij = vijx * xij + vijy * yij;
     const double rhoij = 0.5 * (a.rho + b.rho);
@@ -168,21 +187,37 @@ __device__ inline pair_acc pair_terms(const dev_consts &k, const rec64 &a, bool 
       const double hij = 0.5 * (a.h + b.h);
       const double muij = (hij * vijposij) / (rr2 + k.av_eta * k.av_eta * hij * hij);
       const double piij = (-k.av_alpha * cij * muij + k.av_beta * muij * muij) / rhoij;
-      t.vt0 = -mass * piij * w_x;
-      t.vt1 = -mass * piij * w_y;
+      add.viscosity(-mass * piij * w_x, -mass * piij * w_y);
     }
-    t.xt0 = -k.xsph_eps * w * mass / rhoij * vijx;
-    t.xt1 = -k.xsph_eps * w * mass / rhoij * vijy;
+    const double xs = over(-k.xsph_eps * w * mass, rhoij);
+    add.advection(xs * vijx, xs * vijy);
   }
   if (ta != 0.) {  // Brookshaw
-    const double rij = sqrt(rr2);
+    const double rij = FINITE ? root(rr2) : sqrt(rr2);
     if (rij > 1e-8) {
-      const double rij1 = 1. / rij;
+      const double rij1 = over(1., rij);
       const double eijx = FINITE ? div_by(xij, rij, rij1) : xij / rij, eijy = FINITE ? div_by(yij, rij, rij1) : yij / rij;
-      t.tl = 2.0 * b.vol * (a.T - b.T) * rij1 * (eijx * w_x + eijy * w_y);
+      add.conduction(2.0 * b.vol * (a.T - b.T) * rij1 * (eijx * w_x + eijy * w_y));
     }
   }
-  return t;
 }
+
+// the terms added to a particle's sums
+struct pair_sums : pair_acc {
+  __device__ inline void strain(double a, double b, double c, double d) { vd0 += a; vd1 += b; vd2 += c; vd3 += d; }
+  __device__ inline void stress(double a, double b, double c, double d) { sd0 += a; sd1 += b; sd2 += c; sd3 += d; }
+  __device__ inline void viscosity(double a, double b) { vt0 += a; vt1 += b; }
+  __device__ inline void advection(double a, double b) { xt0 += a; xt1 += b; }
+  __device__ inline void conduction(double a) { tl += a; }
+};
+// the terms of a pair by themselves
+struct pair_row {
+  double t[14] = {};  // in the order of ACC_N
+  __device__ inline void strain(double a, double b, double c, double d) { t[0] = a; t[1] = b; t[2] = c; t[3] = d; }
+  __device__ inline void stress(double a, double b, double c, double d) { t[4] = a; t[5] = b; t[6] = c; t[7] = d; }
+  __device__ inline void viscosity(double a, double b) { t[8] = a; t[9] = b; }
+  __device__ inline void advection(double a, double b) { t[10] = a; t[11] = b; }
+  __device__ inline void conduction(double a) { t[12] = a; }
+};
 
 }  // namespace mfc
