@@ -76,7 +76,7 @@ struct adj_args {
   char *state;                      // start states in storage order (state_block_bytes each)
   size_t state_bytes;
   double *normal;                   // normals before the step, nx then ny (2 N)
-  int *perm, *spos, *key_sorted;    // N each
+  int *tags, *spos, *key_sorted;    // N each
   int *offsets;                     // num_cell + 1 each
   int2 *plist;                      // list of patches (list_len each) and its length
   int *plen;
@@ -182,7 +182,7 @@ __global__ __launch_bounds__(TILE) void kb_adj_tail(const adj_args *__restrict__
       const int fl = slot_flags(d, slot + 1)[i] & FLAG_MASK;
       record_vjp(k, s, fl, eos_pressure(k, s, fl), br, ob);
     }
-    const int sidx = d.perm[(size_t)slot * N + i];
+    const unsigned sidx = tag_index(d.tags[(size_t)slot * N + i]);
     const double *__restrict__ st = slot_state(d, slot);
     tail_in in;
 #pragma unroll
@@ -504,7 +504,7 @@ __global__ __launch_bounds__(TILE) void kb_adj_record(const adj_args *__restrict
   const int a = it.y * TILE + threadIdx.x;
   if (a >= k.N) return;
   const size_t N = k.N;
-  const int dst = d.perm[a];
+  const unsigned dst = tag_index(d.tags[a]);
   const double *__restrict__ st = slot_state(d, 0);
   double s[TS_N], gs[TS_N], br[REC_DOUBLES];
 #pragma unroll
@@ -549,7 +549,7 @@ struct adj_work {
   // the slots of a segment's steps (adj_args)
   char *state = nullptr;
   double *normal = nullptr;
-  int *perm = nullptr, *spos = nullptr, *key_sorted = nullptr, *offsets = nullptr, *plen = nullptr;
+  int *tags = nullptr, *spos = nullptr, *key_sorted = nullptr, *offsets = nullptr, *plen = nullptr;
   int2 *plist = nullptr;
   mfc_tool_state *tool = nullptr;
   double *acc = nullptr;
@@ -607,7 +607,7 @@ int setup_work(mfc_sim *s, int nsteps, int K, int w0, int w1) {
     const size_t n = (size_t)N, k = (size_t)K;
     w->patches = patches_for(s, ADJ_LANES);
     if ((rc = w->alloc(&w->state, (k + 1) * state_block_bytes(N))) || (rc = w->alloc(&w->normal, (k + 1) * 2 * n)) ||
-        (rc = w->alloc(&w->perm, k * n)) || (rc = w->alloc(&w->spos, k * n)) || (rc = w->alloc(&w->key_sorted, k * n)) ||
+        (rc = w->alloc(&w->tags, k * n)) || (rc = w->alloc(&w->spos, k * n)) || (rc = w->alloc(&w->key_sorted, k * n)) ||
         (rc = w->alloc(&w->offsets, k * ((size_t)s->k.ncell_table + 1))) || (rc = w->alloc(&w->plen, k + 1)) ||
         (rc = w->alloc(&w->plist, k * w->patches.list)) || (rc = w->alloc(&w->tool, k + 1)) ||
         (rc = w->alloc(&w->acc, k * (L_N + 1) * n)) ||
@@ -799,7 +799,7 @@ int adj_backward(mfc_sim *const *sims, int n, const batch_work &fw, hipStream_t 
       carve_state(w->state + (j + 1) * sb, N, a.nxt);
       a.b = s->bins;
       a.b.key_sorted = w->key_sorted + (size_t)j * N;
-      a.b.perm = w->perm + (size_t)j * N;
+      a.b.tags = w->tags + (size_t)j * N;
       a.b.spos = w->spos + (size_t)j * N;
       a.b.offsets = w->offsets + j * nc1;
       a.b.plist = w->plist + (size_t)j * w->patches.list;
@@ -829,7 +829,7 @@ int adj_backward(mfc_sim *const *sims, int n, const batch_work &fw, hipStream_t 
     d.state = w->state;
     d.state_bytes = sb;
     d.normal = w->normal;
-    d.perm = w->perm; d.spos = w->spos; d.key_sorted = w->key_sorted;
+    d.tags = w->tags; d.spos = w->spos; d.key_sorted = w->key_sorted;
     d.offsets = w->offsets;
     d.plist = w->plist; d.plen = w->plen;
     d.list_len = w->patches.list; d.ncell1 = (int)nc1;

@@ -25,8 +25,8 @@ struct dbins {
   int *key_sorted;   // cell id per particle in sorted order (= reference's sorted hash)
   int *offsets;      // num_cell + 1 exclusive prefix sums: cell c = [offsets[c], offsets[c+1])
   int *bucket;       // particle indices grouped by cell, unordered inside a cell
-  int *perm;         // sorted position -> current position
-  int *spos;         // current position -> sorted position
+  int *tags;         // sorted position -> current position and flags of the record there (make_tag)
+  int *spos;         // current position -> sorted position (the reverse mode's replay; else null)
   int *bsum;         // particles counted in each scan chunk of cells (the start state's)
   int *bsum_next;    // the same for the next step: cleared by the sort, counted by the interaction
   int2 *clist;       // per scan chunk, (current position, cell id) of the particles counted in
@@ -53,7 +53,7 @@ constexpr int REC = 16;    // doubles per neighbour record (FP64; FP32C: floats)
 constexpr int ACC_N = 14;  // neighbour sums per particle
 
 // neighbour records in the storage order of the start state (sorted index j is particle
-// perm[j]): rec (FP64 path, 128 bytes: x y flags h u v rho vol Axx Axy Ayy Rxx Rxy Ryy c T) or
+// tag_index(tags[j])): rec (FP64 path, 128 bytes: x y flags h u v rho vol Axx Axy Ayy Rxx Rxy Ryy c T) or
 // rec32 (FP32C path, 64 bytes: x y in FP64, then u v rho vol Axx Axy Ayy c Rxx Rxy Ryy T), and the
 // flags of the record, vfl. h is the state's (it does not change). The interaction writes those
 // of the next step into the other of two sets

@@ -147,7 +147,9 @@ __device__ inline void hash_count(const dev_consts &k, int i, const double *__re
 //    here, so no separate scan of the chunk sums);
 // 3. every particle into its cell's bucket at its arrival slot;
 // 4. each one ranked in its cell by current position, the order thrust::sort_by_key gives on
-//    (cell id, 0..N-1): its sorted position (spos), perm and the sorted cell id there.
+//    (cell id, 0..N-1): its sorted position, its tag and the sorted cell id there. (The tag joins
+//    the flags to the position here, where their load hides behind the counting, so that the
+//    interaction's staging has one load fewer before the records'.)
 // The chunks' cells, bucket ranges and particles are disjoint, so the work-groups share nothing
 // but the chunk sums they read. A chunk of at most SCAN_THREADS * SORT_BATCH particles (a dense
 // chunk holds about 2.25 per cell at the lattice spacing) keeps them in registers and their
@@ -157,7 +159,8 @@ __device__ inline void hash_count(const dev_consts &k, int i, const double *__re
 // thread keep most work-groups of a large table resident at once (a 500k-particle cut has 1.18
 // million cells: 2,310 work-groups). sort_fast and sort_list (launch settings, 0: none) lower
 // the two bounds, so that the other paths can be run on any cut.
-__device__ inline void sort_chunk(int blk, int N, int n, const dbins &b, int sort_fast, int sort_list) {
+__device__ inline void sort_chunk(int blk, int N, int n, const dbins &b, const int *__restrict__ vfl, int sort_fast,
+                                  int sort_list) {
   __shared__ int off_l[SCAN_CHUNK], cnt_l[SCAN_CHUNK], fill_l[SCAN_CHUNK];
   __shared__ int bk_l[SCAN_THREADS * SORT_BATCH];
   const int c0 = blk * SCAN_CHUNK;
@@ -200,12 +203,13 @@ __device__ inline void sort_chunk(int blk, int N, int n, const dbins &b, int sor
   const bool listed = members <= list_cap;
   const int lim = listed ? members : N;
   __syncthreads();
-  int ls[SORT_BATCH];
+  int ls[SORT_BATCH], fl[SORT_BATCH];
   if (fast) {
 #pragma unroll
     for (int u = 0; u < SORT_BATCH; u++) {
       const int p = u * SCAN_THREADS + threadIdx.x;
       if (p >= members) e[u].x = -1;
+      fl[u] = e[u].x >= 0 ? vfl[e[u].x] : 0;
       ls[u] = e[u].x >= 0 ? atomicAdd(&cnt_l[e[u].y - c0], 1) : 0;
     }
   } else {
@@ -241,13 +245,13 @@ __device__ inline void sort_chunk(int blk, int N, int n, const dbins &b, int sor
   const int base = off_l[0];
   // the sorted position of particle i (cell h of the chunk): its rank among the entries of the
   // cell's bucket (bk, indexed from offset bbase)
-  auto rank = [&](int i, int h, const int *bk, int bbase) {
+  auto rank = [&](int i, int h, int flags, const int *bk, int bbase) {
     const int cb = off_l[h], ce = cb + cnt_l[h];
     int rnk = 0;
     for (int q = cb; q < ce; q++) rnk += bk[q - bbase] < i;
     const int j = cb + rnk;
-    b.spos[i] = j;
-    b.perm[j] = i;
+    if (b.spos) b.spos[i] = j;  // the same in every thread
+    b.tags[j] = make_tag(i, flags);
     b.key_sorted[j] = h + c0;
   };
   if (fast) {
@@ -257,7 +261,7 @@ __device__ inline void sort_chunk(int blk, int N, int n, const dbins &b, int sor
     __syncthreads();  // the chunk's buckets
 #pragma unroll
     for (int u = 0; u < SORT_BATCH; u++)
-      if (e[u].x >= 0) rank(e[u].x, e[u].y - c0, bk_l, base);
+      if (e[u].x >= 0) rank(e[u].x, e[u].y - c0, fl[u], bk_l, base);
   } else {
     int *__restrict__ bucket = b.bucket;
     for (int p = threadIdx.x; p < lim; p += SCAN_THREADS) {
@@ -269,7 +273,7 @@ __device__ inline void sort_chunk(int blk, int N, int n, const dbins &b, int sor
     for (int p = threadIdx.x; p < lim; p += SCAN_THREADS) {
       const int2 q = listed ? list[p] : make_int2(p, b.key[p]);
       const int h = q.y - c0;
-      if (h >= 0 && h < SCAN_CHUNK) rank(q.x, h, bucket, 0);
+      if (h >= 0 && h < SCAN_CHUNK) rank(q.x, h, vfl[q.x], bucket, 0);
     }
   }
 }
@@ -478,7 +482,7 @@ __device__ inline dstate load_state(MFC_CONST(dstate) * c) {
 }
 __device__ inline dbins load_bins(MFC_CONST(dbins) * c) {
   dbins o;
-  MFC_F(key); MFC_F(key_sorted); MFC_F(offsets); MFC_F(bucket); MFC_F(perm);
+  MFC_F(key); MFC_F(key_sorted); MFC_F(offsets); MFC_F(bucket); MFC_F(tags);
   MFC_F(spos); MFC_F(bsum); MFC_F(bsum_next); MFC_F(pcnt); MFC_F(plist); MFC_F(plen); MFC_F(plen_next); MFC_F(clist); MFC_F(ccap); MFC_F(offsets_r); MFC_F(clamped);
   return o;
 }
@@ -617,17 +621,17 @@ struct lds_source {
   }
 };
 
-// or the records in memory through the sort permutation (index: sorted index)
+// or the records in memory through the tags (index: sorted index)
 template <bool F32>
 struct mem_source {
   const drecords &r;
-  const int *perm;
+  const int *tags;
   const double *h;  // the start state's
   __device__ inline void cand(int j, double2 &p, int &tag) const {
-    const int s = perm[j];
+    tag = tags[j];
+    const unsigned s = tag_index(tag);
     if constexpr (F32) p = *reinterpret_cast<const double2 *>(r.rec32 + (size_t)REC32_PIECES * s);
     else p = *reinterpret_cast<const double2 *>(r.rec + (size_t)REC * s);
-    tag = make_tag(s, r.vfl[s]);
   }
   __device__ inline void heat(int j, int tag, rec_t<F32> &q) const {
     if constexpr (F32) {
@@ -1081,7 +1085,7 @@ struct deferred_return {
 // everything after the neighbour sums for particle i (sorted index), in the reference's order;
 // returns the particle's fc and ft for the tool force. The secant of a Johnson-Cook return runs
 // for the whole wave after this call (finish_return); the other results do not depend on it
-// reads particle s of the unsorted start state src (s = perm[i]) and writes the updated
+// reads particle s of the unsorted start state src (tags[i]) and writes the updated
 // particle to position i of dst: the gather into sorted order happens here, once. Also writes the
 // step's positional values and, with the state before a return, the next step's record (rn)
 template <bool F32>
@@ -1253,10 +1257,11 @@ __device__ inline sum_flags flags_of(const dev_consts &k, int tag) {
   return f;
 }
 
-// everything that follows the sums for the particle at sorted index i (all 64 lanes of the wave;
-// live: the lane has one)
+// everything that follows the sums for the particle at sorted index i, index s of the start state
+// (all 64 lanes of the wave; live: the lane has one)
 template <bool F32>
-__device__ inline void finish_particle(const inst_args *ap, int i, bool live, const pair_acc &acc, double tpse) {
+__device__ inline void finish_particle(const inst_args *ap, int i, unsigned s, bool live, const pair_acc &acc,
+                                       double tpse) {
   const inst_args &a = *ap;
   MFC_CONST(inst_args) *c = const_args(ap, 0);
   const dev_consts &k = a.k;
@@ -1268,7 +1273,7 @@ __device__ inline void finish_particle(const inst_args *ap, int i, bool live, co
   double *acc_out = a.acc_out;
   if (live) {
     if (acc_out) store_acc(acc_out, k.N, i, acc, tpse);  // the same in every thread
-    update_particle<F32>(k, i, c->b.perm[i], acc, tpse, a.cur, a.nxt, a.pos, load_recs(&c->r), load_recs(&c->rn),
+    update_particle<F32>(k, i, s, acc, tpse, a.cur, a.nxt, a.pos, load_recs(&c->r), load_recs(&c->rn),
                          *a.tool_out, fsum, xn, yn, fln, dr);
     if (fsum[0] != 0. || fsum[1] != 0. || fsum[2] != 0. || fsum[3] != 0.) c->f.gflag[i >> 6] = 1;
   }
@@ -1300,7 +1305,7 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, const inst_args *A, 
   const dev_consts &k = a_.k;
   const drecords r = load_recs(&c_->r);
   const int *__restrict__ offsets = k.rothlin ? c_->b.offsets_r : c_->b.offsets;
-  const int *__restrict__ perm = c_->b.perm;
+  const int *__restrict__ tags = c_->b.tags;
   const int *__restrict__ key_sorted = c_->b.key_sorted;
   constexpr int SLOTS = TILE / G;  // particles at a time
   const int tid = threadIdx.x;
@@ -1347,8 +1352,8 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, const inst_args *A, 
   for (int q = tid; q < ncand; q += TILE) {
     int c = 0;
     for (int e = 1; e < ncol; e++) c += q >= m.col_first[e];
-    const int s = perm[q - m.col_shift[c]], fl = r.vfl[s];
-    m.tag[q] = make_tag(s, fl);
+    const int tag = tags[q - m.col_shift[c]], fl = tag & ((1 << TAG_BITS) - 1);
+    m.tag[q] = tag;
     if constexpr (!patch_mem<F32, G>::ALL_IN_LDS) m.fl[q] = (unsigned char)fl;
     if (fl & ~MFC_FLAG_FIXED) atomicOr(&m.flags, fl & ~MFC_FLAG_FIXED);
   }
@@ -1408,16 +1413,25 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, const inst_args *A, 
     const int n = base + tid / G;  // the particle whose sums this thread takes part in
     const bool mine = n < nown;
     [[maybe_unused]] int i_mine = 0;
+    unsigned s_mine = 0;  // loaded before the sums, which hide its latency
     // the exchange area of the wave; the sums of its particles end there too
     constexpr int WAVE_BYTES = patch_mem<F32, G>::TERM_BYTES / (TILE / 64);
     static_assert(G == 1 || WAVE_BYTES >= 64 / G * ACC_N * (int)sizeof(double), "a wave's sums fit its exchange area");
     [[maybe_unused]] char *terms = m.terms + (size_t)(tid >> 6) * WAVE_BYTES;
     [[maybe_unused]] double *out = reinterpret_cast<double *>(terms) + (size_t)((tid & 63) / G) * ACC_N;
+    int i_own = 0;  // of the particle this thread updates (G > 1)
+    if constexpr (G > 1)
+      if (tid < SLOTS && base + tid < nown) {
+        int col, li;
+        i_own = locate(base + tid, col, li);
+        s_mine = tag_index(m.tag[li]);
+      }
     if (mine) {
       int col, li;
       const int i = locate(n, col, li);
       i_mine = i;
       const int key = key_sorted[i];
+      if constexpr (G == 1) s_mine = tag_index(tags[i]);
       double2 p;
       int tag;
       rec_t<F32> a;
@@ -1448,8 +1462,7 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, const inst_args *A, 
       __syncthreads();
       live = tid < SLOTS && base + tid < nown;
       if (live) {
-        int col, li;
-        i = locate(base + tid, col, li);
+        i = i_own;
         // summed by wave tid / (64 / G)
         const double *o = reinterpret_cast<const double *>(m.terms + (size_t)(tid / (64 / G)) * WAVE_BYTES) +
                           (size_t)(tid % (64 / G)) * ACC_N;
@@ -1459,7 +1472,7 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, const inst_args *A, 
       }
     }
     if (G == 1 || tid < (SLOTS < 64 ? 64 : SLOTS))  // whole waves
-      finish_particle<F32>(A + inst, i, live, acc, tpse);
+      finish_particle<F32>(A + inst, i, s_mine, live, acc, tpse);
   }
   return true;
 }
@@ -1487,7 +1500,7 @@ __device__ __attribute__((noinline)) void interact_rest(const inst_args *ap, int
   pair_acc acc = {};
   double tpse = 0.;
   if (live) {
-    const mem_source<F32> mem = {a_.r, b.perm, a_.cur.h};
+    const mem_source<F32> mem = {a_.r, b.tags, a_.cur.h};
     double2 p;
     int tag;
     rec_t<F32> a;
@@ -1499,7 +1512,7 @@ __device__ __attribute__((noinline)) void interact_rest(const inst_args *ap, int
     if (!f.run_mech && !f.run_pse) w.total = 0;
     sums_mem<F32>(k, mem, w, a, f, acc, tpse);
   }
-  finish_particle<F32>(ap, i, live, acc, tpse);
+  finish_particle<F32>(ap, i, live ? tag_index(b.tags[i]) : 0u, live, acc, tpse);
 }
 
 constexpr int FF_BATCH = 8;  // group sums a thread of force_final loads at a time
@@ -1722,7 +1735,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void kb_sort(const inst_args *__restr
     return;
   }
   const dev_consts &k = A[it.x].k;
-  sort_chunk(it.y, k.N, k.ncell_table, load_bins(&c->b), k.sort_fast, k.sort_list);
+  sort_chunk(it.y, k.N, k.ncell_table, load_bins(&c->b), load_recs(&c->r).vfl, k.sort_fast, k.sort_list);
 }
 
 // the records of a start state that no interaction wrote
