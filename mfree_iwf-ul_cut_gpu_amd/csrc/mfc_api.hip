@@ -7,6 +7,7 @@
 
 #include <algorithm>
 #include <cstdio>
+#include <cmath>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -111,14 +112,17 @@ namespace {
 // rows and columns of the patches for `lanes` threads per particle: the largest near-square
 // rectangle of cells that a full lattice (cells of h = hdx dx: hdx^2 particles each) fills with at
 // most TILE / lanes particles, a lattice line more than the whole ones on each side included, and
-// whose windows fit the LDS stage
+// whose windows fit the LDS stage with every lattice line they can touch (a patch whose window does
+// not fit goes the slower way: with the lines rounded to the nearest whole number, at hdx 1.7
+// a window of the largest patches did not, and a step of 250k particles took 177 us instead of 143)
 void patch_shape(double hdx, bool f32, int lanes, int &s, int &w) {
   const int most = mfc::TILE / lanes, cap = mfc::patch_cap(f32, lanes);
   auto lines = [&](int cells, double more) { return (int)(cells * hdx + more); };
   auto fits = [&](int a, int b) {
     const double more = lanes == 1 ? 1. : 0.5;
-    return lines(a, more) * lines(b, more) <= most && lines(a + 4, 1.) * lines(b + 4, 1.) <= cap && b + 4 <= mfc::PATCH_COLS &&
-           (b + 4) * (a + 5) <= mfc::PATCH_TABLE;
+    auto window = [&](int cells) { return std::ceil(cells * hdx - 1e-6); };
+    return lines(a, more) * lines(b, more) <= most && window(a + 4) * window(b + 4) <= cap &&
+           b + 4 <= mfc::PATCH_COLS && (b + 4) * (a + 5) <= mfc::PATCH_TABLE;
   };
   s = w = 1;
   for (;;) {
