@@ -336,11 +336,26 @@ __device__ __attribute__((noinline)) double rr_residual_jc_lib(double dl, double
   return norm - 2 * G * dl - s23 * sY;
 }
 
-// The secant for every returning particle of a wave: neighbouring lanes (4, or 2 with the residuals of the
-// FP32C path and of the tanh model) take a returning particle of the pass each. Called by all 64 lanes of the wave
-// together; need marks the lanes whose particle returns, with their inputs. Returns dl on those
-// lanes, and in folded whether the last update took the fold branch (the reverse mode differentiates
-// the fold's fixed point there). LIB: the FP32C path.
+// lanes per returning particle: 4, or 2 with the residuals of the FP32C path and of the tanh model
+template <bool LIB>
+__device__ inline int secant_lanes_log2(const dev_consts &k) { return LIB || k.jc_tanh ? 1 : 2; }
+
+// the secant of a returning particle by its lanes. LIB: the FP32C path
+template <bool LIB>
+__device__ inline double rr_secant(const dev_consts &k, double dl, double norm, double e0, double t, double TC) {
+  if (k.jc_tanh) return secant(dl, k.secant_tol, [&](double x) { return rr_residual_tanh(k, x, norm, e0, t, TC); });
+  if constexpr (LIB) {
+    const double A = k.jc_A, B = k.jc_B, n = k.jc_n, C = k.jc_C, edr = k.jc_eps_dot_ref, dt = k.dt, G = k.G;
+    return secant(dl, k.secant_tol, [&](double x) { return rr_residual_jc_lib(x, norm, e0, TC, A, B, n, C, edr, dt, G); });
+  } else {
+    return rr_secant_jc(k, dl, norm, e0, TC);
+  }
+}
+
+// The secant for every returning particle of a wave: neighbouring lanes take a returning particle of
+// the pass each. Called by all 64 lanes of the wave together; need marks the lanes whose particle
+// returns, with their inputs. Returns dl on those lanes, and in folded whether the last update took
+// the fold branch (the reverse mode differentiates the fold's fixed point there).
 template <bool LIB>
 __device__ inline double rr_secant_wave(const dev_consts &k, bool need, const rr_input &in, double eps0, double t,
                                         bool &folded) {
@@ -348,10 +363,7 @@ __device__ inline double rr_secant_wave(const dev_consts &k, bool need, const rr
   unsigned long long pending = __ballot(need);
   double out = 0.;
   folded = false;
-  const double A = k.jc_A, B = k.jc_B, n = k.jc_n, C = k.jc_C, edr = k.jc_eps_dot_ref, dt = k.dt, G = k.G;
-  const double tol = k.secant_tol;
-  const bool tanh_model = k.jc_tanh != 0;
-  const int lanes_log2 = LIB || tanh_model ? 1 : 2, per_pass = 64 >> lanes_log2;
+  const int lanes_log2 = secant_lanes_log2<LIB>(k), per_pass = 64 >> lanes_log2;
   while (pending) {  // the same in every lane
     const int cnt = __popcll(pending);
     const int take = cnt < per_pass ? cnt : per_pass;
@@ -362,12 +374,7 @@ __device__ inline double rr_secant_wave(const dev_consts &k, bool need, const rr
     const double norm = __shfl(in.norm, owner, 64), TC = __shfl(in.TC, owner, 64);
     const double e0 = __shfl(eps0, owner, 64), tt = __shfl(t, owner, 64);
     double dl = __shfl(in.init, owner, 64);
-    if (active) {
-      if (tanh_model) dl = secant(dl, tol, [&](double x) { return rr_residual_tanh(k, x, norm, e0, tt, TC); });
-      else if constexpr (LIB)
-        dl = secant(dl, tol, [&](double x) { return rr_residual_jc_lib(x, norm, e0, TC, A, B, n, C, edr, dt, G); });
-      else dl = rr_secant_jc(k, dl, norm, e0, TC);
-    }
+    if (active) dl = rr_secant<LIB>(k, dl, norm, e0, tt, TC);
     // the owner of slot r reads the result of the slot's first lane
     const bool mine = (pass >> lane) & 1ull;
     const int src = mine ? __popcll(pass & ((1ull << lane) - 1)) << lanes_log2 : lane;
@@ -379,6 +386,41 @@ __device__ inline double rr_secant_wave(const dev_consts &k, bool need, const rr
     pending &= ~pass;
   }
   return out;
+}
+
+// The same for the returning particles of the first wave of a work-group of 256, by all its waves, so that
+// they take one pass: the others have no particles of their own to update. Called by every thread;
+// need is read in the first wave
+struct return_slots {
+  double norm[64], TC[64], e0[64], t[64], dl[64];
+  int count;
+};
+template <bool LIB>
+__device__ inline double rr_secant_group(const dev_consts &k, return_slots &q, bool need, const rr_input &in,
+                                         double eps0, double t, bool &folded) {
+  const int tid = threadIdx.x;
+  const unsigned long long all = __ballot(tid < 64 && need);
+  const int mine = __popcll(all & ((1ull << (tid & 63)) - 1));
+  if (tid < 64) {
+    if (need) {
+      q.norm[mine] = in.norm; q.TC[mine] = in.TC; q.e0[mine] = eps0; q.t[mine] = t; q.dl[mine] = in.init;
+    }
+    if (tid == 0) q.count = __popcll(all);
+  }
+  __syncthreads();
+  const int cnt = q.count;
+  folded = false;
+  if (cnt == 0) return 0.;  // the same in every thread
+  const int lanes_log2 = secant_lanes_log2<LIB>(k), slot = tid >> lanes_log2;
+  if (slot < cnt) {
+    const double dl = rr_secant<LIB>(k, q.dl[slot], q.norm[slot], q.e0[slot], q.t[slot], q.TC[slot]);
+    if ((tid & ((1 << lanes_log2) - 1)) == 0) q.dl[slot] = dl;  // read by the slot's lanes only, before
+  }
+  __syncthreads();
+  if (!(tid < 64 && need)) return 0.;
+  const double got = q.dl[mine];
+  folded = got < 0.;
+  return fabs(got);
 }
 
 // ---------------------------------------------------------------- tool contact (tool_gpu.cu)

@@ -1072,7 +1072,7 @@ __device__ inline void sums_group(const dev_consts &k, const lds_source<F32, G> 
   }
 }
 
-// a particle's Johnson-Cook return, left for the whole wave's secant after update_particle: the
+// a particle's Johnson-Cook return, left for the secant after update_particle: the
 // yield test's inputs and the state the return starts from (the stress, plastic strain and rate
 // and temperature that update_particle stored are replaced once the return is done)
 struct deferred_return {
@@ -1084,7 +1084,7 @@ struct deferred_return {
 
 // everything after the neighbour sums for particle i (sorted index), in the reference's order;
 // returns the particle's fc and ft for the tool force. The secant of a Johnson-Cook return runs
-// for the whole wave after this call (finish_return); the other results do not depend on it
+// after this call (finish_return); the other results do not depend on it
 // reads particle s of the unsorted start state src (tags[i]) and writes the updated
 // particle to position i of dst: the gather into sorted order happens here, once. Also writes the
 // step's positional values and, with the state before a return, the next step's record (rn)
@@ -1223,18 +1223,6 @@ __device__ inline void finish_return(const dev_consts &k, int i, double dl, defe
   write_record<F32>(k, q, i, rn);
 }
 
-// the deferred returns of the wave (all 64 lanes together); dl_out (the reverse mode's replay,
-// the same in every thread): each particle's secant result, -dl where its last update folded,
-// 0 for no return. F32: the FP32C path's secant (rr_secant_wave<true>)
-template <bool F32>
-__device__ inline void wave_returns(const dev_consts &k, int i, bool live, deferred_return &dr, const dstate &dst,
-                                    const drecords &rn, double *__restrict__ dl_out) {
-  bool folded;
-  const double dl = rr_secant_wave<F32>(k, dr.need, dr.in, dr.eps, dr.T, folded);
-  if (dr.need) finish_return<F32>(k, i, dl, dr, dst, rn);
-  if (dl_out && live) dl_out[i] = dr.need ? (folded ? -dl : dl) : 0.;
-}
-
 // the next step's first binning pass for the updated particle i (its storage position in the
 // next step): cell id, arrival slot and patch, as hash_count would take them from the updated
 // state (the bins are passed by value so that they stay in registers). An adaptive grid bins the
@@ -1257,28 +1245,51 @@ __device__ inline sum_flags flags_of(const dev_consts &k, int tag) {
   return f;
 }
 
-// everything that follows the sums for the particle at sorted index i, index s of the start state
-// (all 64 lanes of the wave; live: the lane has one)
+// What follows the sums for the particle at sorted index i, index s of the start state, up to its
+// return: the particle's next cell is left in the struct
+struct after_update {
+  deferred_return dr;
+  double x, y;
+  int fl;
+};
 template <bool F32>
-__device__ inline void finish_particle(const inst_args *ap, int i, unsigned s, bool live, const pair_acc &acc,
-                                       double tpse) {
+__device__ inline void begin_update(const inst_args *ap, int i, unsigned s, bool live, const pair_acc &acc, double tpse,
+                                    after_update &u) {
   const inst_args &a = *ap;
   MFC_CONST(inst_args) *c = const_args(ap, 0);
   const dev_consts &k = a.k;
+  u.dr.need = false;
+  u.x = u.y = 0.;
+  u.fl = 0;
+  if (!live) return;
   double fsum[4] = {0., 0., 0., 0.};
-  double xn = 0., yn = 0.;
-  int fln = 0;
-  deferred_return dr;
-  dr.need = false;
-  double *acc_out = a.acc_out;
-  if (live) {
-    if (acc_out) store_acc(acc_out, k.N, i, acc, tpse);  // the same in every thread
-    update_particle<F32>(k, i, s, acc, tpse, a.cur, a.nxt, a.pos, load_recs(&c->r), load_recs(&c->rn),
-                         *a.tool_out, fsum, xn, yn, fln, dr);
-    if (fsum[0] != 0. || fsum[1] != 0. || fsum[2] != 0. || fsum[3] != 0.) c->f.gflag[i >> 6] = 1;
-  }
-  wave_returns<F32>(k, i, live, dr, a.nxt, load_recs(&c->rn), acc_out ? acc_out + (size_t)ACC_N * k.N : nullptr);
-  next_cell(k, i, live, xn, yn, fln, load_bins(&c->b));
+  if (a.acc_out) store_acc(a.acc_out, k.N, i, acc, tpse);  // the same in every thread
+  update_particle<F32>(k, i, s, acc, tpse, a.cur, a.nxt, a.pos, load_recs(&c->r), load_recs(&c->rn), *a.tool_out, fsum,
+                       u.x, u.y, u.fl, u.dr);
+  if (fsum[0] != 0. || fsum[1] != 0. || fsum[2] != 0. || fsum[3] != 0.) c->f.gflag[i >> 6] = 1;
+}
+
+// The rest (all 64 lanes of the wave): the return with the secant's dl, kept for the reverse mode's
+// replay (-dl where its last update folded, 0 for no return), and the next step's binning
+template <bool F32>
+__device__ inline void end_update(const inst_args *ap, int i, bool live, double dl, bool folded, after_update &u) {
+  const inst_args &a = *ap;
+  MFC_CONST(inst_args) *c = const_args(ap, 0);
+  const dev_consts &k = a.k;
+  if (u.dr.need) finish_return<F32>(k, i, dl, u.dr, a.nxt, load_recs(&c->rn));
+  if (a.acc_out && live) a.acc_out[(size_t)ACC_N * k.N + i] = u.dr.need ? (folded ? -dl : dl) : 0.;
+  next_cell(k, i, live, u.x, u.y, u.fl, load_bins(&c->b));
+}
+
+// both, each wave by itself
+template <bool F32>
+__device__ inline void finish_particle(const inst_args *ap, int i, unsigned s, bool live, const pair_acc &acc,
+                                       double tpse) {
+  after_update u;
+  begin_update<F32>(ap, i, s, live, acc, tpse, u);
+  bool folded;
+  const double dl = rr_secant_wave<F32>(ap->k, u.dr.need, u.dr.in, u.dr.eps, u.dr.T, folded);
+  end_update<F32>(ap, i, live, dl, folded, u);
 }
 
 // One patch of cells by one work-group, G threads per particle: the cell starts and the records of
@@ -1471,8 +1482,18 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, const inst_args *A, 
         tpse = o[ACC_N - 1];
       }
     }
-    if (G == 1 || tid < (SLOTS < 64 ? 64 : SLOTS))  // whole waves
+    if constexpr (G == 1) {
       finish_particle<F32>(A + inst, i, s_mine, live, acc, tpse);
+    } else {  // by the first wave, the returns by all
+      static_assert(SLOTS <= 64 && sizeof(return_slots) <= sizeof(m.piece), "one wave's particles");
+      after_update u;
+      u.dr.need = false;
+      if (tid < 64) begin_update<F32>(A + inst, i, s_mine, live, acc, tpse, u);
+      bool folded;
+      const double dl = rr_secant_group<F32>(k, reinterpret_cast<return_slots &>(m.piece), u.dr.need, u.dr.in, u.dr.eps,
+                                             u.dr.T, folded);
+      if (tid < 64) end_update<F32>(A + inst, i, live, dl, folded, u);
+    }
   }
   return true;
 }
