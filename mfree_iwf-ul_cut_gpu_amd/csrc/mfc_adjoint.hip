@@ -260,13 +260,14 @@ __device__ inline void add_theta(const __attribute__((address_space(4))) adj_arg
 // particle: they list its pairs in the window's order, lane r takes the pairs r, r + PULL_LANES,
 // ..., and the lanes' partial sums are added by a butterfly of shuffles, which gives every lane the
 // same bits (((g0 + g1) + (g2 + g3)) + ...). The count is fixed, and so is the lanes' split of a
-// window, so that an instance's gradient has the same bits alone and in a batch. A work-group takes
-// a part of a patch of cells, as the interaction does, with the records and the adjoints of the sums
-// of its window candidates staged in LDS (240 bytes each; three work-groups to a CU): read from
-// memory per pair, by one work-group per 32 particles of the sorted order, they were 30 gathers of
-// 64 scattered lines, and the pass took 95 us at 37.5k particles.
+// window, so that an instance's gradient has the same bits alone and in a batch, whatever the patches.
+// A work-group takes a part of a patch of cells, as the interaction does, with the records and the
+// adjoints of the sums of its window candidates staged in LDS (240 bytes each; three work-groups to a
+// CU): read from memory per pair, by one work-group per 32 particles of the sorted order, they were 30
+// gathers of 64 scattered lines, and the pass took 95 us at 37.5k particles, now 43.
 constexpr int PULL_LANES = 8;
-constexpr int PULL_CAP = 192;  // window candidates a work-group stages
+constexpr int PULL_AT_ONCE = TILE / PULL_LANES;  // particles a work-group takes at once
+constexpr int PULL_CAP = 208;  // window candidates a work-group stages: 5 x 5 cells at hdx 1.5 have 196 at most
 constexpr int PULL_PIECES = REC_DOUBLES / 2 + ACC_N / 2;  // 16-byte pieces: the record, then the adjoints
 
 struct pull_mem {
@@ -299,10 +300,88 @@ __device__ inline void pull_store(double *gb, int r, double *__restrict__ dst) {
   }
 }
 
+// where the pull reads the window members from (piece p, 16 bytes, of member j): the patch's copy in
+// LDS, by index in the copy, or memory, by sorted index
+struct pull_lds {
+  const pull_mem &m;
+  __device__ inline double2 piece(int p, int j) const { return m.piece[p][j]; }
+};
+struct pull_memory {
+  const double2 *rec, *lam;
+  __device__ inline double2 piece(int p, int j) const {
+    return p < REC_DOUBLES / 2 ? rec[(size_t)j * (REC_DOUBLES / 2) + p] : lam[(size_t)j * (LAM / 2) + p - REC_DOUBLES / 2];
+  }
+};
+
+// the pairs of particle b (index in src; all h equal) over its window, lane r of its lanes; gl: its
+// first lane in the wave, list: 64 bytes of LDS of its own
+template <class SRC>
+__device__ inline void pull_particle(const dev_consts &k, const SRC &src, int b, const window &w, int r, int gl,
+                                     unsigned char *list, double *gb) {
+  auto value = [&](int j, int q) { const double2 v = src.piece(q / 2, j); return q % 2 ? v.y : v.x; };
+  auto load = [&](int j, double *rec, double *la) {
+#pragma unroll
+    for (int q = 0; q < REC_DOUBLES; q++) rec[q] = value(j, q);
+#pragma unroll
+    for (int q = 0; q < L_N; q++) la[q] = value(j, REC_DOUBLES + q);
+  };
+#pragma unroll
+  for (int q = 0; q < REC_DOUBLES; q++) gb[q] = 0.;
+  const double2 pb = src.piece(0, b);
+  const int fb = double_to_bits(value(b, R_FLAGS));
+  const bool pse = k.pse != 0, tool_b = fb & MFC_FLAG_TOOL;
+  const bool pse_b = !(fb & MFC_FLAG_BLANKED) && pse && k.thermal_wp;
+  const double ta_b = pse ? 0. : (tool_b ? k.alpha_tool : k.alpha_wp);
+  for (int b0 = 0; b0 < w.total; b0 += 64) {
+    const int nb = w.total - b0 < 64 ? w.total - b0 : 64;
+    int cnt = 0;
+    for (int u0 = 0; u0 < nb; u0 += PULL_LANES) {
+      const bool in = u0 + r < nb;
+      const int t = in ? u0 + r : nb - 1, a = w.at(b0 + t);
+      const double2 pa = src.piece(0, a);
+      const int fa = double_to_bits(value(a, R_FLAGS));
+      const double dx = pa.x - pb.x, dy = pa.y - pb.y, rr2 = dx * dx + dy * dy;
+      const pull_pair pm = pull_flags(k, fa, fb);
+      const bool hit = in && a != b && pm.of_a && pm.of_b && rr2 < 4 * k.h0 * k.h0 && rr2 >= 1e-8;
+      const unsigned bits = (unsigned)(__ballot(hit) >> gl) & ((1u << PULL_LANES) - 1u);
+      if (hit) list[cnt + __popc(bits & ((1u << r) - 1u))] = (unsigned char)t;
+      cnt += __popc(bits);
+      if (pse && in && a != b) {
+        const bool pse_a = !(fa & MFC_FLAG_BLANKED) && k.thermal_wp;
+        if (pse_a || pse_b) {
+          double ra[REC_DOUBLES], la[LAM], rb[REC_DOUBLES], lb[LAM], dummy[REC_DOUBLES];
+          load(a, ra, la);
+          load(b, rb, lb);
+          if (pse_a) pse_vjp(k, ra, rb, la[L_TPSE], false, true, dummy, gb);
+          if (pse_b) pse_vjp(k, rb, ra, lb[L_TPSE], true, false, gb, dummy);
+        }
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the list, by lanes of the same wave
+    __builtin_amdgcn_wave_barrier();
+    for (int p = r; p < cnt; p += PULL_LANES) {
+      // both records are read where a value is used: held in registers across the pair (the
+      // particle's own across the pairs) they spill
+      const int a = w.at(b0 + list[p]);
+      const bool tool_a = double_to_bits(value(a, R_FLAGS)) & MFC_FLAG_TOOL;
+      // the mechanical sums of both take a pair without a tool particle; each conduction sum
+      // counts where its particle conducts
+      const double ta_a = pse ? 0. : (tool_a ? k.alpha_tool : k.alpha_wp);
+      auto adj = [&](int j, double ta, int q) { return q == L_TL && ta == 0. ? 0. : value(j, REC_DOUBLES + q); };
+      asm volatile("" ::: "memory");
+      pair_vjp_sym(
+          k, [&](int q) { return value(b, q); }, [&](int q) { return value(a, q); }, !tool_a && !tool_b,
+          ta_a != 0. || ta_b != 0., [&](int q) { return adj(b, ta_b, q); }, [&](int q) { return adj(a, ta_a, q); }, gb);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
 // one entry of the list from the records in memory: what the staged path does not take (more
-// candidates than the stage holds, an h that is not uniform, entries past the work items). Lane r
-// tests and takes the candidates r, r + PULL_LANES, ...
-__device__ inline void pull_rest(const adj_args *__restrict__ D, int inst, int slot, int patch, int part) {
+// candidates than the stage holds, an h that is not uniform, entries past the work items). With a
+// uniform h the same bits; else each pair's two terms one after the other, with the h of each
+__device__ inline void pull_rest(pull_mem &m, const adj_args *__restrict__ D, int inst, int slot, int patch, int part) {
   MFC_ADJ_ARGS(d, inst);
   const dev_consts &k = D[inst].k;
   const size_t N = k.N;
@@ -310,44 +389,52 @@ __device__ inline void pull_rest(const adj_args *__restrict__ D, int inst, int s
   const int nrb = patch_rows(k), pc = patch / nrb, pr = patch - pc * nrb;
   const int r0 = pr * k.patch_s, r1 = r0 + k.patch_s < k.gny ? r0 + k.patch_s : k.gny;
   const int c0 = pc * k.patch_w, c1 = c0 + k.patch_w < k.gnx ? c0 + k.patch_w : k.gnx;
-  const int r = threadIdx.x % PULL_LANES;
-  int n = part * k.patch_slots + (int)threadIdx.x / PULL_LANES, b = -1;
-  for (int c = c0; c < c1 && b < 0; c++) {
-    const int first = offsets[c * k.gny + r0], count = offsets[c * k.gny + r1] - first;
-    if (n < count) b = first + n;
-    n -= count;
-  }
-  if (b < 0) return;  // whole groups of lanes
+  const int lane = threadIdx.x & 63, r = lane % PULL_LANES, gl = lane - r;
   const double *__restrict__ rec = d.rec, *__restrict__ lam = d.lam_acc;
-  const double *rb = rec + (size_t)REC_DOUBLES * b, *lb = lam + (size_t)LAM * b;
-  double gb[REC_DOUBLES], dummy[REC_DOUBLES];
+  for (int s0 = 0; s0 < k.patch_slots; s0 += PULL_AT_ONCE) {
+    int n = part * k.patch_slots + s0 + (int)threadIdx.x / PULL_LANES, b = -1;
+    for (int c = c0; c < c1 && b < 0; c++) {
+      const int first = offsets[c * k.gny + r0], count = offsets[c * k.gny + r1] - first;
+      if (n < count) b = first + n;
+      n -= count;
+    }
+    if (b < 0) return;  // whole groups of lanes
+    double gb[REC_DOUBLES];
+    const window w = make_window(k, offsets, keys[b]);
+    if (k.uniform_h) {
+      const pull_memory src = {reinterpret_cast<const double2 *>(rec), reinterpret_cast<const double2 *>(lam)};
+      pull_particle(k, src, b, w, r, gl, m.list[threadIdx.x / PULL_LANES], gb);
+    } else {
+      const double *rb = rec + (size_t)REC_DOUBLES * b, *lb = lam + (size_t)LAM * b;
+      double dummy[REC_DOUBLES];
 #pragma unroll
-  for (int q = 0; q < REC_DOUBLES; q++) gb[q] = 0.;
-  const int fb = double_to_bits(rb[R_FLAGS]);
-  const bool pse = k.pse != 0, tool_b = fb & MFC_FLAG_TOOL;
-  const double ta_b = pse ? 0. : (tool_b ? k.alpha_tool : k.alpha_wp);
-  const bool pse_b = !(fb & MFC_FLAG_BLANKED) && pse && k.thermal_wp;
-  const window w = make_window(k, offsets, keys[b]);
-  for (int t = r; t < w.total; t += PULL_LANES) {
-    const int a = w.at(t);
-    if (a == b) continue;
-    asm volatile("" ::: "memory");  // b's record is read again for each pair: kept, it spills
-    const double *ra = rec + (size_t)REC_DOUBLES * a, *la = lam + (size_t)LAM * a;
-    const int fa = double_to_bits(ra[R_FLAGS]);
-    const bool tool_a = fa & MFC_FLAG_TOOL;
-    const double dx = ra[R_X] - rb[R_X], dy = ra[R_Y] - rb[R_Y], rr2 = dx * dx + dy * dy;
-    const pull_pair m = pull_flags(k, fa, fb);
-    const double ha = ra[R_H], hb = rb[R_H];
-    const bool of_a = m.of_a && rr2 < 4 * ha * ha && rr2 >= 1e-8, of_b = m.of_b && rr2 < 4 * hb * hb && rr2 >= 1e-8;
-    const bool pse_a = !(fa & MFC_FLAG_BLANKED) && pse && k.thermal_wp;
-    const double ta_a = pse ? 0. : (tool_a ? k.alpha_tool : k.alpha_wp);
-    if (of_a) pair_vjp(k, ra, rb, tool_a, tool_b, ta_a, la, false, true, dummy, gb);
-    if (pse_a) pse_vjp(k, ra, rb, la[L_TPSE], false, true, dummy, gb);
-    asm volatile("" ::: "memory");
-    if (of_b) pair_vjp(k, rb, ra, tool_b, tool_a, ta_b, lb, true, false, gb, dummy);
-    if (pse_b) pse_vjp(k, rb, ra, lb[L_TPSE], true, false, gb, dummy);
+      for (int q = 0; q < REC_DOUBLES; q++) gb[q] = 0.;
+      const int fb = double_to_bits(rb[R_FLAGS]);
+      const bool pse = k.pse != 0, tool_b = fb & MFC_FLAG_TOOL;
+      const double ta_b = pse ? 0. : (tool_b ? k.alpha_tool : k.alpha_wp);
+      const bool pse_b = !(fb & MFC_FLAG_BLANKED) && pse && k.thermal_wp;
+      for (int t = r; t < w.total; t += PULL_LANES) {
+        const int a = w.at(t);
+        if (a == b) continue;
+        asm volatile("" ::: "memory");  // b's record is read again for each pair: kept, it spills
+        const double *ra = rec + (size_t)REC_DOUBLES * a, *la = lam + (size_t)LAM * a;
+        const int fa = double_to_bits(ra[R_FLAGS]);
+        const bool tool_a = fa & MFC_FLAG_TOOL;
+        const double dx = ra[R_X] - rb[R_X], dy = ra[R_Y] - rb[R_Y], rr2 = dx * dx + dy * dy;
+        const pull_pair pm = pull_flags(k, fa, fb);
+        const double ha = ra[R_H], hb = rb[R_H];
+        const bool of_a = pm.of_a && rr2 < 4 * ha * ha && rr2 >= 1e-8, of_b = pm.of_b && rr2 < 4 * hb * hb && rr2 >= 1e-8;
+        const bool pse_a = !(fa & MFC_FLAG_BLANKED) && pse && k.thermal_wp;
+        const double ta_a = pse ? 0. : (tool_a ? k.alpha_tool : k.alpha_wp);
+        if (of_a) pair_vjp(k, ra, rb, tool_a, tool_b, ta_a, la, false, true, dummy, gb);
+        if (pse_a) pse_vjp(k, ra, rb, la[L_TPSE], false, true, dummy, gb);
+        asm volatile("" ::: "memory");
+        if (of_b) pair_vjp(k, rb, ra, tool_b, tool_a, ta_b, lb, true, false, gb, dummy);
+        if (pse_b) pse_vjp(k, rb, ra, lb[L_TPSE], true, false, gb, dummy);
+      }
+    }
+    pull_store(gb, r, d.g_rec + (size_t)REC_DOUBLES * b);
   }
-  pull_store(gb, r, d.g_rec + (size_t)REC_DOUBLES * b);
 }
 
 // returns false, with nothing done, for an entry that pull_rest takes
@@ -401,75 +488,21 @@ __device__ inline bool pull_patch(pull_mem &m, const adj_args *__restrict__ D, i
   }
   if (tid < ncol * nrow) m.table[tid] += m.col_shift[te];
   __syncthreads();
-  const int n = part * (TILE / PULL_LANES) + tid / PULL_LANES;
-  if (n >= nown) return true;  // whole groups of lanes
   const int lane = tid & 63, r = lane % PULL_LANES, gl = lane - r;
-  int col = 0;
-  for (int e = 1; e < ncol; e++) col += n >= m.own_first[e];
-  const int li = m.table[col * nrow + r0 - s0] + (n - m.own_first[col]);
-  const int b = li - m.col_shift[col];
-  auto load = [&](int j, double *rec, double *la) {
-#pragma unroll
-    for (int q = 0; q < REC_DOUBLES / 2; q++) { const double2 v = m.piece[q][j]; rec[2 * q] = v.x; rec[2 * q + 1] = v.y; }
-#pragma unroll
-    for (int q = 0; q < L_N / 2; q++) { const double2 v = m.piece[REC_DOUBLES / 2 + q][j]; la[2 * q] = v.x; la[2 * q + 1] = v.y; }
-  };
-  double gb[REC_DOUBLES];
-#pragma unroll
-  for (int q = 0; q < REC_DOUBLES; q++) gb[q] = 0.;
-  const double2 pb = m.piece[0][li];
-  const int fb = double_to_bits(m.piece[R_FLAGS / 2][li].x);
-  const bool pse = k.pse != 0, tool_b = fb & MFC_FLAG_TOOL;
-  const bool pse_b = !(fb & MFC_FLAG_BLANKED) && pse && k.thermal_wp;
-  const double ta_b = pse ? 0. : (tool_b ? k.alpha_tool : k.alpha_wp);
-  const int gi = q0 + col, gj = d.key_sorted[(size_t)slot * N + b] - gi * k.gny;
-  const window w = make_window_at(k, gi, gj, [&](int c, int row) { return m.table[(c - q0) * nrow + row - s0]; });
-  unsigned char *list = m.list[tid / PULL_LANES];
-  for (int b0 = 0; b0 < w.total; b0 += 64) {
-    const int nb = w.total - b0 < 64 ? w.total - b0 : 64;
-    int cnt = 0;
-    for (int u0 = 0; u0 < nb; u0 += PULL_LANES) {
-      const bool in = u0 + r < nb;
-      const int a = w.at(b0 + (in ? u0 + r : nb - 1));
-      const double2 pa = m.piece[0][a];
-      const int fa = double_to_bits(m.piece[R_FLAGS / 2][a].x);
-      const double dx = pa.x - pb.x, dy = pa.y - pb.y, rr2 = dx * dx + dy * dy;
-      const pull_pair pm = pull_flags(k, fa, fb);
-      const bool hit = in && a != li && pm.of_a && pm.of_b && rr2 < 4 * k.h0 * k.h0 && rr2 >= 1e-8;
-      const unsigned bits = (unsigned)(__ballot(hit) >> gl) & ((1u << PULL_LANES) - 1u);
-      if (hit) list[cnt + __popc(bits & ((1u << r) - 1u))] = (unsigned char)a;
-      cnt += __popc(bits);
-      if (pse && in && a != li) {
-        const bool pse_a = !(fa & MFC_FLAG_BLANKED) && k.thermal_wp;
-        if (pse_a || pse_b) {
-          double ra[REC_DOUBLES], la[LAM], rb[REC_DOUBLES], lb[LAM], dummy[REC_DOUBLES];
-          load(a, ra, la);
-          load(li, rb, lb);
-          if (pse_a) pse_vjp(k, ra, rb, la[L_TPSE], false, true, dummy, gb);
-          if (pse_b) pse_vjp(k, rb, ra, lb[L_TPSE], true, false, gb, dummy);
-        }
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the list, by lanes of the same wave
-    __builtin_amdgcn_wave_barrier();
-    for (int p = r; p < cnt; p += PULL_LANES) {
-      // both records are read from LDS where a value is used: held in registers across the pair (the
-      // particle's own across the pairs) they spill
-      const int a = list[p];
-      const bool tool_a = double_to_bits(m.piece[R_FLAGS / 2][a].x) & MFC_FLAG_TOOL;
-      // the mechanical sums of both take a pair without a tool particle; each conduction sum
-      // counts where its particle conducts
-      const double ta_a = pse ? 0. : (tool_a ? k.alpha_tool : k.alpha_wp);
-      auto rec = [&](int j, int q) { return q % 2 ? m.piece[q / 2][j].y : m.piece[q / 2][j].x; };
-      auto adj = [&](int j, double ta, int q) { return q == L_TL && ta == 0. ? 0. : rec(j, REC_DOUBLES + q); };
-      pair_vjp_sym(
-          k, [&](int q) { return rec(li, q); }, [&](int q) { return rec(a, q); }, !tool_a && !tool_b,
-          ta_a != 0. || ta_b != 0., [&](int q) { return adj(li, ta_b, q); }, [&](int q) { return adj(a, ta_a, q); }, gb);
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+  const pull_lds src = {m};
+  for (int t0 = 0; t0 < k.patch_slots; t0 += PULL_AT_ONCE) {
+    const int n = part * k.patch_slots + t0 + tid / PULL_LANES;
+    if (n >= nown) return true;  // whole groups of lanes
+    int col = 0;
+    for (int e = 1; e < ncol; e++) col += n >= m.own_first[e];
+    const int li = m.table[col * nrow + r0 - s0] + (n - m.own_first[col]);
+    const int b = li - m.col_shift[col];
+    const int gi = q0 + col, gj = d.key_sorted[(size_t)slot * N + b] - gi * k.gny;
+    const window w = make_window_at(k, gi, gj, [&](int c, int row) { return m.table[(c - q0) * nrow + row - s0]; });
+    double gb[REC_DOUBLES];
+    pull_particle(k, src, li, w, r, gl, m.list[tid / PULL_LANES], gb);
+    pull_store(gb, r, d.g_rec + (size_t)REC_DOUBLES * b);
   }
-  pull_store(gb, r, d.g_rec + (size_t)REC_DOUBLES * b);
   return true;
 }
 
@@ -489,7 +522,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(3))) void 
   const int2 *__restrict__ plist = d.plist + (size_t)slot * d.list_len;
   const int2 p = plist[it.y];
   const bool staged = pull_patch(m, D, it.x, slot, p.x, p.y);
-  for (int q = staged ? it.y + step : it.y; q < count; q += step) pull_rest(D, it.x, slot, plist[q].x, plist[q].y);
+  for (int q = staged ? it.y + step : it.y; q < count; q += step) pull_rest(m, D, it.x, slot, plist[q].x, plist[q].y);
 }
 
 // ------------------------------------------------------------------ B3: record VJP + unsort
@@ -520,12 +553,17 @@ __global__ __launch_bounds__(TILE) void kb_adj_record(const adj_args *__restrict
 }  // namespace
 
 // ------------------------------------------------------------------ workspace
-constexpr int ADJ_LANES = PULL_LANES;  // threads per particle of the replayed interaction: the
-                                       // pull takes the same patches
+// threads per particle of the replayed interaction, whose patches the pull takes too: those of the
+// forward steps, or 4 where they have one (whose patches' windows do not fit the pull's stage)
+int replay_lanes(mfc_sim *const *sims, int n) {
+  const int lanes = interaction_lanes(sims, n);
+  return lanes > 4 ? lanes : 4;
+}
 
 // device memory of the backward pass of a group of instances, kept between calls with the first
 // instance's workspace; the descriptors are written at every call
 struct adj_group {
+  int lanes = 0;                // replay_lanes
   std::vector<int> items;       // work items of each instance's patches
   int nck = 0;
   char *mem = nullptr;
@@ -553,7 +591,6 @@ struct adj_work {
   int2 *plist = nullptr;
   mfc_tool_state *tool = nullptr;
   double *acc = nullptr;
-  patch_plan patches = {};
   int uniform_h = 0;  // of the recorded run's states
   double h0 = 0.;
   char *posw = nullptr;                 // replay positional block (pressure and artificial stress)
@@ -605,11 +642,11 @@ int setup_work(mfc_sim *s, int nsteps, int K, int w0, int w1) {
     for (auto &c : w->ckpt)
       if ((rc = w->alloc_snapshot(c))) return rc;
     const size_t n = (size_t)N, k = (size_t)K;
-    w->patches = patches_for(s, ADJ_LANES);
+    const size_t list = std::max(patches_for(s, 4).list, patches_for(s, 8).list);
     if ((rc = w->alloc(&w->state, (k + 1) * state_block_bytes(N))) || (rc = w->alloc(&w->normal, (k + 1) * 2 * n)) ||
         (rc = w->alloc(&w->tags, k * n)) || (rc = w->alloc(&w->spos, k * n)) || (rc = w->alloc(&w->key_sorted, k * n)) ||
         (rc = w->alloc(&w->offsets, k * ((size_t)s->k.ncell_table + 1))) || (rc = w->alloc(&w->plen, k + 1)) ||
-        (rc = w->alloc(&w->plist, k * w->patches.list)) || (rc = w->alloc(&w->tool, k + 1)) ||
+        (rc = w->alloc(&w->plist, k * list)) || (rc = w->alloc(&w->tool, k + 1)) ||
         (rc = w->alloc(&w->acc, k * (L_N + 1) * n)) ||
         (rc = w->alloc(&w->posw, positional_block_bytes(N))) ||
         (rc = w->alloc(&w->partials, 16 * (size_t)s->ntiles)) || (rc = w->alloc(&w->force_last, 2)) ||
@@ -637,13 +674,15 @@ int setup_work(mfc_sim *s, int nsteps, int K, int w0, int w1) {
 int setup_group(mfc_sim *const *sims, int n, hipStream_t st) {
   adj_work *w0 = sims[0]->adj;
   const int K = w0->K, nck = (w0->nsteps + K - 1) / K;
+  const int lanes = replay_lanes(sims, n);
   std::vector<int> per(n);
-  for (int i = 0; i < n; i++) per[i] = sims[i]->adj->patches.items;
+  for (int i = 0; i < n; i++) per[i] = patches_for(sims[i], lanes).items;
   adj_group *g = w0->group.get();
-  if (g && g->items == per && g->nck >= nck) return MFC_OK;
+  if (g && g->lanes == lanes && g->items == per && g->nck >= nck) return MFC_OK;
   HIP_TRY(hipStreamSynchronize(st));  // nothing queued uses the old one
   w0->group.reset(new adj_group());
   g = w0->group.get();
+  g->lanes = lanes;
   g->items = per;
   g->nck = nck;
   std::vector<int2> items;
@@ -679,7 +718,7 @@ void enqueue_segment(const adj_group &g, const adj_work &w, const batch_work &fw
   batch_work rw = fw;
   rw.patches = g.patches;
   rw.npatches = g.npatches;
-  rw.v.lanes = ADJ_LANES;
+  rw.v.lanes = g.lanes;
   rw.args = g.rep;
   const dim3 gt(padded(fw.ntiles)), gp(chunked_blocks(g.npatches));
   hipLaunchKernelGGL(kb_adj_restore, dim3(copy_blocks, n), dim3(256), 0, st, g.adj, sg);
@@ -785,9 +824,10 @@ int adj_backward(mfc_sim *const *sims, int n, const batch_work &fw, hipStream_t 
     const size_t sb = state_block_bytes(N), nc1 = (size_t)s->k.ncell_table + 1;
     maxN = N > maxN ? N : maxN;
     dev_consts k = s->k;
-    k.patch_s = w->patches.s;
-    k.patch_w = w->patches.w;
-    k.patch_slots = w->patches.slots;
+    const patch_plan &plan = patches_for(s, g.lanes);
+    k.patch_s = plan.s;
+    k.patch_w = plan.w;
+    k.patch_slots = plan.slots;
     k.uniform_h = w->uniform_h;
     k.h0 = w->h0;
     for (int j = 0; j < slots; j++) {
@@ -802,7 +842,7 @@ int adj_backward(mfc_sim *const *sims, int n, const batch_work &fw, hipStream_t 
       a.b.tags = w->tags + (size_t)j * N;
       a.b.spos = w->spos + (size_t)j * N;
       a.b.offsets = w->offsets + j * nc1;
-      a.b.plist = w->plist + (size_t)j * w->patches.list;
+      a.b.plist = w->plist + (size_t)j * plan.list;
       a.b.plen = w->plen + j;
       a.b.plen_next = w->plen + j + 1;
       a.b.bsum = s->chunk_sums[p];
@@ -820,7 +860,7 @@ int adj_backward(mfc_sim *const *sims, int n, const batch_work &fw, hipStream_t 
       a.acc_out = w->acc + (size_t)j * (L_N + 1) * N;
       a.ntiles = s->ntiles;
       a.nscan = scan_blocks(s->k.ncell_table);
-      a.npatch_items = w->patches.items;
+      a.npatch_items = plan.items;
     }
     adj_args &d = da[i];
     std::memset(&d, 0, sizeof(d));
@@ -832,7 +872,7 @@ int adj_backward(mfc_sim *const *sims, int n, const batch_work &fw, hipStream_t 
     d.tags = w->tags; d.spos = w->spos; d.key_sorted = w->key_sorted;
     d.offsets = w->offsets;
     d.plist = w->plist; d.plen = w->plen;
-    d.list_len = w->patches.list; d.ncell1 = (int)nc1;
+    d.list_len = plan.list; d.ncell1 = (int)nc1;
     d.tool = w->tool;
     d.acc = w->acc;
     d.lam = w->lam; d.lam_n = w->lam_n;

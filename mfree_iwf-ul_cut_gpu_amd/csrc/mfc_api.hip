@@ -100,11 +100,20 @@ void patch_items(std::vector<int2> &items, mfc_sim *const *sims, int n) {
     for (int q = 0; q < sims[i]->npatch_items; q++) items.push_back(make_int2(i, q));
 }
 
-// Measured, us per step with 1 / 4 / 8 threads per particle (FP64; FP32C): 6k 48 / 34 / 32
-// (39 / 30 / 29), 7.6k 50 / 34 / 30 (38 / 29 / 27), 27k 55 / 50 / 62 (43 / 38 / 43), 37k 62 / 53 / 62
-// (51 / 45 / 51), 71k 67 / 80 / 107 (47 / 60 / 72): more threads pay as long as they find idle SIMDs
-int interaction_lanes(int64_t total) {
-  return total > 48000 ? 1 : total > 13000 ? 4 : 8;
+// More threads per particle shorten a particle's chain and pay as long as all the work-groups, one per
+// entry of the patch list, run at once: 256 CUs times 3 (FP64) or 4, less 6 % for the patches that
+// the particles spread to. Measured, us per step with 8 / 4 / 1 threads and the entries that 8 and 4
+// make. FP64: 14.3k particles 36 / 39 / 51 (571, 290), 18.7k 39 / 43 / 56 (758, 366), 23.6k 54 / 43 / 54 (911,
+// 457), 29k 57 / 46 / 56, 42k 74 / 60 / 57 (1658, 782), 72k 105 / 77 / 62; FP32C: 23.6k 35 / 38 / 44 (911,
+// 457), 29k 43 / 38 / 44 (1125, 559), 42k 51 / 40 / 46 (1658, 782), 55k 61 / 55 / 47 (2146, 1044).
+int interaction_lanes(const mfc_sim *const *sims, int n) {
+  const int64_t most = 256 * (sims[0]->recs[0].f32 ? 4 : 3) * 15 / 16;
+  for (int lanes : {8, 4}) {
+    int64_t entries = 0;
+    for (int i = 0; i < n; i++) entries += patches_for(sims[i], lanes).entries;
+    if (entries <= most) return lanes;
+  }
+  return 1;
 }
 
 namespace {
@@ -168,6 +177,7 @@ void plan_patches(mfc_sim *s) {
           for (int e = 0; e < p.s && g < k.gny; e++, g++) in[r] += cells[(size_t)c * k.gny + g];
       for (int n : in) entries += (n + p.slots - 1) / p.slots;
     }
+    p.entries = entries;
     p.patches = patch_bound(k, p.s, p.w);
     const int64_t bound = p.patches + k.N / p.slots, want = entries + entries / 2 + 32;
     p.items = (int)(want < bound ? want : bound);
@@ -447,7 +457,7 @@ int mfc_create(const mfc_config *cfg, mfc_sim **out) {
   if ((rc = s->alloc(&b.pcnt, s->npatch_max)) ||
       (rc = s->alloc(&b.plist, (size_t)s->npatch_max + (size_t)N / (mfc::TILE / 8) + 1)) || (rc = s->alloc(&s->plen, 2)))
     return bail(rc);
-  set_patches(s, interaction_lanes(N));
+  set_patches(s, interaction_lanes(&s, 1));
   check_uniform_h(s, s->sc.h.data());
   for (mfc::drecords &r : s->recs) {
     if ((rc = s->alloc(&r.vfl, N))) return bail(rc);
@@ -534,7 +544,7 @@ int mfc_set_tuning(mfc_sim *s, const mfc_tuning *t) {
   s->k.stage_limit = t->stage_limit;
   s->k.sort_fast = t->sort_fast;
   s->k.sort_list = t->sort_list;
-  const int lanes = t->lanes ? t->lanes : interaction_lanes(s->k.N);
+  const int lanes = t->lanes ? t->lanes : interaction_lanes(&s, 1);
   if (lanes != s->lanes) {
     std::vector<int2> patches;
     set_patches(s, lanes);

@@ -22,11 +22,7 @@ struct mfc_batch {
   int2 *tiles = nullptr, *chunks = nullptr, *patches = nullptr;
   int ntiles = 0, nchunks = 0, npatches = 0;
   int lanes = 1;  // threads per particle of the interaction
-  int auto_lanes() const {
-    int64_t total = 0;
-    for (const mfc_sim *s : sims) total += s->k.N;
-    return interaction_lanes(total);  // the instances run together
-  }
+  int auto_lanes() const { return interaction_lanes(sims.data(), (int)sims.size()); }  // they run together
   int cur = 0;
   int64_t step = 0;
   hipGraphExec_t graph[2] = {nullptr, nullptr};

@@ -52,6 +52,7 @@ struct patch_plan {
   int s, w, slots;  // rows and columns of cells, particles a work-group takes at a time
   int items;        // work items of the interaction launch
   int list;         // entries the list of patches can have
+  int64_t entries;  // entries of the list of patches, for the initial particles
   int64_t patches;  // patches the grid can have
 };
 
@@ -151,9 +152,9 @@ int ensure_keys(mfc_sim *s);
 // the work tables of the sort launch and of the interaction launch over a group of instances
 void sort_items(std::vector<int2> &items, mfc_sim *const *sims, int n);
 void patch_items(std::vector<int2> &items, mfc_sim *const *sims, int n);
-// threads per particle of the interaction for `total` particles stepped together, and a handle's
-// patches for that
-int interaction_lanes(int64_t total);
+// threads per particle of the interaction for n handles stepped together, and a handle's patches
+// for that
+int interaction_lanes(const mfc_sim *const *sims, int n);
 const patch_plan &patches_for(const mfc_sim *s, int lanes);
 void set_patches(mfc_sim *s, int lanes);
 // copies the handle's descriptors to where the kernels read them (synchronises its stream)
