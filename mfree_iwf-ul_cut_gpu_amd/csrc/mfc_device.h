@@ -16,10 +16,13 @@
 namespace mfc {
 
 
-// constants of one simulation, passed by value to every kernel
+// The constants of a simulation, read through the constant address space: they do not change while a
+// kernel runs, so that they stay scalar loads whatever the kernel writes in between
+typedef const __attribute__((address_space(4))) dev_consts kconst;
+
 __device__ inline double f32sqrt(double x) { return (double)sqrtf((float)x); }
 // sqrtf of the reference's FP64 build, or the FP64 square root when its truncations are promoted
-__device__ inline double tsqrt(const dev_consts &k, double x) { return k.promote ? sqrt(x) : f32sqrt(x); }
+__device__ inline double tsqrt(kconst &k, double x) { return k.promote ? sqrt(x) : f32sqrt(x); }
 
 // Work-groups are dispatched round-robin over the 8 XCDs of MI355X; map block b so that
 // each XCD owns one contiguous range of tiles (its neighbour data then stays in that XCD's
@@ -61,7 +64,8 @@ __device__ inline int64_t cell_coord(double f) {
 // reported in `outside` (the reference's id then points into another column or past the cell
 // table); an id outside the table is clamped into it, where the reference would index out of
 // bounds.
-__device__ inline int cell_of(const dev_consts &k, double x, double y, bool &outside) {
+template <class K>  // dev_consts or kconst
+__device__ inline int cell_of(K &k, double x, double y, bool &outside) {
   int64_t ix = cell_coord((x - k.bbmin_x) / k.cell);
   int64_t iy = cell_coord((y - k.bbmin_y) / k.cell);
   int64_t h = ix * k.gny + iy;
@@ -125,13 +129,13 @@ __device__ inline void jaumann(double G, double vx_x, double vx_y, double vy_x, 
 // particle's return evaluates the flow stress at one temperature many times (the yield test, two
 // residuals per secant iteration, the plastic heating), so the factor is evaluated once per
 // particle; it is the same expression of the same values, so the results are unchanged.
-__device__ inline double jc_temperature_factor(const dev_consts &k, double t) {
+__device__ inline double jc_temperature_factor(kconst &k, double t) {
   double theta = (t - k.jc_Tref) / (k.jc_Tmelt - k.jc_Tref);
   return 1.0 - mfcm::pow(theta, k.jc_m);
 }
 
 // Johnson-Cook flow stress (plasticity.cuh:30-46), TC = jc_temperature_factor(k, t)
-__device__ inline double sigma_yield(const dev_consts &k, double eps_pl, double eps_pl_dot, double TC) {
+__device__ inline double sigma_yield(kconst &k, double eps_pl, double eps_pl_dot, double TC) {
   double TA = k.jc_A + k.jc_B * mfcm::pow(eps_pl, k.jc_n);
   double TB = 1.0;
   double ed = eps_pl_dot / k.jc_eps_dot_ref;
@@ -142,7 +146,7 @@ __device__ inline double sigma_yield(const dev_consts &k, double eps_pl, double 
 
 // tanh-modified Johnson-Cook flow stress after Calamaz 2008 (plasticity.cuh:48-70),
 // TC = jc_temperature_factor(k, t)
-__device__ inline double sigma_yield_tanh(const dev_consts &k, double eps_pl, double eps_dot_pl, double t, double TC) {
+__device__ inline double sigma_yield_tanh(kconst &k, double eps_pl, double eps_dot_pl, double t, double TC) {
   double TA = k.jc_A + k.jc_B * mfcm::pow(eps_pl, k.jc_n) * 1.0 / mfcm::exp(mfcm::pow(eps_pl, k.tanh_a));
   double TB = 1.0;
   double ed = eps_dot_pl / k.jc_eps_dot_ref;
@@ -162,7 +166,7 @@ struct rr_input {
 };
 
 // the yield test; false (and eps_pl_dot = 0) for an elastic step
-__device__ inline bool plasticity_test(const dev_consts &k, double p, double Sxx, double Sxy, double Syy, double Szz,
+__device__ inline bool plasticity_test(kconst &k, double p, double Sxx, double Sxy, double Syy, double Szz,
                                        double eps_pl, double &eps_pl_dot, double T, rr_input &in) {
   in.norm = tsqrt(k, Sxx * Sxx + Syy * Syy + Szz * Szz + Sxy * Sxy);
   double cxx = Sxx - p, cyy = Syy - p, czz = Szz - p, cxy = Sxy;
@@ -176,7 +180,7 @@ __device__ inline bool plasticity_test(const dev_consts &k, double p, double Sxx
 }
 
 // the return with the secant's dl: stress, plastic strain and rate, plastic heating
-__device__ inline void plasticity_finish(const dev_consts &k, double rho, double dl, const rr_input &in, double &Sxx,
+__device__ inline void plasticity_finish(kconst &k, double rho, double dl, const rr_input &in, double &Sxx,
                                          double &Sxy, double &Syy, double &Szz, double &eps_pl, double &eps_pl_dot,
                                          double &T) {
   const double s23 = sqrt(2.0 / 3.0);
@@ -285,7 +289,7 @@ __device__ inline double jc_part(bool rate, double e, double es, double A, doubl
 // returns 600 us, now 410, of the 6k cut 475, now 280. The loop is in the outlined function so that
 // the polynomials' constants stay in registers through it (evaluated by a function called in the loop
 // they were loaded again each time, and the two cuts took 480 and 320 us).
-__device__ __attribute__((noinline)) double rr_secant_jc(const dev_consts &k, double dl, double norm, double eps0,
+__device__ __attribute__((noinline)) double rr_secant_jc(kconst &k, double dl, double norm, double eps0,
                                                         double TC) {
   const double A = k.jc_A, B = k.jc_B, n = k.jc_n, C = k.jc_C, edr = k.jc_eps_dot_ref, dt = k.dt, G = k.G;
   const double s23 = sqrt(2.0 / 3.0);
@@ -309,7 +313,7 @@ __device__ __attribute__((noinline)) double rr_secant_jc(const dev_consts &k, do
 }
 
 // the residual with the tanh-modified flow stress
-__device__ __attribute__((noinline)) double rr_residual_tanh(const dev_consts &k, double dl, double norm, double eps0,
+__device__ __attribute__((noinline)) double rr_residual_tanh(kconst &k, double dl, double norm, double eps0,
                                                             double t, double TC) {
   const double s23 = sqrt(2.0 / 3.0);
   double e = eps0 + s23 * fmax(dl, 0.);
@@ -338,11 +342,11 @@ __device__ __attribute__((noinline)) double rr_residual_jc_lib(double dl, double
 
 // lanes per returning particle: 4, or 2 with the residuals of the FP32C path and of the tanh model
 template <bool LIB>
-__device__ inline int secant_lanes_log2(const dev_consts &k) { return LIB || k.jc_tanh ? 1 : 2; }
+__device__ inline int secant_lanes_log2(kconst &k) { return LIB || k.jc_tanh ? 1 : 2; }
 
 // the secant of a returning particle by its lanes. LIB: the FP32C path
 template <bool LIB>
-__device__ inline double rr_secant(const dev_consts &k, double dl, double norm, double e0, double t, double TC) {
+__device__ inline double rr_secant(kconst &k, double dl, double norm, double e0, double t, double TC) {
   if (k.jc_tanh) return secant(dl, k.secant_tol, [&](double x) { return rr_residual_tanh(k, x, norm, e0, t, TC); });
   if constexpr (LIB) {
     const double A = k.jc_A, B = k.jc_B, n = k.jc_n, C = k.jc_C, edr = k.jc_eps_dot_ref, dt = k.dt, G = k.G;
@@ -357,7 +361,7 @@ __device__ inline double rr_secant(const dev_consts &k, double dl, double norm, 
 // returns, with their inputs. Returns dl on those lanes, and in folded whether the last update took
 // the fold branch (the reverse mode differentiates the fold's fixed point there).
 template <bool LIB>
-__device__ inline double rr_secant_wave(const dev_consts &k, bool need, const rr_input &in, double eps0, double t,
+__device__ inline double rr_secant_wave(kconst &k, bool need, const rr_input &in, double eps0, double t,
                                         bool &folded) {
   const int lane = (int)(threadIdx.x & 63);
   unsigned long long pending = __ballot(need);
@@ -396,7 +400,7 @@ struct return_slots {
   int count;
 };
 template <bool LIB>
-__device__ inline double rr_secant_group(const dev_consts &k, return_slots &q, bool need, const rr_input &in,
+__device__ inline double rr_secant_group(kconst &k, return_slots &q, bool need, const rr_input &in,
                                          double eps0, double t, bool &folded) {
   const int tid = threadIdx.x;
   const unsigned long long all = __ballot(tid < 64 && need);
@@ -494,7 +498,7 @@ __device__ inline bool tool_contact(const mfc_tool_state &t, double qx, double q
 
 // penalty normal force and LS-DYNA style Coulomb friction with history (tool_gpu.cu:151-207);
 // returns false (and zero forces) outside the tool
-__device__ inline bool contact_force(const dev_consts &k, const mfc_tool_state &t, double x, double y, double vx,
+__device__ inline bool contact_force(kconst &k, const mfc_tool_state &t, double x, double y, double vx,
                                      double vy, double &fcx, double &fcy, double &ftx, double &fty, double &nx,
                                      double &ny) {
   double cx = 0., cy = 0.;

@@ -84,7 +84,8 @@ __device__ inline int block_exclusive_scan(int v, int &total) {
 
 // cell id of a particle for the binning (grid.cu:34-51; blanked particles keep their last
 // sorted id, grid.cu:39-41); positions outside the grid are counted
-__device__ inline int particle_cell(const dev_consts &k, double x, double y, int fl, int sorted_id,
+template <class K>  // dev_consts or kconst
+__device__ inline int particle_cell(K &k, double x, double y, int fl, int sorted_id,
                                     unsigned long long *__restrict__ clamped) {
   if (fl & MFC_FLAG_BLANKED) return sorted_id;
   bool cl;
@@ -119,7 +120,8 @@ __device__ inline void count_cell(int i, int h, int *__restrict__ key, int *__re
 
 // counts the particle of cell h in its patch (all 64 lanes of the wave; h = -1: no particle): one
 // atomic per run of equal patches in the wave
-__device__ inline void count_patch(const dev_consts &k, int h, int *__restrict__ pcnt) {
+template <class K>
+__device__ inline void count_patch(K &k, int h, int *__restrict__ pcnt) {
   int p = -1;
   if (h >= 0) {
     const int gi = h / k.gny, gj = h - gi * k.gny;
@@ -132,7 +134,8 @@ __device__ inline void count_patch(const dev_consts &k, int h, int *__restrict__
 }
 
 // cell id of every particle of the start state, counted in its chunk
-__device__ inline void hash_count(const dev_consts &k, int i, const double *__restrict__ px,
+template <class K>
+__device__ inline void hash_count(K &k, int i, const double *__restrict__ px,
                                   const double *__restrict__ py, const int *__restrict__ flags,
                                   const dbins &b) {
   const int h = i < k.N ? particle_cell(k, px[i], py[i], flags[i], b.key_sorted[i], b.clamped) : -1;
@@ -283,7 +286,7 @@ __device__ inline void sort_chunk(int blk, int N, int n, const dbins &b, const i
 // A section's entries follow each other in ascending order, the sections in any (the results do
 // not depend on the order of the list). Clears the patches' counts
 constexpr int PLIST_BATCH = PLIST_SECTION / SCAN_THREADS;  // patches per thread
-__device__ inline void list_patches(const dev_consts &k, int sec, const dbins &b) {
+__device__ inline void list_patches(kconst &k, int sec, const dbins &b) {
   const int np = patch_total(k);
   const int p0 = sec * PLIST_SECTION + threadIdx.x * PLIST_BATCH;
   if (sec == 0 && threadIdx.x == 0) *b.plen_next = 0;
@@ -382,7 +385,7 @@ __device__ inline rec_input load_rec_input(const dstate &c, int s) {
 }
 
 // leap-frog init + predict (in place)
-__device__ inline void predict_input(const dev_consts &k, rec_input &q) {
+__device__ inline void predict_input(kconst &k, rec_input &q) {
   if (q.fl & MFC_FLAG_BLANKED) return;  // leap_frog.cu:42-66
   const double hdt = 0.5 * k.dt;
   q.x = q.x + hdt * q.ptx; q.y = q.y + hdt * q.pty;
@@ -393,7 +396,7 @@ __device__ inline void predict_input(const dev_consts &k, rec_input &q) {
 }
 
 // the FP64 record of predicted input q with pressure p and artificial stress R, written at i
-__device__ inline void store_record(const dev_consts &k, const rec_input &q, double p, double rxx, double rxy,
+__device__ inline void store_record(kconst &k, const rec_input &q, double p, double rxx, double rxy,
                                     double ryy, int i, const drecords &recs) {
   const double r21 = 1. / (q.rho * q.rho);
   double r[REC];
@@ -424,7 +427,7 @@ __device__ inline void store_record(const dev_consts &k, const rec_input &q, dou
 // written at its storage index i. The pressure and artificial stress of a tool particle enter no sum (every term that
 // reads them skips pairs with one) and are 0 in its record.
 template <bool F32>
-__device__ inline void write_record(const dev_consts &k, rec_input q, int i, const drecords &recs) {
+__device__ inline void write_record(kconst &k, rec_input q, int i, const drecords &recs) {
   predict_input(k, q);
   const bool tool = q.fl & MFC_FLAG_TOOL;
   const double p = tool ? 0. : k.c0 * k.c0 * (q.rho - k.rho0);
@@ -678,11 +681,11 @@ __device__ inline double exp_neg(double x) {
 struct math64 {
   using rec = rec64;
   static constexpr int TERMS = 13;
-  const dev_consts &k;
+  kconst &k;
   const rec64 &a;
   const sum_flags &f;
   double h1, fourh2, fac, h2, inv_h2, pse_c, inv_wd;
-  __device__ inline math64(const dev_consts &k_, const rec64 &a_, const sum_flags &f_) : k(k_), a(a_), f(f_) {
+  __device__ inline math64(kconst &k_, const rec64 &a_, const sum_flags &f_) : k(k_), a(a_), f(f_) {
     h1 = 1 / a.h;
     fourh2 = 4 * a.h * a.h;
     fac = PI_FAC * h1 * h1;
@@ -739,11 +742,11 @@ struct sums32 {
 };
 struct math32 {
   using rec = rec32;
-  const dev_consts &k;
+  kconst &k;
   const rec32 &a;
   const sum_flags &f;
   float ta, Ti, h1, fourh2, fac, inv_wd, eta2, alpha, beta, xeps, inv_h2, pse_c, massf;
-  __device__ inline math32(const dev_consts &k_, const rec32 &a_, const sum_flags &f_) : k(k_), a(a_), f(f_) {
+  __device__ inline math32(kconst &k_, const rec32 &a_, const sum_flags &f_) : k(k_), a(a_), f(f_) {
     ta = (float)f.ta;
     Ti = ta != 0.0f ? a.T : 0.0f;
     h1 = 1.0f / a.h;
@@ -824,11 +827,11 @@ using math_t = std::conditional_t<F32, math32, math64>;
 // the sums as update_particle takes them, from the FP32C sums s (in the order of terms32; the
 // stress and viscosity sums enter the acceleration only as sd0 + sd1 + vt0 and sd2 + sd3 + vt1
 // (actions_gpu.cu momentum), so they are accumulated as those two)
-__device__ inline pair_acc acc_of_sums32(const dev_consts &k, const double *s) {
+__device__ inline pair_acc acc_of_sums32(kconst &k, const double *s) {
   return {s[0], s[1], s[2], s[3], k.mass * s[4], 0., k.mass * s[5], 0., 0., 0., k.mass * s[6], k.mass * s[7], 2.0 * s[8]};
 }
 
-__device__ inline pair_acc acc_of(const dev_consts &k, const sums32 &q) {
+__device__ inline pair_acc acc_of(kconst &k, const sums32 &q) {
   double s[9];
 #pragma unroll
   for (int c = 0; c < 9; c++) s[c] = q.s[c].value();
@@ -840,7 +843,7 @@ __device__ inline double value_of(double s) { return s; }
 // The neighbour sums of a particle by one thread from the records in memory: the window's
 // candidates in order, which is the reference's (interactions_gpu.cu:219-331)
 template <bool F32>
-__device__ inline void sums_mem(const dev_consts &k, const mem_source<F32> &src, const window &w, const rec_t<F32> &a,
+__device__ inline void sums_mem(kconst &k, const mem_source<F32> &src, const window &w, const rec_t<F32> &a,
                                 const sum_flags &f, pair_acc &acc, double &tpse) {
   const math_t<F32> mt(k, a, f);
   std::conditional_t<F32, sums32, pair_sums> sum = {};
@@ -877,7 +880,7 @@ __device__ inline void sums_mem(const dev_consts &k, const mem_source<F32> &src,
 // particles at infinity).
 constexpr int WALK_U = 4;  // candidates whose loads are issued together
 template <bool F32, int G, bool PSE>
-__device__ inline void sums_lds(const dev_consts &k, const lds_source<F32, G> &src, int flags, const int b[5],
+__device__ inline void sums_lds(kconst &k, const lds_source<F32, G> &src, int flags, const int b[5],
                                 const int e[5], const rec_t<F32> &a, const sum_flags &f, pair_acc &acc, double &tpse) {
   const math_t<F32> mt(k, a, f);
   std::conditional_t<F32, sums32, pair_sums> sum = {};
@@ -965,7 +968,7 @@ __device__ inline void wave_lds_fence() {
 // pair, and every sum belongs to one of them, which adds the G pairs' terms in order through LDS:
 // the order of every sum, and so its bits, are sums_lds's. The sums end in out[0..ACC_N) (LDS).
 template <bool F32, int G>
-__device__ inline void sums_group(const dev_consts &k, const lds_source<F32, G> &src, const window &w,
+__device__ inline void sums_group(kconst &k, const lds_source<F32, G> &src, const window &w,
                                   const rec_t<F32> &a, const sum_flags &f, unsigned char *list, char *terms,
                                   double *out) {
   const math_t<F32> mt(k, a, f);
@@ -1089,7 +1092,7 @@ struct deferred_return {
 // particle to position i of dst: the gather into sorted order happens here, once. Also writes the
 // step's positional values and, with the state before a return, the next step's record (rn)
 template <bool F32>
-__device__ inline void update_particle(const dev_consts &k, int i, int s, const pair_acc &acc, double tpse,
+__device__ inline void update_particle(kconst &k, int i, int s, const pair_acc &acc, double tpse,
                                        const dstate &src, const dstate &dst, const dpositional &pos,
                                        const drecords &r, const drecords &rn, const mfc_tool_state &tool_now, double fsum[4], double &x_out, double &y_out,
                                        int &fl_out, deferred_return &dr) {
@@ -1210,7 +1213,7 @@ __device__ inline void update_particle(const dev_consts &k, int i, int s, const 
 // rate and temperature at sorted index i (the thermal boundary condition after the return, as in
 // update_particle), and its record again with them
 template <bool F32>
-__device__ inline void finish_return(const dev_consts &k, int i, double dl, deferred_return &dr, const dstate &dst,
+__device__ inline void finish_return(kconst &k, int i, double dl, deferred_return &dr, const dstate &dst,
                                      const drecords &rn) {
   plasticity_finish(k, dr.rho, dl, dr.in, dr.sxx, dr.sxy, dr.syy, dr.szz, dr.eps, dr.epsd, dr.T);
   if (k.thermal_bc && dr.fixed) dr.T = k.T_init;  // actions_gpu.cu:287-294
@@ -1227,14 +1230,14 @@ __device__ inline void finish_return(const dev_consts &k, int i, double dl, defe
 // next step): cell id, arrival slot and patch, as hash_count would take them from the updated
 // state (the bins are passed by value so that they stay in registers). An adaptive grid bins the
 // next step's start state after its geometry pass instead.
-__device__ inline void next_cell(const dev_consts &k, int i, bool live, double x, double y, int fl, const dbins next) {
+__device__ inline void next_cell(kconst &k, int i, bool live, double x, double y, int fl, const dbins next) {
   if (k.adaptive) return;  // the same in every thread
   const int h = live ? particle_cell(k, x, y, fl, next.key_sorted[i], next.clamped) : -1;
   count_cell(i, h, next.key, next.bsum_next, next.clist, next.ccap);
   count_patch(k, h, next.pcnt);
 }
 
-__device__ inline sum_flags flags_of(const dev_consts &k, int tag) {
+__device__ inline sum_flags flags_of(kconst &k, int tag) {
   const bool pse = k.pse != 0, blank = tag & MFC_FLAG_BLANKED, tool = tag & MFC_FLAG_TOOL;
   sum_flags f;
   f.tool = tool;
@@ -1255,16 +1258,15 @@ struct after_update {
 template <bool F32>
 __device__ inline void begin_update(const inst_args *ap, int i, unsigned s, bool live, const pair_acc &acc, double tpse,
                                     after_update &u) {
-  const inst_args &a = *ap;
   MFC_CONST(inst_args) *c = const_args(ap, 0);
-  const dev_consts &k = a.k;
+  kconst &k = c->k;
   u.dr.need = false;
   u.x = u.y = 0.;
   u.fl = 0;
   if (!live) return;
   double fsum[4] = {0., 0., 0., 0.};
-  if (a.acc_out) store_acc(a.acc_out, k.N, i, acc, tpse);  // the same in every thread
-  update_particle<F32>(k, i, s, acc, tpse, a.cur, a.nxt, a.pos, load_recs(&c->r), load_recs(&c->rn), *a.tool_out, fsum,
+  if (c->acc_out) store_acc(c->acc_out, k.N, i, acc, tpse);  // the same in every thread
+  update_particle<F32>(k, i, s, acc, tpse, load_state(&c->cur), load_state(&c->nxt), load_pos(&c->pos), load_recs(&c->r), load_recs(&c->rn), *c->tool_out, fsum,
                        u.x, u.y, u.fl, u.dr);
   if (fsum[0] != 0. || fsum[1] != 0. || fsum[2] != 0. || fsum[3] != 0.) c->f.gflag[i >> 6] = 1;
 }
@@ -1273,11 +1275,10 @@ __device__ inline void begin_update(const inst_args *ap, int i, unsigned s, bool
 // replay (-dl where its last update folded, 0 for no return), and the next step's binning
 template <bool F32>
 __device__ inline void end_update(const inst_args *ap, int i, bool live, double dl, bool folded, after_update &u) {
-  const inst_args &a = *ap;
   MFC_CONST(inst_args) *c = const_args(ap, 0);
-  const dev_consts &k = a.k;
-  if (u.dr.need) finish_return<F32>(k, i, dl, u.dr, a.nxt, load_recs(&c->rn));
-  if (a.acc_out && live) a.acc_out[(size_t)ACC_N * k.N + i] = u.dr.need ? (folded ? -dl : dl) : 0.;
+  kconst &k = c->k;
+  if (u.dr.need) finish_return<F32>(k, i, dl, u.dr, load_state(&c->nxt), load_recs(&c->rn));
+  if (c->acc_out && live) c->acc_out[(size_t)ACC_N * k.N + i] = u.dr.need ? (folded ? -dl : dl) : 0.;
   next_cell(k, i, live, u.x, u.y, u.fl, load_bins(&c->b));
 }
 
@@ -1288,8 +1289,23 @@ __device__ inline void finish_particle(const inst_args *ap, int i, unsigned s, b
   after_update u;
   begin_update<F32>(ap, i, s, live, acc, tpse, u);
   bool folded;
-  const double dl = rr_secant_wave<F32>(ap->k, u.dr.need, u.dr.in, u.dr.eps, u.dr.T, folded);
+  const double dl = rr_secant_wave<F32>(const_args(ap, 0)->k, u.dr.need, u.dr.in, u.dr.eps, u.dr.T, folded);
   end_update<F32>(ap, i, live, dl, folded, u);
+}
+
+// The state of the particle at index s of the start state on its way into L2 while the sums are
+// formed: a load of a word of each field to LDS that nothing reads (no registers), `wave` 256 bytes.
+// For the kernels with several threads per particle, where the update waits for its loads: us per
+// step of 6k particles 31.7 -> 29.5 (FP64), of 37.5k 51 -> 46.5. With one thread per particle the
+// loads of all work-groups together are bound by bandwidth, and it costs (197k FP32C 56 -> 60).
+__device__ inline void fetch_state(const dstate &src, size_t N, unsigned s, unsigned *wave) {
+  typedef const __attribute__((address_space(1))) unsigned *global_word;
+  typedef __attribute__((address_space(3))) unsigned *lds_word;
+  const double *p = src.px + s;
+#pragma unroll
+  for (int c = 0; c < DSTATE_DOUBLES; c++, p += N)
+    __builtin_amdgcn_global_load_lds((global_word)(const unsigned *)p, (lds_word)wave, 4, 0, 0);
+  __builtin_amdgcn_global_load_lds((global_word)(const unsigned *)(src.flags + s), (lds_word)wave, 4, 0, 0);
 }
 
 // One patch of cells by one work-group, G threads per particle: the cell starts and the records of
@@ -1310,10 +1326,10 @@ __device__ inline void finish_particle(const inst_args *ap, int i, unsigned s, b
 // returns false, with nothing done, for a patch whose window candidates do not fit the stage or
 // whose state has no uniform h (interact_rest takes it)
 template <bool F32, int G, bool PSE>
-__device__ inline bool interact_patch(patch_mem<F32, G> &m, const inst_args *A, int inst, int patch, int part) {
+__device__ inline bool interact_patch(patch_mem<F32, G> &m, unsigned *unread, const inst_args *A, int inst, int patch, int part) {
   const inst_args &a_ = A[inst];
   MFC_CONST(inst_args) *c_ = const_args(&a_, 0);
-  const dev_consts &k = a_.k;
+  kconst &k = c_->k;
   const drecords r = load_recs(&c_->r);
   const int *__restrict__ offsets = k.rothlin ? c_->b.offsets_r : c_->b.offsets;
   const int *__restrict__ tags = c_->b.tags;
@@ -1436,6 +1452,7 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, const inst_args *A, 
         int col, li;
         i_own = locate(base + tid, col, li);
         s_mine = tag_index(m.tag[li]);
+        fetch_state(load_state(&c_->cur), k.N, s_mine, unread);
       }
     if (mine) {
       int col, li;
@@ -1466,6 +1483,8 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, const inst_args *A, 
         sums_group<F32, G>(k, lds, w, a, f, m.list[tid / G], terms, out);
       }
     }
+    // fetch_state's words have arrived before the LDS is given back
+    if constexpr (G > 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     // the update, one thread per particle: with G > 1 the first SLOTS threads
     int i = i_mine;
     bool live = mine;
@@ -1504,7 +1523,7 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, const inst_args *A, 
 template <bool F32>
 __device__ __attribute__((noinline)) void interact_rest(const inst_args *ap, int patch, int part) {
   const inst_args &a_ = *ap;
-  const dev_consts &k = a_.k;
+  kconst &k = const_args(ap, 0)->k;
   const dbins &b = a_.b;
   const int *offsets = k.rothlin ? b.offsets_r : b.offsets;
   const int nrb = patch_rows(k);
@@ -1740,7 +1759,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void kb_sort(const inst_args *__restr
   const int2 it = work[w];
   MFC_CONST(inst_args) *c = const_args(A, it.x);
   if (it.y <= SORT_ITEM_PATCHES) {
-    list_patches(A[it.x].k, SORT_ITEM_PATCHES - it.y, load_bins(&c->b));
+    list_patches(c->k, SORT_ITEM_PATCHES - it.y, load_bins(&c->b));
     return;
   }
   if (it.y <= SORT_ITEM_FORCE) {
@@ -1755,7 +1774,7 @@ __global__ __launch_bounds__(SCAN_THREADS) void kb_sort(const inst_args *__restr
     tool_move(A[it.x].tool_in, A[it.x].tool_out, A[it.x].k.dt);
     return;
   }
-  const dev_consts &k = A[it.x].k;
+  kconst &k = c->k;
   sort_chunk(it.y, k.N, k.ncell_table, load_bins(&c->b), load_recs(&c->r).vfl, k.sort_fast, k.sort_list);
 }
 
@@ -1767,7 +1786,7 @@ __global__ __launch_bounds__(TILE) void kb_records(const inst_args *__restrict__
   if (w < 0) return;
   const int2 it = work[w];
   MFC_CONST(inst_args) *c = const_args(A, it.x);
-  const dev_consts &k = A[it.x].k;
+  kconst &k = c->k;
   const int s = it.y * TILE + threadIdx.x;
   if (s >= k.N) return;
   write_record<F32>(k, load_rec_input(load_state(&c->cur), s), s, load_recs(&c->r));
@@ -1807,6 +1826,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(F32 ? 4 : 
   const int2 it = work[w];
   MFC_CONST(inst_args) *c = const_args(A, it.x);
   __shared__ patch_mem<F32, G> m;
+  __shared__ unsigned unread[G > 1 ? 64 : 1];
   if (it.y == PATCH_ITEM_FORCE) {
     const dforce fo = load_force(&c->f);
     // pending: the same value in every thread
@@ -1817,7 +1837,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(F32 ? 4 : 
   const int count = *c->b.plen, step = c->npatch_items;
   if (it.y >= count) return;
   const int2 p = c->b.plist[it.y];
-  if (!interact_patch<F32, G, PSE>(m, A, it.x, p.x, p.y)) interact_rest<F32>(A + it.x, p.x, p.y);
+  if (!interact_patch<F32, G, PSE>(m, unread, A, it.x, p.x, p.y)) interact_rest<F32>(A + it.x, p.x, p.y);
   for (int q = it.y + step; q < count; q += step) interact_rest<F32>(A + it.x, c->b.plist[q].x, c->b.plist[q].y);
 }
 

@@ -10,8 +10,10 @@ constexpr int REC_DOUBLES = 16;  // doubles per FP64 neighbour record
 
 // patches of the grid: patch p holds the cell rows [r patch_s, (r + 1) patch_s) and the columns
 // [c patch_w, (c + 1) patch_w) with p = c patch_rows + r
-__device__ inline int patch_rows(const dev_consts &k) { return (k.gny + k.patch_s - 1) / k.patch_s; }
-__device__ inline int patch_total(const dev_consts &k) { return ((k.gnx + k.patch_w - 1) / k.patch_w) * patch_rows(k); }
+template <class K>  // dev_consts or kconst
+__device__ inline int patch_rows(K &k) { return (k.gny + k.patch_s - 1) / k.patch_s; }
+template <class K>
+__device__ inline int patch_total(K &k) { return ((k.gnx + k.patch_w - 1) / k.patch_w) * patch_rows(k); }
 
 // a tag: the index of a neighbour's record (storage order) and its flags
 constexpr int TAG_BITS = 4;  // FIXED, BLANKED, TOOL, NONFINITE
@@ -37,8 +39,8 @@ struct window {
 
 // the up to 5 column ranges [b, e) of the window of a particle in cell column gi and row gj;
 // at(column, row) is the first index of a cell (the last one past the column's end for row gny)
-template <class AT>
-__device__ inline void window_ranges(const dev_consts &k, int gi, int gj, const AT &at, int b[5], int e[5]) {
+template <class K, class AT>
+__device__ inline void window_ranges(K &k, int gi, int gj, const AT &at, int b[5], int e[5]) {
   const int li = gi - 2 < 0 ? 0 : gi - 2;
   const int lj = gj - 2 < 0 ? 0 : gj - 2;
   const int hi = gi + 3 > k.gnx ? k.gnx : gi + 3;
@@ -67,8 +69,8 @@ __device__ inline window window_of(const int b[5], const int e[5]) {
   return w;
 }
 
-template <class AT>
-__device__ inline window make_window_at(const dev_consts &k, int gi, int gj, const AT &at) {
+template <class K, class AT>
+__device__ inline window make_window_at(K &k, int gi, int gj, const AT &at) {
   int b[5], e[5];
   window_ranges(k, gi, gj, at, b, e);
   return window_of(b, e);
@@ -76,7 +78,8 @@ __device__ inline window make_window_at(const dev_consts &k, int gi, int gj, con
 
 
 // the window of a particle with cell id hsh over the cell ranges in memory
-__device__ inline window make_window(const dev_consts &k, const int *__restrict__ offsets, int hsh) {
+template <class K>
+__device__ inline window make_window(K &k, const int *__restrict__ offsets, int hsh) {
   const int gi = hsh / k.gny, gj = hsh - gi * k.gny;
   return make_window_at(k, gi, gj, [&](int col, int row) { return offsets[col * k.gny + row]; });
 }
@@ -142,7 +145,7 @@ __device__ inline float root32(float x) {
 // the quotients by the same divisor can share its reciprocal (div_by), and quotients and roots of
 // kernel values and distances need no scaling. inv_wd = 1 / wdeltap.
 template <bool FINITE, class ADD>
-__device__ inline void pair_terms(const dev_consts &k, const rec64 &a, bool tool_i, double ta, double h1,
+__device__ inline void pair_terms(kconst &k, const rec64 &a, bool tool_i, double ta, double h1,
                                   double fourh2, double fac, double inv_wd, const rec64 &b, bool tool_j, ADD &add) {
   const double mass = k.mass;
   auto over = [](double n, double d) { return FINITE ? mfcm::quotient(n, d) : n / d; };
