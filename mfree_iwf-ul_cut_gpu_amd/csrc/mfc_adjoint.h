@@ -28,6 +28,14 @@
 namespace mfc {
 namespace adj {
 
+// the constants: on the GPU read through the constant address space (kconst)
+#if defined(__HIP__)
+typedef const __attribute__((address_space(4))) dev_consts adj_consts;
+#else
+typedef const dev_consts adj_consts;
+#endif
+
+
 MFC_HD double sq(double x) { return x * x; }
 
 // ------------------------------------------------------------------ neighbour record
@@ -56,7 +64,7 @@ MFC_HD void spline(double r, double h, double &w, double &dw, double &F, double 
 }
 
 // contribution of neighbour j to the sums of particle i (promoted pair_terms); adds to out[L_*]
-MFC_HD void pair_fwd(const dev_consts &k, const double *ri, const double *rj, bool tool_i, bool tool_j, double ta,
+MFC_HD void pair_fwd(adj_consts &k, const double *ri, const double *rj, bool tool_i, bool tool_j, double ta,
                      double *out) {
   const double xij = ri[R_X] - rj[R_X], yij = ri[R_Y] - rj[R_Y];
   const double rr2 = xij * xij + yij * yij;
@@ -90,7 +98,7 @@ MFC_HD void pair_fwd(const dev_consts &k, const double *ri, const double *rj, bo
 
 // VJP of pair_fwd. lam: adjoints of i's sums. Adds d/d(record of i) to gi and d/d(record of j)
 // to gj (want_i / want_j select which are needed).
-MFC_HD void pair_vjp(const dev_consts &k, const double *ri, const double *rj, bool tool_i, bool tool_j, double ta,
+MFC_HD void pair_vjp(adj_consts &k, const double *ri, const double *rj, bool tool_i, bool tool_j, double ta,
                      const double *lam, bool want_i, bool want_j, double *gi, double *gj) {
   const double xij = ri[R_X] - rj[R_X], yij = ri[R_Y] - rj[R_Y];
   const double rr2 = xij * xij + yij * yij;
@@ -194,7 +202,7 @@ MFC_HD void pair_vjp(const dev_consts &k, const double *ri, const double *rj, bo
 // with the other one's volume. Adds to gb what pair_vjp(b, a, want_i) and pair_vjp(a, b, want_j)
 // add. mech: neither is a tool particle; heat: the conduction sums are used.
 template <class RB, class RA, class LB, class LA>
-MFC_HD void pair_vjp_sym(const dev_consts &k, const RB &rb, const RA &ra, bool mech, bool heat, const LB &lb,
+MFC_HD void pair_vjp_sym(adj_consts &k, const RB &rb, const RA &ra, bool mech, bool heat, const LB &lb,
                          const LA &la, double *gb) {
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma clang fp contract(fast)
@@ -291,13 +299,13 @@ MFC_HD void pair_vjp_sym(const dev_consts &k, const RB &rb, const RA &ra, bool m
 
 // one term of the PSE sum of particle i (interactions_gpu.cu:130-139, no cutoff, promoted):
 // (T_j - T_i) 4/(pi h^4) exp(-r^2/h^2) m / rho_j
-MFC_HD double pse_fwd(const dev_consts &k, const double *ri, const double *rj) {
+MFC_HD double pse_fwd(adj_consts &k, const double *ri, const double *rj) {
   const double rr2 = sq(ri[R_X] - rj[R_X]) + sq(ri[R_Y] - rj[R_Y]);
   const double h2 = ri[R_H] * ri[R_H];
   return (rj[R_T] - ri[R_T]) * (4. / (h2 * h2 * M_PI)) * mfcm::exp(-rr2 / h2) * k.mass / rj[R_RHO];
 }
 
-MFC_HD void pse_vjp(const dev_consts &k, const double *ri, const double *rj, double lam_tpse, bool want_i,
+MFC_HD void pse_vjp(adj_consts &k, const double *ri, const double *rj, double lam_tpse, bool want_i,
                     bool want_j, double *gi, double *gj) {
   const double xij = ri[R_X] - rj[R_X], yij = ri[R_Y] - rj[R_Y];
   const double rr2 = xij * xij + yij * yij;
@@ -376,7 +384,7 @@ struct jc_grad { double s, e, ed, T, A, B, n, C, m; };
 
 // sigma_Y = (A + B e^n)(1 + C ln ed* or (1 + ed*)^C)(1 - theta^m) and its partials
 // (plasticity.cuh:30-46)
-MFC_HD jc_grad sigma_yield_grad(const dev_consts &k, double e, double ed, double t) {
+MFC_HD jc_grad sigma_yield_grad(adj_consts &k, double e, double ed, double t) {
   jc_grad g;
   const double th = (t - k.jc_Tref) / (k.jc_Tmelt - k.jc_Tref);
   const double en = mfcm::pow(e, k.jc_n);
@@ -406,11 +414,11 @@ MFC_HD jc_grad sigma_yield_grad(const dev_consts &k, double e, double ed, double
 // the temperature factor 1 - theta^m of sigma_yield_grad, and its value sigma_Y alone with that
 // factor given: the same expressions, for the secant's residuals, which evaluate the flow stress
 // at one temperature many times
-MFC_HD double jc_temperature_factor(const dev_consts &k, double t) {
+MFC_HD double jc_temperature_factor(adj_consts &k, double t) {
   const double th = (t - k.jc_Tref) / (k.jc_Tmelt - k.jc_Tref);
   return 1.0 - mfcm::pow(th, k.jc_m);
 }
-MFC_HD double sigma_yield_value(const dev_consts &k, double e, double ed, double TC) {
+MFC_HD double sigma_yield_value(adj_consts &k, double e, double ed, double TC) {
   const double TA = k.jc_A + k.jc_B * mfcm::pow(e, k.jc_n);
   const double es = ed / k.jc_eps_dot_ref;
   double TB;
@@ -428,7 +436,7 @@ struct contact_io {
   bool inside;
 };
 
-MFC_HD contact_io contact_fwd_vjp(const dev_consts &k, const mfc_tool_state &tool, double X, double Y, double U,
+MFC_HD contact_io contact_fwd_vjp(adj_consts &k, const mfc_tool_state &tool, double X, double Y, double U,
                                   double V, double ftx0, double fty0, double bfcx, double bfcy, double bftx,
                                   double bfty, double bnx, double bny, double &bX, double &bY, double &bU, double &bV,
                                   double &bftx0, double &bfty0, double &bmu) {
@@ -553,7 +561,7 @@ struct tail_grad {
 // forward recomputation and VJP of the tail of one particle. out_bar: adjoint of the state at the
 // end of the step (TS_*) and of the normal written by this step; Fbar: adjoint of this step's
 // tool force (F = sum fc + sum ft). fwd (optional): the forward outputs, TS_* then nx, ny.
-MFC_HD void tail_vjp(const dev_consts &k, const mfc_tool_state &tool, const tail_in &in, const double *out_bar,
+MFC_HD void tail_vjp(adj_consts &k, const mfc_tool_state &tool, const tail_in &in, const double *out_bar,
                      double nbar_x, double nbar_y, double Fbar_x, double Fbar_y, tail_grad &g, double *fwd) {
   for (int q = 0; q < TS_N; q++) g.s[q] = 0;
   g.nx = 0; g.ny = 0;
@@ -831,7 +839,7 @@ MFC_HD void tail_vjp(const dev_consts &k, const mfc_tool_state &tool, const tail
 // ------------------------------------------------------------------ record
 // the neighbour record of one particle from its sorted start-of-step state (predict, promoted);
 // p: in/out positional pressure (recomputed unless tool particle), R3: in/out artificial stress
-MFC_HD void record_fwd(const dev_consts &k, const double *s, int flags, double &p, double *R3, double *rec) {
+MFC_HD void record_fwd(adj_consts &k, const double *s, int flags, double &p, double *R3, double *rec) {
   const bool blank = flags & MFC_FLAG_BLANKED, tool_p = flags & MFC_FLAG_TOOL;
   const double hdt = 0.5 * k.dt;
   double x = s[TS_X], y = s[TS_Y], u = s[TS_U], v = s[TS_V], sxx = s[TS_SXX], sxy = s[TS_SXY], syy = s[TS_SYY];
@@ -854,7 +862,7 @@ MFC_HD void record_fwd(const dev_consts &k, const double *s, int flags, double &
 
 // VJP of record_fwd: b_rec (adjoint of the record) -> adjoint of the sorted start-of-step state
 // (added to gs, TS_*)
-MFC_HD void record_vjp(const dev_consts &k, const double *s, int flags, double p, const double *b_rec, double *gs) {
+MFC_HD void record_vjp(adj_consts &k, const double *s, int flags, double p, const double *b_rec, double *gs) {
   const bool blank = flags & MFC_FLAG_BLANKED, tool_p = flags & MFC_FLAG_TOOL;
   const double hdt = 0.5 * k.dt;
   double sxx = s[TS_SXX], sxy = s[TS_SXY], syy = s[TS_SYY], rho = s[TS_RHO];

@@ -144,7 +144,7 @@ __device__ inline const int *slot_flags(const __attribute__((address_space(4))) 
   return (const int *)(slot_state(d, slot) + (size_t)DSTATE_DOUBLES * d.k.N);
 }
 // EOS pressure of the predicted density (0 for a tool particle: no sum reads it)
-__device__ inline double eos_pressure(const dev_consts &k, const double *s, int flags) {
+__device__ inline double eos_pressure(adj_consts &k, const double *s, int flags) {
   if (flags & MFC_FLAG_TOOL) return 0.;
   const double rho = flags & MFC_FLAG_BLANKED ? s[TS_RHO] : s[TS_RHO] + 0.5 * k.dt * s[TS_RHOT];
   return k.c0 * k.c0 * (rho - k.rho0);
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(TILE) void kb_adj_tail(const adj_args *__restrict__
   if (w < 0) return;
   const int2 it = work[w];
   MFC_ADJ_ARGS(d, it.x);
-  const dev_consts &k = D[it.x].k;
+  adj_consts &k = d.k;
   const int t = it.y;
   const int i = t * TILE + threadIdx.x;
   const size_t N = k.N;
@@ -264,7 +264,7 @@ __device__ inline void add_theta(const __attribute__((address_space(4))) adj_arg
 // A work-group takes a part of a patch of cells, as the interaction does, with the records and the
 // adjoints of the sums of its window candidates staged in LDS (240 bytes each; three work-groups to a
 // CU): read from memory per pair, by one work-group per 32 particles of the sorted order, they were 30
-// gathers of 64 scattered lines, and the pass took 95 us at 37.5k particles, now 43.
+// gathers of 64 scattered lines, and the pass took 95 us at 37.5k particles, now 41.
 constexpr int PULL_LANES = 8;
 constexpr int PULL_AT_ONCE = TILE / PULL_LANES;  // particles a work-group takes at once
 constexpr int PULL_CAP = 208;  // window candidates a work-group stages: 5 x 5 cells at hdx 1.5 have 196 at most
@@ -282,7 +282,7 @@ struct pull_mem {
 struct pull_pair {
   bool of_a, of_b;
 };
-__device__ inline pull_pair pull_flags(const dev_consts &k, int fa, int fb) {
+__device__ inline pull_pair pull_flags(adj_consts &k, int fa, int fb) {
   const bool blank = (fa | fb) & MFC_FLAG_BLANKED, pse = k.pse != 0;
   return {!blank && (!pse || !(fa & MFC_FLAG_TOOL)), !blank && (!pse || !(fb & MFC_FLAG_TOOL))};
 }
@@ -316,7 +316,7 @@ struct pull_memory {
 // the pairs of particle b (index in src; all h equal) over its window, lane r of its lanes; gl: its
 // first lane in the wave, list: 64 bytes of LDS of its own
 template <class SRC>
-__device__ inline void pull_particle(const dev_consts &k, const SRC &src, int b, const window &w, int r, int gl,
+__device__ inline void pull_particle(adj_consts &k, const SRC &src, int b, const window &w, int r, int gl,
                                      unsigned char *list, double *gb) {
   auto value = [&](int j, int q) { const double2 v = src.piece(q / 2, j); return q % 2 ? v.y : v.x; };
   auto load = [&](int j, double *rec, double *la) {
@@ -383,7 +383,7 @@ __device__ inline void pull_particle(const dev_consts &k, const SRC &src, int b,
 // uniform h the same bits; else each pair's two terms one after the other, with the h of each
 __device__ inline void pull_rest(pull_mem &m, const adj_args *__restrict__ D, int inst, int slot, int patch, int part) {
   MFC_ADJ_ARGS(d, inst);
-  const dev_consts &k = D[inst].k;
+  adj_consts &k = d.k;
   const size_t N = k.N;
   const int *__restrict__ offsets = d.offsets + (size_t)slot * d.ncell1, *__restrict__ keys = d.key_sorted + (size_t)slot * N;
   const int nrb = patch_rows(k), pc = patch / nrb, pr = patch - pc * nrb;
@@ -440,7 +440,7 @@ __device__ inline void pull_rest(pull_mem &m, const adj_args *__restrict__ D, in
 // returns false, with nothing done, for an entry that pull_rest takes
 __device__ inline bool pull_patch(pull_mem &m, const adj_args *__restrict__ D, int inst, int slot, int patch, int part) {
   MFC_ADJ_ARGS(d, inst);
-  const dev_consts &k = D[inst].k;
+  adj_consts &k = d.k;
   const size_t N = k.N;
   const int *__restrict__ offsets = d.offsets + (size_t)slot * d.ncell1;
   const int tid = threadIdx.x;
@@ -533,7 +533,7 @@ __global__ __launch_bounds__(TILE) void kb_adj_record(const adj_args *__restrict
   if (w < 0) return;
   const int2 it = work[w];
   MFC_ADJ_ARGS(d, it.x);
-  const dev_consts &k = D[it.x].k;
+  adj_consts &k = d.k;
   const int a = it.y * TILE + threadIdx.x;
   if (a >= k.N) return;
   const size_t N = k.N;
