@@ -261,17 +261,19 @@ __device__ inline double secant(double dl, double tol, const F &residual) {
 
 // One lane's part of the Johnson-Cook flow stress TA TB TC (sigma_yield): the strain factor TA, or
 // the rate factor TB (rate), at the strain e and the relative rate es. One evaluation of the
-// logarithm's series serves both.
+// logarithm's series serves both. NORMAL: e, es, n and C are as log_series and pow_of need them to be
+// without special cases.
+template <bool NORMAL>
 __device__ inline double jc_part(bool rate, double e, double es, double A, double B, double n, double C) {
   const bool lg = rate && es > 1.0;
   const double x = !rate ? e : lg ? es : 1.0 + es, y = rate ? C : n;
   double v;
-  if (x > 0.0 && !mfcm::is_inf(x) && mfcm::abs_d(y) <= 1e290) {  // as mfcm::log and mfcm::pow there
+  if (NORMAL || (x > 0.0 && !mfcm::is_inf(x) && mfcm::abs_d(y) <= 1e290)) {  // as mfcm::log and mfcm::pow there
     int k;
     double f, s, R;
-    mfcm::log_series(x, k, f, s, R);
+    mfcm::log_series<NORMAL>(x, k, f, s, R);
     v = mfcm::log_of(k, f, s, R);
-    if (!lg) v = mfcm::pow_of(k, f, s, R, y);
+    if (!lg) v = mfcm::pow_of<NORMAL>(k, f, s, R, y);
   } else if (x == 0.0 && y > 0.0) {
     v = 0.0;
   } else {
@@ -281,33 +283,32 @@ __device__ inline double jc_part(bool rate, double e, double es, double A, doubl
 }
 
 // The FP64 path's secant, four lanes per particle: lane bit 1 takes one of the two factors of the flow
-// stress that depend on dl. What bounds it is one iteration's chain of dependent FP64 operations (about
-// 300 instructions, 220 of them FP64, 0.7 us): a wave with a long return is the last of its launch (a
-// fold at a tolerance of 1e-14 runs to 101 iterations, the steps of a cut at 1e-6 to 16). With both
-// factors in one lane, full divisions by dt and the reference rate and the pow's special cases on
-// the way an iteration took 1.7 us; a taped and reversed step of the 37.5k cut with 20-100 folding
-// returns 600 us, now 410, of the 6k cut 475, now 280. The loop is in the outlined function so that
-// the polynomials' constants stay in registers through it (evaluated by a function called in the loop
-// they were loaded again each time, and the two cuts took 480 and 320 us).
+// stress that depend on dl. What bounds it is one iteration's chain of dependent FP64 operations (some
+// 250 instructions): a wave with a long return is the last of its launch (a fold at a tolerance of
+// 1e-14 runs to 101 iterations, the steps of a cut at 1e-6 to 16). Measured, us per taped and reversed
+// step of the 37.5k and 6k cuts with 20-100 folding returns: 600 and 475 with both factors in one lane,
+// full divisions by dt and the reference rate and the special cases of pow on the way; 410 and 280
+// with two lanes for them and pow_of; 340 and 265 with the returns of a patch in one pass; 295 and 230
+// without a check for special cases at each value. The loop is in the outlined function so that the
+// polynomials' constants stay in registers through it (evaluated by a function called in the loop they
+// were loaded again each time: 480 and 320 instead of 410 and 280).
 __device__ __attribute__((noinline)) double rr_secant_jc(kconst &k, double dl, double norm, double eps0,
                                                         double TC) {
   const double A = k.jc_A, B = k.jc_B, n = k.jc_n, C = k.jc_C, edr = k.jc_eps_dot_ref, dt = k.dt, G = k.G;
   const double s23 = sqrt(2.0 / 3.0);
   const bool rate = threadIdx.x & 2;
   const double ydt = 1.0 / dt, yedr = 1.0 / edr;
-  // dt and edr in a range where div_by's quotients are those of the division
-  const bool in_range = dt > 0x1p-400 && dt < 0x1p400 && edr > 0x1p-400 && edr < 0x1p400;
+  // the return's start and the constants are such that, with inc below, every value of the residual is
+  // a normal number, and div_by's quotients are those of the division
+  const bool normal = dt > 0x1p-100 && dt < 0x1p100 && edr > 0x1p-100 && edr < 0x1p100 && mfcm::abs_d(n) < 0.98 &&
+                      mfcm::abs_d(C) < 0.98 && eps0 >= 0. && eps0 < 0x1p100;
   return secant(dl, k.secant_tol, [&](double x) {
     const double inc = s23 * fmax(x, 0.);
-    double ed, es;
-    if (in_range && (inc == 0. || (inc > 0x1p-100 && inc < 0x1p100))) {
-      ed = div_by(inc, dt, ydt);
-      es = div_by(ed, edr, yedr);
-    } else {
-      ed = inc / dt;
-      es = ed / edr;
-    }
-    const double T = jc_part(rate, eps0 + inc, es, A, B, n, C);
+    double T;
+    if (normal && inc > 0x1p-500 && inc < 0x1p100)
+      T = jc_part<true>(rate, eps0 + inc, div_by(div_by(inc, dt, ydt), edr, yedr), A, B, n, C);
+    else
+      T = jc_part<false>(rate, eps0 + inc, inc / dt / edr, A, B, n, C);
     return norm - 2 * G * x - s23 * (T * quad_xor<2>(T) * TC);
   });
 }

@@ -95,13 +95,18 @@ MFC_HD double exp_reduced(double r) {
   return 1.0 + (r + (r * r) * p);
 }
 
+// e^x where it is a normal number
+MFC_HD double exp_normal(double x) {
+  const double kd = floor(x * INV_LN2 + 0.5);
+  const double r = (x - kd * LN2_HI) - kd * LN2_LO;
+  return __builtin_ldexp(exp_reduced(r), (int)kd);
+}
+
 // e^x
 MFC_HD double exp(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
   // without branches: the scaling is one instruction, exact or rounded once, as below
-  const double kd = floor(x * INV_LN2 + 0.5);
-  const double r = (x - kd * LN2_HI) - kd * LN2_LO;
-  const double v = __builtin_ldexp(exp_reduced(r), (int)kd);
+  const double v = exp_normal(x);
   return is_nan(x) ? x : x > 709.782712893384 ? u2d(0x7ff0000000000000ULL) : x < -745.1332191019412 ? 0.0 : v;
 #else
   if (is_nan(x)) return x;
@@ -116,10 +121,12 @@ MFC_HD double exp(double x) {
   return e * pow2i(k);
 #endif
 }
-// x = 2^e (1 + f) for x positive and finite, and the series R of log(1 + f) (above) with s = f/(2+f)
+// x = 2^e (1 + f) for x positive and finite, and the series R of log(1 + f) (above) with s = f/(2+f).
+// NORMAL: x is a normal number
+template <bool NORMAL = false>
 MFC_HD void log_series(double x, int &e, double &f, double &s, double &R) {
   int eadj = 0;
-  if (x < 2.2250738585072014e-308) { x = x * 18014398509481984.0; eadj = -54; }  // 2^54
+  if (!NORMAL && x < 2.2250738585072014e-308) { x = x * 18014398509481984.0; eadj = -54; }  // 2^54
   uint64_t u = d2u(x);
   e = (int)((u >> 52) & 0x7ff) - 1023 + eadj;
   double m = u2d((u & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL);
@@ -210,14 +217,20 @@ MFC_HD void log_dd(int e, double f, double s, double R, double &hi, double &lo) 
   lo = l - (hi - s2);
 }
 
-// x^y from the series of log(x); y log(x) is formed in double-double before exp
+// x^y from the series of log(x); y log(x) is formed in double-double before exp. NORMAL: |y| < 0.98,
+// so that every value on the way is a normal number
+template <bool NORMAL = false>
 MFC_HD double pow_of(int k, double f, double s, double R, double y) {
   double lh, ll;
   log_dd(k, f, s, R, lh, ll);
-  if (abs_d(y) > 1e290) return exp(y * lh);
+  if (!NORMAL && abs_d(y) > 1e290) return exp(y * lh);
   double p, pe;
   two_prod(y, lh, p, pe);
   double plo = pe + y * ll;
+  if (NORMAL) {
+    const double e = exp_normal(p);
+    return e + e * plo;
+  }
   double e = exp(p);
   if (is_inf(e) || e == 0.0) return exp(p + plo);
   return e + e * plo;

@@ -130,3 +130,19 @@ def test_gradient_of_both_pull_paths(thermal):
     a, b = grads[0][1], grads[1][1]
     assert np.all(np.isfinite(a)) and np.abs(a).max() > 0
     assert np.abs(a - b).max() <= 1e-9 * np.abs(a).max()
+
+
+@pytest.mark.parametrize("lanes", [1, 8])
+@pytest.mark.parametrize("n,C,tol", [(0.34, 0.014, 1e-14), (0.97, 0.97, 1e-6), (1.0, 0.014, 1e-6), (0.34, 1.0, 1e-6),
+                                     (1.3, 2.0, 1e-14)])
+def test_returns_match_the_oracle(lanes, n, C, tol):
+    """The return's secant with exponents on both sides of the bound below which no value on its way
+    needs a special case, to its end and folding, by a wave and by a whole work-group."""
+    cfg = cut(thermal="adiabatic")
+    cfg.jc_n, cfg.jc_C, cfg.secant_tol = n, C, tol
+    g, o = pymfc.Sim(cfg), ob.OracleSim(cfg)
+    g.set_tuning(lanes=lanes)
+    g.step(120)
+    o.step(120)
+    assert np.count_nonzero(o.field("eps_pl")) > 10
+    assert_bitwise(g, o, context=f"n {n} C {C}")
