@@ -45,11 +45,11 @@ STEP_BYTES = 256 + 224 + 12
 KERNEL_BYTES = {"binning": 12, "interact": 256 + 224}
 assert sum(KERNEL_BYTES.values()) == STEP_BYTES
 # HBM bytes per particle of one launch of the interaction kernel on thermal_contact_150k, by
-# precision, XCD chunk length and LDS stage limit (0: all candidates), measured with rocprofv3
-# --pmc FETCH_SIZE / WRITE_SIZE passes and scaled by a 512 MiB copy (the commands and tables are in
-# profiles/traffic_thermal_contact_150k.md); a table of measurements, not measured in this run, and
-# reported as `traffic` only for the tuning it was measured with
-MEASURED_TRAFFIC = {}
+# precision and XCD chunk length (a stage limit above the stage's own size changes nothing), measured
+# with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE passes and scaled by a 512 MiB copy (the commands and
+# tables are in profiles/traffic_thermal_contact_150k.md); a table of measurements, not measured in
+# this run, and reported as `traffic` only for the tuning it was measured with
+MEASURED_TRAFFIC = {("kb_interact", "fp32c", 8): 791, ("kb_interact", "fp64", 8): 987}
 MEASURED_TRAFFIC_SOURCE = ("table: rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, thermal_contact_150k, fused interaction, "
                            "profiles/traffic_thermal_contact_150k.md")
 
@@ -350,7 +350,7 @@ def main() -> int:
     # kernel's roofline
     t_int = r["phases"]["interact"] * 1e-3 if r["phases"] else None
     achieved = N * kbytes / t_int / 1e9 if t_int else None
-    tkey = ("kb_interact", head, r["tuning"].get("xcd_chunk", 8), r["tuning"]["stage_limit"])
+    tkey = ("kb_interact", head, r["tuning"].get("xcd_chunk", 8))
     traffic = None
     if args.workload == "thermal_contact_150k" and tkey in MEASURED_TRAFFIC:
         traffic = MEASURED_TRAFFIC[tkey] * N

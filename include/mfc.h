@@ -319,7 +319,7 @@ int mfc_vjp(mfc_sim *sim, mfc_vjp_req *req, double grad[6]);
 
 /* launch configuration of the step kernels (results do not depend on it: every variant
  * evaluates the same expressions in the same order). lanes: threads per particle of the
- * interaction, 1, 4 or 8 (0: by the number of particles that are stepped together; more lanes
+ * interaction, 1, 4 or 8 (0: by the number of work-groups they make; more lanes
  * shorten a particle's chain of operations where the particles alone would not fill the chip).
  * stage_limit: the most window candidates a patch of cells copies into LDS (0 or anything above
  * what the kernel has room for: all of them); a patch with more reads them from the records in

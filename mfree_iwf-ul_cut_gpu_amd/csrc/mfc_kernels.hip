@@ -1320,9 +1320,9 @@ __device__ inline void fetch_state(const dstate &src, size_t N, unsigned s, unsi
 // its loads and stores move in a burst, since one round of work-groups fills the chip (FP32C four,
 // FP64 three to a CU). With 4 or 8 threads per particle the sums of 6k particles take 13 or 8 us
 // instead of 21 (FP64). Measured, us per step (tiles of the sorted order with candidate positions
-// in LDS and a launch for the records, then this): FP32C 6k 55 -> 29, 27k 68 -> 38, 71k 63 -> 48,
-// 197k 80 -> 60, 500k PSE 276 -> 179; FP64 6k 63 -> 32, 27k 77 -> 50, 71k 93 -> 62, 197k 137 -> 110,
-// 500k PSE 403 -> 351.
+// in LDS and a launch for the records, then this): FP32C 6k 55 -> 26, 27k 68 -> 35, 71k 63 -> 45,
+// 197k 80 -> 56, 500k PSE 276 -> 169; FP64 6k 63 -> 29, 27k 77 -> 46, 71k 93 -> 61, 197k 137 -> 102,
+// 500k PSE 403 -> 299.
 // returns false, with nothing done, for a patch whose window candidates do not fit the stage or
 // whose state has no uniform h (interact_rest takes it)
 template <bool F32, int G, bool PSE>
