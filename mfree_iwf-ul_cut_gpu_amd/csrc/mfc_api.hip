@@ -250,6 +250,8 @@ mfc::inst_args instance_args(const mfc_sim *s, int c) {
   a.rn = s->recs[1 - c];
   a.tool_in = s->tool + c;
   a.tool_out = s->tool + (1 - c);
+  a.tape_in = s->tape + c;
+  a.tape_out = s->tape + (1 - c);
   a.f = s->force(c);
   a.geo = s->geo;
   a.ntiles = s->ntiles;
@@ -412,6 +414,11 @@ void mfc_destroy(mfc_sim *s) {
 }
 
 int mfc_create(const mfc_config *cfg, mfc_sim **out) {
+  // what each step passes on to the next beside the state, two of each, in one allocation
+  struct carried {
+    mfc_tool_state tool[2];
+    mfc::return_tape tape[2];
+  };
   if (!cfg || !out) return fail(MFC_E_INVALID, "null argument");
   *out = nullptr;
   int ndev = 0;
@@ -467,11 +474,14 @@ int mfc_create(const mfc_config *cfg, mfc_sim **out) {
       return bail(rc);
     }
   }
-  if ((rc = s->alloc(&s->tool, 2)) ||
+  carried *two = nullptr;
+  if ((rc = s->alloc(&two, 1)) ||
       (rc = s->alloc(&s->partials, (size_t)16 * s->ntiles)) || (rc = s->alloc(&s->force_last, 2)) ||
       (rc = s->alloc(&s->hist, (size_t)2 * HIST_CAP)) || (rc = s->alloc(&s->hist_ctr, 1)) ||
       (rc = s->alloc(&s->force_pending, 2)) || (rc = s->alloc(&s->force_groups, (size_t)4 * s->ntiles)))
     return bail(rc);
+  s->tool = two->tool;
+  s->tape = two->tape;
   // zero everything, then upload the initial state (particle_gpu.cu:20-125); with the zeros uploaded
   // too, creating a handle took 0.9 ms at 6k particles and 14 at 500k, now 0.4 and 10
   {
@@ -506,8 +516,8 @@ int mfc_create(const mfc_config *cfg, mfc_sim **out) {
         hipMemsetAsync(s->chunk_sums[1], 0, sizeof(int) * (size_t)mfc::scan_blocks(c.ncell_table), s->stream) != hipSuccess ||
         hipMemsetAsync(s->force_last, 0, 2 * sizeof(double), s->stream) != hipSuccess)
       return bail(fail(MFC_E_HIP, "memset"));
-    mfc_tool_state t2[2] = {S.tool, S.tool};
-    if (up(s->tool, t2, sizeof(t2)) != hipSuccess) return bail(fail(MFC_E_HIP, "upload tool"));
+    const carried first = {{S.tool, S.tool}, {{nullptr, 0}, {nullptr, 0}}};
+    if (up(two, &first, sizeof(first)) != hipSuccess) return bail(fail(MFC_E_HIP, "upload tool"));
     const mfc::grid_geo g0 = {c.bbmin_x, c.bbmin_y, c.cell, c.gnx, c.gny, c.num_cell, 0};
     if (up(s->geo, &g0, sizeof(g0)) != hipSuccess) return bail(fail(MFC_E_HIP, "upload grid"));
     // descriptors and work tables of the step kernels (a batch of one)

@@ -103,6 +103,15 @@ struct variant {
   int chunk;  // work items per XCD chunk of the interaction's map (1..XCD_CHUNK_MAX)
 };
 
+// The secant results of a run that the reverse mode recorded: the next step's place (a double per
+// particle in sorted order, written where the particle returns: dl, or -dl where its last update
+// folded) and how many steps have one. Passed on from step to step on the device as the tool is,
+// since a captured step cannot be told its number.
+struct return_tape {
+  double *at;
+  long long left;
+};
+
 // one instance of a batch as the batched kernels see it (an array of these lives in device
 // memory, one per instance and step parity)
 struct inst_args {
@@ -116,11 +125,14 @@ struct inst_args {
   dforce f;
   double *acc_out;  // when set, the interaction also stores its neighbour sums there (ACC_N
                     // arrays of N doubles), then each particle's secant result (N doubles,
-                    // end_update); the reverse mode's replay keeps them
+                    // end_update); the reverse mode's replay keeps them, and takes the secant
+                    // results from the tape where it has some instead of iterating again
   grid_geo *geo;  // adaptive grid: the geometry of the current step (written by the device)
   int ntiles;   // particle tiles of TILE
   int nscan;    // scan chunks of the cell table
   int npatch_items;  // patch work items of the instance: item q takes the entries q, q + npatch_items, ... of plist
+  const return_tape *tape_in;
+  return_tape *tape_out;
 };
 
 // the work of one batched step: instance descriptors and (instance, block) work tables

@@ -85,6 +85,7 @@ struct mfc_sim {
   int *plen = nullptr;                      // bins.plen of parity 0 / 1
   int precision = MFC_PREC_FP64;
   mfc_tool_state *tool = nullptr;  // two states, alternating each step
+  mfc::return_tape *tape = nullptr;  // two, alternating each step
   double *partials = nullptr, *force_last = nullptr, *hist = nullptr;
   int64_t *hist_ctr = nullptr;
   int *force_pending = nullptr;  // per parity: the force of the step that produced it is not yet reduced

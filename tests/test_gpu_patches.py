@@ -146,3 +146,30 @@ def test_returns_match_the_oracle(lanes, n, C, tol):
     o.step(120)
     assert np.count_nonzero(o.field("eps_pl")) > 10
     assert_bitwise(g, o, context=f"n {n} C {C}")
+
+
+@pytest.mark.parametrize("lanes,limit", [(0, 0), (1, 0), (0, 1)])
+def test_gradient_with_recorded_returns(lanes, limit):
+    """A replay that takes the secant results of the recorded run, and one that iterates again (a run
+    so long that its tape would be larger than its checkpoints and slots; the steps past the window
+    carry no adjoint): the same expressions on the same values, so the same bits. Steps after a
+    recorded run write nothing to its tape."""
+    cfg = cut(thermal="adiabatic")
+    cfg.promote_fp64, cfg.secant_tol = 1, 1e-14
+    grads = []
+    for n, K in ((60, 13), (14000, 75)):
+        g = pymfc.Sim(cfg)
+        g.set_tuning(lanes=lanes, stage_limit=limit)
+        g.step(60)
+        F = g.vjp_forward(n, K, 10, 60)
+        grads.append((F, g.vjp_backward([1.0, 0.5])))
+        if n == 60:
+            o = ob.OracleSim(cfg)
+            o.step(140)
+            g.step(20)
+            assert np.count_nonzero(o.field("eps_pl")) > 10
+            assert_bitwise(g, o, context="after a recorded run")
+            assert equal(grads[0][1], g.vjp_backward([1.0, 0.5]))  # its tape is as it was
+    assert equal(grads[0][0], grads[1][0])
+    assert np.all(np.isfinite(grads[0][1])) and np.abs(grads[0][1]).max() > 0
+    assert equal(grads[0][1], grads[1][1])
