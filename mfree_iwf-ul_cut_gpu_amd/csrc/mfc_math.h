@@ -156,7 +156,26 @@ MFC_HD double log_of(int e, double f, double s, double R) {
   return dk * LN2_HI - ((hfsq - (s * (hfsq + R) + dk * LN2_LO)) - f);
 }
 
+// a number with the series of its magnitude's logarithm, for several functions of it
+struct log_parts {
+  double x;
+  int e;
+  double f, s, R;
+};
+MFC_HD log_parts parts_of(double x) {
+  log_parts l;
+  l.x = x;
+  log_series(abs_d(x), l.e, l.f, l.s, l.R);
+  return l;
+}
+
 // natural logarithm
+MFC_HD double log_special(double x) {
+  if (is_nan(x)) return x;
+  if (x < 0.0) return u2d(0x7ff8000000000000ULL);
+  if (x == 0.0) return -u2d(0x7ff0000000000000ULL);
+  return x;
+}
 MFC_HD double log(double x) {
   if (x > 0.0 && !is_inf(x)) {
     int e;
@@ -164,10 +183,10 @@ MFC_HD double log(double x) {
     log_series(x, e, f, s, R);
     return log_of(e, f, s, R);
   }
-  if (is_nan(x)) return x;
-  if (x < 0.0) return u2d(0x7ff8000000000000ULL);
-  if (x == 0.0) return -u2d(0x7ff0000000000000ULL);
-  return x;
+  return log_special(x);
+}
+MFC_HD double log(const log_parts &l) {
+  return l.x > 0.0 && !is_inf(l.x) ? log_of(l.e, l.f, l.s, l.R) : log_special(l.x);
 }
 
 MFC_HD bool is_int(double y) { return floor(y) == y; }
@@ -236,16 +255,9 @@ MFC_HD double pow_of(int k, double f, double s, double R, double y) {
   return e + e * plo;
 }
 
-// x^y with IEEE 754 special cases
-MFC_HD double pow(double x, double y) {
+// x^y with IEEE 754 special cases, given v = |x|^y where x and y are finite and x is not 0
+MFC_HD double pow_special(double x, double y, double v) {
   const double INF = u2d(0x7ff0000000000000ULL);
-  double v = 0.0;
-  if (abs_d(x) > 0.0 && !is_inf(x) && !is_inf(y)) {
-    int e;
-    double f, s, R;
-    log_series(abs_d(x), e, f, s, R);
-    v = pow_of(e, f, s, R, y);
-  }
   if (x > 0.0 && !is_inf(x) && !is_inf(y) && !is_nan(y)) return v;
   if (y == 0.0) return 1.0;
   if (x == 1.0) return 1.0;
@@ -269,6 +281,21 @@ MFC_HD double pow(double x, double y) {
   }
   if (!is_int(y)) return u2d(0x7ff8000000000000ULL);
   return is_odd_int(y) ? -v : v;
+}
+MFC_HD double pow(double x, double y) {
+  double v = 0.0;
+  if (abs_d(x) > 0.0 && !is_inf(x) && !is_inf(y)) {
+    int e;
+    double f, s, R;
+    log_series(abs_d(x), e, f, s, R);
+    v = pow_of(e, f, s, R, y);
+  }
+  return pow_special(x, y, v);
+}
+MFC_HD double pow(const log_parts &l, double y) {
+  double v = 0.0;
+  if (abs_d(l.x) > 0.0 && !is_inf(l.x) && !is_inf(y)) v = pow_of(l.e, l.f, l.s, l.R, y);
+  return pow_special(l.x, y, v);
 }
 
 // atan(x)
