@@ -877,8 +877,9 @@ __device__ inline void sums_mem(kconst &k, const mem_source<F32> &src, const win
 // a wave for windows of 56 candidates, whose columns hold 8 or 16 by turns), because a candidate
 // numbered through the columns costs 11 instructions to find and one of a column none; in the
 // loop over the pairs a lane moves its next column's mask up when its current one is used up.
-// flags: what the patch's candidates have of TOOL and BLANKED (without PSE, the copy holds blanked
-// particles at infinity).
+// flags: what the patch's candidates have of TOOL and BLANKED (without PSE, the copy holds both
+// coordinates of a blanked particle at infinity, whatever they are: one that is not a number would
+// pass the test of near).
 constexpr int WALK_U = 4;  // candidates whose loads are issued together
 template <bool F32, int G, bool PSE>
 __device__ inline void sums_lds(kconst &k, const lds_source<F32, G> &src, int flags, const int b[5],
@@ -1442,7 +1443,7 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, unsigned *unread, co
         if (c >= ncand) break;
         if (!PSE && (flags & MFC_FLAG_BLANKED) && pl == 0 &&
             ((patch_mem<F32, G>::ALL_IN_LDS ? m.tag[c] : (int)m.fl[patch_mem<F32, G>::ALL_IN_LDS ? 0 : c]) & MFC_FLAG_BLANKED))
-          reinterpret_cast<double2 &>(v[u]).x = __builtin_huge_val();
+          reinterpret_cast<double2 &>(v[u]) = make_double2(__builtin_huge_val(), __builtin_huge_val());
         if constexpr (F32) {
           m.piece[pl][c] = v[u];
         } else if (pl != 1) {  // piece 1 of a record: flags (in the tag) and h (uniform)
