@@ -144,9 +144,10 @@ void patch_shape(double hdx, bool f32, int lanes, int &s, int &w) {
 
 int64_t patch_bound(const mfc::dev_consts &k, int s, int w) {
   if (!k.adaptive) return (int64_t)((k.gnx + w - 1) / w) * ((k.gny + s - 1) / s);
-  // any nx by ny cells with nx ny < ncell_table: (nx / w + 1) (ny / s + 1)
+  // any nx by ny cells with nx ny < ncell_table: ((nx - 1) / w + 1) ((ny - 1) / s + 1) at most, where
+  // nx + ny <= ncell_table; and the particles past the grid
   const int64_t t = k.ncell_table;
-  return t / ((int64_t)s * w) + t / (s < w ? s : w) + 2;
+  return t / ((int64_t)s * w) + t / (s < w ? s : w) + 2 + 1;
 }
 
 }  // namespace

@@ -118,15 +118,16 @@ __device__ inline void count_cell(int i, int h, int *__restrict__ key, int *__re
   if (c >= 0 && place < ccap) clist[(size_t)c * ccap + place] = make_int2(i, h);
 }
 
-// counts the particle of cell h in its patch (all 64 lanes of the wave; h = -1: no particle): one
-// atomic per run of equal patches in the wave
-template <class K>
-__device__ inline void count_patch(K &k, int h, int *__restrict__ pcnt) {
-  int p = -1;
-  if (h >= 0) {
-    const int gi = h / k.gny, gj = h - gi * k.gny;
-    p = (gi / k.patch_w) * patch_rows(k) + gj / k.patch_s;
-  }
+// the patch of a cell of the grid
+template <class K>  // dev_consts or kconst
+__device__ inline int patch_of(K &k, int h) {
+  const int gi = h / k.gny, gj = h - gi * k.gny;
+  return (gi / k.patch_w) * patch_rows(k) + gj / k.patch_s;
+}
+
+// counts a particle in its patch p (all 64 lanes of the wave; p = -1: no particle): one atomic per
+// run of equal patches in the wave
+__device__ inline void count_patch(int p, int *__restrict__ pcnt) {
   const int lane = threadIdx.x & 63, prev = __shfl_up(p, 1, 64);
   const bool head = lane == 0 || prev != p;
   const unsigned long long after = lane == 63 ? 0ull : __ballot(head) & ~((2ull << lane) - 1ull);
@@ -140,7 +141,9 @@ __device__ inline void hash_count(K &k, int i, const double *__restrict__ px,
                                   const dbins &b) {
   const int h = i < k.N ? particle_cell(k, px[i], py[i], flags[i], b.key_sorted[i], b.clamped) : -1;
   count_cell(i, h, b.key, b.bsum, b.clist, b.ccap);
-  count_patch(k, h, b.pcnt);
+  // a blanked particle keeps its cell id, which an adaptive grid can shrink below: such particles
+  // are sorted past the grid's cells and make a patch of their own behind the grid's
+  count_patch(h < 0 ? -1 : h >= k.num_cell ? patch_total(k) : patch_of(k, h), b.pcnt);
 }
 
 // The counting sort of one chunk of SCAN_CHUNK cells (SCAN_ITEMS per thread), by one work-group,
@@ -287,7 +290,7 @@ __device__ inline void sort_chunk(int blk, int N, int n, const dbins &b, const i
 // not depend on the order of the list). Clears the patches' counts
 constexpr int PLIST_BATCH = PLIST_SECTION / SCAN_THREADS;  // patches per thread
 __device__ inline void list_patches(kconst &k, int sec, const dbins &b) {
-  const int np = patch_total(k);
+  const int np = patch_total(k) + (k.adaptive ? 1 : 0);  // and that past the grid (hash_count)
   const int p0 = sec * PLIST_SECTION + threadIdx.x * PLIST_BATCH;
   if (sec == 0 && threadIdx.x == 0) *b.plen_next = 0;
   if (sec * PLIST_SECTION >= np) return;
@@ -1236,7 +1239,7 @@ __device__ inline void next_cell(kconst &k, int i, bool live, double x, double y
   if (k.adaptive) return;  // the same in every thread
   const int h = live ? particle_cell(k, x, y, fl, next.key_sorted[i], next.clamped) : -1;
   count_cell(i, h, next.key, next.bsum_next, next.clist, next.ccap);
-  count_patch(k, h, next.pcnt);
+  count_patch(h < 0 ? -1 : patch_of(k, h), next.pcnt);
 }
 
 __device__ inline sum_flags flags_of(kconst &k, int tag) {
@@ -1356,7 +1359,7 @@ __device__ inline void fetch_state(const dstate &src, size_t N, unsigned s, unsi
 // 197k 80 -> 56, 500k PSE 276 -> 169; FP64 6k 63 -> 29, 27k 77 -> 46, 71k 93 -> 61, 197k 137 -> 102,
 // 500k PSE 403 -> 299.
 // returns false, with nothing done, for a patch whose window candidates do not fit the stage or
-// whose state has no uniform h (interact_rest takes it)
+// whose state has no uniform h, and for the particles past the grid (interact_rest takes them)
 template <bool F32, int G, bool PSE>
 __device__ inline bool interact_patch(patch_mem<F32, G> &m, unsigned *unread, const inst_args *A, int inst, int patch, int part) {
   const inst_args &a_ = A[inst];
@@ -1373,6 +1376,7 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, unsigned *unread, co
   // own cells: rows [r0, r1), columns [g0, g1); staged: rows [s0, s1), columns [q0, q1)
   const int r0 = pr * k.patch_s, r1 = r0 + k.patch_s < k.gny ? r0 + k.patch_s : k.gny;
   const int g0 = pc * k.patch_w, g1 = g0 + k.patch_w < k.gnx ? g0 + k.patch_w : k.gnx;
+  if (g0 >= k.gnx) return false;  // the particles past the grid
   const int s0 = r0 < 2 ? 0 : r0 - 2, s1 = r1 + 2 < k.gny ? r1 + 2 : k.gny;
   const int q0 = g0 < 2 ? 0 : g0 - 2, q1 = g1 + 2 < k.gnx ? g1 + 2 : k.gnx;
   const int ncol = q1 - q0, nrow = s1 - s0 + 1;  // cell starts per column, with the end of the last
@@ -1573,6 +1577,10 @@ __device__ __attribute__((noinline)) void interact_rest(const inst_args *ap, int
     const int first = offsets[c * k.gny + r0], count = offsets[c * k.gny + r1] - first;
     if (i < 0 && n < count) i = first + n;
     if (n != 0x7fffffff) n -= count;
+  }
+  if (g0 >= k.gnx) {  // the particles past the grid: blanked ones, which have no sums
+    const int first = offsets[k.num_cell];
+    if (n < k.N - first) i = first + n;
   }
   const bool live = i >= 0;
   pair_acc acc = {};

@@ -9,7 +9,8 @@ namespace mfc {
 constexpr int REC_DOUBLES = 16;  // doubles per FP64 neighbour record
 
 // patches of the grid: patch p holds the cell rows [r patch_s, (r + 1) patch_s) and the columns
-// [c patch_w, (c + 1) patch_w) with p = c patch_rows + r
+// [c patch_w, (c + 1) patch_w) with p = c patch_rows + r; the number of them is also the patch of the
+// particles sorted past the grid's cells (an adaptive grid's blanked ones)
 template <class K>  // dev_consts or kconst
 __device__ inline int patch_rows(K &k) { return (k.gny + k.patch_s - 1) / k.patch_s; }
 template <class K>

@@ -4,7 +4,8 @@ import numpy as np
 import pytest
 
 import pymfc
-from parity import equal
+import oracle_binding as ob
+from parity import assert_bitwise, equal
 
 pytestmark = pytest.mark.gpu
 
@@ -41,3 +42,33 @@ def test_fp32c_blanked_particles_stay_excluded(component, value):
     for g in runs[1:]:
         for f in FIELDS:
             assert equal(runs[0].field(f), g.field(f)), f
+
+
+@pytest.mark.parametrize("many", [False, True])
+@pytest.mark.parametrize("lanes", [1, 4, 8])
+def test_adaptive_grid_shrinks_below_a_blanked_particle(lanes, many):
+    """Blanked particles keep their cell ids, which lie past the cells of an adaptive grid once the
+    bodies have come closer: they are sorted last and carried along as all others are (one, with the
+    neighbours it takes along, or enough for several parts of a work-group)."""
+    gs = [pymfc.Sim(pymfc.config_impact(20, p)) for p in (pymfc.PREC_FP64, pymfc.PREC_FP32C)]
+    o = ob.OracleSim(pymfc.config_impact(20))
+    for s in gs:
+        s.set_tuning(lanes=lanes)
+    for s in [o] + gs:
+        s.step(2)
+        free = np.nonzero(s.field("flags") == 0)[0]
+        last = free[np.argsort(s.field("hash")[free], kind="stable")[-100 if many else -1:]]
+        vt = s.field("vel_t")
+        vt[last, 0] = np.nan
+        s.set_field("vel_t", vt)
+    for _ in range(9):
+        for s in [o] + gs:
+            s.step(5)
+            assert np.array_equal(np.sort(s.field("id")), np.arange(s.N))
+        assert_bitwise(gs[0], o, context="grid shrinks")
+        assert equal(gs[0].cells(), o.cells())
+        assert (gs[1].info.grid_nx, gs[1].info.grid_ny) == (o.info.grid_nx, o.info.grid_ny)
+    for s in gs:
+        past = s.field("hash") >= s.info.num_cell
+        assert past.sum() > (40 if many else 4)
+        assert np.all(s.field("flags")[past] & pymfc.FLAG_BLANKED)
