@@ -556,15 +556,21 @@ int mfc_set_tuning(mfc_sim *s, const mfc_tuning *t) {
   s->k.sort_fast = t->sort_fast;
   s->k.sort_list = t->sort_list;
   const int lanes = t->lanes ? t->lanes : interaction_lanes(&s, 1);
-  if (lanes != s->lanes) {
+  const bool reshaped = lanes != s->lanes;
+  if (reshaped) {
     std::vector<int2> patches;
     set_patches(s, lanes);
     patch_items(patches, &s, 1);
     HIP_TRY(hipMemcpy(s->dpatches, patches.data(), sizeof(int2) * patches.size(), hipMemcpyHostToDevice));
     s->npatches = (int)patches.size();
-    s->keys_fresh = false;  // the patches' counts are those of the old shape
   }
   if ((rc = upload_descriptors(s))) return rc;
+  if (reshaped && s->keys_fresh) {  // the counts are those of the old shape (binning the state again
+                                    // would count its particles outside the grid twice)
+    HIP_TRY(hipMemsetAsync(s->bins.pcnt, 0, sizeof(int) * (size_t)s->npatch_max, s->stream));
+    mfc::launch_batch_patch_counts(s->work(s->cur), s->stream);
+    HIP_TRY(hipGetLastError());
+  }
   for (int p = 0; p < 2; p++)
     if (s->graph[p]) {
       (void)hipGraphExecDestroy(s->graph[p]);

@@ -197,12 +197,10 @@ int mfc_batch_set_tuning(mfc_batch *b, const mfc_tuning *t) {
   b->tuning = *t;
   const size_t n = b->sims.size();
   const int lanes = t->lanes ? t->lanes : b->auto_lanes();
-  if (lanes != b->lanes) {
+  const bool reshaped = lanes != b->lanes;
+  if (reshaped) {
     std::vector<int2> patches;
-    for (mfc_sim *s : b->sims) {
-      set_patches(s, lanes);
-      s->keys_fresh = false;  // the patches' counts are those of the old shape
-    }
+    for (mfc_sim *s : b->sims) set_patches(s, lanes);
     patch_items(patches, b->sims.data(), (int)n);
     HIP_TRY(hipMemcpy(b->patches, patches.data(), sizeof(int2) * patches.size(), hipMemcpyHostToDevice));
     b->npatches = (int)patches.size();
@@ -220,6 +218,12 @@ int mfc_batch_set_tuning(mfc_batch *b, const mfc_tuning *t) {
   }
   HIP_TRY(hipMemcpy(b->args[0], a0.data(), sizeof(mfc::inst_args) * n, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(b->args[1], a1.data(), sizeof(mfc::inst_args) * n, hipMemcpyHostToDevice));
+  if (reshaped) {  // the patches' counts are those of the old shape (batch_keys clears them where it bins)
+    for (mfc_sim *s : b->sims)
+      HIP_TRY(hipMemsetAsync(s->bins.pcnt, 0, sizeof(int) * (size_t)s->npatch_max, b->stream));
+    mfc::launch_batch_patch_counts(b->work(b->cur), b->stream);
+    HIP_TRY(hipGetLastError());
+  }
   b->drop_graphs();
   return MFC_OK;
 }

@@ -156,9 +156,11 @@ struct batch_work {
 // one step of every instance of a batch: 2 launches, and its phases. The
 // cell ids, chunk lists, chunk sums and neighbour records of a step's start state are computed by
 // the previous step's interaction; launch_batch_hash and launch_batch_records compute them from
-// the state itself (chunk sums zeroed before)
+// the state itself (chunk sums zeroed before); launch_batch_patch_counts counts its patches again
+// (counts zeroed before), for another number of lanes
 void launch_batch_step(const batch_work &w, hipStream_t s);
 void launch_batch_hash(const batch_work &w, hipStream_t s);
+void launch_batch_patch_counts(const batch_work &w, hipStream_t s);
 void launch_batch_binning(const batch_work &w, hipStream_t s);
 void launch_batch_records(const batch_work &w, hipStream_t s);
 // with events t0 and t1 the launch records the kernel's own start and end in them

@@ -1727,6 +1727,19 @@ __global__ __launch_bounds__(256) void kb_hash_count(const inst_args *__restrict
   hash_count(a.k, it.y * 256 + threadIdx.x, a.cur.px, a.cur.py, a.cur.flags, a.b);
 }
 
+// the patches' counts of the start state again, from its cell ids: for another shape of the patches
+// (an adaptive grid counts them in its geometry pass)
+__global__ __launch_bounds__(256) void kb_count_patches(const inst_args *__restrict__ A, const int2 *__restrict__ work,
+                                                        int nwork) {
+  const int w = xcd_tile(blockIdx.x, nwork);
+  if (w < 0) return;
+  const int2 it = work[w];
+  const inst_args &a = A[it.x];
+  if (a.k.adaptive) return;
+  const int i = it.y * 256 + threadIdx.x;
+  count_patch(i < a.k.N ? patch_of(a.k, a.b.key[i]) : -1, a.b.pcnt);
+}
+
 // Adaptive grid (grid_base::update_geometry, grid.cu:97-136), one work-group per instance: the
 // box of all positions (blanked particles included, as thrust::min_element / max_element over
 // the whole array) and the largest h give this step's geometry, which the work-group writes
@@ -1980,6 +1993,10 @@ int chunk_list_cap(int N) { return N < 4 * SCAN_CHUNK ? N : 4 * SCAN_CHUNK; }
 
 void launch_batch_hash(const batch_work &w, hipStream_t s) {
   hipLaunchKernelGGL(kb_hash_count, dim3(padded_tiles(w.ntiles)), dim3(256), 0, s, w.args, w.tiles, w.ntiles);
+}
+
+void launch_batch_patch_counts(const batch_work &w, hipStream_t s) {
+  hipLaunchKernelGGL(kb_count_patches, dim3(padded_tiles(w.ntiles)), dim3(256), 0, s, w.args, w.tiles, w.ntiles);
 }
 
 void launch_batch_binning(const batch_work &w, hipStream_t s) {
