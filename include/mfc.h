@@ -304,7 +304,11 @@ int mfc_write_tool_vtk(mfc_sim *sim, const char *path);
  * the steps [w0, w1) of the run (0 <= w0 < w1 <= nsteps).
  * mfc_vjp_backward: grad[j] = cot . dFmean/dtheta_j for the last mfc_vjp_forward; may be
  * called again with other cotangents; leaves the handle's state as mfc_vjp_forward left it.
- * Memory: about 290 B per particle per checkpoint plus checkpoint_every snapshots more.
+ * Memory: about 290 B per particle per checkpoint and about 400 B per particle for each of
+ * checkpoint_every steps. The secant results of the run, 8 B per particle and step, are kept as well
+ * (a pass is a fifth shorter with them) unless they take more than the rest or, all of a
+ * batch's together, more than a quarter of the memory that is free after it. All of it stays with
+ * the handle until a run of another checkpoint_every, or one of more checkpoints, or its end.
  * mfc_vjp: both calls for a cotangent known in advance. */
 typedef struct mfc_vjp_req {
   int nsteps;

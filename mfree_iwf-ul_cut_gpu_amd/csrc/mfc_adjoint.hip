@@ -602,7 +602,8 @@ struct adj_work {
   mfc_tool_state *tool = nullptr;
   return_tape *tape = nullptr;
   double *acc = nullptr;
-  double *returns = nullptr;            // secant results of the run's steps, N each, or null (keeps_returns)
+  double *returns = nullptr;            // secant results of the run's steps, N each, or null (adj_keep_returns)
+  bool returns_decided = false;
   size_t held = 0;                      // bytes of all the other allocations
   int uniform_h = 0;  // of the recorded run's states
   double h0 = 0.;
@@ -641,16 +642,6 @@ void adj_free(adj_work *w) { delete w; }
 
 namespace {
 
-// Whether a run's secant results are recorded for its replay: they take 8 bytes per particle and step, and
-// a tape that would be larger than the checkpoints and the slots of a segment (`held`), or than a
-// quarter of the memory that is free, isn't kept (the replay then iterates again). Runs of up to about
-// 9,000 steps with a checkpoint every sqrt(steps) keep one. It makes a pass 21 to 24 % shorter
-// (the figures stand at on_tape), whatever the length: the line is drawn by memory alone.
-bool keeps_returns(size_t bytes, size_t held) {
-  size_t avail = 0, total = 0;
-  return bytes <= held && hipMemGetInfo(&avail, &total) == hipSuccess && bytes <= avail / 4;
-}
-
 int setup_work(mfc_sim *s, int nsteps, int K, int w0, int w1) {
   const int N = s->k.N;
   adj_work *w = s->adj;
@@ -682,16 +673,6 @@ int setup_work(mfc_sim *s, int nsteps, int K, int w0, int w1) {
         (rc = w->alloc(&w->rec, REC_DOUBLES * n)) || (rc = w->alloc(&w->g_rec, REC_DOUBLES * n)) ||
         (rc = w->alloc(&w->theta_part, 6 * (size_t)s->ntiles)) || (rc = w->alloc(&w->theta_acc, 6)))
       return rc;
-    const size_t tape = (size_t)nck * k * n * sizeof(double);
-    if (keeps_returns(tape, w->held)) {
-      void *q = nullptr;
-      if (hipMalloc(&q, tape) == hipSuccess) {
-        w->allocs.push_back(q);
-        w->returns = (double *)q;
-      } else {
-        (void)hipGetLastError();  // none kept
-      }
-    }
     // the replay's force reduction keeps no history (cap 0) but counts steps
     HIP_TRY(hipMemsetAsync(w->ctr, 0, sizeof(int64_t), s->stream));
     HIP_TRY(hipMemsetAsync(w->pending, 0, 2 * sizeof(int), s->stream));
@@ -799,6 +780,36 @@ int adj_begin(mfc_sim *s, int nsteps, int checkpoint_every, int w0, int w1) {
   s->adj->uniform_h = s->k.uniform_h;
   s->adj->h0 = s->k.h0;
   return MFC_OK;
+}
+
+// Whether the runs' secant results are recorded for their replay: they take 8 bytes per particle and step,
+// and a tape that would be larger than its instance's checkpoints and slots of a segment (`held`) isn't kept,
+// nor are tapes of a group that together take more than a quarter of the memory that is free once every
+// instance has all it needs (the replay then iterates again). Runs of up to about 9,000 steps with a
+// checkpoint every sqrt(steps) keep one. It makes a pass 21 to 24 % shorter (the figures stand at
+// on_tape), whatever the length: the line is drawn by memory alone.
+void adj_keep_returns(mfc_sim *const *sims, int n) {
+  size_t avail = 0, total = 0;
+  if (hipMemGetInfo(&avail, &total) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
+  size_t left = avail / 4;
+  for (int i = 0; i < n; i++) {
+    adj_work *w = sims[i]->adj;
+    if (w->returns_decided) continue;
+    w->returns_decided = true;
+    const size_t tape = w->ckpt.size() * (size_t)w->K * w->N * sizeof(double);
+    void *q = nullptr;
+    if (tape > w->held || tape > left) continue;
+    if (hipMalloc(&q, tape) != hipSuccess) {
+      (void)hipGetLastError();  // none kept
+      continue;
+    }
+    w->allocs.push_back(q);
+    w->returns = (double *)q;
+    left -= tape;
+  }
 }
 
 int adj_segment(const mfc_sim *s) { return s->adj->K; }
@@ -970,7 +981,9 @@ int mfc_vjp_forward(mfc_sim *s, int nsteps, int checkpoint_every, int w0, int w1
   if (!s || !Fmean) return fail(MFC_E_INVALID, "null argument");
   if (s->batched) return fail(MFC_E_INVALID, "instance of a batch: use mfc_batch_vjp_forward");
   int rc = adj_begin(s, nsteps, checkpoint_every, w0, w1);
-  if (rc || (rc = ensure_keys(s))) return rc;
+  if (rc) return rc;
+  mfc::adj_keep_returns(&s, 1);
+  if ((rc = ensure_keys(s))) return rc;
   const int K = mfc::adj_segment(s);
   for (int t = 0; t < nsteps; t += K) {
     if ((rc = adj_checkpoint(s, t)) || (rc = queue_steps(s, nsteps - t < K ? nsteps - t : K))) return rc;

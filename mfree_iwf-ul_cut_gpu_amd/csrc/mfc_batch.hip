@@ -262,6 +262,7 @@ int mfc_batch_vjp_forward(mfc_batch *b, int nsteps, int checkpoint_every, int w0
   int rc;
   for (mfc_sim *s : b->sims)
     if ((rc = mfc::adj_begin(s, nsteps, checkpoint_every, w0, w1))) return rc;
+  mfc::adj_keep_returns(b->sims.data(), (int)b->sims.size());
   if ((rc = batch_keys(b))) return rc;
   for (int t = 0; t < nsteps; t++) {
     for (mfc_sim *s : b->sims)

@@ -35,6 +35,7 @@ void adj_free(adj_work *w);
 // taped forward in three parts, so that a batch can interleave its instances: validate and
 // allocate, keep the state at the start of step t when t is a checkpoint, and mean the window
 int adj_begin(mfc_sim *s, int nsteps, int checkpoint_every, int w0, int w1);
+void adj_keep_returns(mfc_sim *const *sims, int n);  // after adj_begin of every instance of the group
 int adj_checkpoint(mfc_sim *s, int t);
 int adj_segment(const mfc_sim *s);  // steps between its checkpoints
 int adj_finish(mfc_sim *s, double Fmean[2]);
