@@ -1418,7 +1418,9 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, unsigned *unread, co
     const int tag = tags[q - m.col_shift[c]], fl = tag & ((1 << TAG_BITS) - 1);
     m.tag[q] = tag;
     if constexpr (!patch_mem<F32, G>::ALL_IN_LDS) m.fl[q] = (unsigned char)fl;
-    if (fl & ~MFC_FLAG_FIXED) atomicOr(&m.flags, fl & ~MFC_FLAG_FIXED);
+    // a blanked particle enters no sum but those of PSE, so its record may hold anything
+    const int no = MFC_FLAG_FIXED | ((fl & MFC_FLAG_BLANKED) && !k.pse ? FLAG_NONFINITE : 0);
+    if (fl & ~no) atomicOr(&m.flags, fl & ~no);
   }
   __syncthreads();
   const int flags = m.flags;

@@ -72,3 +72,23 @@ def test_adaptive_grid_shrinks_below_a_blanked_particle(lanes, many):
         past = s.field("hash") >= s.info.num_cell
         assert past.sum() > (40 if many else 4)
         assert np.all(s.field("flags")[past] & pymfc.FLAG_BLANKED)
+
+
+@pytest.mark.parametrize("lanes", [1, 4, 8])
+@pytest.mark.parametrize("thermal", ["adiabatic", "contact", "pse"])
+def test_blanked_particles_in_a_patch(lanes, thermal):
+    """Particles blanked with positions and stresses that are not finite, in the patches of others:
+    without PSE they stay in the patch's copy, with PSE they enter the heat sums of all that see them."""
+    cfg = pymfc.cut_config(61, 17, 10.0, thermal=thermal, speed_m_min=1000.0, jitter=0.01)
+    g, o = pymfc.Sim(cfg), ob.OracleSim(cfg)
+    g.set_tuning(lanes=lanes)
+    for s in (g, o):
+        s.step(10)
+        free = np.nonzero(s.field("flags") == 0)[0]
+        vt = s.field("vel_t")
+        vt[free[free.size // 2], 1] = np.nan
+        vt[free[free.size // 5], 0] = np.inf
+        s.set_field("vel_t", vt)
+        s.step(8)
+    assert len(blanked_ids(o)) >= 2
+    assert_bitwise(g, o, context=thermal)
