@@ -254,7 +254,8 @@ __device__ inline double secant(double dl, double tol, const F &residual) {
     dl = dl - g / slope;
     const bool fold = dl < 0.;
     if (fold) dl = -0.1 * dl;
-    if (fabs(dl - dl_old) < tol || iter > 100) return fold ? -dl : dl;
+    // (every iterate after one that is not a number is none either)
+    if (fabs(dl - dl_old) < tol || iter > 100 || dl != dl) return fold ? -dl : dl;
     iter++;
   }
 }

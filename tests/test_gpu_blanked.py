@@ -1,5 +1,7 @@
 """Blanked particles in every path of the interaction: they stay where they were blanked, with whatever
 position made them so, and no mechanical sum takes them."""
+import time
+
 import numpy as np
 import pytest
 
@@ -92,3 +94,33 @@ def test_blanked_particles_in_a_patch(lanes, thermal):
         s.step(8)
     assert len(blanked_ids(o)) >= 2
     assert_bitwise(g, o, context=thermal)
+
+
+def step_time(s, n=64):
+    s.step(32)
+    best = np.inf
+    for _ in range(5):
+        s.sync()
+        t = time.perf_counter()
+        s.step(n)
+        s.sync()
+        best = min(best, time.perf_counter() - t)
+    return best
+
+
+@pytest.mark.parametrize("lanes", [1, 8])
+def test_blanked_particles_cost_no_time(lanes):
+    """A blanked particle is in no pair and has no return: the same steps with some take as long as
+    without (1.5 times as long at most, where a patch off its fast path or a return that iterates
+    on what is not a number makes them three to seven times as long)."""
+    cfg = pymfc.cut_config(150, 40, 10.0, jitter=0.01, seed=1)
+    sims = [pymfc.Sim(cfg), pymfc.Sim(cfg)]
+    for s in sims:
+        s.set_tuning(lanes=lanes)
+        s.step(2)
+    vt, free = sims[1].field("vel_t"), np.nonzero(sims[1].field("flags") == 0)[0]
+    vt[free[free.size // 2], 0] = np.nan
+    sims[1].set_field("vel_t", vt)
+    times = [step_time(s) for s in sims]
+    assert blanked_ids(sims[1]) and not blanked_ids(sims[0])
+    assert times[1] < 1.5 * times[0], times
