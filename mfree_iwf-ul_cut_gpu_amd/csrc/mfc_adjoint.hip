@@ -844,7 +844,7 @@ int adj_finish(mfc_sim *s, double Fmean[2]) {
   return MFC_OK;
 }
 
-int adj_backward(mfc_sim *const *sims, int n, const batch_work &fw, hipStream_t st, const double *cot, double *grad) {
+int adj_backward(mfc_sim *const *sims, int n, const batch_work &handle_work, hipStream_t st, const double *cot, double *grad) {
   if (n < 1) return fail(MFC_E_INVALID, "empty group");
   const adj_work *w0 = sims[0]->adj;
   for (int i = 0; i < n; i++) {
@@ -856,6 +856,8 @@ int adj_backward(mfc_sim *const *sims, int n, const batch_work &fw, hipStream_t 
   int rc = setup_group(sims, n, st);
   if (rc) return rc;
   adj_group &g = *w0->group;
+  batch_work fw = handle_work;
+  for (int i = 0; i < n; i++) fw.general = fw.general || !sims[i]->adj->uniform_h;  // of the recorded states
   const int nsteps = w0->nsteps, K = w0->K, nseg = (nsteps + K - 1) / K;
   const int slots = K < nsteps ? K : nsteps;
   // the descriptors: a replay step each (inst_args, the step kernels' view of a slot), the reverse

@@ -125,7 +125,7 @@ namespace {
 // not fit goes the slower way: with the lines rounded to the nearest whole number, at hdx 1.7
 // a window of the largest patches did not, and a step of 250k particles took 177 us instead of 143)
 void patch_shape(double hdx, bool f32, int lanes, int &s, int &w) {
-  const int most = mfc::TILE / lanes, cap = mfc::patch_cap(f32, lanes);
+  const int most = mfc::TILE / lanes, cap = mfc::patch_cap(f32, lanes, mfc::dense_cells(hdx, f32, lanes));
   auto lines = [&](int cells, double more) { return (int)(cells * hdx + more); };
   auto fits = [&](int a, int b) {
     const double more = lanes == 1 ? 1. : 0.5;
@@ -359,9 +359,22 @@ int copy_out(mfc_sim *s, void *dst, const void *src, size_t bytes) {
 
 }  // namespace
 
+void mfc_sim::drop_graphs() {
+  for (hipGraphExec_t &g : graph)
+    if (g) {
+      (void)hipGraphExecDestroy(g);
+      g = nullptr;
+    }
+}
+
 int queue_steps(mfc_sim *s, int nsteps) {
   int rc;
   int done = 0;
+  if (s->graph_general != s->general()) {
+    HIP_TRY(hipStreamSynchronize(s->stream));
+    s->drop_graphs();
+    s->graph_general = s->general();
+  }
   if (s->use_graphs && nsteps >= GRAPH_STEPS) {
     while (nsteps - done >= GRAPH_STEPS) {
       int par = s->cur;
@@ -406,8 +419,7 @@ int mfc_config_impact(mfc_config *cfg, int nbox) {
 void mfc_destroy(mfc_sim *s) {
   if (!s) return;
   if (s->stream) (void)hipStreamSynchronize(s->stream);
-  for (int p = 0; p < 2; p++)
-    if (s->graph[p]) (void)hipGraphExecDestroy(s->graph[p]);
+  s->drop_graphs();
   mfc::adj_free(s->adj);
   for (void *q : s->allocs) (void)hipFree(q);
   if (s->stream) (void)hipStreamDestroy(s->stream);
@@ -571,11 +583,7 @@ int mfc_set_tuning(mfc_sim *s, const mfc_tuning *t) {
     mfc::launch_batch_patch_counts(s->work(s->cur), s->stream);
     HIP_TRY(hipGetLastError());
   }
-  for (int p = 0; p < 2; p++)
-    if (s->graph[p]) {
-      (void)hipGraphExecDestroy(s->graph[p]);
-      s->graph[p] = nullptr;
-    }
+  s->drop_graphs();
   return MFC_OK;
 }
 

@@ -30,9 +30,15 @@ struct mfc_batch {
   bool adaptive = false;  // some instance has an adaptive grid
   bool pse = false;       // some instance conducts heat by PSE
   bool rothlin = false;   // some instance uses grid_gpu_rothlin's ranges
+  bool general() const {  // some instance needs the general variant of the interaction
+    for (const mfc_sim *s : sims)
+      if (s->general()) return true;
+    return false;
+  }
+  bool graph_general = false;  // of the variant the graphs were captured with
   mfc::batch_work work(int parity) const {
     return {args[parity], (int)sims.size(), tiles, ntiles, chunks, nchunks, patches, npatches, f32,
-            {lanes, tuning.xcd_chunk ? tuning.xcd_chunk : mfc::XCD_CHUNK}, adaptive, pse, rothlin};
+            {lanes, tuning.xcd_chunk ? tuning.xcd_chunk : mfc::XCD_CHUNK}, adaptive, pse, general(), rothlin};
   }
   void drop_graphs() {
     for (int p = 0; p < 2; p++)
@@ -233,6 +239,11 @@ int mfc_batch_step(mfc_batch *b, int nsteps) {
   int rc = batch_keys(b);
   if (rc) return rc;
   int done = 0;
+  if (b->graph_general != b->general()) {
+    HIP_TRY(hipStreamSynchronize(b->stream));
+    b->drop_graphs();
+    b->graph_general = b->general();
+  }
   if (nsteps >= GRAPH_STEPS) {
     while (nsteps - done >= GRAPH_STEPS) {
       const int par = b->cur;

@@ -68,13 +68,17 @@ constexpr int REC32_PIECES = 4;  // float4 per FP32C record
 // The interaction runs over patches: rectangles of cells whose particles one work-group of TILE
 // threads takes, `lanes` threads per particle. The records of every window candidate of a patch
 // (its cells and two more on each side) are staged in LDS: up to patch_cap of them; a patch with
-// more candidates (or of a state whose h is not uniform) reads them from memory. The FP64 kernel with
+// more candidates reads them from memory. The FP64 kernel with
 // one thread per particle gets three work-groups to a CU only up to 53,760 bytes (LDS is given out
 // in pieces of 1,280): with 484 candidates, 54,256 bytes, there were two, and a step of 197k particles
 // took 109 us instead of 102, of 500k with PSE 350 instead of 299.
 constexpr int PATCH_TABLE = 256;  // cell starts a patch holds in LDS: (patch_w + 4) (patch_s + 5) at most
 constexpr int PATCH_COLS = 24;    // patch_w + 4 at most
-__host__ __device__ constexpr int patch_cap(bool f32, int lanes) { return lanes > 1 ? 256 : f32 ? 512 : 479; }
+// The general variant (gen) copies less of each (of 128 bytes 64, of 64 32, with several threads per
+// particle 16 of both, and the tag), so that as many work-groups run at once.
+__host__ __device__ constexpr int patch_cap(bool f32, int lanes, bool gen) {
+  return gen ? (lanes > 1 ? 1408 : f32 ? 1080 : 760) : lanes > 1 ? 256 : f32 ? 512 : 479;
+}
 
 // tool-force reduction: the interaction flags the groups of 64 particles (storage order) in which
 // some contact or friction force is not zero; the next step's sort launch sums those groups from
@@ -150,6 +154,7 @@ struct batch_work {
   variant v;
   bool adaptive;          // some instance has an adaptive grid (a geometry pass starts the step)
   bool pse;               // some instance conducts heat by PSE
+  bool general;           // some instance needs the general variant of the interaction
   bool rothlin;           // some instance uses grid_gpu_rothlin's cell ranges (a pass after the sort)
 };
 

@@ -542,11 +542,17 @@ using rec_t = std::conditional_t<F32, rec32, rec64>;
 // record is staged; else one of the two (X) is there and c or T, whichever the sums read less, in
 // memory. (With the c of each pair gathered from memory, through a pointer that could be to either memory,
 // and full quotients and roots in the pair's terms the interaction of 197k particles took 116 us, now 104.)
-template <bool F32, int G>
+//
+// GEN: the variant of the kernel for states that do not suit that copy (mfc_sim::general): an h of its
+// own for each particle, or so many particles per cell that few cells' windows fit. Only some pieces
+// of a record are staged, and the others are read from memory for each pair (with positions and tags alone
+// staged, a step of 197k particles took 287 us at hdx 2.3 instead of 222, 141 instead of 116 with an uneven h, FP64;
+// with whole records and the h's for two work-groups to a CU 257 and 115).
+template <bool F32, int G, bool GEN>
 struct patch_mem {
-  static constexpr int CAP = patch_cap(F32, G);
-  static constexpr bool ALL_IN_LDS = F32 || G > 1;
-  static constexpr int PIECES = F32 ? 4 : ALL_IN_LDS ? 7 : 6;
+  static constexpr int CAP = patch_cap(F32, G, GEN);
+  static constexpr bool ALL_IN_LDS = F32 || G > 1 || GEN;
+  static constexpr int PIECES = GEN ? (G > 1 ? 1 : F32 ? 2 : 4) : F32 ? 4 : ALL_IN_LDS ? 7 : 6;
   // the terms of one pair per thread, exchanged between the threads of a particle: FP32C all nine,
   // FP64 in two halves (an odd stride keeps the rows on different banks)
   static constexpr int TERM_BYTES = G == 1 ? 0 : TILE * (F32 ? 9 * (int)sizeof(float) : 7 * (int)sizeof(double));
@@ -554,28 +560,48 @@ struct patch_mem {
   double X[ALL_IN_LDS ? 1 : CAP];
   int tag[CAP];            // or, without ALL_IN_LDS and promote, c
   unsigned char fl[ALL_IN_LDS ? 1 : CAP];  // the flags of the tag
-  int flags;               // of all the candidates, and PATCH_DENSE
+  int flags;               // of all the candidates, PATCH_DENSE, PATCH_DENSER and PATCH_HEAPED
   int table[PATCH_TABLE];  // LDS index of the first candidate of each cell (row-major in a column)
   int col_first[PATCH_COLS + 1];  // of each staged column
   int col_shift[PATCH_COLS];      // LDS index minus sorted index in each staged column
   int own_first[PATCH_COLS + 1];  // number of the first particle of each own column
-  unsigned char list[G == 1 ? 1 : TILE / G][64];  // the pairs of a particle, as LDS indices
+  using place = std::conditional_t<GEN, unsigned short, unsigned char>;  // holds an LDS index
+  place list[G == 1 ? 1 : TILE / G][64];  // the pairs of a particle
   alignas(16) char terms[TERM_BYTES ? TERM_BYTES : 16];
   return_tape tape;  // G > 1
 };
 
-// a column range of some window of the patch holds more candidates than a mask of sums_lds has bits
-constexpr int PATCH_DENSE = 16;
+// a column range of some window of the patch holds more candidates than a mask of sums_lds (G == 1) has
+// bits, than two of them have, or than five (without GEN: than one)
+constexpr int PATCH_DENSE = 16, PATCH_DENSER = 32, PATCH_HEAPED = 64;
 
 // where a sum reads the window candidates from: a patch's copy in LDS (index: place in the copy)
-template <bool F32, int G>
+template <bool F32, int G, bool GEN>
 struct lds_source {
-  using mem = patch_mem<F32, G>;
+  using mem = patch_mem<F32, G, GEN>;
   const mem *m;
-  const __attribute__((address_space(1))) double *rec;  // a global pointer: no load of either memory
+  template <class T>
+  using global = const __attribute__((address_space(1))) T *;  // no load of either memory
+  global<double> rec;
+  using float4v = float __attribute__((ext_vector_type(4)));
+  using double2v = double __attribute__((ext_vector_type(2)));
+  global<float4v> rec32;
+  global<double> h;  // the start state's
+  bool uniform_h;
   double h0;
   bool c_in_tag;  // mem::X holds T and mem::tag c
   bool t_in_lds;  // else mem::X holds T (some particle conducts heat), or c
+  // GEN: piece Q of a record (without that of its flags and h), from the copy or from storage index s
+  template <int Q>
+  __device__ inline float4v part32(int j, size_t s) const {
+    if constexpr (Q < mem::PIECES) return reinterpret_cast<const float4v *>(m->piece[Q])[j];
+    else return rec32[REC32_PIECES * s + Q];
+  }
+  template <int Q>
+  __device__ inline double2v part64(int j, size_t s) const {
+    if constexpr (Q < mem::PIECES) return reinterpret_cast<const double2v *>(m->piece[Q])[j];
+    else return ((global<double2v>)rec)[REC / 2 * s + Q + 1];
+  }
   __device__ inline double2 pos(int j) const { return reinterpret_cast<const double2 *>(m->piece[0])[j]; }
   __device__ inline int tag(int j) const {  // its flags
     if constexpr (mem::ALL_IN_LDS) return m->tag[j];
@@ -586,7 +612,14 @@ struct lds_source {
     t = tag(j);
   }
   __device__ inline void heat(int j, int t, rec_t<F32> &q) const {  // T and rho
-    if constexpr (F32) {
+    if constexpr (GEN) {
+      const size_t s = tag_index(t);
+      if constexpr (F32) {
+        q.rho = part32<1>(j, s).z; q.T = part32<3>(j, s).w;
+      } else {
+        q.rho = part64<2>(j, s).x; q.T = part64<6>(j, s).y;
+      }
+    } else if constexpr (F32) {
       q.rho = m->piece[1][j].z; q.T = m->piece[3][j].w;
     } else {
       q.rho = reinterpret_cast<const double2 *>(m->piece[2])[j].x;
@@ -596,7 +629,22 @@ struct lds_source {
     }
   }
   __device__ inline void record(int j, rec_t<F32> &q) const {
-    if constexpr (F32) {
+    if constexpr (GEN) {
+      const size_t s = tag_index(m->tag[j]);
+      if constexpr (F32) {
+        const float4v a = part32<1>(j, s), b = part32<2>(j, s), c = part32<3>(j, s);
+        q.u = a.x; q.v = a.y; q.rho = a.z; q.vol = a.w;
+        q.Axx = b.x; q.Axy = b.y; q.Ayy = b.z; q.c = b.w;
+        q.Rxx = c.x; q.Rxy = c.y; q.Ryy = c.z; q.T = c.w;
+        q.h = (float)(uniform_h ? h0 : h[s]);
+      } else {
+        const double2v a = part64<1>(j, s), b = part64<2>(j, s), c = part64<3>(j, s), d = part64<4>(j, s),
+                       e = part64<5>(j, s), f = part64<6>(j, s);
+        q.u = a.x; q.v = a.y; q.rho = b.x; q.vol = b.y;
+        q.Axx = c.x; q.Axy = c.y; q.Ayy = d.x; q.Rxx = d.y; q.Rxy = e.x; q.Ryy = e.y; q.c = f.x; q.T = f.y;
+        q.h = uniform_h ? h0 : rec[REC * s + 3];
+      }
+    } else if constexpr (F32) {
       const float4 a = m->piece[1][j], b = m->piece[2][j], c = m->piece[3][j];
       q.u = a.x; q.v = a.y; q.rho = a.z; q.vol = a.w;
       q.Axx = b.x; q.Axy = b.y; q.Ayy = b.z; q.c = b.w;
@@ -883,9 +931,11 @@ __device__ inline void sums_mem(kconst &k, const mem_source<F32> &src, const win
 // flags: what the patch's candidates have of TOOL and BLANKED (without PSE, the copy holds both
 // coordinates of a blanked particle at infinity, whatever they are: one that is not a number would
 // pass the test of near).
+// Where a column has more candidates than a mask has bits (GEN), two columns are taken at a time, each in two
+// masks, or one in five.
 constexpr int WALK_U = 4;  // candidates whose loads are issued together
-template <bool F32, int G, bool PSE>
-__device__ inline void sums_lds(kconst &k, const lds_source<F32, G> &src, int flags, const int b[5],
+template <bool F32, int G, bool PSE, bool GEN>
+__device__ inline void sums_lds(kconst &k, const lds_source<F32, G, GEN> &src, int flags, const int b[5],
                                 const int e[5], const rec_t<F32> &a, const sum_flags &f, pair_acc &acc, double &tpse) {
   const math_t<F32> mt(k, a, f);
   std::conditional_t<F32, sums32, pair_sums> sum = {};
@@ -910,50 +960,63 @@ __device__ inline void sums_lds(kconst &k, const lds_source<F32, G> &src, int fl
       }
     }
   }
-  unsigned m[5];
-  int at[5];
+  const bool dense = GEN && (flags & PATCH_DENSE), denser = GEN && (flags & PATCH_DENSER);
+  for (int pass = 0; pass < (denser ? 5 : dense ? 3 : 1); pass++) {
+    unsigned m[5];
+    int at[5];
 #pragma unroll
-  for (int r = 0; r < 5; r++) {
-    const int n = f.run_mech ? e[r] - b[r] : 0;
-    unsigned mr = 0u;
-    for (int q = 0; q < n; q += WALK_U) {
-      double2 p[WALK_U];
-#pragma unroll
-      for (int u = 0; u < WALK_U; u++) p[u] = src.pos(b[r] + q + u);  // past the range: some other entry of the copy
-      unsigned hits = 0u;
-#pragma unroll
-      for (int u = 0; u < WALK_U; u++) {
-        bool hit = q + u < n;
-        if (PSE && (flags & MFC_FLAG_BLANKED)) hit = hit && !(src.tag(b[r] + q + u) & MFC_FLAG_BLANKED);
-        const bool in = mt.near(p[u]);
-        hits |= (hit & in) ? 1u << u : 0u;
+    for (int r = 0; r < 5; r++) {
+      int first = b[r], n = e[r] - b[r];
+      if (denser) {
+        first = (pass == 0 ? b[0] : pass == 1 ? b[1] : pass == 2 ? b[2] : pass == 3 ? b[3] : b[4]) + 32 * r;
+        n = (pass == 0 ? e[0] : pass == 1 ? e[1] : pass == 2 ? e[2] : pass == 3 ? e[3] : e[4]) - first;
+      } else if (dense) {
+        first = (r < 2 ? (pass == 0 ? b[0] : pass == 1 ? b[2] : b[4]) : pass == 0 ? b[1] : b[3]) + (r & 1 ? 32 : 0);
+        n = (r < 2 ? (pass == 0 ? e[0] : pass == 1 ? e[2] : e[4]) : pass == 0 ? e[1] : e[3]) - first;
+        if (r == 4 || (pass == 2 && r >= 2)) n = 0;
       }
-      mr |= hits << q;
+      if (GEN) n = n < 32 ? n : 32;
+      if (!f.run_mech) n = 0;
+      unsigned mr = 0u;
+      for (int q = 0; q < n; q += WALK_U) {
+        double2 p[WALK_U];
+#pragma unroll
+        for (int u = 0; u < WALK_U; u++) p[u] = src.pos(first + q + u);  // past the range: some other entry of the copy
+        unsigned hits = 0u;
+#pragma unroll
+        for (int u = 0; u < WALK_U; u++) {
+          bool hit = q + u < n;
+          if (PSE && (flags & MFC_FLAG_BLANKED)) hit = hit && !(src.tag(first + q + u) & MFC_FLAG_BLANKED);
+          const bool in = mt.near(p[u]);
+          hits |= (hit & in) ? 1u << u : 0u;
+        }
+        mr |= hits << q;
+      }
+      m[r] = mr;
+      at[r] = first;
     }
-    m[r] = mr;
-    at[r] = b[r];
-  }
 #pragma unroll
-  for (int r = 3; r >= 0; r--)  // columns without a pair to the end
-    if (m[r] == 0u) {
+    for (int r = 3; r >= 0; r--)  // columns without a pair to the end
+      if (m[r] == 0u) {
 #pragma unroll
-      for (int q = r; q < 4; q++) { m[q] = m[q + 1]; at[q] = at[q + 1]; }
-      m[4] = 0u;
+        for (int q = r; q < 4; q++) { m[q] = m[q + 1]; at[q] = at[q + 1]; }
+        m[4] = 0u;
+      }
+    while (m[0]) {
+      const int j = at[0] + __builtin_ctz(m[0]);
+      m[0] &= m[0] - 1u;
+      const double2 p = src.pos(j);
+      rec_t<F32> c;
+      src.record(j, c);
+      bool tool_j = false;
+      if (flags & MFC_FLAG_TOOL) tool_j = src.tag(j) & MFC_FLAG_TOOL;  // the same branch in every lane
+      const bool used = m[0] == 0u;  // selects: under a branch every mask is moved twice
+#pragma unroll
+      for (int q = 0; q < 4; q++) { m[q] = used ? m[q + 1] : m[q]; at[q] = used ? at[q + 1] : at[q]; }
+      m[4] = used ? 0u : m[4];
+      if constexpr (F32) mt.pair(p, tool_j, c, sum);
+      else mt.template pair<true>(p, tool_j, c, sum);
     }
-  while (m[0]) {
-    const int j = at[0] + __builtin_ctz(m[0]);
-    m[0] &= m[0] - 1u;
-    const double2 p = src.pos(j);
-    rec_t<F32> c;
-    src.record(j, c);
-    bool tool_j = false;
-    if (flags & MFC_FLAG_TOOL) tool_j = src.tag(j) & MFC_FLAG_TOOL;  // the same branch in every lane
-    const bool used = m[0] == 0u;  // selects: under a branch every mask is moved twice
-#pragma unroll
-    for (int q = 0; q < 4; q++) { m[q] = used ? m[q + 1] : m[q]; at[q] = used ? at[q + 1] : at[q]; }
-    m[4] = used ? 0u : m[4];
-    if constexpr (F32) mt.pair(p, tool_j, c, sum);
-    else mt.template pair<true>(p, tool_j, c, sum);
   }
   if constexpr (F32) acc = acc_of(k, sum);
   else acc = sum;
@@ -972,9 +1035,9 @@ __device__ inline void wave_lds_fence() {
 // The threads test G candidates at a time and list the pairs in order; then each evaluates one
 // pair, and every sum belongs to one of them, which adds the G pairs' terms in order through LDS:
 // the order of every sum, and so its bits, are sums_lds's. The sums end in out[0..ACC_N) (LDS).
-template <bool F32, int G>
-__device__ inline void sums_group(kconst &k, const lds_source<F32, G> &src, const window &w,
-                                  const rec_t<F32> &a, const sum_flags &f, unsigned char *list, char *terms,
+template <bool F32, int G, bool GEN>
+__device__ inline void sums_group(kconst &k, const lds_source<F32, G, GEN> &src, const window &w,
+                                  const rec_t<F32> &a, const sum_flags &f, typename patch_mem<F32, G, GEN>::place *list, char *terms,
                                   double *out) {
   const math_t<F32> mt(k, a, f);
   const int lane = threadIdx.x & 63, r = lane % G, g0 = lane - r;
@@ -1010,7 +1073,7 @@ __device__ inline void sums_group(kconst &k, const lds_source<F32, G> &src, cons
       }
       const bool hit = f.run_mech && in && mt.support(p, tag);
       const unsigned bits = (unsigned)(__ballot(hit) >> g0) & ((1u << G) - 1u);
-      if (hit) list[cnt + __popc(bits & ((1u << r) - 1u))] = (unsigned char)j;
+      if (hit) list[cnt + __popc(bits & ((1u << r) - 1u))] = (typename patch_mem<F32, G, GEN>::place)j;
       cnt += __popc(bits);
     }
     wave_lds_fence();
@@ -1358,10 +1421,10 @@ __device__ inline void fetch_state(const dstate &src, size_t N, unsigned s, unsi
 // in LDS and a launch for the records, then this): FP32C 6k 55 -> 26, 27k 68 -> 35, 71k 63 -> 45,
 // 197k 80 -> 56, 500k PSE 276 -> 169; FP64 6k 63 -> 29, 27k 77 -> 46, 71k 93 -> 61, 197k 137 -> 102,
 // 500k PSE 403 -> 299.
-// returns false, with nothing done, for a patch whose window candidates do not fit the stage or
-// whose state has no uniform h, and for the particles past the grid (interact_rest takes them)
-template <bool F32, int G, bool PSE>
-__device__ inline bool interact_patch(patch_mem<F32, G> &m, unsigned *unread, const inst_args *A, int inst, int patch, int part) {
+// returns false, with nothing done, for a patch whose window candidates do not fit the stage or the masks
+// and for the particles past the grid (interact_rest takes them)
+template <bool F32, int G, bool PSE, bool GEN>
+__device__ inline bool interact_patch(patch_mem<F32, G, GEN> &m, unsigned *unread, const inst_args *A, int inst, int patch, int part) {
   const inst_args &a_ = A[inst];
   MFC_CONST(inst_args) *c_ = const_args(&a_, 0);
   kconst &k = c_->k;
@@ -1405,26 +1468,27 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, unsigned *unread, co
   }
   __syncthreads();
   const int ncand = m.col_first[ncol], nown = m.own_first[ncol];
-  constexpr int CAP = patch_mem<F32, G>::CAP;
+  using mem = patch_mem<F32, G, GEN>;
+  constexpr int CAP = mem::CAP;
   const int cap = k.stage_limit > 0 && k.stage_limit < CAP ? k.stage_limit : CAP;
-  if (ncand > cap || !k.uniform_h) return false;  // the same in every thread
-  if (tid < ncol * nrow) {
-    const int last = (te + 1) * nrow - 1;
-    if (m.table[tid + 5 < last ? tid + 5 : last] - m.table[tid] > 32) atomicOr(&m.flags, PATCH_DENSE);
+  if (ncand > cap || (!GEN && !k.uniform_h)) return false;  // the same in every thread
+  if (G == 1 && tid < ncol * nrow) {
+    const int last = (te + 1) * nrow - 1, n = m.table[tid + 5 < last ? tid + 5 : last] - m.table[tid];
+    if (n > 32) atomicOr(&m.flags, !GEN || n > 5 * 32 ? PATCH_HEAPED : n > 2 * 32 ? PATCH_DENSER : PATCH_DENSE);
   }
   for (int q = tid; q < ncand; q += TILE) {
     int c = 0;
     for (int e = 1; e < ncol; e++) c += q >= m.col_first[e];
     const int tag = tags[q - m.col_shift[c]], fl = tag & ((1 << TAG_BITS) - 1);
     m.tag[q] = tag;
-    if constexpr (!patch_mem<F32, G>::ALL_IN_LDS) m.fl[q] = (unsigned char)fl;
+    if constexpr (!mem::ALL_IN_LDS) m.fl[q] = (unsigned char)fl;
     // a blanked particle enters no sum but those of PSE, so its record may hold anything
     const int no = MFC_FLAG_FIXED | ((fl & MFC_FLAG_BLANKED) && !k.pse ? FLAG_NONFINITE : 0);
     if (fl & ~no) atomicOr(&m.flags, fl & ~no);
   }
   __syncthreads();
   const int flags = m.flags;
-  if (flags & (PATCH_DENSE | FLAG_NONFINITE)) return false;  // the same in every thread
+  if (flags & (PATCH_HEAPED | FLAG_NONFINITE)) return false;  // the same in every thread
   const bool t_in_lds = k.alpha_wp != 0. || k.alpha_tool != 0., c_in_tag = k.promote == 0;
   {
     return_tape tape = {nullptr, 0};
@@ -1434,7 +1498,14 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, unsigned *unread, co
     constexpr int LPR = F32 ? 4 : 8;  // lanes per record
     const int pl = tid % LPR;
     constexpr int STAGE_U = 4;
-    for (int q = tid / LPR; q < ncand; q += STAGE_U * (TILE / LPR)) {
+    if constexpr (GEN) {
+      constexpr int P = mem::PIECES;
+      const int p = tid % P;
+      for (int q = tid / P; q < ncand; q += TILE / P) {
+        const size_t s = tag_index(m.tag[q]);
+        m.piece[p][q] = F32 ? r.rec32[s * REC32_PIECES + p] : reinterpret_cast<const float4 *>(r.rec)[s * (REC / 2) + (p ? p + 1 : 0)];
+      }
+    } else for (int q = tid / LPR; q < ncand; q += STAGE_U * (TILE / LPR)) {
       float4 v[STAGE_U];
 #pragma unroll
       for (int u = 0; u < STAGE_U; u++) {
@@ -1448,13 +1519,13 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, unsigned *unread, co
         const int c = q + u * (TILE / LPR);
         if (c >= ncand) break;
         if (!PSE && (flags & MFC_FLAG_BLANKED) && pl == 0 &&
-            ((patch_mem<F32, G>::ALL_IN_LDS ? m.tag[c] : (int)m.fl[patch_mem<F32, G>::ALL_IN_LDS ? 0 : c]) & MFC_FLAG_BLANKED))
+            ((mem::ALL_IN_LDS ? m.tag[c] : (int)m.fl[mem::ALL_IN_LDS ? 0 : c]) & MFC_FLAG_BLANKED))
           reinterpret_cast<double2 &>(v[u]) = make_double2(__builtin_huge_val(), __builtin_huge_val());
         if constexpr (F32) {
           m.piece[pl][c] = v[u];
         } else if (pl != 1) {  // piece 1 of a record: flags (in the tag) and h (uniform)
           const int p = pl == 0 ? 0 : pl - 1;
-          if (patch_mem<F32, G>::ALL_IN_LDS || p < 6) m.piece[p][c] = v[u];
+          if (mem::ALL_IN_LDS || p < 6) m.piece[p][c] = v[u];
           else {
             const double2 ct = reinterpret_cast<const double2 &>(v[u]);
             m.X[c] = c_in_tag || t_in_lds ? ct.y : ct.x;
@@ -1483,7 +1554,7 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, unsigned *unread, co
     [[maybe_unused]] int i_mine = 0;
     unsigned s_mine = 0;  // loaded before the sums, which hide its latency
     // the exchange area of the wave; the sums of its particles end there too
-    constexpr int WAVE_BYTES = patch_mem<F32, G>::TERM_BYTES / (TILE / 64);
+    constexpr int WAVE_BYTES = mem::TERM_BYTES / (TILE / 64);
     static_assert(G == 1 || WAVE_BYTES >= 64 / G * ACC_N * (int)sizeof(double), "a wave's sums fit its exchange area");
     [[maybe_unused]] char *terms = m.terms + (size_t)(tid >> 6) * WAVE_BYTES;
     [[maybe_unused]] double *out = reinterpret_cast<double *>(terms) + (size_t)((tid & 63) / G) * ACC_N;
@@ -1504,7 +1575,9 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, unsigned *unread, co
       double2 p;
       int tag;
       rec_t<F32> a;
-      const lds_source<F32, G> lds = {&m, (const __attribute__((address_space(1))) double *)r.rec, k.h0, c_in_tag, t_in_lds};
+      using src = lds_source<F32, G, GEN>;
+      const src lds = {&m, (typename src::template global<double>)r.rec, (typename src::template global<typename src::float4v>)r.rec32,
+                       (typename src::template global<double>)(GEN ? load_state(&c_->cur).h : nullptr), k.uniform_h != 0, k.h0, c_in_tag, t_in_lds};
       lds.cand(li, p, tag);
       lds.record(li, a);
       a.x = p.x; a.y = p.y;
@@ -1517,11 +1590,11 @@ __device__ inline bool interact_patch(patch_mem<F32, G> &m, unsigned *unread, co
         if (!f.run_mech && !f.run_pse)
 #pragma unroll
           for (int q = 0; q < 5; q++) e[q] = b[q];
-        sums_lds<F32, G, PSE>(k, lds, flags, b, e, a, f, acc, tpse);
+        sums_lds<F32, G, PSE, GEN>(k, lds, flags, b, e, a, f, acc, tpse);
       } else {
         window w = make_window_at(k, gi, gj, at);
         if (!f.run_mech && !f.run_pse) w.total = 0;
-        sums_group<F32, G>(k, lds, w, a, f, m.list[tid / G], terms, out);
+        sums_group<F32, G, GEN>(k, lds, w, a, f, m.list[tid / G], terms, out);
       }
     }
     // fetch_state's words have arrived before the LDS is given back
@@ -1884,14 +1957,14 @@ __global__ __launch_bounds__(256) void kb_rothlin_cells(const inst_args *__restr
     for (int q = h + 1; q <= hn; q++) b.offsets_r[q] = i + 1;
 }
 
-template <bool F32, int G, bool PSE>
+template <bool F32, int G, bool PSE, bool GEN>
 __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(F32 ? 4 : 3))) void kb_interact(
     const inst_args *__restrict__ A, const int2 *__restrict__ work, int nwork, int chunk) {
   const int w = xcd_chunk_tile(blockIdx.x, nwork, chunk);
   if (w < 0) return;
   const int2 it = work[w];
   MFC_CONST(inst_args) *c = const_args(A, it.x);
-  __shared__ patch_mem<F32, G> m;
+  __shared__ patch_mem<F32, G, GEN> m;
   __shared__ unsigned unread[G > 1 ? 64 : 1];
   if (it.y == PATCH_ITEM_FORCE) {
     const dforce fo = load_force(&c->f);
@@ -1903,7 +1976,7 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(F32 ? 4 : 
   const int count = *c->b.plen, step = c->npatch_items;
   if (it.y >= count) return;
   const int2 p = c->b.plist[it.y];
-  if (!interact_patch<F32, G, PSE>(m, unread, A, it.x, p.x, p.y)) interact_rest<F32>(A + it.x, p.x, p.y);
+  if (!interact_patch<F32, G, PSE, GEN>(m, unread, A, it.x, p.x, p.y)) interact_rest<F32>(A + it.x, p.x, p.y);
   for (int q = it.y + step; q < count; q += step) interact_rest<F32>(A + it.x, c->b.plist[q].x, c->b.plist[q].y);
 }
 
@@ -2026,8 +2099,9 @@ static void launch_patches(K kern, const batch_work &w, hipStream_t s, hipEvent_
 }
 
 void launch_batch_interact(const batch_work &w, hipStream_t s, hipEvent_t t0, hipEvent_t t1) {
-#define MFC_PICK(lanes, pse) (w.f32 ? kb_interact<true, lanes, pse> : kb_interact<false, lanes, pse>)
-#define MFC_PICK_PSE(lanes) launch_patches(w.pse ? MFC_PICK(lanes, true) : MFC_PICK(lanes, false), w, s, t0, t1)
+#define MFC_PICK(lanes, pse, gen) (w.f32 ? kb_interact<true, lanes, pse, gen> : kb_interact<false, lanes, pse, gen>)
+#define MFC_PICK_PSE(lanes) launch_patches(w.general ? MFC_PICK(lanes, true, true) : \
+                                           w.pse ? MFC_PICK(lanes, true, false) : MFC_PICK(lanes, false, false), w, s, t0, t1)
   switch (w.v.lanes) {
     case 1: MFC_PICK_PSE(1); break;
     case 4: MFC_PICK_PSE(4); break;

@@ -1,6 +1,7 @@
 // mfc_sim.h — the simulation handle behind the C ABI (internal to the library).
 #pragma once
 
+#include <cmath>
 #include <memory>
 #include <mutex>
 #include <hip/hip_runtime.h>
@@ -71,6 +72,16 @@ struct read_stage {
   }
 };
 
+namespace mfc {
+// Whether the cells hold so many lattice points that a patch's copy of whole records does not do: with one
+// thread per particle where a column of a window (5 h by h) has more than 32 (from hdx 2.1 on),
+// with several where the window of a single cell has more than the copy (from 3.2 on)
+inline bool dense_cells(double hdx, bool f32, int lanes) {
+  const auto lines = [](double cells) { return std::ceil(cells - 1e-6); };
+  return lanes == 1 ? lines(5 * hdx) * lines(hdx) > 32 : lines(5 * hdx) * lines(5 * hdx) > patch_cap(f32, lanes, false);
+}
+}  // namespace mfc
+
 struct mfc_sim {
   mfc_config cfg;      // the configuration the handle was created from (checkpoints keep it)
   mfc::scenario sc;
@@ -98,6 +109,8 @@ struct mfc_sim {
   int cur = 0;                     // set holding the current state, and index of the current tool state
   int64_t step = 0;
   hipGraphExec_t graph[2] = {nullptr, nullptr};  // GRAPH_STEPS steps starting from parity 0 / 1
+  bool graph_general = false;                    // of the variant they were captured with
+  void drop_graphs();
   bool use_graphs = true;
   mfc::adj_work *adj = nullptr;    // reverse-mode tape of the last mfc_vjp_forward
   bool batched = false;            // instance of a batch: stepped by mfc_batch_step only
@@ -109,6 +122,15 @@ struct mfc_sim {
   double wear_accum = 0.;          // accumulated wear, sum of dt * mean rate (tool_wear.cu:59)
   mfc_tuning tuning = {};
   int lanes = 1;  // threads per particle of the interaction (set_patches)
+  // Whether its interaction takes the general variant of the kernel (patch_mem's GEN): for an h of its
+  // own for each particle, or for dense cells. us per step of 197k particles by tiles of the sorted
+  // order (what there was before the patches) / from the records in memory (interact_rest) / with this: FP64
+  // an uneven h 135 / 229 / 116, hdx 2.3 260 / 547 / 222, 3.0 372 / 955 / 287; FP32C 81 / 154 / 65, 138 / 325
+  // / 118, 188 / - / 148; hdx 3.5 536 / - / 569 and 267 / - / 281. Where whole records fit it costs: FP64
+  // an even h 102, FP32C 57.
+  bool general() const {
+    return !k.uniform_h || mfc::dense_cells(cfg.hdx, recs[0].f32, lanes);
+  }
   mfc::variant variant() const { return {lanes, tuning.xcd_chunk ? tuning.xcd_chunk : mfc::XCD_CHUNK}; }
   // the step runs the batched kernels on a batch of one: descriptors of this handle for start
   // parity 0 and 1, and its (instance, block) work tables
@@ -123,7 +145,7 @@ struct mfc_sim {
   mfc::grid_geo *geo = nullptr;    // adaptive grid: the geometry of the last step (device)
   mfc::batch_work work(int c) const {
     return {dargs + c, 1, dtiles, ntiles, dchunks, nchunks, dpatches, npatches, recs[0].f32, variant(),
-            k.adaptive != 0, k.pse != 0, k.rothlin != 0};
+            k.adaptive != 0, k.pse != 0, general(), k.rothlin != 0};
   }
 
   template <class T>

@@ -1,4 +1,6 @@
 """The number of threads per particle is a launch setting: changing it changes no result."""
+import time
+
 import numpy as np
 import pytest
 
@@ -30,3 +32,90 @@ def test_out_of_grid_count_does_not_depend_on_lanes(batch):
         for s in sims:
             assert s.info.out_of_grid == alone.info.out_of_grid > 0
             assert_bitwise(s, o, context=f"lanes {lanes}")
+
+
+def cut(prec=pymfc.PREC_FP64, hdx=1.5, nx=61, ny=17, thermal="contact", **kw):
+    cfg = pymfc.cut_config(nx, ny, 10.0, thermal=thermal, speed_m_min=1000.0, jitter=0.01, precision=prec, **kw)
+    cfg.hdx = hdx
+    return cfg
+
+
+def uneven(s):
+    h = s.field("h")
+    s.set_field("h", h * (1.0 - 0.05 * (s.field("id") % 3)))
+
+
+@pytest.mark.parametrize("thermal", ["contact", "pse"])
+@pytest.mark.parametrize("hdx", [1.0, 2.1, 2.8, 3.4, 6.0])
+@pytest.mark.parametrize("lanes", [1, 4, 8])
+def test_smoothing_lengths(lanes, hdx, thermal):
+    """From less than one to many lattice points per cell: windows whose columns hold up to 32, 64 and 160
+    candidates and more, and windows of more candidates than a patch's copy of whole records, or of
+    their parts, has room for; also with an h of its own for each particle."""
+    g, o = pymfc.Sim(cut(hdx=hdx, thermal=thermal)), ob.OracleSim(cut(hdx=hdx, thermal=thermal))
+    g.set_tuning(lanes=lanes)
+    for s in (g, o):
+        s.step(9)
+    assert_bitwise(g, o, context=f"hdx {hdx}")
+    for s in (g, o):
+        uneven(s)
+        s.step(9)
+    assert_bitwise(g, o, context=f"hdx {hdx}, uneven h")
+
+
+@pytest.mark.parametrize("hdx", [1.5, 2.3])
+def test_fp32c_bits_do_not_depend_on_lanes_or_stage(hdx):
+    runs = []
+    for lanes, limit in ((1, 0), (4, 0), (8, 0), (1, 1)):
+        g = pymfc.Sim(cut(pymfc.PREC_FP32C, hdx=hdx))
+        g.set_tuning(lanes=lanes, stage_limit=limit)
+        g.step(9)
+        uneven(g)
+        g.step(9)
+        runs.append(g)
+    for g in runs[1:]:
+        for f in ("pos", "vel", "S", "rho", "T", "fc", "ft", "id"):
+            assert equal(runs[0].field(f), g.field(f)), f
+
+
+@pytest.mark.parametrize("batch", [False, True])
+def test_kernel_follows_the_h_of_the_state(batch):
+    """h written between blocks of steps that replay captured graphs, to one of its own for each
+    particle and back, in a handle or in one instance of a batch."""
+    cfgs = [cut(), cut(hdx=2.3), cut(nx=41)] if batch else [cut()]
+    handle = pymfc.Batch(cfgs) if batch else pymfc.Sim(cfgs[0])
+    sims = list(handle.instances) if batch else [handle]
+    oracles = [ob.OracleSim(c) for c in cfgs]
+    h0 = sims[0].field("h")
+    for block in range(3):
+        for s in (handle, *oracles):
+            s.step(19)
+        for s, o in zip(sims, oracles):
+            assert_bitwise(s, o, context=f"block {block}")
+        for s in (sims[0], oracles[0]):
+            if block == 0:
+                uneven(s)
+            else:
+                s.set_field("h", h0)
+
+
+def step_time(s, n=64):
+    s.step(32)
+    best = np.inf
+    for _ in range(5):
+        s.sync()
+        t = time.perf_counter()
+        s.step(n)
+        s.sync()
+        best = min(best, time.perf_counter() - t)
+    return best
+
+
+@pytest.mark.parametrize("prec", [pymfc.PREC_FP64, pymfc.PREC_FP32C])
+def test_uneven_h_costs_little_time(prec):
+    """The same pairs and some loads more: 1.6 times as long at most (by themselves from the records in
+    memory, the pairs take 2.2 to 2.8 times as long)."""
+    sims = [pymfc.Sim(pymfc.cut_config(750, 200, 2.0, thermal="contact", jitter=0.01, precision=prec)) for _ in range(2)]
+    uneven(sims[1])
+    times = [step_time(s) for s in sims]
+    assert times[1] < 1.6 * times[0], times
