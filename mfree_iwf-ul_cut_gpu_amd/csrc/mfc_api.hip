@@ -125,7 +125,7 @@ namespace {
 // not fit goes the slower way: with the lines rounded to the nearest whole number, at hdx 1.7
 // a window of the largest patches did not, and a step of 250k particles took 177 us instead of 143)
 void patch_shape(double hdx, bool f32, int lanes, int &s, int &w) {
-  const int most = mfc::TILE / lanes, cap = mfc::patch_cap(f32, lanes, mfc::dense_cells(hdx, f32, lanes));
+  const int most = mfc::TILE / lanes, cap = mfc::patch_plan_cap(f32, lanes, mfc::dense_cells(hdx, f32, lanes));
   auto lines = [&](int cells, double more) { return (int)(cells * hdx + more); };
   auto fits = [&](int a, int b) {
     const double more = lanes == 1 ? 1. : 0.5;

@@ -77,7 +77,14 @@ constexpr int PATCH_COLS = 24;    // patch_w + 4 at most
 // The general variant (gen) copies less of each (of 128 bytes 64, of 64 32, with several threads per
 // particle 16 of both, and the tag), so that as many work-groups run at once.
 __host__ __device__ constexpr int patch_cap(bool f32, int lanes, bool gen) {
-  return gen ? (lanes > 1 ? 1408 : f32 ? 1080 : 760) : lanes > 1 ? 256 : f32 ? 512 : 479;
+  return gen ? (lanes > 1 ? 1408 : f32 ? 1080 : 760) : lanes > 1 ? 256 : f32 ? 576 : 479;
+}
+// What the patches of a full lattice may have of that: a body in compression has more particles in a
+// cell, and a few patches over the copy's room make the launch twice as long (in FP32C, planned up to
+// 512 of 512, steps of the impact of 131k particles went from 65 to 128 us behind the shock and of
+// the rings of 171k from 63 to 113, now 81 and 63)
+__host__ __device__ constexpr int patch_plan_cap(bool f32, int lanes, bool gen) {
+  return patch_cap(f32, lanes, gen) * 12 / 13;
 }
 
 // tool-force reduction: the interaction flags the groups of 64 particles (storage order) in which
