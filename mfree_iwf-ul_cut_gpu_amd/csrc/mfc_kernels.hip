@@ -676,19 +676,18 @@ struct lds_source {
   }
 };
 
-// or the records in memory through the tags (index: sorted index)
+// or the records in memory, their tags and positions there too (index: sorted index) or from a copy of
+// them alone in LDS (index: place in the copy)
 template <bool F32>
-struct mem_source {
-  const drecords &r;
-  const int *tags;
+struct mem_records {
+  const drecords r;
   const double *h;  // the start state's
-  __device__ inline void cand(int j, double2 &p, int &tag) const {
-    tag = tags[j];
-    const unsigned s = tag_index(tag);
-    if constexpr (F32) p = *reinterpret_cast<const double2 *>(r.rec32 + (size_t)REC32_PIECES * s);
-    else p = *reinterpret_cast<const double2 *>(r.rec + (size_t)REC * s);
+  __device__ inline double2 pos_of(int tag) const {
+    const size_t s = tag_index(tag);
+    if constexpr (F32) return *reinterpret_cast<const double2 *>(r.rec32 + REC32_PIECES * s);
+    else return *reinterpret_cast<const double2 *>(r.rec + REC * s);
   }
-  __device__ inline void heat(int j, int tag, rec_t<F32> &q) const {
+  __device__ inline void heat(int tag, rec_t<F32> &q) const {
     if constexpr (F32) {
       const float4 *d = r.rec32 + (size_t)REC32_PIECES * tag_index(tag);
       q.rho = d[1].z; q.T = d[3].w;
@@ -697,7 +696,7 @@ struct mem_source {
       q.rho = d[6]; q.T = d[15];
     }
   }
-  __device__ inline void record(int j, int tag, rec_t<F32> &q) const {
+  __device__ inline void record(int tag, rec_t<F32> &q) const {
     if constexpr (F32) {
       const float4 *d = r.rec32 + (size_t)REC32_PIECES * tag_index(tag);
       const float4 a = d[1], b = d[2], c = d[3];
@@ -710,6 +709,35 @@ struct mem_source {
       q.h = d[3]; q.u = d[4]; q.v = d[5]; q.rho = d[6]; q.vol = d[7];
       q.Axx = d[8]; q.Axy = d[9]; q.Ayy = d[10]; q.Rxx = d[11]; q.Rxy = d[12]; q.Ryy = d[13];
       q.c = d[14]; q.T = d[15];
+    }
+  }
+};
+template <bool F32>
+struct mem_source : mem_records<F32> {
+  const int *tags;
+  template <int U>
+  __device__ inline void cands(const int (&j)[U], double2 (&p)[U], int (&tag)[U]) const {
+#pragma unroll
+    for (int u = 0; u < U; u++) tag[u] = tags[j[u]];
+#pragma unroll
+    for (int u = 0; u < U; u++) p[u] = this->pos_of(tag[u]);
+  }
+};
+template <class T>
+using lds_ptr = __attribute__((address_space(3))) T *;
+struct lds_pos {
+  double x, y;
+};
+template <bool F32>
+struct copy_source : mem_records<F32> {
+  lds_ptr<lds_pos> pos;
+  lds_ptr<int> tags;
+  template <int U>
+  __device__ inline void cands(const int (&j)[U], double2 (&p)[U], int (&tag)[U]) const {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      tag[u] = tags[j[u]];
+      p[u] = make_double2(pos[j[u]].x, pos[j[u]].y);
     }
   }
 };
@@ -893,28 +921,46 @@ __device__ inline double value_of(const kahan &s) { return s.value(); }
 __device__ inline double value_of(double s) { return s; }
 
 // The neighbour sums of a particle by one thread from the records in memory: the window's
-// candidates in order, which is the reference's (interactions_gpu.cu:219-331)
-template <bool F32>
-__device__ inline void sums_mem(kconst &k, const mem_source<F32> &src, const window &w, const rec_t<F32> &a,
-                                const sum_flags &f, pair_acc &acc, double &tpse) {
+// candidates in order, which is the reference's (interactions_gpu.cu:219-331), 64 at a time: first the
+// support tests, whose loads are issued together for WALK_U candidates, then the pairs
+constexpr int WALK_U = 4;  // candidates whose loads are issued together
+template <bool F32, bool FINITE, class SRC>
+__device__ inline void sums_mem(kconst &k, const SRC &src, const window &w, const rec_t<F32> &a, const sum_flags &f,
+                                pair_acc &acc, double &tpse) {
   const math_t<F32> mt(k, a, f);
   std::conditional_t<F32, sums32, pair_sums> sum = {};
   std::conditional_t<F32, kahan, double> tp = {};
-  for (int t = 0; t < w.total; t++) {
-    const int j = w.at(t);
-    double2 p;
-    int tag;
-    rec_t<F32> b;
-    src.cand(j, p, tag);
-    if (f.run_pse) {  // all members of the window
-      src.heat(j, tag, b);
-      if constexpr (F32) tp.add(mt.template pse<false>(p, b));
-      else tp += mt.template pse<false>(p, b);
+  for (int c0 = 0; c0 < w.total; c0 += 64) {
+    const int n = w.total - c0 < 64 ? w.total - c0 : 64;
+    unsigned long long mask = 0ull;
+    for (int q = 0; q < n; q += WALK_U) {
+      int j[WALK_U], tag[WALK_U];
+      double2 p[WALK_U];
+#pragma unroll
+      for (int u = 0; u < WALK_U; u++) j[u] = w.at(c0 + (q + u < n ? q + u : n - 1));
+      src.cands(j, p, tag);
+#pragma unroll
+      for (int u = 0; u < WALK_U; u++) {
+        if (q + u >= n) continue;
+        if (f.run_pse) {  // all members of the window
+          rec_t<F32> b;
+          src.heat(tag[u], b);
+          if constexpr (F32) tp.add(mt.template pse<FINITE>(p[u], b));
+          else tp += mt.template pse<FINITE>(p[u], b);
+        }
+        if (f.run_mech && mt.support(p[u], tag[u])) mask |= 1ull << (q + u);
+      }
     }
-    if (!f.run_mech || !mt.support(p, tag)) continue;
-    src.record(j, tag, b);
-    if constexpr (F32) mt.pair(p, (tag & MFC_FLAG_TOOL) != 0, b, sum);
-    else mt.template pair<false>(p, (tag & MFC_FLAG_TOOL) != 0, b, sum);
+    for (; mask; mask &= mask - 1ull) {
+      const int j[1] = {w.at(c0 + __builtin_ctzll(mask))};
+      double2 p[1];
+      int tag[1];
+      rec_t<F32> b;
+      src.cands(j, p, tag);
+      src.record(tag[0], b);
+      if constexpr (F32) mt.pair(p[0], (tag[0] & MFC_FLAG_TOOL) != 0, b, sum);
+      else mt.template pair<FINITE>(p[0], (tag[0] & MFC_FLAG_TOOL) != 0, b, sum);
+    }
   }
   if constexpr (F32) acc = acc_of(k, sum);
   else acc = sum;
@@ -933,7 +979,6 @@ __device__ inline void sums_mem(kconst &k, const mem_source<F32> &src, const win
 // pass the test of near).
 // Where a column has more candidates than a mask has bits (GEN), two columns are taken at a time, each in two
 // masks, or one in five.
-constexpr int WALK_U = 4;  // candidates whose loads are issued together
 template <bool F32, int G, bool PSE, bool GEN>
 __device__ inline void sums_lds(kconst &k, const lds_source<F32, G, GEN> &src, int flags, const int b[5],
                                 const int e[5], const rec_t<F32> &a, const sum_flags &f, pair_acc &acc, double &tpse) {
@@ -1635,44 +1680,91 @@ __device__ inline bool interact_patch(patch_mem<F32, G, GEN> &m, unsigned *unrea
 }
 
 // The patches that interact_patch leaves, and those past the end of the launch's work items: one
-// thread per particle over the records in memory. A call, so that this rare path takes no
-// registers from the kernel that holds it.
+// thread per particle over the records in memory, with the window's positions and tags copied to
+// LDS where they fit and all records are finite (`lds`, of `bytes`; 20 bytes each, four times as many as
+// whole records). A call, so that this rare path takes no registers from the kernel that holds it. A
+// launch waits for its last patch, so what counts is how long one takes. us per step with every patch sent
+// here: 6k particles FP64 58, 197k 216, FP32C 134 (one candidate after the other from memory,
+// with the pair terms for any value, 81, 234 and 158).
 template <bool F32>
-__device__ __attribute__((noinline)) void interact_rest(const inst_args *ap, int patch, int part) {
-  const inst_args &a_ = *ap;
-  kconst &k = const_args(ap, 0)->k;
-  const dbins &b = a_.b;
+__device__ __attribute__((noinline)) void interact_rest(const inst_args *ap, int patch, int part, lds_ptr<char> lds,
+                                                        int bytes) {
+  MFC_CONST(inst_args) *c_ = const_args(ap, 0);
+  kconst &k = c_->k;
+  const dbins b = load_bins(&c_->b);
   const int *offsets = k.rothlin ? b.offsets_r : b.offsets;
+  const int tid = threadIdx.x;
   const int nrb = patch_rows(k);
   const int pc = patch / nrb, pr = patch - pc * nrb;
   const int r0 = pr * k.patch_s, r1 = r0 + k.patch_s < k.gny ? r0 + k.patch_s : k.gny;
   const int g0 = pc * k.patch_w, g1 = g0 + k.patch_w < k.gnx ? g0 + k.patch_w : k.gnx;
-  int n = (int)threadIdx.x < k.patch_slots ? part * k.patch_slots + (int)threadIdx.x : 0x7fffffff, i = -1;
+  int n = tid < k.patch_slots ? part * k.patch_slots + tid : 0x7fffffff, i = -1;
   for (int c = g0; c < g1; c++) {
     const int first = offsets[c * k.gny + r0], count = offsets[c * k.gny + r1] - first;
     if (i < 0 && n < count) i = first + n;
     if (n != 0x7fffffff) n -= count;
   }
+  pair_acc acc = {};
+  double tpse = 0.;
   if (g0 >= k.gnx) {  // the particles past the grid: blanked ones, which have no sums
     const int first = offsets[k.num_cell];
     if (n < k.N - first) i = first + n;
+  } else {
+    const mem_records<F32> rec = {load_recs(&c_->r), load_state(&c_->cur).h};
+    // where each column of the windows starts in the copy, and its place minus its sorted index
+    const int s0 = r0 < 2 ? 0 : r0 - 2, s1 = r1 + 2 < k.gny ? r1 + 2 : k.gny;
+    const int q0 = g0 < 2 ? 0 : g0 - 2, ncol = (g1 + 2 < k.gnx ? g1 + 2 : k.gnx) - q0;
+    lds_ptr<int> first = (lds_ptr<int>)lds, shift = first + 32, nonfinite = first + 63;
+    constexpr int HEAD = 64 * sizeof(int);
+    const int cap = (bytes - HEAD) / (int)(sizeof(lds_pos) + sizeof(int));
+    lds_ptr<lds_pos> pos = (lds_ptr<lds_pos>)(lds + HEAD);
+    lds_ptr<int> tags = (lds_ptr<int>)(pos + cap);
+    __syncthreads();  // what was in the LDS before is no longer read
+    if (tid < 64) {
+      const int j0 = tid < ncol ? offsets[(q0 + tid) * k.gny + s0] : 0, c = tid < ncol ? offsets[(q0 + tid) * k.gny + s1] - j0 : 0;
+      int x = c;
+#pragma unroll
+      for (int s = 1; s < 32; s <<= 1) {
+        const int y = __shfl_up(x, s, 64);
+        if (tid >= s) x += y;
+      }
+      if (tid <= ncol) {
+        first[tid] = x - c;
+        shift[tid] = x - c - j0;
+      }
+      if (tid == 63) *nonfinite = 0;
+    }
+    __syncthreads();
+    const int ncand = first[ncol];
+    bool copied = ncand <= cap;  // the same in every thread
+    if (copied) {
+      for (int q = tid; q < ncand; q += TILE) {
+        int c = 0;
+        for (int e = 1; e < ncol; e++) c += q >= first[e];
+        const int tag = b.tags[q - shift[c]];
+        const double2 p = rec.pos_of(tag);
+        tags[q] = tag;
+        pos[q].x = p.x; pos[q].y = p.y;
+        if ((tag & FLAG_NONFINITE) && (k.pse || !(tag & MFC_FLAG_BLANKED))) *nonfinite = 1;
+      }
+      __syncthreads();
+      if (*nonfinite) copied = false;
+    }
+    if (i >= 0) {
+      const int tag = b.tags[i], key = b.key_sorted[i];
+      const double2 p = rec.pos_of(tag);
+      rec_t<F32> a;
+      rec.record(tag, a);
+      a.x = p.x; a.y = p.y;
+      const sum_flags f = flags_of(k, tag);
+      const int gi = key / k.gny, gj = key - gi * k.gny;
+      window w = make_window_at(k, gi, gj, [&](int col, int row) { return offsets[col * k.gny + row] + (copied ? shift[col - q0] : 0); });
+      if (!f.run_mech && !f.run_pse) w.total = 0;
+      if (copied) sums_mem<F32, true>(k, copy_source<F32>{rec, pos, tags}, w, a, f, acc, tpse);
+      else sums_mem<F32, false>(k, mem_source<F32>{rec, b.tags}, w, a, f, acc, tpse);
+    }
   }
   const bool live = i >= 0;
-  pair_acc acc = {};
-  double tpse = 0.;
-  if (live) {
-    const mem_source<F32> mem = {a_.r, b.tags, a_.cur.h};
-    double2 p;
-    int tag;
-    rec_t<F32> a;
-    mem.cand(i, p, tag);
-    mem.record(i, tag, a);
-    a.x = p.x; a.y = p.y;
-    const sum_flags f = flags_of(k, tag);
-    window w = make_window(k, offsets, b.key_sorted[i]);
-    if (!f.run_mech && !f.run_pse) w.total = 0;
-    sums_mem<F32>(k, mem, w, a, f, acc, tpse);
-  }
   finish_particle<F32>(ap, i, live ? tag_index(b.tags[i]) : 0u, live, acc, tpse);
 }
 
@@ -1969,8 +2061,10 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(F32 ? 4 : 
   const int count = *c->b.plen, step = c->npatch_items;
   if (it.y >= count) return;
   const int2 p = c->b.plist[it.y];
-  if (!interact_patch<F32, G, PSE, GEN>(m, unread, A, it.x, p.x, p.y)) interact_rest<F32>(A + it.x, p.x, p.y);
-  for (int q = it.y + step; q < count; q += step) interact_rest<F32>(A + it.x, c->b.plist[q].x, c->b.plist[q].y);
+  const lds_ptr<char> lds = (lds_ptr<char>)(char *)&m;
+  if (!interact_patch<F32, G, PSE, GEN>(m, unread, A, it.x, p.x, p.y)) interact_rest<F32>(A + it.x, p.x, p.y, lds, sizeof(m));
+  for (int q = it.y + step; q < count; q += step)
+    interact_rest<F32>(A + it.x, c->b.plist[q].x, c->b.plist[q].y, lds, sizeof(m));
 }
 
 // after the last step of a call: its tool force, by one work-group per instance

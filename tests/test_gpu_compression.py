@@ -1,9 +1,10 @@
-"""Patches of a body in compression."""
+"""Patches of a body in compression, and patches that are read from memory."""
 import time
 
 import pytest
 
 import pymfc
+from test_gpu_lanes import step_time
 
 pytestmark = pytest.mark.gpu
 
@@ -23,3 +24,13 @@ def test_compression_keeps_the_patches_copy():
         s.sync()
         times.append(time.perf_counter() - t)
     assert max(times[2:]) < 1.6 * times[0], times
+
+
+def test_patches_read_from_memory():
+    """A patch whose window does not fit ends its launch late: with all of them read from memory, a
+    step of 6k particles takes twice as long (with one candidate after the other 2.8 times)."""
+    cfg = pymfc.cut_config(150, 40, 10.0, jitter=0.01, seed=1)
+    sims = [pymfc.Sim(cfg), pymfc.Sim(cfg)]
+    sims[1].set_tuning(stage_limit=1)
+    times = [step_time(s) for s in sims]
+    assert times[1] < 2.35 * times[0], times
