@@ -254,8 +254,8 @@ __device__ inline double secant(double dl, double tol, const F &residual) {
     dl = dl - g / slope;
     const bool fold = dl < 0.;
     if (fold) dl = -0.1 * dl;
-    // (every iterate after one that is not a number is none either)
-    if (fabs(dl - dl_old) < tol || iter > 100 || dl != dl) return fold ? -dl : dl;
+    // below the tolerance, or not a number (no iterate after it is one)
+    if (!(fabs(dl - dl_old) >= tol) || iter > 100) return fold ? -dl : dl;
     iter++;
   }
 }
