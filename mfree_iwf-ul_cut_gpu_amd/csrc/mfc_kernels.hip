@@ -1527,9 +1527,12 @@ __device__ inline bool interact_patch(patch_mem<F32, G, GEN> &m, unsigned *unrea
     const int tag = tags[q - m.col_shift[c]], fl = tag & ((1 << TAG_BITS) - 1);
     m.tag[q] = tag;
     if constexpr (!mem::ALL_IN_LDS) m.fl[q] = (unsigned char)fl;
-    // a blanked particle enters no sum but those of PSE, so its record may hold anything
-    const int no = MFC_FLAG_FIXED | ((fl & MFC_FLAG_BLANKED) && !k.pse ? FLAG_NONFINITE : 0);
-    if (fl & ~no) atomicOr(&m.flags, fl & ~no);
+    if (fl & ~MFC_FLAG_FIXED) {
+      int set = fl & ~MFC_FLAG_FIXED;
+      // a blanked particle enters no sum but those of PSE, so its record may hold anything
+      if ((set & MFC_FLAG_BLANKED) && !k.pse) set &= ~FLAG_NONFINITE;
+      atomicOr(&m.flags, set);
+    }
   }
   __syncthreads();
   const int flags = m.flags;
