@@ -35,6 +35,11 @@ struct mfc_batch {
       if (s->general()) return true;
     return false;
   }
+  bool fresh() const {  // every instance's state is binned
+    for (const mfc_sim *s : sims)
+      if (!s->keys_fresh) return false;
+    return true;
+  }
   bool graph_general = false;  // of the variant the graphs were captured with
   mfc::batch_work work(int parity) const {
     return {args[parity], (int)sims.size(), tiles, ntiles, chunks, nchunks, patches, npatches, f32,
@@ -91,9 +96,7 @@ int build_batch_graph(mfc_batch *b, int parity) {
 // the binning and records of every instance's current state (computed by the last step's interaction),
 // recomputed for all instances when any of them lacks it
 int batch_keys(mfc_batch *b) {
-  bool fresh = true;
-  for (mfc_sim *s : b->sims) fresh = fresh && s->keys_fresh;
-  if (fresh) return MFC_OK;
+  if (b->fresh()) return MFC_OK;
   for (mfc_sim *s : b->sims) {
     HIP_TRY(hipMemsetAsync(s->bins.pcnt, 0, sizeof(int) * (size_t)s->npatch_max, b->stream));
     HIP_TRY(hipMemsetAsync(s->plen, 0, 2 * sizeof(int), b->stream));
@@ -224,7 +227,8 @@ int mfc_batch_set_tuning(mfc_batch *b, const mfc_tuning *t) {
   }
   HIP_TRY(hipMemcpy(b->args[0], a0.data(), sizeof(mfc::inst_args) * n, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(b->args[1], a1.data(), sizeof(mfc::inst_args) * n, hipMemcpyHostToDevice));
-  if (reshaped) {  // the patches' counts are those of the old shape (batch_keys clears them where it bins)
+  if (reshaped && b->fresh()) {  // the patches' counts are those of the old shape (else batch_keys bins
+                                 // every instance, and cell ids that were never written must not be read)
     for (mfc_sim *s : b->sims)
       HIP_TRY(hipMemsetAsync(s->bins.pcnt, 0, sizeof(int) * (size_t)s->npatch_max, b->stream));
     mfc::launch_batch_patch_counts(b->work(b->cur), b->stream);

@@ -119,3 +119,47 @@ def test_uneven_h_costs_little_time(prec):
     uneven(sims[1])
     times = [step_time(s) for s in sims]
     assert times[1] < 1.6 * times[0], times
+
+
+@pytest.mark.parametrize("lanes", [1, 4, 8])
+@pytest.mark.parametrize("name", ["rothlin", "impact", "rings", "tanh_jc"])
+def test_scenarios(lanes, name):
+    """The cell ranges of the rothlin grid, whose sort leaves the friction force in place, an adaptive
+    grid, a body without a tool and the tanh flow stress, whose secant takes other lanes."""
+    if name == "impact":
+        cfg = pymfc.config_impact(20)
+    elif name == "rings":
+        cfg = pymfc.config_rings(24)
+    else:
+        cfg = cut(nx=40, ny=12)
+        if name == "rothlin":
+            cfg.grid_kind = pymfc.GRID_ROTHLIN
+        else:
+            cfg.jc_model = pymfc.JC_TANH
+            cfg.jc_tanh_a, cfg.jc_tanh_b, cfg.jc_tanh_c, cfg.jc_tanh_d = 2.0, 5.0, 1.0, 0.5
+    g, o = pymfc.Sim(cfg), ob.OracleSim(cfg)
+    g.set_tuning(lanes=lanes)
+    for _ in range(3):
+        g.step(33)
+        o.step(33)
+        assert_bitwise(g, o, context=name)
+    assert equal(g.force_history(), o.force_history())
+    assert equal(g.cells(), o.cells())
+
+
+@pytest.mark.parametrize("prec", [pymfc.PREC_FP64, pymfc.PREC_FP32C])
+@pytest.mark.parametrize("lanes", [1, 4, 8])
+def test_mixed_batches(lanes, prec):
+    """Cuts of every thermal model beside the bodies, an adaptive grid, the rothlin grid and dense cells."""
+    cfgs = [cut(prec, thermal="adiabatic"), cut(prec, nx=41), cut(prec, thermal="pse", nx=33), cut(prec, hdx=2.3, nx=33),
+            pymfc.config_rings(24, prec), pymfc.config_impact(16, prec), cut(prec, nx=31)]
+    cfgs[-1].grid_kind = pymfc.GRID_ROTHLIN
+    b = pymfc.Batch(cfgs)
+    b.set_tuning(lanes=lanes)
+    b.step(21)
+    for i, c in enumerate(cfgs):
+        s = pymfc.Sim(c)
+        s.step(21)
+        for f in ("pos", "vel", "S", "T", "eps_pl", "fc", "ft", "flags", "id"):
+            assert equal(b[i].field(f), s.field(f)), (i, f)
+        assert equal(b[i].force_history(), s.force_history()), i
