@@ -548,6 +548,7 @@ using rec_t = std::conditional_t<F32, rec32, rec64>;
 // of a record are staged, and the others are read from memory for each pair (with positions and tags alone
 // staged, a step of 197k particles took 287 us at hdx 2.3 instead of 222, 141 instead of 116 with an uneven h, FP64;
 // with whole records and the h's for two work-groups to a CU 257 and 115).
+constexpr int WALK_U = 4;  // candidates of a window whose loads are issued together
 template <bool F32, int G, bool GEN>
 struct patch_mem {
   static constexpr int CAP = patch_cap(F32, G, GEN);
@@ -556,10 +557,12 @@ struct patch_mem {
   // the terms of one pair per thread, exchanged between the threads of a particle: FP32C all nine,
   // FP64 in two halves (an odd stride keeps the rows on different banks)
   static constexpr int TERM_BYTES = G == 1 ? 0 : TILE * (F32 ? 9 * (int)sizeof(float) : 7 * (int)sizeof(double));
-  float4 piece[PIECES][CAP + 1];
+  float4 pieces[PIECES * (CAP + 1) + (PIECES == 1 ? WALK_U : 0)];  // sums_lds reads up to WALK_U - 1 past a candidate
+  __device__ inline float4 *piece(int p) { return pieces + p * (CAP + 1); }
+  __device__ inline const float4 *piece(int p) const { return pieces + p * (CAP + 1); }
   double X[ALL_IN_LDS ? 1 : CAP];
-  int tag[CAP];            // or, without ALL_IN_LDS and promote, c
-  unsigned char fl[ALL_IN_LDS ? 1 : CAP];  // the flags of the tag
+  int tag[CAP + WALK_U - 1];            // or, without ALL_IN_LDS and promote, c
+  unsigned char fl[ALL_IN_LDS ? 1 : CAP + WALK_U - 1];  // the flags of the tag
   int flags;               // of all the candidates, PATCH_DENSE, PATCH_DENSER and PATCH_HEAPED
   int table[PATCH_TABLE];  // LDS index of the first candidate of each cell (row-major in a column)
   int col_first[PATCH_COLS + 1];  // of each staged column
@@ -594,15 +597,15 @@ struct lds_source {
   // GEN: piece Q of a record (without that of its flags and h), from the copy or from storage index s
   template <int Q>
   __device__ inline float4v part32(int j, size_t s) const {
-    if constexpr (Q < mem::PIECES) return reinterpret_cast<const float4v *>(m->piece[Q])[j];
+    if constexpr (Q < mem::PIECES) return reinterpret_cast<const float4v *>(m->piece(Q))[j];
     else return rec32[REC32_PIECES * s + Q];
   }
   template <int Q>
   __device__ inline double2v part64(int j, size_t s) const {
-    if constexpr (Q < mem::PIECES) return reinterpret_cast<const double2v *>(m->piece[Q])[j];
+    if constexpr (Q < mem::PIECES) return reinterpret_cast<const double2v *>(m->piece(Q))[j];
     else return ((global<double2v>)rec)[REC / 2 * s + Q + 1];
   }
-  __device__ inline double2 pos(int j) const { return reinterpret_cast<const double2 *>(m->piece[0])[j]; }
+  __device__ inline double2 pos(int j) const { return reinterpret_cast<const double2 *>(m->piece(0))[j]; }
   __device__ inline int tag(int j) const {  // its flags
     if constexpr (mem::ALL_IN_LDS) return m->tag[j];
     else return m->fl[j];
@@ -620,10 +623,10 @@ struct lds_source {
         q.rho = part64<2>(j, s).x; q.T = part64<6>(j, s).y;
       }
     } else if constexpr (F32) {
-      q.rho = m->piece[1][j].z; q.T = m->piece[3][j].w;
+      q.rho = m->piece(1)[j].z; q.T = m->piece(3)[j].w;
     } else {
-      q.rho = reinterpret_cast<const double2 *>(m->piece[2])[j].x;
-      if constexpr (mem::ALL_IN_LDS) q.T = reinterpret_cast<const double2 *>(m->piece[6])[j].y;
+      q.rho = reinterpret_cast<const double2 *>(m->piece(2))[j].x;
+      if constexpr (mem::ALL_IN_LDS) q.T = reinterpret_cast<const double2 *>(m->piece(6))[j].y;
       else if (c_in_tag || t_in_lds) q.T = m->X[j];
       else q.T = rec[(size_t)REC * tag_index(m->tag[j]) + 15];
     }
@@ -645,14 +648,14 @@ struct lds_source {
         q.h = uniform_h ? h0 : rec[REC * s + 3];
       }
     } else if constexpr (F32) {
-      const float4 a = m->piece[1][j], b = m->piece[2][j], c = m->piece[3][j];
+      const float4 a = m->piece(1)[j], b = m->piece(2)[j], c = m->piece(3)[j];
       q.u = a.x; q.v = a.y; q.rho = a.z; q.vol = a.w;
       q.Axx = b.x; q.Axy = b.y; q.Ayy = b.z; q.c = b.w;
       q.Rxx = c.x; q.Rxy = c.y; q.Ryy = c.z; q.T = c.w;
       q.h = (float)h0;
     } else {
       if constexpr (mem::ALL_IN_LDS) {
-        const double2 f = reinterpret_cast<const double2 *>(m->piece[6])[j];
+        const double2 f = reinterpret_cast<const double2 *>(m->piece(6))[j];
         q.c = f.x; q.T = f.y;
       } else if (c_in_tag) {
         q.c = __int_as_float(m->tag[j]);
@@ -664,11 +667,11 @@ struct lds_source {
         q.c = m->X[j];
         q.T = 0.;  // not read
       }
-      const double2 a = reinterpret_cast<const double2 *>(m->piece[1])[j];
-      const double2 b = reinterpret_cast<const double2 *>(m->piece[2])[j];
-      const double2 c = reinterpret_cast<const double2 *>(m->piece[3])[j];
-      const double2 d = reinterpret_cast<const double2 *>(m->piece[4])[j];
-      const double2 e = reinterpret_cast<const double2 *>(m->piece[5])[j];
+      const double2 a = reinterpret_cast<const double2 *>(m->piece(1))[j];
+      const double2 b = reinterpret_cast<const double2 *>(m->piece(2))[j];
+      const double2 c = reinterpret_cast<const double2 *>(m->piece(3))[j];
+      const double2 d = reinterpret_cast<const double2 *>(m->piece(4))[j];
+      const double2 e = reinterpret_cast<const double2 *>(m->piece(5))[j];
       q.u = a.x; q.v = a.y; q.rho = b.x; q.vol = b.y;
       q.Axx = c.x; q.Axy = c.y; q.Ayy = d.x; q.Rxx = d.y; q.Rxy = e.x; q.Ryy = e.y;
       q.h = h0;
@@ -923,7 +926,6 @@ __device__ inline double value_of(double s) { return s; }
 // The neighbour sums of a particle by one thread from the records in memory: the window's
 // candidates in order, which is the reference's (interactions_gpu.cu:219-331), 64 at a time: first the
 // support tests, whose loads are issued together for WALK_U candidates, then the pairs
-constexpr int WALK_U = 4;  // candidates whose loads are issued together
 template <bool F32, bool FINITE, class SRC>
 __device__ inline void sums_mem(kconst &k, const SRC &src, const window &w, const rec_t<F32> &a, const sum_flags &f,
                                 pair_acc &acc, double &tpse) {
@@ -1026,7 +1028,7 @@ __device__ inline void sums_lds(kconst &k, const lds_source<F32, G, GEN> &src, i
       for (int q = 0; q < n; q += WALK_U) {
         double2 p[WALK_U];
 #pragma unroll
-        for (int u = 0; u < WALK_U; u++) p[u] = src.pos(first + q + u);  // past the range: some other entry of the copy
+        for (int u = 0; u < WALK_U; u++) p[u] = src.pos(first + q + u);  // past the range: some other piece of the copy
         unsigned hits = 0u;
 #pragma unroll
         for (int u = 0; u < WALK_U; u++) {
@@ -1551,7 +1553,7 @@ __device__ inline bool interact_patch(patch_mem<F32, G, GEN> &m, unsigned *unrea
       const int p = tid % P;
       for (int q = tid / P; q < ncand; q += TILE / P) {
         const size_t s = tag_index(m.tag[q]);
-        m.piece[p][q] = F32 ? r.rec32[s * REC32_PIECES + p] : reinterpret_cast<const float4 *>(r.rec)[s * (REC / 2) + (p ? p + 1 : 0)];
+        m.piece(p)[q] = F32 ? r.rec32[s * REC32_PIECES + p] : reinterpret_cast<const float4 *>(r.rec)[s * (REC / 2) + (p ? p + 1 : 0)];
       }
     } else for (int q = tid / LPR; q < ncand; q += STAGE_U * (TILE / LPR)) {
       float4 v[STAGE_U];
@@ -1570,10 +1572,10 @@ __device__ inline bool interact_patch(patch_mem<F32, G, GEN> &m, unsigned *unrea
             ((mem::ALL_IN_LDS ? m.tag[c] : (int)m.fl[mem::ALL_IN_LDS ? 0 : c]) & MFC_FLAG_BLANKED))
           reinterpret_cast<double2 &>(v[u]) = make_double2(__builtin_huge_val(), __builtin_huge_val());
         if constexpr (F32) {
-          m.piece[pl][c] = v[u];
+          m.piece(pl)[c] = v[u];
         } else if (pl != 1) {  // piece 1 of a record: flags (in the tag) and h (uniform)
           const int p = pl == 0 ? 0 : pl - 1;
-          if (mem::ALL_IN_LDS || p < 6) m.piece[p][c] = v[u];
+          if (mem::ALL_IN_LDS || p < 6) m.piece(p)[c] = v[u];
           else {
             const double2 ct = reinterpret_cast<const double2 &>(v[u]);
             m.X[c] = c_in_tag || t_in_lds ? ct.y : ct.x;
@@ -1666,14 +1668,14 @@ __device__ inline bool interact_patch(patch_mem<F32, G, GEN> &m, unsigned *unrea
     if constexpr (G == 1) {
       finish_particle<F32>(A + inst, i, s_mine, live, acc, tpse);
     } else {  // by the first wave, the returns by all
-      static_assert(SLOTS <= 64 && sizeof(return_slots) <= sizeof(m.piece), "one wave's particles");
+      static_assert(SLOTS <= 64 && sizeof(return_slots) <= sizeof(m.pieces), "one wave's particles");
       after_update u;
       u.dr.need = false;
       if (tid < 64) begin_update<F32>(A + inst, i, s_mine, live, acc, tpse, u);
       const return_tape t = m.tape;
       const bool taped = on_tape<F32>(c_, t, u.dr.need);
       bool folded;
-      double dl = rr_secant_group<F32>(k, reinterpret_cast<return_slots &>(m.piece), u.dr.need && !taped, u.dr.in,
+      double dl = rr_secant_group<F32>(k, reinterpret_cast<return_slots &>(m.pieces), u.dr.need && !taped, u.dr.in,
                                        u.dr.eps, u.dr.T, folded);
       if (taped && u.dr.need) dl = from_tape(t, i, folded);
       if (tid < 64) end_update<F32>(A + inst, i, live, dl, folded, t, u);
