@@ -325,9 +325,10 @@ int mfc_vjp(mfc_sim *sim, mfc_vjp_req *req, double grad[6]);
  * evaluates the same expressions in the same order). lanes: threads per particle of the
  * interaction, 1, 4 or 8 (0: by the number of work-groups they make; more lanes
  * shorten a particle's chain of operations where the particles alone would not fill the chip).
- * stage_limit: the most window candidates a patch of cells copies into LDS (0 or anything above
- * what the kernel has room for: all of them); a patch with more reads them from the records in
- * memory. xcd_chunk: the interaction deals its patches to the 8 XCDs in chunks of this many
+ * stage_limit: the most window candidates a patch of cells copies into LDS (0..MFC_STAGE_CAP; 0 or
+ * anything above what the kernel has room for, 256 to 1,408 by lanes, precision and smoothing
+ * lengths: all of them); a patch with more reads them from the records in memory. xcd_chunk: the
+ * interaction deals its patches to the 8 XCDs in chunks of this many
  * (1..MFC_XCD_CHUNK_MAX; 0 = 8). split_interact and compact_pairs (0 or 1) selected other kernels
  * of the interaction once; they are accepted and change nothing. The Python package's autotuner
  * (pymfc.autotune) times the combinations on a live handle and keeps the fastest. sort_fast and

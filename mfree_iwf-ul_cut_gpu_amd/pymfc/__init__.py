@@ -115,16 +115,18 @@ class VjpReq(C.Structure):
                 ("cot", C.c_double * 2), ("Fmean", C.c_double * 2)]
 
 
-STAGE_CAP = 2048  # MFC_STAGE_CAP: window candidates a tile can stage in LDS
-XCD_CHUNK_MAX = 64  # MFC_XCD_CHUNK_MAX: longest XCD chunk of the interaction kernels' tile map
+STAGE_CAP = 2048  # MFC_STAGE_CAP: the largest stage_limit (a patch stages 1,408 candidates at most)
+XCD_CHUNK_MAX = 64  # MFC_XCD_CHUNK_MAX: longest XCD chunk of the interaction's map
 SORT_FAST_MAX = 1536  # MFC_SORT_FAST_MAX: most particles of a chunk the sort holds in registers
 GRAPH_STEPS = 8   # steps per captured hipGraph of a handle (one graph per buffer parity)
 
 
-# the launch configurations the autotuner tries: LDS stage limit (0: patches stage all the
-# candidates the kernel has room for; n > 0: patches with more than n read them from memory; 1: no
-# patch stages) and XCD chunk; split_interact and compact_pairs change nothing
-TUNING_SPACE = {"split_interact": (0, 1), "compact_pairs": (0, 1), "stage_limit": (0, 1536, 1), "xcd_chunk": (8, 32)}
+# the launch configurations the autotuner tries: threads per particle (0: by size) and XCD chunk. Each
+# selects another kernel or another map, so no candidate is another one again but those of lanes 0.
+# Settings with one value are reported with the others: a stage limit only sends patches the
+# slower way, and split_interact and compact_pairs change nothing
+TUNING_SPACE = {"split_interact": (0,), "compact_pairs": (0,), "stage_limit": (0,), "lanes": (0, 1, 4, 8),
+                "xcd_chunk": (8, 4, 16, 24, 32, 64)}
 
 
 def autotune(handle, steps: int = 100, space: dict | None = None, rounds: int = 2) -> dict:

@@ -163,3 +163,13 @@ def test_mixed_batches(lanes, prec):
         for f in ("pos", "vel", "S", "T", "eps_pl", "fc", "ft", "flags", "id"):
             assert equal(b[i].field(f), s.field(f)), (i, f)
         assert equal(b[i].force_history(), s.force_history()), i
+
+
+def test_autotuner_tries_kernels():
+    """No two candidates of the default space are the same launches twice, but for lanes 0, which stands for
+    one of the others; the threads per particle are among them."""
+    s = pymfc.Sim(cut(nx=40, ny=12))
+    t = pymfc.autotune(s, steps=2, rounds=1)
+    assert {"lanes", "xcd_chunk"} == {k for k, v in pymfc.TUNING_SPACE.items() if len(v) > 1}
+    assert set(pymfc.TUNING_SPACE["lanes"]) == {0, 1, 4, 8}
+    assert s.tuning()["lanes"] == t["lanes"] and s.tuning()["xcd_chunk"] == t["xcd_chunk"]
