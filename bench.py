@@ -44,12 +44,14 @@ STEP_BYTES = 256 + 224 + 12
 # window candidates read by two work-groups) is traffic above the algorithmic bytes.
 KERNEL_BYTES = {"binning": 12, "interact": 256 + 224}
 assert sum(KERNEL_BYTES.values()) == STEP_BYTES
-# HBM bytes per particle of one launch of the interaction kernel on thermal_contact_150k, by
-# precision and XCD chunk length (a stage limit above the stage's own size changes nothing), measured
+# HBM bytes per particle of one launch of the interaction kernel on thermal_contact_150k, one thread
+# per particle, by precision and XCD chunk length (those of the autotuner's space), measured
 # with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE passes and scaled by a 512 MiB copy (the commands and
 # tables are in profiles/traffic_thermal_contact_150k.md); a table of measurements, not measured in
 # this run, and reported as `traffic` only for the tuning it was measured with
-MEASURED_TRAFFIC = {("kb_interact", "fp32c", 8): 791, ("kb_interact", "fp64", 8): 987}
+MEASURED_TRAFFIC = {("fp32c", 4): 826, ("fp32c", 8): 792, ("fp32c", 16): 766, ("fp32c", 24): 752, ("fp32c", 32): 741,
+                    ("fp32c", 64): 730, ("fp64", 4): 1031, ("fp64", 8): 991, ("fp64", 16): 963, ("fp64", 24): 941,
+                    ("fp64", 32): 924, ("fp64", 64): 908}
 MEASURED_TRAFFIC_SOURCE = ("table: rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE, thermal_contact_150k, fused interaction, "
                            "profiles/traffic_thermal_contact_150k.md")
 
@@ -210,7 +212,7 @@ def batch_bench(pymfc, n: int, steps: int, tune_steps: int) -> dict:
         seq = 0.0
         for c in cfgs:
             s = pymfc.Sim(c)
-            s.set_tuning(**best)
+            s.set_tuning(**(best | {"lanes": 0}))  # an instance by itself: by its own size
             s.step(warm)
             s.sync()
             t0 = time.perf_counter()
@@ -268,13 +270,13 @@ def batch_adjoint_bench(pymfc, n: int, nsteps: int = 100, K: int = 25) -> dict:
 COPY_PROBE_BYTES = 512 << 20
 
 
-def counter_probe(pymfc, workload: str, precision: int, steps: int, split: int, compact: int) -> None:
-    """A short run for hardware-counter passes (rocprofv3 --pmc): `steps` steps of one path,
-    then a plain device copy of COPY_PROBE_BYTES read + COPY_PROBE_BYTES written, whose counter
+def counter_probe(pymfc, workload: str, precision: int, steps: int) -> None:
+    """A short run for hardware-counter passes (rocprofv3 --pmc): `steps` steps of one path with the
+    settings of --tuning, then a plain device copy of COPY_PROBE_BYTES read + COPY_PROBE_BYTES written, whose counter
     readings calibrate the bytes per counted unit."""
     import torch
     sim = pymfc.Sim(pymfc.workload(workload, precision))
-    sim.set_tuning(**(FIXED_TUNING | {"split_interact": split, "compact_pairs": compact}))
+    sim.set_tuning(**FIXED_TUNING)
     for _ in range(steps):
         sim.step(1)
     sim.sync()
@@ -283,8 +285,7 @@ def counter_probe(pymfc, workload: str, precision: int, steps: int, split: int, 
     torch.cuda.synchronize()
     b.copy_(a)
     torch.cuda.synchronize()
-    print(json.dumps({"probe": workload, "precision": precision, "steps": steps, "split_interact": split,
-                      "compact_pairs": compact,
+    print(json.dumps({"probe": workload, "precision": precision, "steps": steps, "tuning": FIXED_TUNING,
                       "copy_bytes": COPY_PROBE_BYTES, "N": sim.N}), flush=True)
     sim.close()
 
@@ -300,7 +301,7 @@ def main() -> int:
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--only", choices=["fp64", "fp32c"], default=None)
     ap.add_argument("--tune-steps", type=int, default=100, help="steps per candidate of the autotuner (0: off)")
-    ap.add_argument("--tuning", default="", help="with --tune-steps 0: launch settings k=v,... (e.g. compact_pairs=1)")
+    ap.add_argument("--tuning", default="", help="with --tune-steps 0: launch settings k=v,... (e.g. xcd_chunk=32)")
     ap.add_argument("--adjoint-workload", default="adjoint_40k")
     ap.add_argument("--adjoint-steps", type=int, default=400)
     ap.add_argument("--adjoint-k", type=int, default=50)
@@ -311,8 +312,6 @@ def main() -> int:
     ap.add_argument("--other-steps", type=int, default=500, help="timed steps of the other configurations")
     ap.add_argument("--no-other", action="store_true", help="skip the 6k and 500k configurations")
     ap.add_argument("--probe", action="store_true", help="counter-pass mode: short run + calibration copy")
-    ap.add_argument("--split", type=int, default=0, help="split_interact for --probe")
-    ap.add_argument("--compact", type=int, default=0, help="compact_pairs for --probe")
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py: this build runs on one GPU only; --gpus {args.gpus} is not supported "
@@ -329,7 +328,7 @@ def main() -> int:
         FIXED_TUNING[k] = int(v)
     if args.probe:
         counter_probe(pymfc, args.workload, pymfc.PREC_FP32C if args.only == "fp32c" else pymfc.PREC_FP64,
-                      args.steps, args.split, args.compact)
+                      args.steps)
         return 0
 
     res = {}
@@ -350,9 +349,9 @@ def main() -> int:
     # kernel's roofline
     t_int = r["phases"]["interact"] * 1e-3 if r["phases"] else None
     achieved = N * kbytes / t_int / 1e9 if t_int else None
-    tkey = ("kb_interact", head, r["tuning"].get("xcd_chunk", 8))
+    tkey = (head, r["tuning"].get("xcd_chunk", 8))
     traffic = None
-    if args.workload == "thermal_contact_150k" and tkey in MEASURED_TRAFFIC:
+    if args.workload == "thermal_contact_150k" and r["tuning"].get("lanes", 0) in (0, 1) and tkey in MEASURED_TRAFFIC:
         traffic = MEASURED_TRAFFIC[tkey] * N
     step_s = r["wall"] / args.steps
     result = {

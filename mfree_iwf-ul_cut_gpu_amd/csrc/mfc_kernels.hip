@@ -7,8 +7,8 @@
 //                grid_gpu_green.cu:22-116,177-201) from the cell ids (grid.cu:34-51), per-cell
 //                and per-chunk counts and the chunks' particle lists that the previous step's
 //                interaction computed for the updated state (hash_count computes them when the
-//                state was written from outside, and for every state the reverse mode
-//                restores); a few more work-groups of the launch move the tool, list the patches of
+//                state was written from outside, for every state the reverse mode restores, and
+//                behind an adaptive grid's geometry pass); a few more work-groups of the launch move the tool, list the patches of
 //                cells that hold particles and sum the previous step's tool force
 //                (output.cu:30-39) over groups of 64 particles
 //   interact     neighbour sums (interactions_gpu.cu:88-345) fused with every per-particle action

@@ -45,9 +45,10 @@ MFC_HD double abs_d(double x) { return u2d(d2u(x) & 0x7fffffffffffffffULL); }
 // 2^k for k in [-1022, 1023], exact.
 MFC_HD double pow2i(int k) { return u2d((uint64_t)(k + 1023) << 52); }
 
-// a / b where neither operand nor the quotient is near the ends of the exponent range: on the GPU
-// the Newton iterations for 1/b and the corrected quotient that its division expands to, without the
-// scaling and special cases around them (correctly rounded, as the division)
+// a / b where neither operand nor the quotient is near the ends of the exponent range: on the GPU two
+// Newton iterations for 1/b from the hardware's estimate, and the quotient corrected by its exact
+// remainder (P. Markstein, IBM J. Res. Dev. 34, 1990), without the scaling and special cases of a
+// division around them (correctly rounded, as the division)
 MFC_HD double quotient(double a, double b) {
 #if defined(__HIP_DEVICE_COMPILE__)
   double y = __builtin_amdgcn_rcp(b);

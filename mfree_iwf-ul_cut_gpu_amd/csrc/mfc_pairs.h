@@ -118,8 +118,10 @@ struct rec64 {
   double x, y, u, v, rho, vol, Axx, Axy, Ayy, Rxx, Rxy, Ryy, c, T, h;
 };
 
-// sqrt of x far from the ends of the exponent range: the Goldschmidt iterations and corrections of the
-// division-free square root, without the scaling and special cases around them (correctly rounded)
+// sqrt of x far from the ends of the exponent range: Goldschmidt's iterations from the hardware's
+// estimate of 1 / sqrt(x) and corrections by the exact remainder (P. Markstein, Software division and
+// square root using Goldschmidt's algorithms, RNC6, 2004), without scaling and special cases
+// around them (correctly rounded)
 __device__ inline double root(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   double s = x * y, h = 0.5 * y;
@@ -130,7 +132,8 @@ __device__ inline double root(double x) {
   return __builtin_fma(__builtin_fma(-s, s, x), h, s);
 }
 // the same in single precision: the hardware's value (within one unit in the last place), or its
-// neighbour where x is beyond the midpoint to it
+// neighbour where x is beyond the midpoint to it by the sign of the exact remainder (P. Markstein,
+// Computation of elementary functions on the IBM RISC System/6000 processor, IBM J. Res. Dev. 34, 1990)
 __device__ inline float root32(float x) {
   const float s = __builtin_amdgcn_sqrtf(x);
   const float lo = __uint_as_float(__float_as_uint(s) - 1u), hi = __uint_as_float(__float_as_uint(s) + 1u);
