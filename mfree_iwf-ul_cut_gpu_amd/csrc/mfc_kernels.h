@@ -77,7 +77,7 @@ constexpr int PATCH_COLS = 24;    // patch_w + 4 at most
 // The general variant (gen) copies less of each (of 128 bytes 64, of 64 32, with several threads per
 // particle 16 of both, and the tag), so that as many work-groups run at once.
 __host__ __device__ constexpr int patch_cap(bool f32, int lanes, bool gen) {
-  return gen ? (lanes > 1 ? 1408 : f32 ? 1080 : 760) : lanes > 1 ? 256 : f32 ? 576 : 479;
+  return gen ? (f32 ? 1080 : lanes > 1 ? 1408 : 760) : lanes > 1 ? 256 : f32 ? 576 : 479;
 }
 // What the patches of a full lattice may have of that: a body in compression has more particles in a
 // cell, and a few patches over the copy's room make the launch twice as long (in FP32C, planned up to

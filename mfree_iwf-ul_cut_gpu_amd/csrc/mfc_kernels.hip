@@ -1684,93 +1684,123 @@ __device__ inline bool interact_patch(patch_mem<F32, G, GEN> &m, unsigned *unrea
   return true;
 }
 
-// The patches that interact_patch leaves, and those past the end of the launch's work items: one
-// thread per particle over the records in memory, with the window's positions and tags copied to
-// LDS where they fit and all records are finite (`lds`, of `bytes`; 20 bytes each, four times as many as
-// whole records). A call, so that this rare path takes no registers from the kernel that holds it. A
-// launch waits for its last patch, so what counts is how long one takes. us per step with every patch sent
-// here: 6k particles FP64 58, 197k 216, FP32C 134 (one candidate after the other from memory,
-// with the pair terms for any value, 81, 234 and 158).
+// Positions and tags of the window candidates of a patch copied to `lds` (of `bytes`; 20 bytes each, four
+// times as many as whole records): the columns [q0, q0 + ncol) of cells, rows [s0, s1). False where they
+// do not fit or a record of some sum is not finite; shift: a column's places minus its sorted indices
 template <bool F32>
-__device__ __attribute__((noinline)) void interact_rest(const inst_args *ap, int patch, int part, lds_ptr<char> lds,
-                                                        int bytes) {
+__device__ inline bool copy_window(kconst &k, const mem_records<F32> &rec, const int *offsets, const int *tags, int q0,
+                                   int ncol, int s0, int s1, lds_ptr<char> lds, int bytes, lds_ptr<int> &shift,
+                                   copy_source<F32> &copy) {
+  lds_ptr<int> first = (lds_ptr<int>)lds, nonfinite = first + 63;
+  shift = first + 32;  // PATCH_COLS at most of each
+  constexpr int HEAD = 64 * sizeof(int);
+  const int cap = (bytes - HEAD) / (int)(sizeof(lds_pos) + sizeof(int)), tid = threadIdx.x;
+  copy.pos = (lds_ptr<lds_pos>)(lds + HEAD);
+  copy.tags = (lds_ptr<int>)(copy.pos + cap);
+  __syncthreads();  // what was in the LDS before is no longer read
+  if (tid < 64) {
+    int j0 = 0, c = 0;
+    if (tid < ncol) {
+      j0 = offsets[(q0 + tid) * k.gny + s0];
+      c = offsets[(q0 + tid) * k.gny + s1] - j0;
+    }
+    int x = c;
+#pragma unroll
+    for (int s = 1; s < 32; s <<= 1) {
+      const int y = __shfl_up(x, s, 64);
+      if (tid >= s) x += y;
+    }
+    if (tid <= ncol) {
+      first[tid] = x - c;
+      shift[tid] = x - c - j0;
+    }
+    if (tid == 63) *nonfinite = 0;
+  }
+  __syncthreads();
+  const int ncand = first[ncol];
+  if (ncand > cap) return false;  // the same in every thread
+  for (int q = tid; q < ncand; q += TILE) {
+    int c = 0;
+    for (int e = 1; e < ncol; e++) c += q >= first[e];
+    const int tag = tags[q - shift[c]];
+    const double2 p = rec.pos_of(tag);
+    copy.tags[q] = tag;
+    copy.pos[q].x = p.x; copy.pos[q].y = p.y;
+    if ((tag & FLAG_NONFINITE) && (k.pse || !(tag & MFC_FLAG_BLANKED))) *nonfinite = 1;
+  }
+  __syncthreads();
+  return *nonfinite == 0;
+}
+
+// What interact_patch leaves, one thread per particle over the records in memory: a patch that it does not
+// take, an entry past the end of the launch's work items, the particles past the grid, or (patch < 0) tile
+// `part` of the sorted order. A launch waits for its last work-group, so what counts is how long one takes.
+// us per step with every patch sent here: 6k particles FP64 60, 197k 167, FP32C 84 (one candidate
+// after the other from memory, with the pair terms for any value, 81, 234 and 158).
+template <bool F32>
+__device__ __attribute__((always_inline)) inline void interact_rest(const inst_args *ap, int patch, int part,
+                                                                    lds_ptr<char> lds, int bytes) {
   MFC_CONST(inst_args) *c_ = const_args(ap, 0);
   kconst &k = c_->k;
   const dbins b = load_bins(&c_->b);
   const int *offsets = k.rothlin ? b.offsets_r : b.offsets;
-  const int tid = threadIdx.x;
-  const int nrb = patch_rows(k);
-  const int pc = patch / nrb, pr = patch - pc * nrb;
-  const int r0 = pr * k.patch_s, r1 = r0 + k.patch_s < k.gny ? r0 + k.patch_s : k.gny;
-  const int g0 = pc * k.patch_w, g1 = g0 + k.patch_w < k.gnx ? g0 + k.patch_w : k.gnx;
-  int n = tid < k.patch_slots ? part * k.patch_slots + tid : 0x7fffffff, i = -1;
-  for (int c = g0; c < g1; c++) {
-    const int first = offsets[c * k.gny + r0], count = offsets[c * k.gny + r1] - first;
-    if (i < 0 && n < count) i = first + n;
-    if (n != 0x7fffffff) n -= count;
+  const mem_records<F32> rec = {load_recs(&c_->r), load_state(&c_->cur).h};
+  copy_source<F32> copy = {rec, nullptr, nullptr};
+  lds_ptr<int> shift = nullptr;
+  int i = -1, q0 = 0;   // the thread's particle; the first column of the copy
+  bool copied = false;  // the same in every thread
+  if (patch < 0) {
+    const int j = part * TILE + (int)threadIdx.x;
+    if (j < k.N) i = j;
+  } else {
+    const int nrb = patch_rows(k);
+    const int pc = patch / nrb, pr = patch - pc * nrb;
+    const int r0 = pr * k.patch_s, r1 = r0 + k.patch_s < k.gny ? r0 + k.patch_s : k.gny;
+    const int g0 = pc * k.patch_w, g1 = g0 + k.patch_w < k.gnx ? g0 + k.patch_w : k.gnx;
+    int n = (int)threadIdx.x < k.patch_slots ? part * k.patch_slots + (int)threadIdx.x : 0x7fffffff;
+    for (int c = g0; c < g1; c++) {
+      const int first = offsets[c * k.gny + r0], count = offsets[c * k.gny + r1] - first;
+      if (i < 0 && n < count) i = first + n;
+      if (n != 0x7fffffff) n -= count;
+    }
+    if (g0 >= k.gnx) {  // the particles past the grid: blanked ones, which have no sums
+      const int first = offsets[k.num_cell];
+      if (n < k.N - first) i = first + n;
+    } else {
+      q0 = g0 < 2 ? 0 : g0 - 2;
+      copied = copy_window(k, rec, offsets, b.tags, q0, (g1 + 2 < k.gnx ? g1 + 2 : k.gnx) - q0, r0 < 2 ? 0 : r0 - 2,
+                           r1 + 2 < k.gny ? r1 + 2 : k.gny, lds, bytes, shift, copy);
+    }
   }
   pair_acc acc = {};
   double tpse = 0.;
-  if (g0 >= k.gnx) {  // the particles past the grid: blanked ones, which have no sums
-    const int first = offsets[k.num_cell];
-    if (n < k.N - first) i = first + n;
-  } else {
-    const mem_records<F32> rec = {load_recs(&c_->r), load_state(&c_->cur).h};
-    // where each column of the windows starts in the copy, and its place minus its sorted index
-    const int s0 = r0 < 2 ? 0 : r0 - 2, s1 = r1 + 2 < k.gny ? r1 + 2 : k.gny;
-    const int q0 = g0 < 2 ? 0 : g0 - 2, ncol = (g1 + 2 < k.gnx ? g1 + 2 : k.gnx) - q0;
-    lds_ptr<int> first = (lds_ptr<int>)lds, shift = first + 32, nonfinite = first + 63;
-    constexpr int HEAD = 64 * sizeof(int);
-    const int cap = (bytes - HEAD) / (int)(sizeof(lds_pos) + sizeof(int));
-    lds_ptr<lds_pos> pos = (lds_ptr<lds_pos>)(lds + HEAD);
-    lds_ptr<int> tags = (lds_ptr<int>)(pos + cap);
-    __syncthreads();  // what was in the LDS before is no longer read
-    if (tid < 64) {
-      const int j0 = tid < ncol ? offsets[(q0 + tid) * k.gny + s0] : 0, c = tid < ncol ? offsets[(q0 + tid) * k.gny + s1] - j0 : 0;
-      int x = c;
-#pragma unroll
-      for (int s = 1; s < 32; s <<= 1) {
-        const int y = __shfl_up(x, s, 64);
-        if (tid >= s) x += y;
-      }
-      if (tid <= ncol) {
-        first[tid] = x - c;
-        shift[tid] = x - c - j0;
-      }
-      if (tid == 63) *nonfinite = 0;
-    }
-    __syncthreads();
-    const int ncand = first[ncol];
-    bool copied = ncand <= cap;  // the same in every thread
-    if (copied) {
-      for (int q = tid; q < ncand; q += TILE) {
-        int c = 0;
-        for (int e = 1; e < ncol; e++) c += q >= first[e];
-        const int tag = b.tags[q - shift[c]];
-        const double2 p = rec.pos_of(tag);
-        tags[q] = tag;
-        pos[q].x = p.x; pos[q].y = p.y;
-        if ((tag & FLAG_NONFINITE) && (k.pse || !(tag & MFC_FLAG_BLANKED))) *nonfinite = 1;
-      }
-      __syncthreads();
-      if (*nonfinite) copied = false;
-    }
-    if (i >= 0) {
-      const int tag = b.tags[i], key = b.key_sorted[i];
-      const double2 p = rec.pos_of(tag);
-      rec_t<F32> a;
-      rec.record(tag, a);
-      a.x = p.x; a.y = p.y;
-      const sum_flags f = flags_of(k, tag);
-      const int gi = key / k.gny, gj = key - gi * k.gny;
-      window w = make_window_at(k, gi, gj, [&](int col, int row) { return offsets[col * k.gny + row] + (copied ? shift[col - q0] : 0); });
-      if (!f.run_mech && !f.run_pse) w.total = 0;
-      if (copied) sums_mem<F32, true>(k, copy_source<F32>{rec, pos, tags}, w, a, f, acc, tpse);
-      else sums_mem<F32, false>(k, mem_source<F32>{rec, b.tags}, w, a, f, acc, tpse);
-    }
+  unsigned s = 0u;
+  if (i >= 0) {
+    const int tag = b.tags[i], key = b.key_sorted[i];
+    s = tag_index(tag);
+    const double2 p = rec.pos_of(tag);
+    rec_t<F32> a;
+    rec.record(tag, a);
+    a.x = p.x; a.y = p.y;
+    const sum_flags f = flags_of(k, tag);
+    const int gi = key / k.gny, gj = key - gi * k.gny;
+    window w = make_window_at(k, gi, gj, [&](int col, int row) {
+      return offsets[col * k.gny + row] + (copied ? shift[col - q0] : 0);
+    });
+    if (!f.run_mech && !f.run_pse) w.total = 0;
+    if (copied) sums_mem<F32, true>(k, copy, w, a, f, acc, tpse);
+    else sums_mem<F32, false>(k, mem_source<F32>{rec, b.tags}, w, a, f, acc, tpse);
   }
-  const bool live = i >= 0;
-  finish_particle<F32>(ap, i, live ? tag_index(b.tags[i]) : 0u, live, acc, tpse);
+  finish_particle<F32>(ap, i, s, i >= 0, acc, tpse);
+}
+
+// As a call it takes no registers from the kernel, but saves up to 600 bytes of them per thread. In line it makes
+// every patch sent here 197k FP64 214 -> 167 us, FP32C 134 -> 84; but in FP64 with several threads per particle, where it
+// gives less (6k 60 -> 56), the registers it takes cost the kernel 1 % (150 steps of 37.5k 7.85 -> 7.95 ms).
+template <bool F32>
+__device__ __attribute__((noinline)) void call_interact_rest(const inst_args *ap, int patch, int part, lds_ptr<char> lds,
+                                                             int bytes) {
+  interact_rest<F32>(ap, patch, part, lds, bytes);
 }
 
 constexpr int FF_BATCH = 8;  // group sums a thread of force_final loads at a time
@@ -2047,6 +2077,13 @@ __global__ __launch_bounds__(256) void kb_rothlin_cells(const inst_args *__restr
     for (int q = h + 1; q <= hn; q++) b.offsets_r[q] = i + 1;
 }
 
+// Particles spread over so many patches that the entries of the list are more than 1.3 times the launch's
+// work items: a patch then has few particles, and the work-groups take the particles as tiles of the
+// sorted order instead, by interact_rest. us per step of 171k particles, by patches (what does not fit the
+// work items behind the others, one entry after the other) / by tiles, FP64: scattered over the whole grid 504 / 59,
+// a quarter of it 163 / 90, a sixth (1.6 times) 128 / 111; a body of which 0.5 % (1.25 times) are scattered 129 / 174,
+// 1 % (1.8 times) 156 / 175, 3 % 290 / 170. Of 27k FP64: 1.5 % (1.1 times) 60 / 86, 3 % (1.6 times) 76 / 85, a sixth (1.4) 64 / 62.
+__device__ inline bool sparse(int entries, int items) { return 10ll * entries > 13ll * items; }
 template <bool F32, int G, bool PSE, bool GEN>
 __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(F32 ? 4 : 3))) void kb_interact(
     const inst_args *__restrict__ A, const int2 *__restrict__ work, int nwork, int chunk) {
@@ -2064,12 +2101,22 @@ __global__ __launch_bounds__(TILE) __attribute__((amdgpu_waves_per_eu(F32 ? 4 : 
     return;
   }
   const int count = *c->b.plen, step = c->npatch_items;
-  if (it.y >= count) return;
-  const int2 p = c->b.plist[it.y];
   const lds_ptr<char> lds = (lds_ptr<char>)(char *)&m;
-  if (!interact_patch<F32, G, PSE, GEN>(m, unread, A, it.x, p.x, p.y)) interact_rest<F32>(A + it.x, p.x, p.y, lds, sizeof(m));
-  for (int q = it.y + step; q < count; q += step)
-    interact_rest<F32>(A + it.x, c->b.plist[q].x, c->b.plist[q].y, lds, sizeof(m));
+  const bool tiles = sparse(count, step);
+  if (!tiles && it.y >= count) return;
+  int q = it.y;
+  if (!tiles) {
+    const int2 p = c->b.plist[q];
+    if (interact_patch<F32, G, PSE, GEN>(m, unread, A, it.x, p.x, p.y)) q += step;
+  }
+  const int end = tiles ? c->ntiles : count;
+#pragma clang loop unroll(disable)
+  for (; q < end; q += step) {  // of most work-groups none
+    int2 p = make_int2(-1, q);
+    if (!tiles) p = c->b.plist[q];
+    if constexpr (F32 || G == 1) interact_rest<F32>(A + it.x, p.x, p.y, lds, sizeof(m));
+    else call_interact_rest<F32>(A + it.x, p.x, p.y, lds, sizeof(m));
+  }
 }
 
 // after the last step of a call: its tool force, by one work-group per instance
